@@ -157,8 +157,19 @@ __host__ __device__ inline size_t activation_offset(ActivationLayout layout, uin
 }
 constexpr uint32_t kOperandOrderRows = 32;
 
-VxHipStatus launch_prepare_i8(hipStream_t s, const float* x, uint32_t rows, uint32_t k,
-                              int8_t* prepared, ActivationLayout layout, float* scales);
+// row_prepare.hip: rows of d f32 elements, through a row operation, to int8 codes and a scale per row.
+// Swiglu rows hold [gate | up] of 2 * d; delta (Norm, may be null) is added to the rows in place first; values
+// (not Plain, may be null) receives the f32 rows the codes are made of.
+enum class RowOp : int { Plain = 0, Norm = 1, Swiglu = 2 };
+constexpr uint32_t kMaxRowOpLength = 15360;  // Norm and Swiglu hold the whole row in registers
+VxHipStatus launch_row_prepare(hipStream_t s, RowOp op, float* x, const float* delta, const float* gain, double eps,
+                               uint32_t rows, uint32_t d, int8_t* codes, ActivationLayout layout, float* scales,
+                               float* values);
+inline VxHipStatus launch_prepare_i8(hipStream_t s, const float* x, uint32_t rows, uint32_t k, int8_t* prepared,
+                                     ActivationLayout layout, float* scales) {
+    return launch_row_prepare(s, RowOp::Plain, const_cast<float*>(x), nullptr, nullptr, 0.0, rows, k, prepared, layout,
+                              scales, nullptr);
+}
 // operand-order activations (rows <= 32, k codes each) back to row-major rows of ld bytes
 VxHipStatus launch_unblock_activations(hipStream_t s, const int8_t* blocked, uint32_t rows, uint32_t k,
                                        int8_t* row_major, uint32_t ld);
@@ -227,9 +238,9 @@ struct LinearArgs {
     // what the kernel does to the f32 rows before it prepares them (DequantF32 only), the fused decode
     // forms of the reference's device route
     // (native/src/backends/cuda/kernels/cuda_forward_gemv_pair_kernels.inc:1136,1424,408,672):
-    // row_gain: RMSNorm with this gain [k] and row_eps, as rmsnorm_prepare_kernel computes it;
+    // row_gain: RMSNorm with this gain [k] and row_eps, as row_prepare_kernel computes it;
     // row_swiglu: the rows are [gate | up] of 2k elements and the input is silu(gate) * up, as
-    // swiglu_prepare_kernel computes it.  add_to [rows][n] (may be y itself): the output is
+    // row_prepare_kernel computes it.  add_to [rows][n] (may be y itself): the output is
     // add_to + (linear + bias), the residual add behind the linear.
     const float* row_gain;
     double row_eps;

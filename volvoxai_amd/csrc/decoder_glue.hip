@@ -1,11 +1,7 @@
 // The steps either side of the W8A8 linears in a decoder layer, fused so that a decode step
 // is a dozen launches per layer instead of several dozen elementwise ones:
 //
-//   rmsnorm_prepare   RMSNorm (native/src/kernels/softmax_rmsnorm.inc:3-17: double accumulation,
-//                     x * inv_std * gain in double, one rounding to f32) followed by the
-//                     PackedLinear activation preparation of that row
-//                     (native/src/kernels/packed_linear_ops.inc:97-217)
-//   swiglu_prepare    silu(gate) * up, then the same preparation
+//   rmsnorm_prepare, swiglu_prepare   row_prepare.hip
 //   rope_append       non-interleaved rotary embedding of q and k
 //                     (native/src/kernels/llm_math.h:256-274) and the KV-cache append
 //   gqa_attention     grouped-query attention of the new tokens over the cache: f32 scores
@@ -23,105 +19,6 @@ namespace vxhip {
 namespace {
 
 extern __shared__ __attribute__((aligned(16))) char glue_lds[];
-
-// LAST: nothing writes `slots` again before the kernel ends, so no second barrier is needed.
-template <bool LAST = false>
-__device__ __forceinline__ float block_max(float v, float* slots) {
-    v = wave_max(v);
-    if ((threadIdx.x & 63u) == 0u) slots[threadIdx.x >> 6] = v;
-    __syncthreads();
-    float m = slots[0];
-    for (uint32_t w = 1; w < blockDim.x / 64u; w++) m = fmaxf(m, slots[w]);
-    if constexpr (!LAST) __syncthreads();
-    return m;
-}
-
-// Shared tail of the two *_prepare kernels: the row's f32 values are in `vals` (LDS), element j
-// written by thread j % blockDim.x, which is also the thread that reads it here.
-// scale = max|v| / 127 (1.0 for an all-zero row, floored at 2^-126), code = ties-to-even(v / scale)
-// clamped to +-127 with a true f32 divide; a non-finite row gets zero codes and a NaN scale.
-// The codes of row `row` go where `layout` puts them (row-major rows of d bytes, or operand order,
-// whose last 16-byte chunk is filled up with zeros).
-__device__ __forceinline__ void prepare_row(const float* vals, uint32_t d, int8_t* codes, ActivationLayout layout,
-                                            uint32_t row, float* scale_out, float* slots) {
-    // one reduction for both questions: a non-finite element counts as +inf, which no finite
-    // maximum can be
-    float maximum = 0.0f;
-    for (uint32_t j = threadIdx.x; j < d; j += blockDim.x) {
-        const float v = vals[j];
-        maximum = fmaxf(maximum, finite_f32(v) ? fabsf(v) : __builtin_inff());
-    }
-    maximum = block_max<true>(maximum, slots);
-    const float bad = maximum == __builtin_inff() ? 1.0f : 0.0f;
-    float scale = maximum == 0.0f || bad != 0.0f ? 1.0f : __fdiv_rn(maximum, 127.0f);
-    if (scale < 0x1p-126f) scale = 0x1p-126f;
-    for (uint32_t j = threadIdx.x; j < d; j += blockDim.x)
-        codes[activation_offset(layout, row, j)] =
-            bad != 0.0f ? (int8_t)0 : (int8_t)packed_round_i8(__fdiv_rn(vals[j], scale));
-    if (layout.operand_order)
-        for (uint32_t j = d + threadIdx.x; j < layout.ld; j += blockDim.x) codes[activation_offset(layout, row, j)] = 0;
-    if (threadIdx.x == 0) *scale_out = bad != 0.0f ? __builtin_nanf("") : scale;
-}
-
-// delta (may be null): the row is first updated in place, x += delta (the residual add), and the
-// updated row is what gets normalized.
-__global__ __launch_bounds__(1024) void rmsnorm_prepare_kernel(float* __restrict__ x, const float* __restrict__ delta,
-                                                              const float* __restrict__ gain, uint32_t d, double eps,
-                                                              int8_t* __restrict__ prepared,
-                                                              const ActivationLayout layout,
-                                                              float* __restrict__ row_scales,
-                                                              float* __restrict__ normalized) {
-    float* vals = reinterpret_cast<float*>(glue_lds);
-    __shared__ double dslots[16];
-    __shared__ float slots[16];
-    const uint32_t row = blockIdx.x;
-    float* src = x + (size_t)row * d;
-    double sum = 0.0;
-    // the first pass's gain is requested with the row, not after the reduction
-    const float gain_first = threadIdx.x < d ? gain[threadIdx.x] : 0.0f;
-    for (uint32_t j = threadIdx.x; j < d; j += blockDim.x) {
-        float v = src[j];
-        if (delta) {
-            v = __fadd_rn(v, delta[(size_t)row * d + j]);
-            src[j] = v;
-        }
-        vals[j] = v;
-        sum += (double)v * (double)v;
-    }
-    sum = wave_sum_to_lane0(sum);
-    if ((threadIdx.x & 63u) == 0u) dslots[threadIdx.x >> 6] = sum;
-    __syncthreads();
-    double total = 0.0;
-    for (uint32_t w = 0; w < blockDim.x / 64u; w++) total += dslots[w];
-    const double inv_std = rms_inverse(total, d, eps);
-    for (uint32_t j = threadIdx.x; j < d; j += blockDim.x) {
-        const float gj = j == threadIdx.x ? gain_first : gain[j];
-        const float y = rms_scaled(vals[j], inv_std, gj);
-        vals[j] = y;
-        if (normalized) normalized[(size_t)row * d + j] = y;
-    }
-    // (no barrier: prepare_row walks the row with the same stride, a thread reads its own writes)
-    prepare_row(vals, d, prepared, layout, row, row_scales + row, slots);
-}
-
-__global__ __launch_bounds__(1024) void swiglu_prepare_kernel(const float* __restrict__ gate_up, uint32_t inter,
-                                                             int8_t* __restrict__ prepared,
-                                                             const ActivationLayout layout,
-                                                             float* __restrict__ row_scales,
-                                                             float* __restrict__ activated) {
-    float* vals = reinterpret_cast<float*>(glue_lds);
-    __shared__ float slots[16];
-    const uint32_t row = blockIdx.x;
-    const float* gate = gate_up + (size_t)row * 2u * inter;
-    const float* up = gate + inter;
-    for (uint32_t j = threadIdx.x; j < inter; j += blockDim.x) {
-        const float y = swiglu_value(gate[j], up[j]);
-        vals[j] = y;
-        if (activated) activated[(size_t)row * inter + j] = y;
-    }
-    // (no barrier: prepare_row walks the row with the same stride, a thread reads its own writes)
-    prepare_row(vals, inter, prepared, layout, row, row_scales + row, slots);
-}
 
 // grid rows * t, one workgroup per token walking the elements of all its heads (a workgroup per head
 // is a launch of a hundred thousand workgroups that move 512 bytes each).  Token (row, i) sits at cache
@@ -912,12 +809,6 @@ __global__ __launch_bounds__(256) void gqa_prefill_mfma_kernel(const float* __re
     }
 }
 
-// Few rows leave most of the device idle and the kernel latency bound: then a row gets a full
-// 1024-thread workgroup; with many rows 256 threads per row keep more rows resident.
-uint32_t row_block(uint32_t rows, uint32_t d) {
-    return rows <= 256u && d >= 1024u ? 1024u : 256u;
-}
-
 // Query heads that share a workgroup (and with it every key and value row of their KV head):
 // four for wide groups, two for any even group, else one.  With the key and value rows requested
 // ahead of their use the kernel is bound by those reads, and two heads per workgroup (half the
@@ -1067,48 +958,40 @@ extern "C" {
 VxHipStatus vxhip_rmsnorm_prepare_i8(VxHipContext* ctx, const float* input_dev, const float* gain_dev, uint32_t rows,
                                      uint32_t d, double eps, int8_t* prepared_dev, float* row_scales_dev,
                                      float* normalized_dev) {
-    if (!ctx || !input_dev || !gain_dev || !prepared_dev || !row_scales_dev || !d || d > 15360u) {
-        set_error("rmsnorm_prepare_i8: null argument or row length outside 1..15360");
+    if (!ctx || !input_dev || !gain_dev || !prepared_dev || !row_scales_dev || !d || d > kMaxRowOpLength) {
+        set_error("rmsnorm_prepare_i8: null argument or row length outside 1..%u", kMaxRowOpLength);
         return VXHIP_INVALID_ARGUMENT;
     }
     if (!rows) return VXHIP_OK;
     if (!device_ready(ctx)) return VXHIP_BACKEND_UNAVAILABLE;
-    hipLaunchKernelGGL(rmsnorm_prepare_kernel, dim3(rows), dim3(row_block(rows, d)), d * sizeof(float), ctx->stream,
-                       const_cast<float*>(input_dev), (const float*)nullptr, gain_dev, d, eps, prepared_dev,
-                       prepared_layout(ctx, rows, d), row_scales_dev, normalized_dev);
-    VXHIP_TRY(hipGetLastError());
-    return VXHIP_OK;
+    return launch_row_prepare(ctx->stream, RowOp::Norm, const_cast<float*>(input_dev), nullptr, gain_dev, eps, rows, d,
+                              prepared_dev, prepared_layout(ctx, rows, d), row_scales_dev, normalized_dev);
 }
 
 VxHipStatus vxhip_add_rmsnorm_prepare_i8(VxHipContext* ctx, float* residual_dev, const float* delta_dev,
                                          const float* gain_dev, uint32_t rows, uint32_t d, double eps,
                                          int8_t* prepared_dev, float* row_scales_dev) {
-    if (!ctx || !residual_dev || !delta_dev || !gain_dev || !prepared_dev || !row_scales_dev || !d || d > 15360u) {
-        set_error("add_rmsnorm_prepare_i8: null argument or row length outside 1..15360");
+    if (!ctx || !residual_dev || !delta_dev || !gain_dev || !prepared_dev || !row_scales_dev || !d ||
+        d > kMaxRowOpLength) {
+        set_error("add_rmsnorm_prepare_i8: null argument or row length outside 1..%u", kMaxRowOpLength);
         return VXHIP_INVALID_ARGUMENT;
     }
     if (!rows) return VXHIP_OK;
     if (!device_ready(ctx)) return VXHIP_BACKEND_UNAVAILABLE;
-    hipLaunchKernelGGL(rmsnorm_prepare_kernel, dim3(rows), dim3(row_block(rows, d)), d * sizeof(float), ctx->stream,
-                       residual_dev, delta_dev, gain_dev, d, eps, prepared_dev, prepared_layout(ctx, rows, d),
-                       row_scales_dev, (float*)nullptr);
-    VXHIP_TRY(hipGetLastError());
-    return VXHIP_OK;
+    return launch_row_prepare(ctx->stream, RowOp::Norm, residual_dev, delta_dev, gain_dev, eps, rows, d, prepared_dev,
+                              prepared_layout(ctx, rows, d), row_scales_dev, nullptr);
 }
 
 VxHipStatus vxhip_swiglu_prepare_i8(VxHipContext* ctx, const float* gate_up_dev, uint32_t rows, uint32_t inter,
                                     int8_t* prepared_dev, float* row_scales_dev, float* activated_dev) {
-    if (!ctx || !gate_up_dev || !prepared_dev || !row_scales_dev || !inter || inter > 15360u) {
-        set_error("swiglu_prepare_i8: null argument or row length outside 1..15360");
+    if (!ctx || !gate_up_dev || !prepared_dev || !row_scales_dev || !inter || inter > kMaxRowOpLength) {
+        set_error("swiglu_prepare_i8: null argument or row length outside 1..%u", kMaxRowOpLength);
         return VXHIP_INVALID_ARGUMENT;
     }
     if (!rows) return VXHIP_OK;
     if (!device_ready(ctx)) return VXHIP_BACKEND_UNAVAILABLE;
-    hipLaunchKernelGGL(swiglu_prepare_kernel, dim3(rows), dim3(row_block(rows, inter)), inter * sizeof(float),
-                       ctx->stream, gate_up_dev, inter, prepared_dev, prepared_layout(ctx, rows, inter), row_scales_dev,
-                       activated_dev);
-    VXHIP_TRY(hipGetLastError());
-    return VXHIP_OK;
+    return launch_row_prepare(ctx->stream, RowOp::Swiglu, const_cast<float*>(gate_up_dev), nullptr, nullptr, 0.0, rows,
+                              inter, prepared_dev, prepared_layout(ctx, rows, inter), row_scales_dev, activated_dev);
 }
 
 VxHipStatus vxhip_rope_append_kv(VxHipContext* ctx, const float* qkv_dev, const float* cos_dev, const float* sin_dev,

@@ -65,7 +65,7 @@ __device__ __forceinline__ v4i load_stream(const int8_t* p) {
 // the workgroup's channels are parked, folded and stored.
 //
 // PREP: the activations arrive as f32 rows (a.x_f32, at most kMaxPrepRows of them) and the workgroup
-// prepares them itself, exactly as prepare_i8_kernel does (boundary.hip): per row scale = max|x| / 127
+// prepares them itself, exactly as row_prepare_kernel does (row_prepare.hip): per row scale = max|x| / 127
 // with a true division, floored at 2^-126, 1 for a zero row; codes = ties-to-even(x / scale) clamped to
 // +-127; a row holding NaN or Inf gets zero codes and a NaN scale.  The codes live in LDS, where the
 // MFMA's activation operand is then read from.  Every workgroup repeats this for all rows -- a few
@@ -147,7 +147,10 @@ __global__ __launch_bounds__(WAVES * 64, (ROWOP == 2 && WAVES == 8) ? 4 : 1) voi
     constexpr bool ROWOPS = PREP && F;
     // pass i of row r holds elements (whole 16-byte chunks of codes are written, so up to the padded end)
     const uint32_t prep_end = (a.k + 15u) / 16u * 16u;
-    auto live = [&](int r, int i) { return (uint32_t)r < rows && (uint32_t)(i * WAVES * 64) < prep_end; };
+    // (RMSNorm: pairs of elements, as its sum of squares is ordered; eight waves)
+    auto first_of = [&](int i) { return (uint32_t)(NORM ? (i / 2) * 1024 : i * WAVES * 64); };
+    auto element = [&](int i) { return first_of(i) + (NORM ? 2u * threadIdx.x + (uint32_t)(i & 1) : threadIdx.x); };
+    auto live = [&](int r, int i) { return (uint32_t)r < rows && first_of(i) < prep_end; };
     float xrows[PREP_ROWS][PREP_KEPT];
     float xup[SWIGLU ? PREP_ROWS : 1][SWIGLU ? PREP_KEPT : 1];
     float xgain[NORM ? PREP_KEPT : 1];
@@ -157,7 +160,7 @@ __global__ __launch_bounds__(WAVES * 64, (ROWOP == 2 && WAVES == 8) ? 4 : 1) voi
             const float* src = a.x_f32 + (size_t)min((uint32_t)r, rows - 1u) * a.ldx;
 #pragma unroll
             for (int i = 0; i < PREP_KEPT; i++) {
-                const uint32_t j = threadIdx.x + i * WAVES * 64;
+                const uint32_t j = element(i);
                 xrows[r][i] = 0.0f;
                 if constexpr (SWIGLU) xup[r][i] = 0.0f;
                 if (live(r, i)) {  // (scalar: whole passes past the row end, and rows not given, cost nothing)
@@ -169,7 +172,7 @@ __global__ __launch_bounds__(WAVES * 64, (ROWOP == 2 && WAVES == 8) ? 4 : 1) voi
         if constexpr (NORM) {
 #pragma unroll
             for (int i = 0; i < PREP_KEPT; i++) {
-                const uint32_t j = threadIdx.x + i * WAVES * 64;
+                const uint32_t j = element(i);
                 xgain[i] = 0.0f;
                 if (live(0, i)) xgain[i] = j < a.k ? a.row_gain[j] : 0.0f;
             }
@@ -246,7 +249,7 @@ __global__ __launch_bounds__(WAVES * 64, (ROWOP == 2 && WAVES == 8) ? 4 : 1) voi
     // reductions interleave)
     auto prepare_rows_of = [&](auto rows_tag) __attribute__((always_inline)) {
         constexpr int NR = decltype(rows_tag)::value;
-        auto pass = [&](int i) { return (uint32_t)(i * WAVES * 64) < prep_end; };
+        auto pass = [&](int i) { return first_of(i) < prep_end; };
         if constexpr (PREP && !F) {
             // QuantizeLinear in front of a QLinear: q = saturate(ties-to-even(f32(x / s) + f32(zp))), NaN -> zp
             // (native/src/kernels/quantize_linear_ops.inc:156-169), stored as the signed byte the MFMA takes
@@ -259,7 +262,7 @@ __global__ __launch_bounds__(WAVES * 64, (ROWOP == 2 && WAVES == 8) ? 4 : 1) voi
 #pragma unroll
                 for (int i = 0; i < PREP_KEPT; i++) {
                     if (!pass(i)) continue;
-                    const uint32_t j = threadIdx.x + i * WAVES * 64;
+                    const uint32_t j = element(i);
                     const float v = xrows[r][i];
                     int32_t q = a.input_zp + shift;
                     if (v == v) {
@@ -280,32 +283,15 @@ __global__ __launch_bounds__(WAVES * 64, (ROWOP == 2 && WAVES == 8) ? 4 : 1) voi
         }
         if constexpr (NORM) {
             {
-                // The row's sum of squares in the order of rmsnorm_prepare_kernel's 1024 threads: this
-                // thread stands for VT of them (elements 1024 apart belong to the same one).
-                constexpr int VT = (int)kNormThreads / (WAVES * 64);
-                static_assert(VT >= 1 && PREP_KEPT % VT == 0, "a thread holds whole virtual threads");
-                __shared__ double norm_slots[PREP_ROWS][kNormThreads / 64];
+                static_assert(WAVES == 8, "the sum of squares is ordered for a pair of elements a thread of 512");
+                __shared__ double norm_slots[PREP_ROWS][8];
 #pragma unroll
                 for (int r = 0; r < NR; r++) {
-                    double vs[VT];
+                    double pair[1] = {0.0};
 #pragma unroll
-                    for (int v = 0; v < VT; v++) vs[v] = 0.0;
-#pragma unroll
-                    for (int i = 0; i < PREP_KEPT; i++)
-                        if (pass(i)) vs[i % VT] += (double)xrows[r][i] * (double)xrows[r][i];
-#pragma unroll
-                    for (int v = 0; v < VT; v++) {
-                        const double part = wave_sum_to_lane0(vs[v]);
-                        if (lane == 0) norm_slots[r][wave + v * WAVES] = part;
-                    }
-                }
-                __syncthreads();
-#pragma unroll
-                for (int r = 0; r < NR; r++) {
-                    double total = 0.0;
-#pragma unroll
-                    for (uint32_t w = 0; w < kNormThreads / 64u; w++) total += norm_slots[r][w];
-                    const double inv_std = rms_inverse(total, a.k, a.row_eps);
+                    for (int i = 0; i < PREP_KEPT; i += 2)
+                        if (pass(i)) pair[0] += square(xrows[r][i]) + square(xrows[r][i + 1]);
+                    const double inv_std = rms_inverse(norm_total<512>(pair, norm_slots[r]), a.k, a.row_eps);
 #pragma unroll
                     for (int i = 0; i < PREP_KEPT; i++)
                         if (pass(i)) xrows[r][i] = rms_scaled(xrows[r][i], inv_std, xgain[i]);
@@ -345,7 +331,7 @@ __global__ __launch_bounds__(WAVES * 64, (ROWOP == 2 && WAVES == 8) ? 4 : 1) voi
 #pragma unroll
                 for (int i = 0; i < PREP_KEPT; i++) {
                     if (!pass(i)) continue;
-                    const uint32_t j = threadIdx.x + i * WAVES * 64;
+                    const uint32_t j = element(i);
                     // (elements past k were loaded as zeros: the padding of the last 16-byte chunk)
                     if (j < ldk) prep_codes[(size_t)r * ldk + j] = (int8_t)(bad ? 0 : packed_round_i8(__fdiv_rn(xrows[r][i], scale)));
                 }
@@ -495,7 +481,7 @@ __global__ __launch_bounds__(WAVES * 64, (ROWOP == 2 && WAVES == 8) ? 4 : 1) voi
 //     (packed_linear_ops.inc:1498-1504), bit for bit.
 // Measured at M=1, K=4096, N=14336 (sixteen waves of eight blocks): 10.3 us against 12.5 us for the
 // general kernel, with a plain read of the same bytes at 9.3-9.6 us.
-// PREP: one or two f32 rows (a.x_f32) which the workgroup prepares itself, by prepare_i8_kernel's rule to the
+// PREP: one or two f32 rows (a.x_f32) which the workgroup prepares itself, by row_prepare_kernel's rule to the
 // letter, as the reference's single-row route quantizes the row and multiplies in one call
 // (packed_linear_ops.inc:1471-1535).  A wave's 64 lanes hold exactly the elements of the wave's own K-slice
 // (BPW / 2 consecutive ones per lane), so only the row maximum crosses the waves; the codes go straight into
@@ -944,9 +930,8 @@ const char* launch_mode(hipStream_t s, const LinearArgs& a, int cu_count, const 
             a.k > (uint32_t)kPrepPerThread * (uint32_t)waves * 64u || (MODE != (int)Epilogue::DequantF32 && a.zw))
             return nullptr;
         lds += (size_t)a.rows * ((a.k + 15u) / 16u * 16u) + (size_t)a.rows * 4u + 16u;
-        // RMSNorm in front: the sum of squares follows the 1024-thread row kernel, which rows of 1024
-        // elements and more get
-        if (a.row_gain && a.k < kNormThreads) return nullptr;
+        // RMSNorm in front: rows of 1024 elements and more
+        if (a.row_gain && a.k < kNormBlock) return nullptr;
         // (that form is built for eight waves only: its double arithmetic does not fit the registers of sixteen)
         if (a.row_gain) {
             if (a.k > (uint32_t)kPrepPerThread * 8u * 64u) return nullptr;

@@ -39,7 +39,7 @@ const VxHipKernelVariant kVariants[] = {
     {"hip.packed-linear.w4a8-gemv-mfma", 0, kPackedLinear, "gemv_fit_kernel<W4>|gemv_panel_kernel<DequantF32, W4>",
      "hip.packed-linear.w4-dynamic-i8-g32-64-128-256-rows-le32",
      "hip.gfx950-mfma-i32-32x32x32-i8,hip.nontemporal-dwordx4", 400},
-    {"hip.packed-linear.prepare-i8", 0, kPackedLinear, "prepare_i8_kernel|prepare_i8_rows_kernel",
+    {"hip.packed-linear.prepare-i8", 0, kPackedLinear, "row_prepare_kernel",
      "hip.packed-linear.dynamic-i8-row-absmax", "", 100},
 };
 }  // namespace
