@@ -1,0 +1,32 @@
+"""One and two f32 rows through PackedLinear in one launch (gemv_row.hip) at the edges of its instances."""
+import numpy as np
+import pytest
+
+import _cases as cases
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 2])
+@pytest.mark.parametrize("bits,group", [(8, 32), (8, 64), (8, 128), (8, 256), (4, 32), (4, 64), (4, 128), (4, 256)])
+@pytest.mark.parametrize("k,n", [(2, 33), (1023, 40), (1024, 2049), (1025, 31), (2050, 64), (3072, 2080), (3101, 8), (4097, 70),
+                                 (8192, 33), (8200, 2056), (14336, 24)])
+def test_rows_at_the_edges_of_the_instances(ctx, oracle, k, n, bits, group, rows):
+    """Lengths on both sides of every instance, both widths of a workgroup's channels (the line is at 64 panels),
+    every scale group, n that ends inside a panel: the oracle's bits."""
+    import torch
+    import volvoxai_amd as vx
+    c = cases.packed_case(rows, k, n, group, k + n + bits, True)
+    w = c["w"] if bits == 8 else cases.four_bit(c["w"])
+    words = oracle.pack_w8_words(w) if bits == 8 else oracle.pack_w4_words(w)
+    _, want = oracle.packed_linear(c["x"], words, c["scales"], c["bias"], n, group, bits=bits)
+    pl = vx.PackedLinear(words, c["scales"], c["bias"], k, n, group, weight_bits=bits)
+    try:
+        for force in (None, "gemv.nofit.row8", "gemv.nofit.row32"):
+            vx.force_variant(force)
+            st, y = pl.forward_f32(ctx, torch.from_numpy(c["x"]).cuda())
+            ctx.synchronize()
+            assert st == 0 and ctx.last_variant.endswith("-prep"), ctx.last_variant
+            assert (y.cpu().numpy().view(np.uint32) == want.view(np.uint32)).all(), ctx.last_variant
+    finally:
+        vx.force_variant(None)
+        pl.close()

@@ -1159,7 +1159,7 @@ int vxhip_packed_linear_forward_a8(VxHipContext* ctx, const VxHipPackedLinear* p
                          zeros, rows);
 }
 
-// Few f32 rows: one launch, the GEMV preparing the rows itself (gemv_stream.hip, PREP).  0: ran; -2: no
+// Few f32 rows: one launch, the GEMV preparing the rows itself (gemv_row.hip).  0: ran; -2: no
 // such kernel takes the call (shape, forced variant) and nothing was launched.
 struct RowOps {
     const float* gain = nullptr;  // RMSNorm in front of the preparation

@@ -191,7 +191,7 @@ struct LinearArgs {
     Epilogue mode;
     const int8_t* x;        // signed activations [rows][ldx], or in operand order (GEMV only)
     // instead of x (GEMV, rows <= kMaxPrepRows): f32 rows of ldx elements which the kernel turns into codes
-    // itself -- DequantF32: the dynamic per-row preparation; RequantTensor: the QuantizeLinear in front
+    // itself -- DequantF32: the dynamic per-row preparation (gemv_row.hip); RequantTensor: the QuantizeLinear in front
     // of the QLinear (input_scale, input_zp; x_f32_unsigned: that node writes U8)
     const float* x_f32;
     uint32_t x_f32_unsigned;
@@ -267,6 +267,8 @@ inline bool raise_lds_limit(const void* kernel, int bytes, std::atomic<uint64_t>
 }
 
 const char* launch_gemv_stream(hipStream_t s, const LinearArgs& a, int cu_count, const char* force);
+// gemv_row.hip, called by launch_gemv_stream: the variant suffix, or null when the shape is not taken.
+const char* launch_gemv_row(hipStream_t s, const LinearArgs& a, int cu_count, const char* force, bool dry_run);
 // While on (per thread), launch_gemv_stream chooses as always and launches nothing: its result tells
 // whether a call of that description would be taken.
 void set_gemv_dry_run(bool on);

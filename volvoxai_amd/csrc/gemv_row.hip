@@ -1,0 +1,310 @@
+// PackedLinear of one or two f32 rows in one launch, with a decoder's row operation in front and its
+// residual add behind: what the reference's device route does for a decode row
+// (native/src/backends/cuda/kernels/cuda_forward_gemv_pair_kernels.inc:1136 RMSNorm + q/k/v, :1424 RMSNorm +
+// gate/up, :408 SwiGLU, :672 residual add) and its CPU route for a single row
+// (native/src/kernels/packed_linear_ops.inc:1471-1535).
+//
+// Such a launch is bound by latency: its weights (2-6 MB in a decoder) arrive in about the time of one memory
+// round trip once they are all requested at the start.  So the kernel is short straight-line code -- the
+// row, then every weight byte of the workgroup, is requested first; the row operation, the preparation (the
+// rules of row_prepare.hip) and the codes' trip through LDS happen while the weights are under way -- and it is
+// small: the five linears of a decoder layer and its attention kernel then stay in the instruction cache
+// together, which kernels of 20-30 KB each did not.  Cost per launch in a recorded step of one row, before (the
+// same operations as forms of gemv_stream.hip's kernel) and after: RMSNorm + 4096 of K=1024 7.7 -> 3.4 us, 1024 of
+// K=2048 + add 7.0 -> 3.6, RMSNorm + 6144 of K=1024 8.0 -> 3.6, SwiGLU + 1024 of K=3072 + add 8.3 -> 4.6; the step
+// 1.06 -> 0.65 ms.
+//
+// Work split: a workgroup of 512 threads owns CH (8 or 32) output channels of a panel over all of K.  A
+// 16-byte piece of a 1 KiB block (common.h) is one channel's weights of sixteen columns; the 2 * CH lanes that
+// hold the workgroup's channels read whole 128-byte lines, and a wavefront reads 64 / (2 * CH) blocks with one
+// load.  The dots are v_dot4 (a matrix instruction would do 32 rows' work for one or two); a scale group's
+// lanes meet in the register file, the product f32(dot) * (s_a * s_w) goes to LDS, and one thread per output adds
+// the products in ascending group order -- the sum the reference forms (packed_linear_ops.inc:1498-1504), bit
+// for bit.
+#include "common.h"
+#include "device_math.h"
+#include "row_math.h"
+#include "wave_ops.h"
+
+#include <stdio.h>
+#include <string.h>
+
+namespace vxhip {
+namespace {
+
+extern __shared__ __attribute__((aligned(16))) char row_lds[];
+
+constexpr int kThreads = 512, kWaves = kThreads / 64;
+constexpr int kDppRowRor8 = 0x128;
+constexpr uint32_t kMaxRowLength = 14336;  // longest K
+
+typedef float v2f_any __attribute__((ext_vector_type(2), aligned(4)));
+
+// K up to NB * 1024.
+template <RowOp OP, int GK, bool W4, int CH, int NB, int ROWS>
+__global__ __launch_bounds__(kThreads) void gemv_row_kernel(const LinearArgs a) {
+    constexpr int SPB = W4 ? 2 : 1;               // k-steps of 32 per 1 KiB block
+    constexpr int KPAD = NB * 1024, BLOCKS = KPAD / (32 * SPB);
+    constexpr int BPL = 32 / CH;                  // blocks per load of a wavefront
+    constexpr int NSUB = GK < SPB ? 2 : 1;        // scale groups per block (four-bit weights in groups of 32)
+    constexpr int GBLK = GK < SPB ? 1 : GK / SPB; // blocks per scale group
+    constexpr int LG = GBLK > BPL ? GBLK / BPL : 1;                // loads per unit: whole scale groups
+    constexpr int UNITS = BLOCKS / (LG * BPL), NU = (UNITS + kWaves - 1) / kWaves, NL = NU * LG;
+    // weight loads of a wavefront requested before the row is looked at: all of a short run; of a long one four,
+    // which leave registers for a third workgroup per compute unit (one row, K=4096, N=14336: 11.8 us with
+    // eight, 11.1 with four)
+    constexpr int AHEAD = NL <= 8 ? NL : 4;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    constexpr int PARTS = 32 / CH;                // workgroups per panel
+    const uint32_t panel = blockIdx.x / PARTS, sub = blockIdx.x % PARTS, ch0 = panel * 32u + sub * CH;
+    const uint32_t c = lane % CH, half = (lane / CH) & 1, blk = lane / (2 * CH);
+    const uint32_t k = a.k;
+
+    // the rows (elements past k: zeros): a thread holds the pair 2t of every 1024 elements
+    float x[ROWS][NB][2], up[OP == RowOp::Swiglu ? ROWS : 1][OP == RowOp::Swiglu ? NB : 1][2], gain[OP == RowOp::Norm ? NB : 1][2];
+    auto pair_of = [&](const float* src, int b, float (&v)[2]) {
+        const uint32_t j = (uint32_t)b * 1024u + threadIdx.x * 2u, at = min(j, k - 2u);
+        const v2f_any p = *reinterpret_cast<const v2f_any*>(src + at);
+        v[0] = j < k ? (j == at ? p.x : p.y) : 0.0f;
+        v[1] = j + 1u < k ? p.y : 0.0f;
+    };
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) {
+        const float* src = a.x_f32 + (size_t)r * a.ldx;
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            pair_of(src, b, x[r][b]);
+            if constexpr (OP == RowOp::Swiglu) pair_of(src + k, b, up[r][b]);
+        }
+    }
+    if constexpr (OP == RowOp::Norm) {
+#pragma unroll
+        for (int b = 0; b < NB; b++) pair_of(a.row_gain, b, gain[b]);
+    }
+    // (loads return in the order of their issue: the row has to be asked for before the weights)
+    __builtin_amdgcn_sched_barrier(0);
+    const int8_t* wp = a.w + (size_t)panel * a.ksteps * 1024u + (half * 32u + sub * CH + c) * 16u;
+    auto block_of = [&](int l) { return (uint32_t)((((l / LG) * kWaves + wave) * LG + l % LG) * BPL) + blk; };
+    v4i w[AHEAD];
+    auto issue = [&](int l) {
+        w[l % AHEAD] = __builtin_nontemporal_load(
+            reinterpret_cast<const v4i*>(wp + (size_t)min(block_of(l), a.ksteps - 1u) * 1024u));
+    };
+#pragma unroll
+    for (int l = 0; l < AHEAD; l++) issue(l);
+    __builtin_amdgcn_sched_barrier(0);
+    float sw[NU][NSUB];
+#pragma unroll
+    for (int u = 0; u < NU; u++)
+#pragma unroll
+        for (int s = 0; s < NSUB; s++)
+            sw[u][s] = a.scales_t[(size_t)min(block_of(u * LG) / GBLK * NSUB + s, a.groups - 1u) * a.n_pad + ch0 + c];
+    // the tail's operands: output o = row * CH + channel
+    const uint32_t om = threadIdx.x / CH, on = ch0 + threadIdx.x % CH;
+    const bool stores = threadIdx.x < ROWS * CH && on < a.n;
+    float bias = 0.0f, residual = 0.0f;
+    if (stores) {
+        bias = a.bias_f32[on];
+        if (a.add_to) residual = a.add_to[(size_t)om * a.n + on];
+    }
+
+    if constexpr (OP == RowOp::Swiglu) {
+#pragma unroll
+        for (int r = 0; r < ROWS; r++)
+#pragma unroll
+            for (int b = 0; b < NB; b++)
+#pragma unroll
+                for (int e = 0; e < 2; e++) x[r][b][e] = swiglu_value(x[r][b][e], up[r][b][e]);
+    }
+    if constexpr (OP == RowOp::Norm) {
+        __shared__ double norm_slots[ROWS][kWaves];
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+            double pair[1] = {0.0};
+#pragma unroll
+            for (int b = 0; b < NB; b++) pair[0] += square(x[r][b][0]) + square(x[r][b][1]);
+            const double inv_std = rms_inverse(norm_total<kThreads>(pair, norm_slots[r]), k, a.row_eps);
+#pragma unroll
+            for (int b = 0; b < NB; b++)
+#pragma unroll
+                for (int e = 0; e < 2; e++) x[r][b][e] = rms_scaled(x[r][b][e], inv_std, gain[b][e]);
+        }
+    }
+    // preparation: scale = max|v| / 127 (1 for a zero row, floored at 2^-126), codes = ties-to-even(v / scale)
+    // clamped to +-127, true divisions; a row that is not finite gets zero codes and a NaN scale
+    int8_t* codes = reinterpret_cast<int8_t*>(row_lds);
+    float* products = reinterpret_cast<float*>(row_lds + ROWS * KPAD);  // [groups][ROWS][CH]
+    __shared__ float slots[ROWS][kWaves];
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) {
+        float maximum = 0.0f;
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int e = 0; e < 2; e++)
+                maximum = fmaxf(maximum, finite_f32(x[r][b][e]) ? fabsf(x[r][b][e]) : __builtin_inff());
+        maximum = wave_max(maximum);
+        if (lane == 0) slots[r][wave] = maximum;
+    }
+    __syncthreads();
+    float rs[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; r++) {
+        float maximum = slots[r][0];
+#pragma unroll
+        for (int v = 1; v < kWaves; v++) maximum = fmaxf(maximum, slots[r][v]);
+        const bool bad = maximum == __builtin_inff();
+        float scale = maximum == 0.0f || bad ? 1.0f : __fdiv_rn(maximum, 127.0f);
+        if (scale < 0x1p-126f) scale = 0x1p-126f;
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            const uint32_t q0 = bad ? 0u : (uint32_t)packed_round_i8(__fdiv_rn(x[r][b][0], scale));
+            const uint32_t q1 = bad ? 0u : (uint32_t)packed_round_i8(__fdiv_rn(x[r][b][1], scale));
+            *reinterpret_cast<uint16_t*>(codes + r * KPAD + b * 1024 + threadIdx.x * 2u) =
+                (uint16_t)((q0 & 0xffu) | (q1 << 8));
+        }
+        rs[r] = bad ? __builtin_nanf("") : scale;
+    }
+    __syncthreads();
+
+#pragma unroll
+    for (int u = 0; u < NU; u++) {
+        int32_t acc[ROWS][NSUB];
+#pragma unroll
+        for (int r = 0; r < ROWS; r++)
+#pragma unroll
+            for (int s = 0; s < NSUB; s++) acc[r][s] = 0;
+#pragma unroll
+        for (int i = 0; i < LG; i++) {
+            const int l = u * LG + i;
+            const v4i wb = w[l % AHEAD];
+            const int8_t* xc = codes + (min(block_of(l), (uint32_t)BLOCKS - 1u) * SPB * 2u + half) * 16u;
+#pragma unroll
+            for (int r = 0; r < ROWS; r++) {
+#pragma unroll
+                for (int s = 0; s < SPB; s++) {
+                    const v4i xv = *reinterpret_cast<const v4i*>(xc + r * KPAD + s * 32);
+#pragma unroll
+                    for (int d = 0; d < 4; d++) {
+                        // (four-bit weights: the low, then the high nibbles, each at the top of its byte)
+                        const int wd = W4 ? (s == 0 ? wb[d] << 4 : wb[d]) & (int)0xf0f0f0f0u : wb[d];
+                        acc[r][s % NSUB] = __builtin_amdgcn_sdot4(wd, xv[d], acc[r][s % NSUB], false);
+                    }
+                }
+            }
+            if (l + AHEAD < NL) issue(l + AHEAD);
+        }
+        const uint32_t group = block_of(u * LG) / GBLK * NSUB;
+        // the lanes of a channel: both halves of a block, then the blocks of its group
+        constexpr int MEET = GBLK < BPL ? GBLK : BPL;
+        const bool leads = half == 0u && blk % MEET == 0u && group < a.groups;
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+#pragma unroll
+            for (int s = 0; s < NSUB; s++) {
+                uint32_t v = (uint32_t)acc[r][s];
+                if constexpr (CH == 8) v += (uint32_t)lane_exchange<kDppRowRor8>((int)v);
+                if constexpr (CH == 16 || (CH == 8 && MEET >= 2)) v += lane_down16(v);
+                if constexpr (CH == 32 || (CH == 16 && MEET >= 2) || (CH == 8 && MEET == 4)) v += lane_down32(v);
+                const int32_t dot = W4 ? (int32_t)v >> 4 : (int32_t)v;
+                if (leads && group + s < a.groups)
+                    products[((group + s) * ROWS + r) * CH + c] = __fmul_rn((float)dot, __fmul_rn(rs[r], sw[u][s]));
+            }
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x >= ROWS * CH) return;
+    float sum = 0.0f;
+    const float* p = products + threadIdx.x;
+    uint32_t g = 0;
+    for (; g + 8u <= a.groups; g += 8u) {
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = p[(g + i) * ROWS * CH];
+#pragma unroll
+        for (int i = 0; i < 8; i++) sum = __fadd_rn(sum, v[i]);
+    }
+    for (; g < a.groups; g++) sum = __fadd_rn(sum, p[g * ROWS * CH]);
+    sum = __fadd_rn(sum, bias);
+    if (a.add_to) sum = __fadd_rn(residual, sum);
+    if (stores) ((float*)a.y)[(size_t)om * a.n + on] = sum;
+}
+
+template <RowOp OP, int GK, bool W4, int CH, int NB, int ROWS>
+bool launch(hipStream_t s, const LinearArgs& a) {
+    const size_t lds = (size_t)ROWS * NB * 1024u + (size_t)a.groups * ROWS * CH * 4u;
+    auto kern = gemv_row_kernel<OP, GK, W4, CH, NB, ROWS>;
+    if (lds > 48u * 1024u) {
+        static std::atomic<uint64_t> configured{0};
+        if (!raise_lds_limit((const void*)kern, 152 * 1024, configured)) return false;
+    }
+    hipLaunchKernelGGL(kern, dim3((a.n + 31u) / 32u * (32u / CH)), dim3(kThreads), lds, s, a);
+    return hipGetLastError() == hipSuccess;
+}
+
+template <RowOp OP, int GK, bool W4, int CH, int NB>
+bool launch_rows(hipStream_t s, const LinearArgs& a) {
+    return a.rows == 1u ? launch<OP, GK, W4, CH, NB, 1>(s, a) : launch<OP, GK, W4, CH, NB, 2>(s, a);
+}
+
+template <RowOp OP, int GK, bool W4, int CH>
+bool launch_length(hipStream_t s, const LinearArgs& a) {
+    if (a.k <= 1024u) return launch_rows<OP, GK, W4, CH, 1>(s, a);
+    if (a.k <= 2048u) return launch_rows<OP, GK, W4, CH, 2>(s, a);
+    if (a.k <= 3072u) return launch_rows<OP, GK, W4, CH, 3>(s, a);
+    if (a.k <= 4096u) return launch_rows<OP, GK, W4, CH, 4>(s, a);
+    if constexpr (OP != RowOp::Norm) {
+        if (a.k <= 8192u) return launch_rows<OP, GK, W4, CH, 8>(s, a);
+        return launch_rows<OP, GK, W4, CH, 14>(s, a);
+    }
+    return false;
+}
+
+template <RowOp OP, int GK, bool W4>
+bool launch_channels(hipStream_t s, const LinearArgs& a, uint32_t ch) {
+    return ch == 8u ? launch_length<OP, GK, W4, 8>(s, a) : launch_length<OP, GK, W4, 32>(s, a);
+}
+
+template <int GK, bool W4>
+bool launch_op(hipStream_t s, const LinearArgs& a, uint32_t ch) {
+    if (a.row_gain) return launch_channels<RowOp::Norm, GK, W4>(s, a, ch);
+    if (a.row_swiglu) return launch_channels<RowOp::Swiglu, GK, W4>(s, a, ch);
+    return launch_channels<RowOp::Plain, GK, W4>(s, a, ch);
+}
+
+template <bool W4>
+bool launch_group(hipStream_t s, const LinearArgs& a, uint32_t ch) {
+    switch (a.group_size) {
+        case 32: return launch_op<1, W4>(s, a, ch);
+        case 64: return launch_op<2, W4>(s, a, ch);
+        case 128: return launch_op<4, W4>(s, a, ch);
+        case 256: return launch_op<8, W4>(s, a, ch);
+        default: return false;
+    }
+}
+
+}  // namespace
+
+// Channels per workgroup.  One row, eight-bit weights in groups of 128, weights from HBM, us with 8 | 32:
+//   K \ N      1024          4096          6144          14336
+//   1024    2.7 |  2.8    3.4 |  3.1        |         6.0 |  4.6
+//   3072    3.6 |  4.8    5.5 |  5.2    6.7 |  5.7   11.2 |  9.3
+//   4096    4.4 |  5.8    6.5 |  6.5    8.3 |  7.2   14.6 | 11.1
+//   14336   9.8 | 14.7   15.5 | 16.9   22.6 | 19.5   44.1 | 35.0
+// (16 in between at every size.)  Workgroups of eight channels pay while they are no more than the compute
+// units, N = 2048 (3.5 | 3.6 at K = 2048); past that the row operation each of them repeats outweighs them.
+const char* launch_gemv_row(hipStream_t s, const LinearArgs& a, int cu_count, const char* force, bool dry_run) {
+    if (a.mode != Epilogue::DequantF32 || !a.x_f32 || a.rows == 0u || a.rows > kMaxPrepRows || a.k < 2u ||
+        a.k > kMaxRowLength || (a.weight_bits != 8u && a.weight_bits != 4u))
+        return nullptr;
+    if (a.row_gain && (a.k < kNormBlock || a.k > 4096u)) return nullptr;
+    const uint32_t panels = (a.n + 31u) / 32u;
+    uint32_t ch = panels * 4u <= (uint32_t)cu_count ? 8u : 32u;
+    if (force && strstr(force, "row8")) ch = 8u;
+    else if (force && strstr(force, "row32")) ch = 32u;
+    if (!dry_run && !(a.weight_bits == 4u ? launch_group<true>(s, a, ch) : launch_group<false>(s, a, ch))) return nullptr;
+    return ch == 8u ? "row8-prep" : "row32-prep";
+}
+
+}  // namespace vxhip

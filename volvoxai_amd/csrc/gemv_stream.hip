@@ -24,7 +24,6 @@
 #include "common.h"
 #include "device_math.h"
 #include "epilogue.h"
-#include "row_math.h"
 #include "wave_ops.h"
 
 #include <stdio.h>
@@ -44,7 +43,7 @@ thread_local bool gemv_dry_run = false;
 extern __shared__ __attribute__((aligned(16))) char gemv_lds[];
 
 constexpr int kDepth = 4;  // 1 KiB blocks in flight per wave
-constexpr int kPrepPerThread = 8;  // f32 elements of a row that a thread of a preparing kernel holds
+constexpr int kPrepPerThread = 8;  // f32 elements of a row that a thread of a quantizing kernel holds
 constexpr uint32_t kFitLdsRows = 8;  // the exact-fit kernel keeps the activation rows in LDS up to this many rows
 
 __device__ __forceinline__ v4i load_stream(const int8_t* p) {
@@ -64,24 +63,15 @@ __device__ __forceinline__ v4i load_stream(const int8_t* p) {
 // on a full operand whose other rows repeat the workgroup's own, and only the accumulator quads of
 // the workgroup's channels are parked, folded and stored.
 //
-// PREP: the activations arrive as f32 rows (a.x_f32, at most kMaxPrepRows of them) and the workgroup
-// prepares them itself, exactly as row_prepare_kernel does (row_prepare.hip): per row scale = max|x| / 127
-// with a true division, floored at 2^-126, 1 for a zero row; codes = ties-to-even(x / scale) clamped to
-// +-127; a row holding NaN or Inf gets zero codes and a NaN scale.  The codes live in LDS, where the
-// MFMA's activation operand is then read from.  Every workgroup repeats this for all rows -- a few
-// 16 KiB reads that hit L2, issued behind the first weight requests -- and the linear is one launch
-// instead of two: the single-row route of the reference (packed_linear_ops.inc:1471-1535) also
-// quantizes the row and multiplies in one call.
-constexpr int kRowsPrepared = 0, kRowsF32 = 1, kRowsNorm = 2, kRowsSwiglu = 3;
-
-template <int MODE, int GK, int WAVES, bool W4, int SPLIT, int ROWOP>
-__global__ __launch_bounds__(WAVES * 64, (ROWOP == 2 && WAVES == 8) ? 4 : 1) void gemv_panel_kernel(const LinearArgs a) {
+// PREP (QLinear): the activations arrive as the f32 rows in front of the QuantizeLinear that feeds the linear
+// (a.x_f32, at most kMaxPrepRows of them) and the workgroup quantizes them itself with the linear's own input
+// parameters.  The codes live in LDS, where the MFMA's activation operand is then read from.  Every
+// workgroup repeats this for all rows -- a few 16 KiB reads that hit L2, issued in front of the weight
+// requests -- and the two nodes are one launch.
+template <int MODE, int GK, int WAVES, bool W4, int SPLIT, bool PREP>
+__global__ __launch_bounds__(WAVES * 64) void gemv_panel_kernel(const LinearArgs a) {
     constexpr bool F = MODE == (int)Epilogue::DequantF32;
-    // ROWOP: kRowsPrepared (0) int8 rows; kRowsF32 f32 rows prepared here; kRowsNorm, kRowsSwiglu: with
-    // RMSNorm or SwiGLU in front of the preparation
-    constexpr bool PREP = ROWOP != kRowsPrepared, NORM = ROWOP == kRowsNorm, SWIGLU = ROWOP == kRowsSwiglu;
-    static_assert(F || !(NORM || SWIGLU), "row operations ride in front of the dynamic preparation only");
-    static_assert(MODE != (int)Epilogue::RequantRow || !PREP, "f32 activations: PackedLinear, or QLinear behind a QuantizeLinear");
+    static_assert(MODE == (int)Epilogue::RequantTensor || !PREP, "f32 activations: a QLinear behind a QuantizeLinear");
     constexpr int CH = 32 / SPLIT;     // channels of this workgroup
     constexpr int QUADS = 4 / SPLIT;   // accumulator quads (8 channels each) of this workgroup
     static_assert(F || !W4, "four-bit weights exist for the dequantizing epilogue only");
@@ -139,61 +129,37 @@ __global__ __launch_bounds__(WAVES * 64, (ROWOP == 2 && WAVES == 8) ? 4 : 1) voi
     for (int r = 0; r < 16; r++) acc[r] = 0;
 
     // PREP: the f32 rows are requested first of all (loads return in order: behind the weight stream
-    // they would arrive with it, in front of it they are L2 hits whose preparation then runs while the
-    // first weight blocks are on their way) and stay in registers for the two passes.
+    // they would arrive with it, in front of it they are L2 hits whose quantization then runs while the
+    // first weight blocks are on their way).
     constexpr int PREP_ROWS = PREP ? (int)kMaxPrepRows : 1, PREP_KEPT = PREP ? kPrepPerThread : 1;
-    // A row operation of the decoder may ride in front of the preparation (F only): RMSNorm with
-    // a.row_gain, or SwiGLU over rows that hold [gate | up]; its other operands travel with the rows.
-    constexpr bool ROWOPS = PREP && F;
     // pass i of row r holds elements (whole 16-byte chunks of codes are written, so up to the padded end)
     const uint32_t prep_end = (a.k + 15u) / 16u * 16u;
-    // (RMSNorm: pairs of elements, as its sum of squares is ordered; eight waves)
-    auto first_of = [&](int i) { return (uint32_t)(NORM ? (i / 2) * 1024 : i * WAVES * 64); };
-    auto element = [&](int i) { return first_of(i) + (NORM ? 2u * threadIdx.x + (uint32_t)(i & 1) : threadIdx.x); };
-    auto live = [&](int r, int i) { return (uint32_t)r < rows && first_of(i) < prep_end; };
+    auto pass = [&](int i) { return (uint32_t)(i * WAVES * 64) < prep_end; };
     float xrows[PREP_ROWS][PREP_KEPT];
-    float xup[SWIGLU ? PREP_ROWS : 1][SWIGLU ? PREP_KEPT : 1];
-    float xgain[NORM ? PREP_KEPT : 1];
     if constexpr (PREP) {
 #pragma unroll
         for (int r = 0; r < PREP_ROWS; r++) {
             const float* src = a.x_f32 + (size_t)min((uint32_t)r, rows - 1u) * a.ldx;
 #pragma unroll
             for (int i = 0; i < PREP_KEPT; i++) {
-                const uint32_t j = element(i);
+                const uint32_t j = threadIdx.x + i * WAVES * 64;
                 xrows[r][i] = 0.0f;
-                if constexpr (SWIGLU) xup[r][i] = 0.0f;
-                if (live(r, i)) {  // (scalar: whole passes past the row end, and rows not given, cost nothing)
-                    xrows[r][i] = j < a.k ? src[j] : 0.0f;
-                    if constexpr (SWIGLU) xup[r][i] = j < a.k ? src[a.k + j] : 0.0f;
-                }
-            }
-        }
-        if constexpr (NORM) {
-#pragma unroll
-            for (int i = 0; i < PREP_KEPT; i++) {
-                const uint32_t j = element(i);
-                xgain[i] = 0.0f;
-                if (live(0, i)) xgain[i] = j < a.k ? a.row_gain[j] : 0.0f;
+                // (scalar: whole passes past the row end, and rows not given, cost nothing)
+                if ((uint32_t)r < rows && pass(i)) xrows[r][i] = j < a.k ? src[j] : 0.0f;
             }
         }
     }
 
     // The tail's per-output operands (activation scale, bias) are requested now, so that their
     // latency hides behind the stream instead of following it.
-    constexpr int TAIL_ITERS = ((int)(PREP ? kMaxPrepRows : kMaxGemvRows) * CH + WAVES * 64 - 1) / (WAVES * 64);
-    float tail_rs[F ? TAIL_ITERS : 1], tail_bias[F ? TAIL_ITERS : 1], tail_add[ROWOPS ? TAIL_ITERS : 1];
+    constexpr int TAIL_ITERS = ((int)kMaxGemvRows * CH + WAVES * 64 - 1) / (WAVES * 64);
+    float tail_rs[F ? TAIL_ITERS : 1], tail_bias[F ? TAIL_ITERS : 1];
     if constexpr (F) {
 #pragma unroll
         for (int it = 0; it < TAIL_ITERS; it++) {
             const uint32_t o = threadIdx.x + it * WAVES * 64;
-            tail_rs[it] = PREP ? 0.0f : a.row_scale[min(o / CH, rows - 1u)];
+            tail_rs[it] = a.row_scale[min(o / CH, rows - 1u)];
             tail_bias[it] = a.bias_f32[ch0 + o % CH];  // padded to whole panels
-            if constexpr (ROWOPS) {
-                // the residual the output is added to: this thread's element, read before anything writes it
-                const uint32_t om = o / CH, on = ch0 + o % CH;
-                tail_add[it] = (a.add_to && om < rows && on < a.n) ? a.add_to[(size_t)om * a.n + on] : 0.0f;
-            }
         }
     }
 
@@ -238,19 +204,11 @@ __global__ __launch_bounds__(WAVES * 64, (ROWOP == 2 && WAVES == 8) ? 4 : 1) voi
         }
     };
 
-    // PREP: the rows' codes [rows][ldk] and scales [rows] behind the group dots and group scales
-    __shared__ float slot_max[PREP_ROWS][WAVES];
-    __shared__ uint32_t slot_bad[PREP_ROWS][WAVES];
+    // PREP: the rows' codes [rows][ldk] behind the partial dots
     const uint32_t ldk = (a.k + 15u) / 16u * 16u;
-    int8_t* prep_codes = reinterpret_cast<int8_t*>(gemv_lds) +
-                         (F ? (size_t)a.groups * (rows + 1u) * CH * 4u : (size_t)WAVES * rows * CH * 4u);
-    float* prep_scale = reinterpret_cast<float*>(prep_codes + (size_t)rows * ldk);
-    // (NR, the number of rows, is a template tag: without a branch between the rows their chains of
-    // reductions interleave)
-    auto prepare_rows_of = [&](auto rows_tag) __attribute__((always_inline)) {
-        constexpr int NR = decltype(rows_tag)::value;
-        auto pass = [&](int i) { return first_of(i) < prep_end; };
-        if constexpr (PREP && !F) {
+    int8_t* prep_codes = reinterpret_cast<int8_t*>(gemv_lds) + (size_t)WAVES * rows * CH * 4u;
+    auto prepare_rows = [&]() __attribute__((always_inline)) {
+        if constexpr (PREP) {
             // QuantizeLinear in front of a QLinear: q = saturate(ties-to-even(f32(x / s) + f32(zp))), NaN -> zp
             // (native/src/kernels/quantize_linear_ops.inc:156-169), stored as the signed byte the MFMA takes
             // (an unsigned type's bytes have their top bit flipped, as input_zp already is)
@@ -258,11 +216,12 @@ __global__ __launch_bounds__(WAVES * 64, (ROWOP == 2 && WAVES == 8) ? 4 : 1) voi
             const float zp_f = (float)(a.input_zp + shift), lo_f = (float)(a.x_f32_unsigned ? 0 : -128),
                         hi_f = (float)(a.x_f32_unsigned ? 255 : 127);
 #pragma unroll
-            for (int r = 0; r < NR; r++) {
+            for (int r = 0; r < PREP_ROWS; r++) {
+                if ((uint32_t)r >= rows) continue;
 #pragma unroll
                 for (int i = 0; i < PREP_KEPT; i++) {
                     if (!pass(i)) continue;
-                    const uint32_t j = element(i);
+                    const uint32_t j = threadIdx.x + i * WAVES * 64;
                     const float v = xrows[r][i];
                     int32_t q = a.input_zp + shift;
                     if (v == v) {
@@ -273,77 +232,6 @@ __global__ __launch_bounds__(WAVES * 64, (ROWOP == 2 && WAVES == 8) ? 4 : 1) voi
                 }
             }
             __syncthreads();  // every wave reads every row's codes
-        }
-        if constexpr (SWIGLU) {
-#pragma unroll
-            for (int r = 0; r < NR; r++)
-#pragma unroll
-                for (int i = 0; i < PREP_KEPT; i++)
-                    if (pass(i)) xrows[r][i] = swiglu_value(xrows[r][i], xup[r][i]);
-        }
-        if constexpr (NORM) {
-            {
-                static_assert(WAVES == 8, "the sum of squares is ordered for a pair of elements a thread of 512");
-                __shared__ double norm_slots[PREP_ROWS][8];
-#pragma unroll
-                for (int r = 0; r < NR; r++) {
-                    double pair[1] = {0.0};
-#pragma unroll
-                    for (int i = 0; i < PREP_KEPT; i += 2)
-                        if (pass(i)) pair[0] += square(xrows[r][i]) + square(xrows[r][i + 1]);
-                    const double inv_std = rms_inverse(norm_total<512>(pair, norm_slots[r]), a.k, a.row_eps);
-#pragma unroll
-                    for (int i = 0; i < PREP_KEPT; i++)
-                        if (pass(i)) xrows[r][i] = rms_scaled(xrows[r][i], inv_std, xgain[i]);
-                }
-            }
-        }
-        if constexpr (PREP && F) {
-#pragma unroll
-            for (int r = 0; r < NR; r++) {
-                float maximum = 0.0f;
-                uint32_t bad = 0u;
-#pragma unroll
-                for (int i = 0; i < PREP_KEPT; i++) {
-                    if (!pass(i)) continue;
-                    bad |= finite_f32(xrows[r][i]) ? 0u : 1u;
-                    maximum = fmaxf(maximum, fabsf(xrows[r][i]));  // fmaxf ignores a NaN operand; `bad` records it
-                }
-                maximum = wave_max(maximum);
-                bad = __builtin_amdgcn_ballot_w64(bad != 0u) != 0ull ? 1u : 0u;
-                if (lane == 0) {
-                    slot_max[r][wave] = maximum;
-                    slot_bad[r][wave] = bad;
-                }
-            }
-            __syncthreads();
-#pragma unroll
-            for (int r = 0; r < NR; r++) {
-                float maximum = slot_max[r][0];
-                uint32_t bad = slot_bad[r][0];
-#pragma unroll
-                for (int w = 1; w < WAVES; w++) {
-                    maximum = fmaxf(maximum, slot_max[r][w]);
-                    bad |= slot_bad[r][w];
-                }
-                float scale = maximum == 0.0f ? 1.0f : __fdiv_rn(maximum, 127.0f);
-                if (scale < 0x1p-126f) scale = 0x1p-126f;
-#pragma unroll
-                for (int i = 0; i < PREP_KEPT; i++) {
-                    if (!pass(i)) continue;
-                    const uint32_t j = element(i);
-                    // (elements past k were loaded as zeros: the padding of the last 16-byte chunk)
-                    if (j < ldk) prep_codes[(size_t)r * ldk + j] = (int8_t)(bad ? 0 : packed_round_i8(__fdiv_rn(xrows[r][i], scale)));
-                }
-                if (threadIdx.x == 0) prep_scale[r] = bad ? __builtin_nanf("") : scale;
-            }
-            __syncthreads();  // every wave reads every row's codes
-        }
-    };
-    auto prepare_rows = [&]() __attribute__((always_inline)) {
-        if constexpr (PREP) {
-            if (rows >= 2u) prepare_rows_of(std::integral_constant<int, PREP_ROWS>{});
-            else prepare_rows_of(std::integral_constant<int, 1>{});
         }
     };
 
@@ -429,7 +317,7 @@ __global__ __launch_bounds__(WAVES * 64, (ROWOP == 2 && WAVES == 8) ? 4 : 1) voi
             const uint32_t o = threadIdx.x + it * WAVES * 64;
             if (o >= rows * CH) break;
             const uint32_t om = o / CH, on = ch0 + o % CH;
-            const float rs = PREP ? prep_scale[om] : tail_rs[it];
+            const float rs = tail_rs[it];
             float sum = 0.0f;
             const int32_t* dp = parts + o;
             const float* sp = lds_scales + o % CH;
@@ -448,10 +336,7 @@ __global__ __launch_bounds__(WAVES * 64, (ROWOP == 2 && WAVES == 8) ? 4 : 1) voi
             }
             for (; g < a.groups; g++)
                 sum = __fadd_rn(sum, __fmul_rn((float)dp[(size_t)g * slab], __fmul_rn(rs, sp[g * CH])));
-            float out = __fadd_rn(sum, tail_bias[it]);
-            if constexpr (ROWOPS)
-                if (a.add_to) out = __fadd_rn(tail_add[it], out);
-            if (on < a.n) ((float*)a.y)[(size_t)om * a.n + on] = out;
+            if (on < a.n) ((float*)a.y)[(size_t)om * a.n + on] = __fadd_rn(sum, tail_bias[it]);
         }
     } else {
         for (uint32_t o = threadIdx.x; o < rows * CH; o += WAVES * 64) {
@@ -481,19 +366,12 @@ __global__ __launch_bounds__(WAVES * 64, (ROWOP == 2 && WAVES == 8) ? 4 : 1) voi
 //     (packed_linear_ops.inc:1498-1504), bit for bit.
 // Measured at M=1, K=4096, N=14336 (sixteen waves of eight blocks): 10.3 us against 12.5 us for the
 // general kernel, with a plain read of the same bytes at 9.3-9.6 us.
-// PREP: one or two f32 rows (a.x_f32) which the workgroup prepares itself, by row_prepare_kernel's rule to the
-// letter, as the reference's single-row route quantizes the row and multiplies in one call
-// (packed_linear_ops.inc:1471-1535).  A wave's 64 lanes hold exactly the elements of the wave's own K-slice
-// (BPW / 2 consecutive ones per lane), so only the row maximum crosses the waves; the codes go straight into
-// the wave's LDS slice, where the MFMA's activation operand is read from.
 // W4: four-bit weights; a 1 KiB block then carries two k-steps (low nibbles, then high nibbles, each moved to
 // the top of its byte: operands with a factor 16, which the exact dot sheds with a shift when it is parked).
-template <int GK, int WAVES, int BPW, bool XLDS, bool PREP = false, bool RPROD = false, bool W4 = false, int SPLIT = 1>
+template <int GK, int WAVES, int BPW, bool XLDS, bool RPROD = false, bool W4 = false, int SPLIT = 1>
 __global__ __launch_bounds__(WAVES * 64, 8) void gemv_fit_kernel(const LinearArgs a) {
     constexpr int SPB = W4 ? 2 : 1, STEPS = BPW * SPB;  // k-steps per block, per wave
     static_assert(STEPS % GK == 0 && BPW >= kDepth, "a wave's run is whole groups and at least one round");
-    static_assert(!PREP || (XLDS && STEPS % 4 == 0), "prepared rows live in the LDS slices; a lane loads pairs of elements");
-    static_assert(!(PREP && RPROD), "one or two rows form their products lane-parallel");
     static_assert(SPLIT == 1 || SPLIT == 2 || SPLIT == 4, "workgroups per panel");
     constexpr int GPW = STEPS / GK, GROUPS = WAVES * GPW;  // groups per wave, per panel
     // SPLIT workgroups share a panel, each taking CH of its channels, as in gemv_panel_kernel: a lane whose
@@ -521,22 +399,9 @@ __global__ __launch_bounds__(WAVES * 64, 8) void gemv_fit_kernel(const LinearArg
 
     // (XLDS) this wave's activation chunks are requested first: they are cache hits and return ahead
     // of the weight stream
-    constexpr int XPL = XLDS && !PREP ? (2 * STEPS * (int)kFitLdsRows + 63) / 64 : 1;  // chunks per lane
+    constexpr int XPL = XLDS ? (2 * STEPS * (int)kFitLdsRows + 63) / 64 : 1;  // chunks per lane
     v4i xstage[XPL];
-    constexpr int EPL = STEPS / 2;  // PREP: f32 elements of a row per lane
-    float xf[PREP ? (int)kMaxPrepRows : 1][PREP ? EPL : 1];
-    if constexpr (PREP) {
-#pragma unroll
-        for (int r = 0; r < (int)kMaxPrepRows; r++) {
-            const float* src = a.x_f32 + (size_t)min((uint32_t)r, rows - 1u) * a.ldx + (size_t)t0 * 32u + (uint32_t)lane * EPL;
-#pragma unroll
-            for (int i = 0; i < EPL; i += 2) {
-                const float2 v = *reinterpret_cast<const float2*>(src + i);
-                xf[r][i] = v.x;
-                xf[r][i + 1] = v.y;
-            }
-        }
-    } else if constexpr (XLDS) {
+    if constexpr (XLDS) {
 #pragma unroll
         for (int j = 0; j < XPL; j++) {
             const uint32_t e = min((uint32_t)lane + 64u * j, 2u * STEPS * rows - 1u);
@@ -576,61 +441,13 @@ __global__ __launch_bounds__(WAVES * 64, 8) void gemv_fit_kernel(const LinearArg
         sreg[u] = a.scales_t[(size_t)(g0 + e / CH) * a.n_pad + ch0 + e % CH];
     }
     // (RPROD: the scale of the row whose dots the lane holds in its accumulators; else lane r carries row r's)
-    float rs_lane = 0.0f;
-    if constexpr (!PREP) rs_lane = a.row_scale[RPROD ? m : min((uint32_t)lane, rows - 1u)];
+    const float rs_lane = a.row_scale[RPROD ? m : min((uint32_t)lane, rows - 1u)];
     constexpr int OPT_ = ((int)kMaxGemvRows * CH + WAVES * 64 - 1) / (WAVES * 64);  // outputs per thread
     float bias_t[OPT_];
 #pragma unroll
     for (int it = 0; it < OPT_; it++) bias_t[it] = a.bias_f32[ch0 + (threadIdx.x + it * WAVES * 64) % CH];
 
-    if constexpr (PREP) {
-        // per row: scale = max|x| / 127 (true division; 1 for a zero row; floored at 2^-126), codes =
-        // ties-to-even(x / scale) clamped to +-127; a row that is not finite gets zero codes and a NaN scale
-        __shared__ float slot_max[kMaxPrepRows][WAVES];
-        __shared__ uint32_t slot_bad[kMaxPrepRows][WAVES];
-#pragma unroll
-        for (int r = 0; r < (int)kMaxPrepRows; r++) {
-            float maximum = 0.0f;
-            uint32_t bad = 0u;
-#pragma unroll
-            for (int i = 0; i < EPL; i++) {
-                bad |= finite_f32(xf[r][i]) ? 0u : 1u;
-                maximum = fmaxf(maximum, fabsf(xf[r][i]));
-            }
-            maximum = wave_max(maximum);
-            bad = __builtin_amdgcn_ballot_w64(bad != 0u) != 0ull ? 1u : 0u;
-            if (lane == 0) {
-                slot_max[r][wave] = maximum;
-                slot_bad[r][wave] = bad;
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int r = 0; r < (int)kMaxPrepRows; r++) {
-            float maximum = slot_max[r][0];
-            uint32_t bad = slot_bad[r][0];
-#pragma unroll
-            for (int w = 1; w < WAVES; w++) {
-                maximum = fmaxf(maximum, slot_max[r][w]);
-                bad |= slot_bad[r][w];
-            }
-            float scale = maximum == 0.0f ? 1.0f : __fdiv_rn(maximum, 127.0f);
-            if (scale < 0x1p-126f) scale = 0x1p-126f;
-            if ((uint32_t)r < rows) {
-                // element j = lane * EPL + i of the slice lives in chunk j / 16 at byte j % 16: [chunk][row] of 16 bytes
-#pragma unroll
-                for (int i = 0; i < EPL; i += 2) {
-                    const uint32_t j = (uint32_t)lane * EPL + i;
-                    const int32_t q0 = bad ? 0 : packed_round_i8(__fdiv_rn(xf[r][i], scale));
-                    const int32_t q1 = bad ? 0 : packed_round_i8(__fdiv_rn(xf[r][i + 1], scale));
-                    *reinterpret_cast<uint16_t*>(xslice + ((size_t)(j / 16u) * rows + r) * 16u + j % 16u) =
-                        (uint16_t)((uint32_t)(q0 & 0xff) | ((uint32_t)(q1 & 0xff) << 8));
-                }
-            }
-            const float row_scale = bad ? __builtin_nanf("") : scale;
-            if (min((uint32_t)lane, rows - 1u) == (uint32_t)r) rs_lane = row_scale;  // (as the loaded scales: lane r carries row r's)
-        }
-    } else if constexpr (XLDS) {
+    if constexpr (XLDS) {
 #pragma unroll
         for (int j = 0; j < XPL; j++) {
             const uint32_t e = (uint32_t)lane + 64u * j;
@@ -753,16 +570,13 @@ __global__ __launch_bounds__(WAVES * 64, 8) void gemv_fit_kernel(const LinearArg
 
 template <int GK, int WAVES, int BPW, bool W4, int SPLIT = 1>
 bool launch_fit(hipStream_t s, const LinearArgs& a, size_t lds, bool xlds, bool rprod) {
-    auto kern = xlds ? gemv_fit_kernel<GK, WAVES, BPW, true, false, false, W4, SPLIT> : gemv_fit_kernel<GK, WAVES, BPW, false, false, false, W4, SPLIT>;
+    auto kern = xlds ? gemv_fit_kernel<GK, WAVES, BPW, true, false, W4, SPLIT> : gemv_fit_kernel<GK, WAVES, BPW, false, false, W4, SPLIT>;
     if (rprod)
-        kern = xlds ? gemv_fit_kernel<GK, WAVES, BPW, true, false, true, W4, SPLIT> : gemv_fit_kernel<GK, WAVES, BPW, false, false, true, W4, SPLIT>;
-    if constexpr (SPLIT == 1 && (BPW * (W4 ? 2 : 1)) % 4 == 0) {
-        if (a.x_f32) kern = gemv_fit_kernel<GK, WAVES, BPW, true, true, false, W4>;
-    }
+        kern = xlds ? gemv_fit_kernel<GK, WAVES, BPW, true, true, W4, SPLIT> : gemv_fit_kernel<GK, WAVES, BPW, false, true, W4, SPLIT>;
     if (gemv_dry_run) return true;
     if (lds > 64u * 1024u) {
-        static std::atomic<uint64_t> configured[5] = {{0}, {0}, {0}, {0}, {0}};
-        if (!raise_lds_limit((const void*)kern, 160 * 1024, configured[a.x_f32 ? 4 : (rprod ? 2 : 0) + (xlds ? 1 : 0)])) return false;
+        static std::atomic<uint64_t> configured[4] = {{0}, {0}, {0}, {0}};
+        if (!raise_lds_limit((const void*)kern, 160 * 1024, configured[(rprod ? 2 : 0) + (xlds ? 1 : 0)])) return false;
     }
     hipLaunchKernelGGL(kern, dim3((a.n + 31u) / 32u * SPLIT), dim3(WAVES * 64), lds, s, a);
     return hipGetLastError() == hipSuccess;
@@ -777,10 +591,10 @@ const char* launch_fit_mode(hipStream_t s, const LinearArgs& a, int cu_count, co
     constexpr uint32_t SPB = W4 ? 2u : 1u;
     if (force && (strstr(force, "nofit") || strstr(force, "wv"))) return nullptr;  // (wv..: a general-kernel name)
     if (a.row_gain || a.row_swiglu || a.add_to || a.weight_bits != (W4 ? 4u : 8u) || a.x_flip_mask) return nullptr;
-    // f32 rows (prepared in the kernel): one or two whole rows of exactly the stream's length, pairs of elements aligned
+    // One or two f32 rows of exactly the stream's length: gemv_row.hip runs them, under the name of the instance that
+    // takes such a shape's prepared rows.
     const bool prep = a.x_f32 != nullptr;
-    if (prep && (a.rows > kMaxPrepRows || a.k != a.ksteps * 32u * SPB || (a.ldx % 2u) != 0u || ((uintptr_t)a.x_f32 % 8u) != 0u))
-        return nullptr;
+    if (prep && (a.rows > kMaxPrepRows || a.k != a.ksteps * 32u * SPB)) return nullptr;
     const uint32_t panels = (a.n + 31u) / 32u;
     const bool forced = force && strstr(force, "fit");
     // workgroups per panel: the general kernel's rule (and its names: c8, c16 for the channels of a workgroup)
@@ -807,7 +621,7 @@ const char* launch_fit_mode(hipStream_t s, const LinearArgs& a, int cu_count, co
     // in its accumulators' layout (more rows)
     // (measured at K=4096, N=14336: one row 10.8 us either way, 2 / 4 / 8 / 16 / 32 rows 10.8 / 10.9 / 11.0 / 11.9 / 16.3 us
     // against 11.1 / 11.3 / 12.9 / 15.9 / 27.9 lane-parallel and 12.5 / 12.6 / 12.8 / 13.5 / 18.4 in the general kernel)
-    const bool rprod = !prep && (force && strstr(force, "rprod") ? true : force && strstr(force, "lprod") ? false : a.rows > 1u);
+    const bool rprod = force && strstr(force, "rprod") ? true : force && strstr(force, "lprod") ? false : a.rows > 1u;
     static thread_local char name[24];
     bool taken = false, ok = false;
     auto run = [&](auto waves_tag, auto bpw_tag, auto splits_tag) {
@@ -823,12 +637,14 @@ const char* launch_fit_mode(hipStream_t s, const LinearArgs& a, int cu_count, co
             // the activation rows go through LDS while two workgroups still fit a compute unit that way
             bool xlds = a.rows <= kFitLdsRows;
             size_t lds = lds_for(W, STEPS, xlds);
-            if (xlds && lds > 80u * 1024u && !prep) {
+            if (xlds && lds > 80u * 1024u) {
                 xlds = false;
                 lds = lds_for(W, STEPS, false);
             }
-            if (lds > 156u * 1024u || (prep && STEPS % 4 != 0)) return;
-            if constexpr (SPLITS) {
+            if (lds > 156u * 1024u) return;
+            if (prep) {
+                ok = launch_gemv_row(s, a, cu_count, force, gemv_dry_run) != nullptr;
+            } else if constexpr (SPLITS) {
                 if (split == 4u) ok = launch_fit<GK, W, B, W4, 4>(s, a, lds, xlds, rprod);
                 else if (split == 2u) ok = launch_fit<GK, W, B, W4, 2>(s, a, lds, xlds, rprod);
                 else ok = launch_fit<GK, W, B, W4>(s, a, lds, xlds, rprod);
@@ -866,9 +682,9 @@ const char* launch_fit_mode(hipStream_t s, const LinearArgs& a, int cu_count, co
     return ok ? name : nullptr;
 }
 
-template <int MODE, int GK, int WAVES, bool W4, int SPLIT = 1, int ROWOP = kRowsPrepared>
+template <int MODE, int GK, int WAVES, bool W4, int SPLIT = 1, bool PREP = false>
 bool launch_panel(hipStream_t s, const LinearArgs& a, size_t lds) {
-    auto kern = gemv_panel_kernel<MODE, GK, WAVES, W4, SPLIT, ROWOP>;
+    auto kern = gemv_panel_kernel<MODE, GK, WAVES, W4, SPLIT, PREP>;
     if (gemv_dry_run) return true;
     if (lds > 64u * 1024u) {
         static std::atomic<uint64_t> configured{0};
@@ -878,17 +694,19 @@ bool launch_panel(hipStream_t s, const LinearArgs& a, size_t lds) {
     return hipGetLastError() == hipSuccess;
 }
 
-template <int MODE, int GK, int WAVES, bool W4, int ROWOP = kRowsPrepared>
+template <int MODE, int GK, int WAVES, bool W4, bool PREP = false>
 bool launch_split(hipStream_t s, const LinearArgs& a, size_t lds, int split) {
-    if (split == 4) return launch_panel<MODE, GK, WAVES, W4, 4, ROWOP>(s, a, lds);
-    if (split == 2) return launch_panel<MODE, GK, WAVES, W4, 2, ROWOP>(s, a, lds);
-    return launch_panel<MODE, GK, WAVES, W4, 1, ROWOP>(s, a, lds);
+    if (split == 4) return launch_panel<MODE, GK, WAVES, W4, 4, PREP>(s, a, lds);
+    if (split == 2) return launch_panel<MODE, GK, WAVES, W4, 2, PREP>(s, a, lds);
+    return launch_panel<MODE, GK, WAVES, W4, 1, PREP>(s, a, lds);
 }
 
 template <int MODE, int GK, bool W4 = false>
 const char* launch_mode(hipStream_t s, const LinearArgs& a, int cu_count, const char* force) {
     if constexpr (MODE == (int)Epilogue::DequantF32) {
         if (const char* fit = launch_fit_mode<GK, W4>(s, a, cu_count, force)) return fit;
+        // f32 rows; with the general kernel named (wv..), the caller prepares them and comes back
+        if (a.x_f32) return force && strstr(force, "wv") ? nullptr : launch_gemv_row(s, a, cu_count, force, gemv_dry_run);
     }
     // blocks of the stream per panel, and the units a wave's run is made of
     constexpr uint32_t SPB = W4 ? 2 : 1, UNIT = GK > SPB ? GK : SPB;
@@ -907,7 +725,7 @@ const char* launch_mode(hipStream_t s, const LinearArgs& a, int cu_count, const 
     else if (force && strstr(force, "wv8")) waves = 8;
     else if (force && strstr(force, "wv4")) waves = 4;
     else if (force && strstr(force, "wv2")) waves = 2;
-    // f32 rows are prepared by workgroups of eight waves or more (waves past the end of a short row idle)
+    // f32 rows are quantized by workgroups of eight waves or more (waves past the end of a short row idle)
     if (a.x_f32 && waves < 8) waves = 8;
     // Fewer panels than half the compute units: two or four workgroups share each panel's
     // channels (only the 8- and 16-wave kernels are built that way; such shapes have them
@@ -922,40 +740,22 @@ const char* launch_mode(hipStream_t s, const LinearArgs& a, int cu_count, const 
     const size_t ch_bytes = 128u / (size_t)split;  // one row of the workgroup's channels, int32 or f32
     size_t lds = MODE == (int)Epilogue::DequantF32 ? (size_t)a.groups * (a.rows + 1u) * ch_bytes
                                                     : (size_t)waves * a.rows * ch_bytes;
-    // f32 activations: the kernel prepares them itself (codes and scales in LDS behind the rest)
+    // f32 activations: the kernel quantizes them itself (codes in LDS behind the rest)
     const bool prep = a.x_f32 != nullptr;
     if (prep) {
-        // (a thread keeps kPrepPerThread elements of every row in registers between the two passes)
-        if (MODE == (int)Epilogue::RequantRow || a.rows > kMaxPrepRows || waves < 8 ||
-            a.k > (uint32_t)kPrepPerThread * (uint32_t)waves * 64u || (MODE != (int)Epilogue::DequantF32 && a.zw))
+        // (a thread keeps kPrepPerThread elements of every row in registers)
+        if (MODE != (int)Epilogue::RequantTensor || a.rows > kMaxPrepRows || waves < 8 ||
+            a.k > (uint32_t)kPrepPerThread * (uint32_t)waves * 64u || a.zw)
             return nullptr;
-        lds += (size_t)a.rows * ((a.k + 15u) / 16u * 16u) + (size_t)a.rows * 4u + 16u;
-        // RMSNorm in front: rows of 1024 elements and more
-        if (a.row_gain && a.k < kNormBlock) return nullptr;
-        // (that form is built for eight waves only: its double arithmetic does not fit the registers of sixteen)
-        if (a.row_gain) {
-            if (a.k > (uint32_t)kPrepPerThread * 8u * 64u) return nullptr;
-            waves = 8;
-        }
+        lds += (size_t)a.rows * ((a.k + 15u) / 16u * 16u);
     }
     // the MFMA GEMM takes shapes whose group dots or scales do not fit
     if (lds > 156u * 1024u) return nullptr;
     bool ok = false;
-    if constexpr (MODE != (int)Epilogue::RequantRow) {
+    if constexpr (MODE == (int)Epilogue::RequantTensor) {
         if (prep) {
-            if constexpr (MODE == (int)Epilogue::DequantF32) {
-                if (a.row_gain)
-                    ok = launch_split<MODE, GK, 8, W4, kRowsNorm>(s, a, lds, split);
-                else if (a.row_swiglu)
-                    ok = waves == 16 ? launch_split<MODE, GK, 16, W4, kRowsSwiglu>(s, a, lds, split)
-                                     : launch_split<MODE, GK, 8, W4, kRowsSwiglu>(s, a, lds, split);
-                else
-                    ok = waves == 16 ? launch_split<MODE, GK, 16, W4, kRowsF32>(s, a, lds, split)
-                                     : launch_split<MODE, GK, 8, W4, kRowsF32>(s, a, lds, split);
-            } else {
-                ok = waves == 16 ? launch_split<MODE, GK, 16, W4, kRowsF32>(s, a, lds, split)
-                                 : launch_split<MODE, GK, 8, W4, kRowsF32>(s, a, lds, split);
-            }
+            ok = waves == 16 ? launch_split<MODE, GK, 16, W4, true>(s, a, lds, split)
+                             : launch_split<MODE, GK, 8, W4, true>(s, a, lds, split);
             if (!ok) return nullptr;
             static const char* const prep_names[3][2] = {{"wv8-prep", "wv16-prep"},
                                                          {"wv8c16-prep", "wv16c16-prep"},
