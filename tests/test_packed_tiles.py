@@ -1,0 +1,40 @@
+"""The narrow tiles of the dequantizing GEMM (gemm_k64.hip) at the edges of their rows, channels and k-blocks."""
+import numpy as np
+import pytest
+
+import _cases as cases
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("grouped", [True, False])
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("group", [32, 64, 128, 256])
+@pytest.mark.parametrize("rows,k,n", [(33, 31, 5), (64, 32, 64), (65, 128, 65), (33, 129, 31), (129, 161, 130), (47, 640, 257),
+                                      (96, 1153, 34), (257, 2050, 300)])
+def test_narrow_tiles_at_their_edges(ctx, oracle, rows, k, n, group, bits, grouped):
+    """One k-block and many, a last k-block with one to four groups of 32, rows and channels that end inside a tile, one
+    scale per channel and a scale per group: the oracle's bits, on every tile and on the one the rule picks."""
+    import torch
+    import volvoxai_amd as vx
+    c = cases.packed_case(rows, k, n, group, rows + k + n + bits, True, special_rows=rows == 47)
+    scales = c["scales"] if grouped else np.ascontiguousarray(np.broadcast_to(c["scales"][:, :1], c["scales"].shape))
+    w = c["w"] if bits == 8 else cases.four_bit(c["w"])
+    words = oracle.pack_w8_words(w) if bits == 8 else oracle.pack_w4_words(w)
+    _, want = oracle.packed_linear(c["x"], words, scales, c["bias"], n, group, bits=bits)
+    pl = vx.PackedLinear(words, scales, c["bias"], k, n, group, weight_bits=bits)
+    x = torch.from_numpy(c["x"]).cuda()
+    seen = set()
+    try:
+        for force in (None, "a8-mfma.t64x64k64", "a8-mfma.t64x32k64", "a8-mfma.t32x32k64"):
+            vx.force_variant(force)
+            st, y = pl.forward_f32(ctx, x)
+            ctx.synchronize()
+            got = y.cpu().numpy()
+            nan = np.isnan(want)
+            assert st == 0 and "k64" in ctx.last_variant, ctx.last_variant
+            assert (np.isnan(got) == nan).all() and (got.view(np.uint32)[~nan] == want.view(np.uint32)[~nan]).all(), ctx.last_variant
+            seen.add(ctx.last_variant.rsplit(".", 1)[1])
+    finally:
+        vx.force_variant(None)
+        pl.close()
+    assert seen == {"t64x64k64", "t64x32k64", "t32x32k64"}, seen

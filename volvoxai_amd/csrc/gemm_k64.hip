@@ -331,31 +331,40 @@ __global__ __launch_bounds__(WN* WM * 64) void gemm_k64_kernel(const GemmParams 
     }
 }
 
+// eight codes' low nibbles (two's complement) as four signed bytes, every second one: ((v ^ 8) - 8) without a
+// borrow between the bytes
+__device__ __forceinline__ uint32_t signed_nibbles(uint32_t v) {
+    return (((v & 0x0f0f0f0fu) ^ 0x08080808u) + 0x78787878u) ^ 0x80808080u;
+}
+
 // ---- the dequantizing form (PackedLinear under DYNAMIC_I8) ----------------------------------------
 // sum += f32(dot_g) * (s_a * s_w[n][g]) in ascending group order with every product and sum rounded
 // on its own (packed_linear_ops.inc:1498-1504): four VALU operations per output and group against
 // 2 * group_size matrix operations, so the kernel is bound by the vector pipe, not by the MFMAs.
-// It therefore runs small wave tiles (64 channels x 32 rows) at four waves per SIMD and leaves the
-// overlap of one wave's fold with the other waves' MFMAs to the hardware: two workgroups of
-// 128 x 128 per compute unit, each with its own barrier.  GK: 64-wide MFMA steps per scale group
-// (1, 2 or 4).  W4: four-bit weights; a 1 KiB block then holds the block pair of one MFMA step, low
+// It therefore runs small wave tiles (16 x TN channels x 16 x TM rows, at most 64 x 32) at four waves per
+// SIMD and leaves the overlap of one wave's fold with the other waves' MFMAs to the hardware: two workgroups
+// of 128 x 128 per compute unit, each with its own barrier, or more of the narrow tiles that put a small
+// launch on every SIMD (see pick_f32_tile).  GK: 64-wide MFMA steps per scale group (1, 2 or 4; 0: two groups
+// of 32 per step, on 16x16x32 MFMAs, which take the same cycles).  W4: four-bit weights; a 1 KiB block then holds the block pair of one MFMA step, low
 // nibbles for its first 32 k, high nibbles for the rest, and a lane shifts its half into place.
 // The scales of the groups that end in a k-block travel as the tail of that k-block's LDS stage.
 // UNI: every channel has one scale for all its groups (a per-channel scale replicated, which is what
 // per-channel quantization exports); s_a * s_w is then formed once per output instead of once per
 // output and group -- the same products, so the same bits -- and the fold is three operations.
-template <int GK, bool W4, int WM, int NS, bool UNI>
-__global__ __launch_bounds__(WM * 128, 4) void gemm_k64_f32_kernel(const GemmParams p) {
-    constexpr int WN = 2, TN = 4, TM = 2, NWAVES = WN * WM;
-    constexpr int BN = WN * TN * 16, BM = WM * TM * 16;  // 128 channels x 128 or 256 rows
+template <int GK, bool W4, int WN, int WM, int TN, int TM, int NS, bool UNI>
+__global__ __launch_bounds__(WN * WM * 64, 4) void gemm_k64_f32_kernel(const GemmParams p) {
+    constexpr int NWAVES = WN * WM;
+    constexpr int BN = WN * TN * 16, BM = WM * TM * 16;
     constexpr int KS = 4, KB = W4 ? 2 : 4;  // 32-byte k-steps and 1 KiB weight blocks per panel and stage
+    static_assert(BN % 32 == 0 && BM % 8 == 0 && (TN == 1 || TN % 2 == 0), "whole panels, whole loads");
     constexpr int WBLK = (BN / 32) * KB, XBLK = BM / 8;
-    constexpr int WLOADS = WBLK / NWAVES, XLOADS = XBLK / NWAVES;
-    static_assert(WBLK % NWAVES == 0 && XBLK % NWAVES == 0, "blocks must divide over waves");
-    constexpr int GPB = GK == 1 ? 2 : 1;  // scale groups that end in a k-block (GK == 4: every second block)
+    constexpr int GPB = GK == 0 ? 4 : GK == 1 ? 2 : 1;  // scale groups that end in a k-block (GK == 4: every second block)
+    constexpr int SBLK = UNI ? 0 : (GPB * BN + 63) / 64;  // loads of 64 scales
+    constexpr int WLOADS = (WBLK + NWAVES - 1) / NWAVES, XLOADS = (XBLK + NWAVES - 1) / NWAVES;
+    constexpr int SLOADS = (SBLK + NWAVES - 1) / NWAVES;
     constexpr int SCALE_OFF = (WBLK + XBLK) * 1024;
-    constexpr int STAGE_BYTES = SCALE_OFF + GPB * BN * 4;
-    constexpr int NLOADS = WLOADS + XLOADS;
+    constexpr int STAGE_BYTES = SCALE_OFF + SBLK * 256;
+    constexpr int NLOADS = WLOADS + XLOADS + SLOADS;
     const LinearArgs& a = p.a;
 
     const int lane = threadIdx.x & 63;
@@ -374,10 +383,12 @@ __global__ __launch_bounds__(WM * 128, 4) void gemm_k64_f32_kernel(const GemmPar
     const int8_t* const w_tile = a.w + (size_t)(n0 / 32u) * panel_bytes;
     const uint32_t last_chunk = (a.k - 1u) / 16u;
     const uint32_t my_chunk = (lane & 7) ^ ((lane >> 3) & 7);
+    // (a wave without a block of its own in the last round of loads repeats another's: the same bytes to the
+    // same place, and every wave has the same number of loads in flight)
     uint32_t xrow[XLOADS];
 #pragma unroll
     for (int i = 0; i < XLOADS; i++) {
-        const int b = wave + i * NWAVES;
+        const int b = (wave + i * NWAVES) % XBLK;
         uint32_t row = m0 + b * 8 + (lane >> 3);
         row = min(row, a.rows - 1u);
         xrow[i] = row * a.ldx;
@@ -386,23 +397,22 @@ __global__ __launch_bounds__(WM * 128, 4) void gemm_k64_f32_kernel(const GemmPar
     const uint32_t nkb = (ksteps_real + KS - 1) / KS;
     auto issue_block = [&](uint32_t kb, int stage) {
         char* base = lds_raw + stage * STAGE_BYTES;
-        // the scales of the groups that end in this k-block: 64 channels per wavefront, 4 bytes per lane
-        if (!UNI && wave < GPB * (BN / 64)) {
-            const uint32_t slot = wave / (BN / 64), half = wave % (BN / 64);
-            const uint32_t g = min(GK == 1 ? kb * 2u + slot : GK == 2 ? kb : kb / 2u, a.groups - 1u);
-            load_to_lds4(a.scales_t + (size_t)g * a.n_pad + n0 + half * 64 + lane,
-                         base + SCALE_OFF + (slot * BN + half * 64) * 4);
-        }
         static_for<NLOADS>([&](auto t_tag) {
             constexpr int t = decltype(t_tag)::value;
-            if constexpr (t < WLOADS) {
-                const uint32_t b = wave + t * NWAVES;
+            if constexpr (t < SLOADS) {
+                // the scales of the groups that end in this k-block, [group][channel]: 4 bytes per lane
+                const uint32_t b = (wave + t * NWAVES) % (SBLK > 0 ? SBLK : 1), e = b * 64u + lane;
+                const uint32_t slot = e / BN, g = GK == 0 ? kb * 4u + slot : GK == 1 ? kb * 2u + slot : GK == 2 ? kb : kb / 2u;
+                load_to_lds4(a.scales_t + (size_t)min(g, a.groups - 1u) * a.n_pad + n0 + e % BN, base + SCALE_OFF + b * 256);
+            } else if constexpr (t < SLOADS + WLOADS) {
+                const uint32_t b = (wave + (t - SLOADS) * NWAVES) % WBLK;
                 const int8_t* src = w_tile + (size_t)(b / KB) * panel_bytes + (size_t)(kb * KB + b % KB) * 1024u;
                 load_to_lds16(src + w_lane, base + b * 1024);
             } else {
+                constexpr int i = t - SLOADS - WLOADS;
                 const uint32_t chunk16 = min(kb * 8u + my_chunk, last_chunk) * 16u;
-                const uint32_t b = wave + (t - WLOADS) * NWAVES;
-                load_to_lds16(a.x + (xrow[t - WLOADS] + chunk16), base + (WBLK + b) * 1024);
+                const uint32_t b = (wave + i * NWAVES) % XBLK;
+                load_to_lds16(a.x + (xrow[i] + chunk16), base + (WBLK + b) * 1024);
             }
         });
     };
@@ -425,14 +435,22 @@ __global__ __launch_bounds__(WM * 128, 4) void gemm_k64_f32_kernel(const GemmPar
 
     // fragment addressing (see the requantizing kernel); four-bit weights: one block per MFMA step,
     // the lane's 16-byte slot is the same for both halves of the step
-    const uint32_t a_frag = W4 ? (uint32_t)(wave_n * (TN / 2) * KB) * 1024u + (uint32_t)((lane & 15) + 32 * ((lane >> 4) & 1)) * 16u
-                               : (uint32_t)(wave_n * (TN / 2) * KB) * 1024u + (uint32_t)(lane >> 5) * 1024u +
-                                     (uint32_t)((lane & 15) + 32 * ((lane >> 4) & 1)) * 16u;
+    const uint32_t tile0 = (uint32_t)wave_n * TN;  // the wave's first 16 channels
+    const uint32_t a_tile = (tile0 / 2u) * KB * 1024u + (tile0 & 1u) * 256u;
+    // (groups of 32: the MFMA takes eight bytes a lane, of one k-step)
+    const uint32_t a_frag = GK == 0 ? a_tile + (uint32_t)((lane & 15) + 32 * (lane >> 5)) * 16u + ((lane >> 4) & 1) * 8u
+                            : W4    ? a_tile + (uint32_t)((lane & 15) + 32 * ((lane >> 4) & 1)) * 16u
+                                    : a_tile + (uint32_t)(lane >> 5) * 1024u + (uint32_t)((lane & 15) + 32 * ((lane >> 4) & 1)) * 16u;
     const uint32_t nib_shift = lane < 32 ? 4u : 0u;
     const uint32_t x_row = WBLK * 1024u + ((uint32_t)(wave_m * TM * 16) + (lane & 15)) * 128u;
-    uint32_t x_slot[2];
+    uint32_t x_slot[GK == 0 ? KS : 2];
+    if constexpr (GK == 0) {
 #pragma unroll
-    for (int s = 0; s < 2; s++) x_slot[s] = (((4u * s + (lane >> 4)) ^ (lane & 7u)) << 4);
+        for (int s = 0; s < KS; s++) x_slot[s] = (((2u * s + (lane >> 5)) ^ (lane & 7u)) << 4) + ((lane >> 4) & 1) * 8u;
+    } else {
+#pragma unroll
+        for (int s = 0; s < 2; s++) x_slot[s] = (((4u * s + (lane >> 4)) ^ (lane & 7u)) << 4);
+    }
     const uint32_t sw_lane = SCALE_OFF + (uint32_t)(wave_n * TN * 16 + (lane >> 4) * 4) * 4u;
 
     // UNI: the products s_a * s_w of the lane's outputs
@@ -448,6 +466,7 @@ __global__ __launch_bounds__(WM * 128, 4) void gemm_k64_f32_kernel(const GemmPar
         }
     }
     // fold of scale-group slot `slot` of the stage: every tile of the wave
+    constexpr int DOT_SHIFT = W4 && GK != 0 ? 4 : 0;
     auto fold = [&](const char* stage, int slot) {
 #pragma unroll
         for (int i = 0; i < TN; i++) {
@@ -459,7 +478,7 @@ __global__ __launch_bounds__(WM * 128, 4) void gemm_k64_f32_kernel(const GemmPar
                 for (int e = 0; e < 4; e++) {
                     const float gs = UNI ? gs_all[UNI ? i : 0][UNI ? j : 0][e] : __fmul_rn(row_scale[j], sw[e]);
                     // four-bit operands carry a factor 16; the dot is exact, so is the shift
-                    const float term = __fmul_rn((float)(acc[i][j][e] >> (W4 ? 4 : 0)), gs);
+                    const float term = __fmul_rn((float)(acc[i][j][e] >> DOT_SHIFT), gs);
                     fsum[i][j][e] = __fadd_rn(fsum[i][j][e], term);
                 }
             }
@@ -472,47 +491,84 @@ __global__ __launch_bounds__(WM * 128, 4) void gemm_k64_f32_kernel(const GemmPar
     // last one, so the count of loads in flight is the same in every iteration.)
     static_for<NS - 1>([&](auto b_tag) { issue_block(min((uint32_t)decltype(b_tag)::value, nkb - 1u), decltype(b_tag)::value); });
     int cur = 0, refill = NS - 1;
-    for (uint32_t kb = 0; kb < nkb; kb++) {
-        wait_vmcnt<(NS - 2) * NLOADS>();  // (waves that also carry a scale load wait for one load more than they must)
+    const v4i zero = {0, 0, 0, 0};
+    auto k_block = [&](uint32_t kb, auto ends_tag) {
+        constexpr bool ENDS = decltype(ends_tag)::value;  // may be the last k-block, with fewer groups
+        wait_vmcnt<(NS - 2) * NLOADS>();
         wg_barrier();
         issue_block(min(kb + NS - 1u, nkb - 1u), refill);
         const char* stage = lds_raw + cur * STAGE_BYTES;
+        if constexpr (GK == 0) {
+            // a group per k-step of 32.  Four-bit weights are spread to signed bytes here, which the many outputs
+            // of a group are cheaper for than a shift each.
 #pragma unroll
-        for (int s = 0; s < 2; s++) {
-            v4i af[TN], bf[TM];
+            for (int s = 0; s < KS; s++) {
+                long bf[TM], af[TN];
 #pragma unroll
-            for (int j = 0; j < TM; j++) bf[j] = *reinterpret_cast<const v4i*>(stage + x_row + j * 16 * 128 + x_slot[s]);
+                for (int j = 0; j < TM; j++) bf[j] = *reinterpret_cast<const long*>(stage + x_row + j * 16 * 128 + x_slot[s]);
 #pragma unroll
-            for (int i = 0; i < TN; i++) {
-                if constexpr (W4) {
-                    const v4i raw = *reinterpret_cast<const v4i*>(stage + a_frag + ((i / 2) * KB + s) * 1024 + (i & 1) * 256);
-#pragma unroll
-                    for (int d = 0; d < 4; d++) af[i][d] = (raw[d] << nib_shift) & (int)0xf0f0f0f0u;
-                } else {
-                    af[i] = *reinterpret_cast<const v4i*>(stage + a_frag + ((i / 2) * KB + 2 * s) * 1024 + (i & 1) * 256);
+                for (int i = 0; i < TN; i++) {
+                    const long raw = *reinterpret_cast<const long*>(stage + a_frag + ((i / 2) * KB + (W4 ? s / 2 : s)) * 1024 + (i & 1) * 256);
+                    if constexpr (W4) {
+                        const uint32_t lo = signed_nibbles((uint32_t)raw >> (s & 1) * 4);
+                        const uint32_t hi = signed_nibbles((uint32_t)((uint64_t)raw >> 32) >> (s & 1) * 4);
+                        af[i] = (long)(((uint64_t)hi << 32) | lo);
+                    } else {
+                        af[i] = raw;
+                    }
                 }
+#pragma unroll
+                for (int i = 0; i < TN; i++)
+#pragma unroll
+                    for (int j = 0; j < TM; j++)
+                        acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x32_i8(af[i], bf[j], zero, 0, 0, 0);
+                if (!ENDS || kb * 4u + s < a.groups) fold(stage, s);
             }
-            // first MFMA step of a scale group: accumulate onto zero instead of clearing registers
-            const bool fresh = GK == 1 || (GK == 2 && s == 0) || (GK == 4 && s == 0 && (kb & 1u) == 0u);
-            const v4i zero = {0, 0, 0, 0};
+        } else {
 #pragma unroll
-            for (int i = 0; i < TN; i++)
+            for (int s = 0; s < 2; s++) {
+                v4i af[TN], bf[TM];
 #pragma unroll
-                for (int j = 0; j < TM; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[i], bf[j], fresh ? zero : acc[i][j], 0, 0, 0);
-            // last MFMA step of a scale group (or of the row): fold it.  A group that starts past the
-            // end of k does not exist (its dot would be zero, but adding +0.0 can flip a -0.0 sum).
-            if constexpr (GK == 1) {
-                if (kb * 2u + s < a.groups) fold(stage, s);
-            } else if constexpr (GK == 2) {
-                if (s == 1) fold(stage, 0);
-            } else {
-                if (s == 1 && ((kb & 1u) == 1u || kb + 1u == nkb)) fold(stage, 0);
+                for (int j = 0; j < TM; j++) bf[j] = *reinterpret_cast<const v4i*>(stage + x_row + j * 16 * 128 + x_slot[s]);
+#pragma unroll
+                for (int i = 0; i < TN; i++) {
+                    if constexpr (W4) {
+                        const v4i raw = *reinterpret_cast<const v4i*>(stage + a_frag + ((i / 2) * KB + s) * 1024 + (i & 1) * 256);
+#pragma unroll
+                        for (int d = 0; d < 4; d++) af[i][d] = (raw[d] << nib_shift) & (int)0xf0f0f0f0u;
+                    } else {
+                        af[i] = *reinterpret_cast<const v4i*>(stage + a_frag + ((i / 2) * KB + 2 * s) * 1024 + (i & 1) * 256);
+                    }
+                }
+                // first MFMA step of a scale group: accumulate onto zero instead of clearing registers
+                const bool fresh = GK == 1 || (GK == 2 && s == 0) || (GK == 4 && s == 0 && (kb & 1u) == 0u);
+#pragma unroll
+                for (int i = 0; i < TN; i++)
+#pragma unroll
+                    for (int j = 0; j < TM; j++)
+                        acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af[i], bf[j], fresh ? zero : acc[i][j], 0, 0, 0);
+                // last MFMA step of a scale group (or of the row): fold it.  A group that starts past the
+                // end of k does not exist (its dot would be zero, but adding +0.0 can flip a -0.0 sum).
+                if constexpr (GK == 1) {
+                    if (!ENDS || kb * 2u + s < a.groups) fold(stage, s);
+                } else if constexpr (GK == 2) {
+                    if (s == 1) fold(stage, 0);
+                } else {
+                    if (s == 1 && ((kb & 1u) == 1u || (ENDS && kb + 1u == nkb))) fold(stage, 0);
+                }
             }
         }
         refill = cur;
         cur = cur + 1 == NS ? 0 : cur + 1;
+    };
+    // (narrow wave tiles take the last k-block by itself, so that nothing in the others is conditional; the wide
+    // ones would spill)
+    constexpr bool PEEL = TN * TM <= 4;
+    uint32_t kb = 0;
+    if constexpr (PEEL) {
+        for (; kb + 1u < nkb; kb++) k_block(kb, std::false_type{});
     }
+    for (; kb < nkb; kb++) k_block(kb, std::true_type{});
     wait_vmcnt<0>();
 
     // ---- epilogue: + bias, 16-byte stores (a lane owns row l%16 and four consecutive channels) ----
@@ -543,27 +599,13 @@ __global__ __launch_bounds__(WM * 128, 4) void gemm_k64_f32_kernel(const GemmPar
     }
 }
 
-template <int GK, bool W4, int WM, int NS, bool UNI>
-bool launch_f32_as(hipStream_t s, const LinearArgs& a);
-
-template <int GK, bool W4, int WM, int NS>
-bool launch_f32(hipStream_t s, const LinearArgs& a) {
-    // (the instances listed keep the products in registers without spilling at four waves per SIMD;
-    // the others would lose more to scratch traffic than the fourth operation costs)
-    constexpr bool kUniformFits = GK == 1 || (GK == 2 && (W4 || WM == 8));
-    if constexpr (kUniformFits) {
-        if (a.uniform_group_scales) return launch_f32_as<GK, W4, WM, NS, true>(s, a);
-    }
-    return launch_f32_as<GK, W4, WM, NS, false>(s, a);
-}
-
-template <int GK, bool W4, int WM, int NS, bool UNI>
+template <int GK, bool W4, int WN, int WM, int TN, int TM, int NS, bool UNI>
 bool launch_f32_as(hipStream_t s, const LinearArgs& a) {
-    constexpr int BN = 128, BM = WM * 32;
-    constexpr int LDS = NS * (((BN / 32) * (W4 ? 2 : 4) + BM / 8) * 1024 + (GK == 1 ? 2 : 1) * BN * 4);
+    constexpr int BN = WN * TN * 16, BM = WM * TM * 16, GPB = GK == 0 ? 4 : GK == 1 ? 2 : 1;
+    constexpr int LDS = NS * (((BN / 32) * (W4 ? 2 : 4) + BM / 8) * 1024 + (UNI ? 0 : (GPB * BN + 63) / 64 * 256));
     static_assert(LDS <= 160 * 1024, "stages do not fit the LDS");
     static std::atomic<uint64_t> configured{0};
-    auto kern = gemm_k64_f32_kernel<GK, W4, WM, NS, UNI>;
+    auto kern = gemm_k64_f32_kernel<GK, W4, WN, WM, TN, TM, NS, UNI>;
     if (!raise_lds_limit((const void*)kern, LDS, configured)) return false;
     GemmParams p;
     p.a = a;
@@ -571,8 +613,39 @@ bool launch_f32_as(hipStream_t s, const LinearArgs& a) {
     p.tiles_m = (a.rows + BM - 1) / BM;
     const uint32_t total = p.tiles_n * p.tiles_m;
     const uint32_t grid = ((total + 7u) / 8u) * 8u;
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(WM * 128), LDS, s, p);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(WN * WM * 64), LDS, s, p);
     return hipGetLastError() == hipSuccess;
+}
+
+template <int GK, bool W4, int WN, int WM, int TN, int TM, int NS>
+bool launch_f32(hipStream_t s, const LinearArgs& a) {
+    // (the instances listed keep the products in registers without spilling at four waves per SIMD;
+    // the others would lose more to scratch traffic than the fourth operation costs)
+    constexpr bool kUniformFits = TN * TM <= 4 || GK == 1 || (GK == 2 && (W4 || WM == 8));
+    if constexpr (kUniformFits) {
+        if (a.uniform_group_scales) return launch_f32_as<GK, W4, WN, WM, TN, TM, NS, true>(s, a);
+    }
+    return launch_f32_as<GK, W4, WN, WM, TN, TM, NS, false>(s, a);
+}
+
+template <bool W4, int WN, int WM, int TN, int TM, int NS>
+bool launch_f32_group(hipStream_t s, const LinearArgs& a) {
+    switch (a.group_size) {
+        case 32:
+            // (only narrow wave tiles: the wide ones have no registers left)
+            if constexpr (TN * TM <= 4) return launch_f32<0, W4, WN, WM, TN, TM, NS>(s, a);
+            else return false;
+        case 64: return launch_f32<1, W4, WN, WM, TN, TM, NS>(s, a);
+        case 128: return launch_f32<2, W4, WN, WM, TN, TM, NS>(s, a);
+        case 256: return launch_f32<4, W4, WN, WM, TN, TM, NS>(s, a);
+        default: return false;
+    }
+}
+
+template <int WN, int WM, int TN, int TM, int NS>
+bool launch_f32_bits(hipStream_t s, const LinearArgs& a) {
+    return a.weight_bits == 4u ? launch_f32_group<true, WN, WM, TN, TM, NS>(s, a)
+                               : launch_f32_group<false, WN, WM, TN, TM, NS>(s, a);
 }
 
 template <int WN, int WM, int TN, int TM, int MODE, bool FLIP = false, bool DQ = false>
@@ -621,36 +694,50 @@ const char* launch_gemm_k64(hipStream_t s, const LinearArgs& a, int tile) {
     return tile == 0 ? (dq ? "t256x256k64-dq" : "t256x256k64") : (dq ? "t256x128k64-dq" : "t256x128k64");
 }
 
-// The dequantizing GEMM on 16x16x64 MFMAs; group sizes 64, 128 and 256.  deep: one workgroup of
-// sixteen waves per compute unit on a 128 x 256 tile with three LDS stages (eight-bit weights only),
-// else two workgroups of eight waves on 128 x 128 tiles with two stages each.
-const char* launch_gemm_k64_f32(hipStream_t s, const LinearArgs& a, bool deep) {
+// The dequantizing GEMM on 16x16x64 MFMAs (16x16x32 for groups of 32, on the three narrow tiles only).
+const char* launch_gemm_k64_f32(hipStream_t s, const LinearArgs& a, F32Tile tile) {
     if (a.mode != Epilogue::DequantF32 || a.acc_out || !a.y) return nullptr;
-    bool ok = false;
-    if (a.weight_bits == 4u) {
-        deep = false;
-        switch (a.group_size) {
-            case 64: ok = launch_f32<1, true, 4, 2>(s, a); break;
-            case 128: ok = launch_f32<2, true, 4, 2>(s, a); break;
-            case 256: ok = launch_f32<4, true, 4, 2>(s, a); break;
-            default: return nullptr;
-        }
-    } else if (deep) {
-        switch (a.group_size) {
-            case 64: ok = launch_f32<1, false, 8, 3>(s, a); break;
-            case 128: ok = launch_f32<2, false, 8, 3>(s, a); break;
-            case 256: ok = launch_f32<4, false, 8, 3>(s, a); break;
-            default: return nullptr;
-        }
-    } else {
-        switch (a.group_size) {
-            case 64: ok = launch_f32<1, false, 4, 2>(s, a); break;
-            case 128: ok = launch_f32<2, false, 4, 2>(s, a); break;
-            case 256: ok = launch_f32<4, false, 4, 2>(s, a); break;
-            default: return nullptr;
-        }
+    switch (tile) {
+        case F32Tile::T128x256: return launch_f32_group<false, 2, 8, 4, 2, 3>(s, a) ? "t128x256k64s3" : nullptr;
+        case F32Tile::T128x128: return launch_f32_bits<2, 4, 4, 2, 2>(s, a) ? "t128x128k64" : nullptr;
+        case F32Tile::T64x64: return launch_f32_bits<2, 2, 2, 2, 3>(s, a) ? "t64x64k64" : nullptr;
+        case F32Tile::T64x32: return launch_f32_bits<2, 2, 2, 1, 4>(s, a) ? "t64x32k64" : nullptr;
+        case F32Tile::T32x32: return launch_f32_bits<2, 2, 1, 1, 4>(s, a) ? "t32x32k64" : nullptr;
     }
-    return !ok ? nullptr : deep ? "t128x256k64s3" : "t128x128k64";
+    return nullptr;
+}
+
+// Which tile.  Few rows or channels: the narrow tiles, which put the outputs on more wavefronts -- a wavefront
+// walks all of K with a barrier, the fragments and a fold per group in its way, so what counts first is that no
+// SIMD is without one, then that it has two.  us with 64x64 | 64x32 | 32x32 tiles, preparation included
+// (and with the 32x32x32 kernels of gemm_mfma.hip that these launches took before):
+//   8 bits, groups of 128   64 x 4096 -> 4096     18.1 | 15.0 | 12.3 (21.6)   200 x 4096 -> 4096   19.8 | 18.2 | 18.4 (23.2)
+//                           512 x 4096 -> 4096    26.2 | 32.2 | 34.9 (32.7)   333 x 3000 -> 5001   22.7 | 27.8 | 27.1 (29.6)
+//                           1000 x 8192 -> 1024   40.2 | 37.2 | 40.7 (46.4)   128 x 3000 -> 5001   16.5 | 15.3 | 13.8 (19.7)
+//   4 bits, groups of 32    64 x 4096 -> 4096     40.8 | 27.1 | 19.1 (54.9)   333 x 3000 -> 5001   41.0 | 40.0 | 39.2 (67.1)
+//                           512 x 4096 -> 4096    52.1 | 51.1 | 54.2 (94.2)   1024 x 3000 -> 5001  82.3 | 88.6 | 94.4 (227)
+// The lines: 1.5 workgroups of a tile per compute unit.
+// Past them the 128-channel tiles against 64x64, by how many a compute unit gets (in units of one 128x128 tile;
+// an odd one of those has no second workgroup to take turns with, four 64x64 tiles cost 1.2 of it -- 1.07 with four-bit
+// weights -- and one 128x256 tile 1.75 where its products fit the registers).  64x64 | 128x128 | 128x256, 8 bits,
+// one scale per channel:
+//   1024 x 3000 -> 5001  43.8 | 52.7         700 x 1024 -> 4096   14.0 | 16.9 | 21.0   4096 x 1024 -> 4096  47.0 | 43.7 | 48.0
+//   333 x 4096 -> 14336  48.9 | 55.9 | 53.4  700 x 4096 -> 14336  77.7 | 81.4 | 89.9   2048 x 14336 -> 4096  211 | 195 | 172
+// 4 bits, groups of 128:  4096 x 2048 -> 1024  33.1 | 36.9   700 x 4096 -> 14336  88.5 | 96.5   2048 x 4096 -> 14336  230 | 214
+F32Tile pick_f32_tile(const LinearArgs& a, int cu_count) {
+    const auto tiles = [&](uint32_t bn, uint32_t bm) { return (uint64_t)((a.n + bn - 1) / bn) * ((a.rows + bm - 1) / bm); };
+    const uint64_t cu = (uint64_t)cu_count, busy = cu * 3 / 2;
+    if (tiles(64, 64) < busy) return tiles(64, 32) < busy ? F32Tile::T32x32 : F32Tile::T64x32;
+    if (a.group_size < 64u) return F32Tile::T64x64;
+    const auto per_cu = [&](uint64_t t) { return (t + cu - 1) / cu; };
+    const uint64_t c128 = per_cu(tiles(128, 128));
+    const float narrow = (float)per_cu(tiles(64, 64)) * (a.weight_bits == 4u ? 0.2675f : 0.3f);
+    const float wide = (float)c128 + (c128 % 2 ? 0.15f : 0.0f);
+    if (a.uniform_group_scales && a.weight_bits == 8u && a.group_size <= 128u && a.k >= 4096u) {
+        const float deep = 1.75f * (float)per_cu(tiles(128, 256));
+        if (deep < wide && deep < narrow) return F32Tile::T128x256;
+    }
+    return narrow < wide ? F32Tile::T64x64 : F32Tile::T128x128;
 }
 
 }  // namespace vxhip

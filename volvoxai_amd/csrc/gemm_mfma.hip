@@ -598,26 +598,22 @@ const char* dispatch_tile(hipStream_t s, const LinearArgs& a, int cu_count, cons
     auto forced = [&](const char* tag) { return force && strstr(force, tag) != nullptr; };
     if constexpr (MODE == (int)Epilogue::DequantF32) {
         // int32 tile accumulators plus f32 running sums: the wave tile is at most 64x64, and with
-        // a scale group per k-step the eight-wave tile runs out of registers.  A wave folds a
-        // group (four VALU operations per output) strictly after that group's MFMAs, so its time
-        // per k-block grows with its tile: few rows or few channels take narrower tiles, which
-        // also puts more workgroups on the device.
+        // a scale group per k-step the eight-wave tile runs out of registers.
         const auto tiles = [&](uint32_t bn, uint32_t bm) {
             return (uint64_t)((a.n + bn - 1) / bn) * ((a.rows + bm - 1) / bm);
         };
         const uint64_t enough = (uint64_t)cu_count * 3 / 4;
         int pick = a.rows <= 64u ? 3 : tiles(128, 256) >= enough && GK > 1 ? 0 : tiles(128, 128) >= enough ? 1
                    : tiles(64, 128) >= enough ? 2 : 3;
-        // Enough 128 x 128 tiles for every compute unit to hold its two workgroups, or most of them: the
-        // 16x16x64 kernel of gemm_k64.hip (group sizes of 64 and more), unless a tile of this file is named.
-        const bool named = forced("t256x") || forced("t128x") || forced("t64x");
-        if (a.group_size >= 64u && (forced("k64") || (!named && tiles(128, 128) >= enough))) {
-            // long rows with one scale per channel: sixteen waves on a 128 x 256 tile, three stages
-            // (K = 14336, N = 4096, 2048 rows: 211 against 232 us; short rows favour the small tile)
-            const bool deep = forced("t128x256k64") || (!forced("k64") && a.uniform_group_scales && a.weight_bits == 8u &&
-                                                        a.group_size <= 128u && a.k >= 4096u && tiles(128, 256) >= enough);
-            const char* t = launch_gemm_k64_f32(s, a, deep);
-            if (t) return t;
+        // The 16x16x64 kernel of gemm_k64.hip, unless a tile of this file is named (or it declines).
+        if (forced("k64") || !(forced("t256x") || forced("t128x") || forced("t64x"))) {
+            const F32Tile tile = forced("t128x256k64") ? (a.weight_bits == 8u ? F32Tile::T128x256 : F32Tile::T128x128)
+                                 : forced("t64x64k64") ? F32Tile::T64x64
+                                 : forced("t64x32k64") ? F32Tile::T64x32
+                                 : forced("t32x32k64") ? F32Tile::T32x32
+                                 : forced("k64")       ? F32Tile::T128x128
+                                                       : pick_f32_tile(a, cu_count);
+            if (const char* t = launch_gemm_k64_f32(s, a, tile)) return t;
         }
         if (forced("t256x256")) pick = GK > 1 ? 0 : 1;
         if (forced("t128x128")) pick = 1;

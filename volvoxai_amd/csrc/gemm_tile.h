@@ -72,6 +72,9 @@ __device__ __forceinline__ TileOrigin tile_of_workgroup(const GemmParams& p) {
 
 // gemm_k64.hip
 const char* launch_gemm_k64(hipStream_t s, const LinearArgs& a, int tile);
-const char* launch_gemm_k64_f32(hipStream_t s, const LinearArgs& a, bool deep);
+enum class F32Tile { T128x256, T128x128, T64x64, T64x32, T32x32 };  // channels x rows
+F32Tile pick_f32_tile(const LinearArgs& a, int cu_count);
+// the tile's name, or null if it does not exist for these weights
+const char* launch_gemm_k64_f32(hipStream_t s, const LinearArgs& a, F32Tile tile);
 
 }  // namespace vxhip
