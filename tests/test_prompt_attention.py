@@ -1,0 +1,77 @@
+"""The matrix-pipe prompt attention (head sizes 64 and 128) at the edges of its tiles: 32 queries a wavefront, 32
+slots a tile, a workgroup's wavefronts on neighbouring tokens (many query blocks, or at most 32 tokens) or sharing
+their queries (few)."""
+import numpy as np
+import pytest
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    import torch
+    import volvoxai_amd as vx
+    c = vx.Context(0, torch.cuda.current_stream())
+    yield c
+    c.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,t,start,q_heads,kv_heads,head_dim,max_seq,order", [
+    (128, 33, 0, 16, 8, 128, 33, "rising"),     # neighbouring tokens: ragged last block and last group of four
+    (64, 97, 7, 16, 16, 64, 111, "rising"),     # the same at head size 64, a full cache but for the last slots
+    (1, 33, 0, 2, 1, 128, 65, "rising"),        # shared queries: a second tile of one slot, wavefronts without a tile
+    (2, 64, 64, 8, 4, 64, 160, "rising"),       # the same at head size 64: whole tiles, a prompt continued
+    (1, 129, 60, 32, 1, 128, 190, "rising"),    # 32 query heads per KV head: one token a wavefront
+    (3, 32, 1, 6, 2, 64, 34, "rising"),         # three heads per KV head: 30 of 32 queries
+    (2, 8, 0, 4, 2, 128, 16, "rising"),         # fewest tokens of the path
+    (2, 45, 3, 4, 2, 128, 60, "shuffled"),      # positions in any order: no wavefront's span follows from its place
+])
+def test_prompt_attention_tiles(ctx, rows, t, start, q_heads, kv_heads, head_dim, max_seq, order):
+    """Against the definition in float64; cache slots no token sees hold NaN.  A score is head_dim products of about
+    unit variance summed in f32 (error about 1e-6), which is the relative error of its probability."""
+    import torch
+    import volvoxai_amd.w8a8 as vx
+    rng = np.random.default_rng(rows * 1000 + t)
+    q = rng.normal(0, 1, (rows, t, q_heads, head_dim)).astype(np.float32)
+    k = rng.normal(0, 1, (rows, kv_heads, max_seq, head_dim)).astype(np.float32)
+    v = rng.normal(0, 1, (rows, kv_heads, max_seq, head_dim)).astype(np.float32)
+    positions = np.arange(start, start + t, dtype=np.int64)
+    if order == "shuffled":
+        positions = rng.permutation(positions)
+    k[:, :, start + t:] = np.nan
+    v[:, :, start + t:] = np.nan
+    k[0, 0, start + 2, :] *= 40.0  # one slot takes most of the weight: the running maximum jumps
+    out = vx.gqa_attention(ctx, *(torch.from_numpy(a).cuda() for a in (q, k, v, positions)))
+    ctx.synchronize()
+    got = out.cpu().numpy().reshape(rows, t, q_heads, head_dim)
+    seen, rep = start + t, q_heads // kv_heads
+    hidden = np.arange(seen)[None, :] > positions[:, None]
+    for h in range(q_heads):
+        kk, vv = (a[:, h // rep, :seen].astype(np.float64) for a in (k, v))
+        sc = np.matmul(q[:, :, h].astype(np.float64), kk.transpose(0, 2, 1)) / np.sqrt(head_dim)
+        sc[:, hidden] = -np.inf
+        p = np.exp(sc - sc.max(-1, keepdims=True))
+        p /= p.sum(-1, keepdims=True)
+        # (a score of the strong slot is up to about 200: its f32 rounding is 1e-5 of a probability)
+        assert np.allclose(got[:, :, h], np.matmul(p, vv), rtol=2e-5, atol=1e-4 if h < rep else 5e-6), h
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("head_dim,t", [(128, 20), (128, 70), (64, 70)])
+def test_prompt_attention_of_infinite_scores(ctx, head_dim, t):
+    """Scores of -inf count nothing, also where a whole first tile has no other; a NaN or +inf score makes its row NaN."""
+    import torch
+    import volvoxai_amd.w8a8 as vx
+    rng = np.random.default_rng(t)
+    q = np.ones((1, t, 1, head_dim), np.float32)
+    k = np.zeros((1, 1, 96, head_dim), np.float32)
+    v = rng.normal(0, 1, (1, 1, 96, head_dim)).astype(np.float32)
+    low, bad = (32, 50) if t > 60 else (5, 12)
+    k[0, 0, :low, 0] = -np.inf
+    k[0, 0, bad, 0] = np.inf
+    positions = np.arange(t, dtype=np.int64)
+    out = vx.gqa_attention(ctx, *(torch.from_numpy(a).cuda() for a in (q, k, v, positions)))
+    ctx.synchronize()
+    got = out.cpu().numpy().reshape(t, head_dim)
+    assert np.isnan(got[:low]).all() and np.isnan(got[bad:]).all()  # (nothing but -inf: 0 / 0, as exp(-inf + inf) gives)
+    for i in range(low, bad):
+        assert np.allclose(got[i], v[0, 0, low:i + 1].astype(np.float64).mean(0), rtol=1e-5, atol=1e-6), i

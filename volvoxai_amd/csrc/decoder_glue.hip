@@ -10,6 +10,7 @@
 // All are row-sized, latency-bound kernels; none of them is on the int8 roofline.
 #include "common.h"
 #include "device_math.h"
+#include "gemm_tile.h"
 #include "row_math.h"
 #include "wave_ops.h"
 
@@ -642,171 +643,232 @@ __global__ __launch_bounds__(256) void gqa_prefill_kernel(const float* __restric
     }
 }
 
-// The same prompt attention for head size 128 on the f32 matrix pipes (v_mfma_f32_32x32x2f32: full
-// f32 products and sums, not a reduced-precision format).  The queries of a workgroup are the 32
-// rows of the A operand and stay in registers for the whole kernel: lane l holds query l % 32 and,
-// for the scores, 32 of its 128 channels.  Per 64-slot block:
-//   scores  wavefront w takes slots 32 * (w & 1) .. +31 and channels 64 * (w >> 1) .. +63: 32 MFMAs,
-//           each adding the channel pair (c, c + 32) of the lane halves; the two channel halves of
-//           a slot tile are added through the score rows in LDS (one stores, one adds and scales)
-//   P.V     wavefront w takes output channels 32 * w .. +31: 32 MFMAs, each adding the slot pair
-//           (s, s + 32); the sums stay in 16 accumulator registers across the blocks
-// Softmax and staging are those of the kernel above.  A workgroup's score rows are always 32.
-// (The kernel above reads its queries through the scalar cache, which two workgroups per compute
-// unit overflow: 189 us per launch of a 32-row, 128-token prompt against 102 us here.)
+// The same prompt attention for head sizes 64 and 128 on the f32 matrix pipes (v_mfma_f32_32x32x2f32:
+// full f32 products and sums, not a reduced-precision format), every wavefront by itself: no LDS stage,
+// no barrier, nothing but matrix instructions with loads between them.  A wavefront takes `tq`
+// consecutive tokens of one row and the query heads of one KV head, up to 32 queries, and walks the
+// visible slots 32 at a time with a running maximum and sum (softmax rescaled as the maximum grows).
+// Lane l is r = l % 32, h = l / 32:
+//   scores  transposed, keys as the A operand: MFMA (j, e) adds channels 8j + e (h = 0) and 8j + 4 + e
+//           (h = 1) of key row r and query r, so lane l ends with query r's scores of the 16 slots
+//           8 * (v / 4) + 4h + v % 4
+//   P.V     transposed, values as the A operand: MFMA v adds just those two slots (one per h), so the
+//           probabilities are the B operand from the registers where they already are.  Row r of
+//           channel tile c is channel VW * r + c (VW = head size / 32): a value load is VW consecutive
+//           floats a lane, and the output leaves the same way.
+// Bound by the matrix pipes (128 MFMAs of 64 cycles per 32 slots and 128 channels: 17 us for 32 prompts of
+// 128 tokens, 16 query and 8 KV heads) and by 100 MB of queries, cache and outputs (20 us); measured 43 us.
+// With keys and values staged through LDS by four wavefronts and the scores kept there, three barriers per
+// 64 slots, the same launch took 99.7 us; heads of 64 on the vector kernel above 76.6, here 17.2.  The loads are a ring of RING 16-byte
+// registers, RING * 256 cycles of MFMAs ahead of their use; the fence behind each refill keeps the
+// scheduler from collecting them.
+// SPLIT wavefronts of a workgroup share their queries and take the 32-slot tiles in turn, then merge
+// their sums through LDS; 1: the four take the queries of four neighbouring token blocks.
 typedef float v16f __attribute__((ext_vector_type(16)));
 
-__global__ __launch_bounds__(256) void gqa_prefill_mfma_kernel(const float* __restrict__ q,
-                                                               const float* __restrict__ k_cache,
-                                                               const float* __restrict__ v_cache,
-                                                               const int64_t* __restrict__ positions, uint32_t t,
-                                                               uint32_t tq, uint32_t q_heads, uint32_t kv_heads,
-                                                               uint32_t max_seq, float scale, float* __restrict__ out,
-                                                               uint32_t* __restrict__ fault) {
-    constexpr uint32_t HD = 128u, HD4 = HD / 4u, PITCH = HD + 4u;
-    __shared__ uint32_t visible[kPrefillQueries];
-    const uint32_t rep = q_heads / kv_heads, qw = tq * rep;
-    const uint32_t blocks = (t + tq - 1u) / tq;
-    const uint32_t row = blockIdx.x / blocks, i0 = (blockIdx.x % blocks) * tq, kvh = blockIdx.y;
-    const uint32_t score_pitch = (max_seq + 63u) & ~63u;
-    float* sc = reinterpret_cast<float*>(glue_lds);             // [32][score_pitch]
-    float* stage = sc + (size_t)kPrefillQueries * score_pitch;  // [64][PITCH]
-    const float* kbase = k_cache + ((size_t)row * kv_heads + kvh) * max_seq * HD;
-    const float* vbase = v_cache + ((size_t)row * kv_heads + kvh) * max_seq * HD;
+template <int HD, int SPLIT>
+__global__ __launch_bounds__(256, 2) void gqa_prefill_mfma_kernel(const float* __restrict__ q,
+                                                                  const float* __restrict__ k_cache,
+                                                                  const float* __restrict__ v_cache,
+                                                                  const int64_t* __restrict__ positions, uint32_t rows,
+                                                                  uint32_t t, uint32_t tq, uint32_t q_heads,
+                                                                  uint32_t kv_heads, uint32_t max_seq, float scale,
+                                                                  float* __restrict__ out, uint32_t* __restrict__ fault) {
+    static_assert((HD == 64 || HD == 128) && (SPLIT == 1 || SPLIT == 4), "see the launch");
+    constexpr int RING = 8, KE = HD / 8, VE = HD / 8, VW = HD / 32;  // 16-byte loads of keys and values per tile
+    static_assert((KE + VE) % RING == 0 && RING <= KE, "a ring register keeps its place from tile to tile");
+    typedef float out_vec __attribute__((ext_vector_type(VW), aligned(4)));  // (`out` may start at any float)
     const uint32_t lane = threadIdx.x & 63u, r = lane & 31u, h = lane >> 5;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    auto token_of = [&](uint32_t qi) { return i0 + qi / rep; };
-    auto head_of = [&](uint32_t qi) { return kvh * rep + qi % rep; };
-
-    if (threadIdx.x < kPrefillQueries) {
-        const uint32_t qi = threadIdx.x;
-        uint32_t v = 0u;
-        if (qi < qw && token_of(qi) < t) {
-            const uint64_t named = (uint64_t)positions[token_of(qi)];
-            if (named >= max_seq) atomicOr(fault, (uint32_t)kFaultBadPosition);  // (its output row is left as it is)
-            else v = (uint32_t)named + 1u;
-        }
-        visible[qi] = v;
+    const uint32_t rep = q_heads / kv_heads, qw = tq * rep, blocks = (t + tq - 1u) / tq;
+    // The workgroups of the last tokens, which see the most slots, come first, and every other one has
+    // its wavefronts in reverse: a SIMD that holds one of the long and one of the short ones is even.
+    const uint32_t pairs = rows * kv_heads, pair = blockIdx.x % pairs, turn = blockIdx.x / pairs;
+    const uint32_t row = pair / kv_heads, kvh = pair % kv_heads;
+    uint32_t block;
+    if constexpr (SPLIT > 1) {
+        block = blocks - 1u - turn;
+    } else {
+        const uint32_t from_end = turn * 4u + ((turn & 1u) ? 3u - wave : wave);
+        if (from_end >= blocks) return;
+        block = blocks - 1u - from_end;
     }
-    // this lane's 32 channels of query r for the scores (zeros for a query that does not exist)
-    const uint32_t score_channel = 64u * (wave >> 1) + 32u * h;
-    float qreg[32];
+    const float* kbase = k_cache + ((size_t)row * kv_heads + kvh) * max_seq * HD;
+    const float* vbase = v_cache + ((size_t)row * kv_heads + kvh) * max_seq * HD;
+
+    const uint32_t token = block * tq + r / rep, head = kvh * rep + r % rep;
+    const bool exists = r < qw && token < t;
+    uint32_t visible = 0u;  // slots query r may see
+    if (exists) {
+        const uint64_t named = (uint64_t)positions[token];
+        if (named >= max_seq) atomicOr(fault, (uint32_t)kFaultBadPosition);  // (its output row is left as it is)
+        else visible = (uint32_t)named + 1u;
+    }
+    uint32_t span = visible;
+#pragma unroll
+    for (int d = 1; d < 32; d <<= 1) span = max(span, (uint32_t)__shfl_xor((int)span, d));
+    span = __builtin_amdgcn_readfirstlane(span);
+    if (span == 0u) return;  // (the same in every wavefront that shares these queries)
+
+    float4 qreg[KE];  // channels 8j + 4h .. +3 of query r (zeros for a query that does not exist)
     {
-        const bool exists = r < qw && token_of(r) < t;
-        const float* src = q + ((size_t)(row * t + (exists ? token_of(r) : 0u)) * q_heads + head_of(exists ? r : 0u)) * HD +
-                           score_channel;
+        const float* src = q + ((size_t)(row * t + (exists ? token : 0u)) * q_heads + (exists ? head : 0u)) * HD + 4u * h;
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const float4 v = exists ? *reinterpret_cast<const float4*>(src + 4 * j) : make_float4(0.f, 0.f, 0.f, 0.f);
-            qreg[4 * j] = v.x, qreg[4 * j + 1] = v.y, qreg[4 * j + 2] = v.z, qreg[4 * j + 3] = v.w;
-        }
+        for (int j = 0; j < KE; j++)
+            qreg[j] = exists ? *reinterpret_cast<const float4*>(src + 8 * j) : make_float4(0.f, 0.f, 0.f, 0.f);
     }
-    __syncthreads();
-    uint32_t span = 0u;
-    for (uint32_t qi = 0; qi < qw; qi++) span = max(span, visible[qi]);
-    const uint32_t span_blocks = (span + kPrefillSlots - 1u) / kPrefillSlots * kPrefillSlots;
-
-    constexpr int kStageRegs = 8;  // 64 rows x 128 floats over 256 threads, as 16-byte words
-    auto fetch_rows = [&](const float* base, uint32_t s0, float4 (&v)[kStageRegs]) {
-#pragma unroll
-        for (int u = 0; u < kStageRegs; u++) {
-            const uint32_t e = threadIdx.x + u * 256u, srow = s0 + e / HD4;
-            v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (srow < span) v[u] = *reinterpret_cast<const float4*>(base + (size_t)srow * HD + 4u * (e % HD4));
+    // Load e of the tile at s0: key chunks first, then value slots.  Slots past the span repeat its last
+    // (their probabilities are zero, and what the cache holds there is nobody's).
+    float4 ring[RING];
+    auto fetch = [&](auto e_tag, uint32_t s0) {
+        constexpr int e = decltype(e_tag)::value;
+        if constexpr (e < KE) {
+            ring[e % RING] = *reinterpret_cast<const float4*>(kbase + (size_t)min(s0 + r, span - 1u) * HD + 8 * e + 4u * h);
+        } else if constexpr (VW == 4) {
+            constexpr int v = e - KE;
+            const uint32_t slot = min(s0 + 8u * (v / 4) + 4u * h + v % 4, span - 1u);
+            ring[e % RING] = *reinterpret_cast<const float4*>(vbase + (size_t)slot * HD + 4u * r);
+        } else {
+            constexpr int v = 2 * (e - KE);
+            const uint32_t slot = s0 + 8u * (v / 4) + 4u * h + v % 4;
+            const float2 a = *reinterpret_cast<const float2*>(vbase + (size_t)min(slot, span - 1u) * HD + 2u * r);
+            const float2 b = *reinterpret_cast<const float2*>(vbase + (size_t)min(slot + 1u, span - 1u) * HD + 2u * r);
+            ring[e % RING] = make_float4(a.x, a.y, b.x, b.y);
         }
     };
-    auto commit_rows = [&](const float4 (&v)[kStageRegs]) {
-#pragma unroll
-        for (int u = 0; u < kStageRegs; u++) {
-            const uint32_t e = threadIdx.x + u * 256u;
-            *reinterpret_cast<float4*>(stage + (size_t)(e / HD4) * PITCH + 4u * (e % HD4)) = v[u];
-        }
-    };
-    float4 ahead[kStageRegs];
-    fetch_rows(kbase, 0u, ahead);
+    constexpr uint32_t STEP = 32u * SPLIT;
+    const uint32_t first = SPLIT > 1 ? 32u * wave : 0u;
+    static_for<RING>([&](auto e_tag) { fetch(e_tag, first); });
 
-    // The 16 accumulator registers of a lane are rows 8 * (v / 4) + 4 * h + v % 4 of column r.
-    auto tile_row = [&](int v) { return 8u * (uint32_t)(v / 4) + 4u * h + (uint32_t)(v % 4); };
+    float m = -INFINITY, sum = 0.0f;  // of query r, the same in both lanes that hold it
+    v16f o[VW];
+#pragma unroll
+    for (int c = 0; c < VW; c++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) o[c][v] = 0.0f;
+    for (uint32_t s0 = first; s0 < span; s0 += STEP) {
+        auto refill = [&](auto e_tag) {  // the ring register of load e takes load e + RING
+            constexpr int e = decltype(e_tag)::value + RING;
+            if constexpr (e < KE + VE) fetch(IC<e>{}, s0);
+            else fetch(IC<e - KE - VE>{}, s0 + STEP);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        v16f s;
+#pragma unroll
+        for (int v = 0; v < 16; v++) s[v] = 0.0f;
+        static_for<KE>([&](auto e_tag) {
+            constexpr int e = decltype(e_tag)::value;
+            const float4 kv = ring[e % RING];
+            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.x, qreg[e].x, s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.y, qreg[e].y, s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.z, qreg[e].z, s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.w, qreg[e].w, s, 0, 0, 0);
+            refill(e_tag);
+        });
+        auto both_halves = [&](float x) {  // the values of the two lanes that hold a query
+            return __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+        };
+        float top = -INFINITY;
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+            const uint32_t slot = s0 + 8u * (v / 4) + 4u * h + v % 4;
+            s[v] = slot < visible ? __fmul_rn(s[v], scale) : -INFINITY;
+            top = fmaxf(top, s[v]);
+        }
+        const auto tops = both_halves(top);
+        const float grown = fmaxf(m, fmaxf(__uint_as_float(tops[0]), __uint_as_float(tops[1])));
+        // (nothing visible yet, or only scores of -inf: any finite reference gives zeros)
+        const float reference = grown == -INFINITY ? 0.0f : grown;
+        const float keep = expf(m - reference);
+        m = grown;
+        float part = 0.0f;
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+            // (a slot that is not visible counts nothing, also beside a score that makes the reference NaN or infinite)
+            const uint32_t slot = s0 + 8u * (v / 4) + 4u * h + v % 4;
+            s[v] = slot < visible ? expf(s[v] - reference) : 0.0f;
+            part += s[v];
+        }
+        const auto parts = both_halves(part);
+        sum = __builtin_fmaf(sum, keep, __uint_as_float(parts[0]) + __uint_as_float(parts[1]));
+#pragma unroll
+        for (int c = 0; c < VW; c++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) o[c][v] *= keep;
+        static_for<VE>([&](auto e_tag) {
+            constexpr int e = decltype(e_tag)::value;
+            const float4 vv = ring[(KE + e) % RING];
+            if constexpr (VW == 4) {
+                o[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.x, s[e], o[0], 0, 0, 0);
+                o[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.y, s[e], o[1], 0, 0, 0);
+                o[2] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.z, s[e], o[2], 0, 0, 0);
+                o[3] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.w, s[e], o[3], 0, 0, 0);
+            } else {
+                o[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.x, s[2 * e], o[0], 0, 0, 0);
+                o[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.y, s[2 * e], o[1], 0, 0, 0);
+                o[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.z, s[2 * e + 1], o[0], 0, 0, 0);
+                o[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.w, s[2 * e + 1], o[1], 0, 0, 0);
+            }
+            refill(IC<KE + e>{});
+        });
+    }
 
-    for (uint32_t s0 = 0; s0 < span; s0 += kPrefillSlots) {  // scores
-        commit_rows(ahead);
-        __syncthreads();
-        if (s0 + kPrefillSlots < span) fetch_rows(kbase, s0 + kPrefillSlots, ahead);
-        else fetch_rows(vbase, 0u, ahead);
-        const uint32_t slot_tile = 32u * (wave & 1u);
-        const float* krow = stage + (size_t)(slot_tile + r) * PITCH + score_channel;
-        v16f acc;
+    float* dst = out + ((size_t)(row * t + token) * q_heads + head) * HD;
+    if constexpr (SPLIT == 1) {
+        if (visible == 0u) return;
 #pragma unroll
-        for (int v = 0; v < 16; v++) acc[v] = 0.0f;
+        for (int v = 0; v < 16; v++) {
+            out_vec y;
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const float4 kv = *reinterpret_cast<const float4*>(krow + 4 * j);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(qreg[4 * j], kv.x, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(qreg[4 * j + 1], kv.y, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(qreg[4 * j + 2], kv.z, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(qreg[4 * j + 3], kv.w, acc, 0, 0, 0);
+            for (int c = 0; c < VW; c++) y[c] = __fdiv_rn(o[c][v], sum);
+            *reinterpret_cast<out_vec*>(dst + VW * (8u * (v / 4) + 4u * h + v % 4)) = y;
         }
-        float* tile = sc + s0 + slot_tile + r;  // + query * score_pitch
-        if ((wave >> 1) == 0u) {
+    } else {
+        // [wavefront][2 + 16 * VW][64]: maximum, sum, then the outputs; wavefront w merges the registers
+        // 4w .. 4w + 3 of every channel tile
+        constexpr uint32_t PART = (2u + 16u * VW) * 64u;
+        float* mine = reinterpret_cast<float*>(glue_lds) + wave * PART + lane;
+        mine[0] = m;
+        mine[64] = sum;
 #pragma unroll
-            for (int v = 0; v < 16; v++) tile[(size_t)tile_row(v) * score_pitch] = acc[v];
-        }
+        for (int c = 0; c < VW; c++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) mine[(2 + v * VW + c) * 64] = o[c][v];
         __syncthreads();
-        if ((wave >> 1) == 1u) {
+        const float* parts = reinterpret_cast<const float*>(glue_lds) + lane;
+        float top = -INFINITY, weight[SPLIT], total = 0.0f;
 #pragma unroll
-            for (int v = 0; v < 16; v++) {
-                float* at = tile + (size_t)tile_row(v) * score_pitch;
-                *at = __fmul_rn(__fadd_rn(*at, acc[v]), scale);
+        for (int w = 0; w < SPLIT; w++) top = fmaxf(top, parts[w * PART]);
+        const float reference = top == -INFINITY ? 0.0f : top;
+#pragma unroll
+        for (int w = 0; w < SPLIT; w++) {
+            weight[w] = expf(parts[w * PART] - reference);
+            total = __builtin_fmaf(parts[w * PART + 64], weight[w], total);
+        }
+        if (visible == 0u) return;
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            out_vec y;
+#pragma unroll
+            for (int c = 0; c < VW; c++) {
+                float x = 0.0f;
+#pragma unroll
+                for (int w = 0; w < SPLIT; w++)
+                    x = __builtin_fmaf(parts[w * PART + (2u + (4u * wave + u) * VW + c) * 64u], weight[w], x);
+                y[c] = __fdiv_rn(x, total);
             }
-        }
-        __syncthreads();
-    }
-    {   // softmax: probabilities over the visible slots, zeros from there to the end of the last block
-        for (uint32_t qi = wave; qi < kPrefillQueries; qi += 4u) {
-            float* mine = sc + (size_t)qi * score_pitch;
-            const uint32_t seen = qi < qw ? visible[qi] : 0u;
-            if (seen != 0u) {
-                float m = -INFINITY;
-                for (uint32_t s = lane; s < seen; s += 64u) m = fmaxf(m, mine[s]);
-                m = wave_max(m);
-                float sum = 0.0f;
-                for (uint32_t s = lane; s < seen; s += 64u) {
-                    const float e = expf(mine[s] - m);
-                    mine[s] = e;
-                    sum += e;
-                }
-                sum = wave_sum(sum);
-                for (uint32_t s = lane; s < seen; s += 64u) mine[s] = __fdiv_rn(mine[s], sum);
-            }
-            for (uint32_t s = seen + lane; s < span_blocks; s += 64u) mine[s] = 0.0f;
+            *reinterpret_cast<out_vec*>(dst + VW * (8u * wave + 4u * h + u)) = y;
         }
     }
-    __syncthreads();
-    v16f o;
-#pragma unroll
-    for (int v = 0; v < 16; v++) o[v] = 0.0f;
-    for (uint32_t s0 = 0; s0 < span; s0 += kPrefillSlots) {  // P.V
-        commit_rows(ahead);
-        __syncthreads();
-        if (s0 + kPrefillSlots < span) fetch_rows(vbase, s0 + kPrefillSlots, ahead);
-        const float* prow = sc + (size_t)r * score_pitch + s0 + 32u * h;      // probabilities of query r
-        const float* vcol = stage + (size_t)(32u * h) * PITCH + 32u * wave + r;  // channel 32 * wave + r
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const float4 pv = *reinterpret_cast<const float4*>(prow + 4 * j);
-            o = __builtin_amdgcn_mfma_f32_32x32x2f32(pv.x, vcol[(size_t)(4 * j) * PITCH], o, 0, 0, 0);
-            o = __builtin_amdgcn_mfma_f32_32x32x2f32(pv.y, vcol[(size_t)(4 * j + 1) * PITCH], o, 0, 0, 0);
-            o = __builtin_amdgcn_mfma_f32_32x32x2f32(pv.z, vcol[(size_t)(4 * j + 2) * PITCH], o, 0, 0, 0);
-            o = __builtin_amdgcn_mfma_f32_32x32x2f32(pv.w, vcol[(size_t)(4 * j + 3) * PITCH], o, 0, 0, 0);
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int v = 0; v < 16; v++) {
-        const uint32_t qi = tile_row(v);
-        if (qi >= qw || token_of(qi) >= t || visible[qi] == 0u) continue;
-        out[((size_t)(row * t + token_of(qi)) * q_heads + head_of(qi)) * HD + 32u * wave + r] = o[v];
-    }
+}
+
+// Whether the wavefronts of a workgroup share their queries and split the slots (see the kernel above): while
+// the launch has not one wavefront for every SIMD, and more than one tile to split.  Measured, shared against
+// apart (16 query / 8 KV heads of 128): 128 tokens of 1 row 10.6 / 24.6 us, of 8 rows (512 query blocks)
+// 18.5 / 26.3, of 16 rows (1024) 33.1 / 28.2, of 32 rows 55.9 / 43.0; 190 tokens of 8 rows (768) 34.1 / 36.0;
+// 64 tokens of 16 rows (512) 17.9 / 17.0.  Heads of 64, 128 tokens: 512 blocks 11.6 / 16.4, 1024 20.1 / 17.2.
+bool split_prompt_slots(uint32_t query_blocks, uint32_t t, int compute_units) {
+    return t > 32u && query_blocks < 4u * (uint32_t)(compute_units > 0 ? compute_units : 256);
 }
 
 // Query heads that share a workgroup (and with it every key and value row of their KV head):
@@ -1025,24 +1087,30 @@ VxHipStatus vxhip_gqa_attention(VxHipContext* ctx, const float* q_dev, const flo
     if (!device_ready(ctx)) return VXHIP_BACKEND_UNAVAILABLE;
     const float scale = (float)(1.0 / sqrt((double)head_dim));
     const uint32_t rep = q_heads / kv_heads;
-    if (t >= 8u && rep <= kPrefillQueries && head_dim == 128u) {
-        // a prompt at head size 128: the matrix-pipe kernel, if its 32 score rows fit
-        const size_t lds = ((size_t)kPrefillQueries * ((max_seq + 63u) & ~63u) + (size_t)kPrefillSlots * (128u + 4u)) *
-                           sizeof(float);
-        if (lds <= 150u * 1024u) {
-            static std::atomic<uint64_t> configured{0};
-            if (!raise_lds_limit((const void*)gqa_prefill_mfma_kernel, 152 * 1024, configured)) {
-                set_error("gqa_attention: the prompt kernel's LDS limit could not be raised");
-                return VXHIP_EXECUTION_FAILED;
-            }
-            const uint32_t tq = kPrefillQueries / rep;
-            const dim3 grid(rows * ((t + tq - 1u) / tq), kv_heads);
-            hipLaunchKernelGGL(gqa_prefill_mfma_kernel, grid, dim3(256), lds, ctx->stream, q_dev, k_cache_dev,
-                               v_cache_dev, positions_dev, t, tq, q_heads, kv_heads, max_seq, scale, out_dev,
-                               ctx->fault_dev);
-            VXHIP_TRY(hipGetLastError());
-            return VXHIP_OK;
-        }
+    if (t >= 8u && rep <= kPrefillQueries && (head_dim == 128u || head_dim == 64u)) {
+        // a prompt at the common head sizes: the matrix-pipe kernel
+        const uint32_t tq = kPrefillQueries / rep, blocks = (t + tq - 1u) / tq, pairs = rows * kv_heads;
+        const bool split = split_prompt_slots(pairs * blocks, t, ctx->cu_count);
+        const uint32_t grid = pairs * (split ? blocks : (blocks + 3u) / 4u);
+        const size_t lds = split ? 4u * (2u + head_dim / 2u) * 64u * sizeof(float) : 0u;
+#define VXHIP_PROMPT(HD, SPLIT)                                                                                       \
+    do {                                                                                                              \
+        static std::atomic<uint64_t> configured{0};                                                                   \
+        if (lds > 64u * 1024u && !raise_lds_limit((const void*)gqa_prefill_mfma_kernel<HD, SPLIT>, (int)lds, configured)) { \
+            set_error("gqa_attention: the prompt kernel's LDS limit could not be raised");                            \
+            return VXHIP_EXECUTION_FAILED;                                                                            \
+        }                                                                                                             \
+        hipLaunchKernelGGL((gqa_prefill_mfma_kernel<HD, SPLIT>), dim3(grid), dim3(256), lds, ctx->stream, q_dev,      \
+                           k_cache_dev, v_cache_dev, positions_dev, rows, t, tq, q_heads, kv_heads, max_seq, scale,   \
+                           out_dev, ctx->fault_dev);                                                                  \
+    } while (0)
+        if (head_dim == 128u && split) VXHIP_PROMPT(128, 4);
+        else if (head_dim == 128u) VXHIP_PROMPT(128, 1);
+        else if (split) VXHIP_PROMPT(64, 4);
+        else VXHIP_PROMPT(64, 1);
+#undef VXHIP_PROMPT
+        VXHIP_TRY(hipGetLastError());
+        return VXHIP_OK;
     }
     if (t >= 8u && rep <= kPrefillQueries && head_dim <= 256u) {
         // a prompt: tokens share the walk over the cache, as many per workgroup as the LDS holds
