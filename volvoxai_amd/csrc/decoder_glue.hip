@@ -128,7 +128,7 @@ __global__ __launch_bounds__(256) void rope_append_chunks_kernel(const float* __
 // from the caches, so workgroups do not depend on each other.  Every slot is still handled by
 // the thread, and in the order, that the unfused kernel gives it: the results are the same bits.
 //
-// Scores, NC = head_dim / 32 in {1, 2, 4, 8}: eight lanes share a key row, each loading the 16-byte
+// Scores, NC = head_dim / 32 in {1, 4, 8}: eight lanes share a key row, each loading the 16-byte
 // chunks c = lane%8 + 8*i, so one load instruction of a wavefront covers eight rows with whole
 // 128-byte lines (a thread per row touches 64 lines with every load and refetches each of them
 // eight times once the rows outgrow the L1); the eight partial dots meet in three xor-shuffles.
@@ -514,7 +514,226 @@ __global__ __launch_bounds__(256) void gqa_attention_kernel(const float* __restr
     }
 }
 
-// Prompt attention (t > 1 tokens per row).  The kernel above gives every (token, head) its own
+// The same attention for head size 64 and few tokens a row (decode), in one walk over keys and values together.  Eight wavefronts a workgroup; eight lanes share a slot, key and value row alike (16-byte chunks
+// c = lane % 8 + 8 * i), so a slot's probability is in the lanes that weigh its value row and nothing is exchanged
+// but the three steps of a dot's sum: each group of eight lanes keeps its own running maximum, sum and output, and
+// the 64 groups of a workgroup meet once, at the end.  A wavefront takes 16 slots of every 128; the rows of the
+// first 256 slots, values too, are requested before the query is ready.
+// Bound by the latency of a launch and of its reads; the kernel above asks for its values only once the keys have
+// come, and its three phases are behind barriers.  At slot 145, 8 query and 4 KV heads: 1 row 6.0 -> 4.6 us, 32 rows
+// 7.2 -> 5.9.  (At head size 128 twice the bytes are in flight either way and the reads themselves bound it: 1 row
+// 7.4 against 7.0 us, but 32 rows 12.7 against 13.3 and at slot 220 14.7 against 16.6, so it keeps the kernel above.)
+template <int REP, bool FUSED>
+__global__ __launch_bounds__(512, 2) void decode_attention_kernel(const float* __restrict__ q,
+                                                                  float* __restrict__ k_cache,
+                                                                  float* __restrict__ v_cache,
+                                                                  const int64_t* __restrict__ positions, uint32_t t,
+                                                                  uint32_t q_heads, uint32_t kv_heads,
+                                                                  uint32_t max_seq, float scale, float* __restrict__ out,
+                                                                  const float* __restrict__ cos_table,
+                                                                  const float* __restrict__ sin_table,
+                                                                  uint32_t* __restrict__ fault) {
+    constexpr int HD = 64, KC = HD / 32, WAVES = 8, PASSES = 2;
+    constexpr int BUFS = 2;  // blocks of 128 slots in flight
+    constexpr int STAGED = (REP + (FUSED ? 2 : 0)) * HD, ITEMS = (STAGED + 511) / 512;
+    constexpr uint32_t BLOCK = WAVES * PASSES * 8u;
+    __shared__ __attribute__((aligned(16))) float staged[STAGED];  // queries; FUSED: the appended key and value
+    __shared__ __attribute__((aligned(16))) float partial[WAVES][REP][HD];
+    __shared__ float maxima[WAVES][REP], sums[WAVES][REP];
+    const uint32_t token = blockIdx.x, head0 = blockIdx.y * REP;
+    const uint32_t row = token / t, i = token % t;
+    const uint32_t rep = q_heads / kv_heads, kvh = head0 / rep;
+    const uint64_t named = (uint64_t)positions[i];
+    if (named >= max_seq) {  // (the whole workgroup) outside the caches: touch nothing, say so
+        if (threadIdx.x == 0) atomicOr(fault, (uint32_t)kFaultBadPosition);
+        return;
+    }
+    const uint32_t position = (uint32_t)named;
+    const uint32_t cached = FUSED ? position : position + 1u;  // slots read from the caches
+    const uint32_t last_cached = max(cached, 1u) - 1u;
+    float* kbase = k_cache + ((size_t)row * kv_heads + kvh) * max_seq * HD;
+    float* vbase = v_cache + ((size_t)row * kv_heads + kvh) * max_seq * HD;
+    const uint32_t lane8 = threadIdx.x & 7u, group = (threadIdx.x >> 3) & 7u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+
+    // operands of the queries (and of the appended row) first: loads return in order
+    float own[ITEMS], mate[ITEMS], c[ITEMS], sn[ITEMS];
+#pragma unroll
+    for (int j = 0; j < ITEMS; j++) {
+        own[j] = mate[j] = c[j] = sn[j] = 0.0f;
+        const uint32_t e = threadIdx.x + 512u * j, which = e / HD, dd = e % HD;
+        if (e < STAGED) {
+            if constexpr (FUSED) {
+                const uint32_t head = which < REP ? head0 + which : which == REP ? q_heads + kvh : q_heads + kv_heads + kvh;
+                const float* src = q + ((size_t)token * (q_heads + 2u * kv_heads) + head) * HD;
+                own[j] = src[dd];
+                mate[j] = src[dd ^ (HD / 2u)];
+                c[j] = cos_table[(size_t)position * HD + dd];
+                sn[j] = sin_table[(size_t)position * HD + dd];
+            } else {
+                own[j] = q[((size_t)token * q_heads + head0 + which) * HD + dd];
+            }
+        }
+    }
+    // Slots past the end repeat the last cached one (row 0 where there is none) and are not counted.
+    float4 kb[BUFS][PASSES][KC], vb[BUFS][PASSES][KC];
+    auto slot_of = [&](uint32_t block, int u) { return block * BLOCK + wave * (PASSES * 8u) + u * 8u + group; };
+    auto request = [&](auto b_tag, uint32_t block) {
+        constexpr int b = decltype(b_tag)::value;
+#pragma unroll
+        for (int u = 0; u < PASSES; u++) {
+            const size_t at = (size_t)min(slot_of(block, u), last_cached) * HD;
+#pragma unroll
+            for (int n = 0; n < KC; n++) kb[b][u][n] = *reinterpret_cast<const float4*>(kbase + at + 4u * (lane8 + 8u * n));
+        }
+#pragma unroll
+        for (int u = 0; u < PASSES; u++) {
+            const size_t at = (size_t)min(slot_of(block, u), last_cached) * HD;
+#pragma unroll
+            for (int n = 0; n < KC; n++) vb[b][u][n] = *reinterpret_cast<const float4*>(vbase + at + 4u * (lane8 + 8u * n));
+        }
+    };
+    static_for<BUFS>([&](auto b_tag) { request(b_tag, (uint32_t)decltype(b_tag)::value); });
+#pragma unroll
+    for (int j = 0; j < ITEMS; j++) {
+        const uint32_t e = threadIdx.x + 512u * j, which = e / HD, dd = e % HD;
+        if (e < STAGED) {
+            float y = own[j];
+            if (FUSED && which <= REP)  // the arithmetic of rope_append_kernel
+                y = __fadd_rn(__fmul_rn(own[j], c[j]), __fmul_rn(dd < HD / 2u ? -mate[j] : mate[j], sn[j]));
+            staged[e] = y;
+            if (FUSED && which >= REP && head0 % rep == 0u) (which == REP ? kbase : vbase)[(size_t)position * HD + dd] = y;
+        }
+    }
+    __syncthreads();
+    float4 qv[REP][KC], acc[REP][KC];
+    float m[REP], sum[REP];
+#pragma unroll
+    for (int h = 0; h < REP; h++) {
+        m[h] = -INFINITY;
+        sum[h] = 0.0f;
+#pragma unroll
+        for (int n = 0; n < KC; n++) {
+            qv[h][n] = *reinterpret_cast<const float4*>(staged + h * HD + 4u * (lane8 + 8u * n));
+            acc[h][n] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    }
+    // one slot of this group of eight lanes (all 64 lanes take part; `counts` is false for a slot past the end)
+    auto take = [&](const float4 (&kr)[KC], const float4 (&vr)[KC], bool counts) {
+        float dot[REP];
+#pragma unroll
+        for (int h = 0; h < REP; h++) {
+            float d = 0.0f;
+#pragma unroll
+            for (int n = 0; n < KC; n++) {
+                d = __builtin_fmaf(qv[h][n].x, kr[n].x, d);
+                d = __builtin_fmaf(qv[h][n].y, kr[n].y, d);
+                d = __builtin_fmaf(qv[h][n].z, kr[n].z, d);
+                d = __builtin_fmaf(qv[h][n].w, kr[n].w, d);
+            }
+            d += lane_exchange<kDppXor1>(d);
+            d += lane_exchange<kDppXor2>(d);
+            d += lane_exchange<kDppHalfMirror>(d);
+            dot[h] = __fmul_rn(d, scale);
+        }
+        if (!counts) return;
+#pragma unroll
+        for (int h = 0; h < REP; h++) {
+            const float grown = fmaxf(m[h], dot[h]);
+            const float reference = grown == -INFINITY ? 0.0f : grown;  // (only scores of -inf so far: zeros)
+            const float keep = expf(m[h] - reference), p = expf(dot[h] - reference);
+            m[h] = grown;
+            sum[h] = __builtin_fmaf(sum[h], keep, p);
+#pragma unroll
+            for (int n = 0; n < KC; n++) {
+                acc[h][n].x = __builtin_fmaf(p, vr[n].x, acc[h][n].x * keep);
+                acc[h][n].y = __builtin_fmaf(p, vr[n].y, acc[h][n].y * keep);
+                acc[h][n].z = __builtin_fmaf(p, vr[n].z, acc[h][n].z * keep);
+                acc[h][n].w = __builtin_fmaf(p, vr[n].w, acc[h][n].w * keep);
+            }
+        }
+    };
+    const uint32_t blocks = (cached + BLOCK - 1u) / BLOCK;
+    for (uint32_t block = 0; block < blocks; block += BUFS) {
+        static_for<BUFS>([&](auto b_tag) {
+            constexpr int b = decltype(b_tag)::value;
+            if (block + b < blocks) {  // (a scalar branch)
+#pragma unroll
+                for (int u = 0; u < PASSES; u++) take(kb[b][u], vb[b][u], slot_of(block + b, u) < cached);
+            }
+            request(b_tag, block + b + BUFS);
+        });
+    }
+    if constexpr (FUSED) {
+        // the appended slot, from LDS, by the group that has it in the unfused form and behind the same slots
+        if (wave == position % BLOCK / (PASSES * 8u)) {
+            float4 kr[KC], vr[KC];
+#pragma unroll
+            for (int n = 0; n < KC; n++) {
+                kr[n] = *reinterpret_cast<const float4*>(staged + REP * HD + 4u * (lane8 + 8u * n));
+                vr[n] = *reinterpret_cast<const float4*>(staged + (REP + 1) * HD + 4u * (lane8 + 8u * n));
+            }
+            take(kr, vr, group == position % 8u);
+        }
+    }
+    // The groups of a wavefront meet: lanes 32, then 16, then 8 apart.  The first step exchanges one half of the
+    // channels for the other and leaves half as many to the next.
+    constexpr int kDppRor8 = 0x128;  // lane ^ 8 within a row of 16
+    auto halves = [](float a, float b) {  // lower half: a summed over both, upper half: b
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    };
+    auto row_pair = [](float a) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(a), false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    };
+#pragma unroll
+    for (int h = 0; h < REP; h++) {
+        const float top = wave_max(m[h]);
+        const float keep = expf(m[h] - (top == -INFINITY ? 0.0f : top));
+        float total = sum[h] * keep;
+        total = halves(total, total);
+        total = row_pair(total);
+        total += lane_exchange<kDppRor8>(total);
+        float x[KC * 4];
+#pragma unroll
+        for (int n = 0; n < KC; n++)
+            x[4 * n] = acc[h][n].x * keep, x[4 * n + 1] = acc[h][n].y * keep, x[4 * n + 2] = acc[h][n].z * keep,
+                  x[4 * n + 3] = acc[h][n].w * keep;
+#pragma unroll
+        for (int e = 0; e < KC * 2; e++) x[e] = halves(x[e], x[e + KC * 2]);
+        const uint32_t chunk = (threadIdx.x >> 5) & 1u;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            x[e] = row_pair(x[e]);
+            x[e] += lane_exchange<kDppRor8>(x[e]);
+        }
+        if ((threadIdx.x & 24u) == 0u)
+            *reinterpret_cast<float4*>(&partial[wave][h][4u * (lane8 + 8u * chunk)]) = make_float4(x[0], x[1], x[2], x[3]);
+        if ((threadIdx.x & 63u) == 0u) {
+            maxima[wave][h] = top;
+            sums[wave][h] = total;
+        }
+    }
+    __syncthreads();
+    for (uint32_t e = threadIdx.x; e < REP * HD; e += 512u) {
+        const uint32_t h = e / HD, dd = e % HD;
+        float top = maxima[0][h];
+#pragma unroll
+        for (int w = 1; w < WAVES; w++) top = fmaxf(top, maxima[w][h]);
+        const float reference = top == -INFINITY ? 0.0f : top;
+        float total = 0.0f, y = 0.0f;
+#pragma unroll
+        for (int w = 0; w < WAVES; w++) {
+            const float weight = expf(maxima[w][h] - reference);
+            total = __builtin_fmaf(sums[w][h], weight, total);
+            y = __builtin_fmaf(partial[w][h][dd], weight, y);
+        }
+        out[((size_t)token * q_heads + head0 + h) * HD + dd] = __fdiv_rn(y, total);
+    }
+}
+
+// Prompt attention (t > 1 tokens per row).  The kernels above give every (token, head) its own
 // workgroup, so a prompt of t tokens reads each key and value row t times.  Here a workgroup takes
 // `tq` consecutive tokens of one row and the `rep` query heads of one KV head, qw = tq * rep <= 32
 // queries, and walks that KV head's rows once for all of them, 64 slots at a time through LDS:
@@ -964,6 +1183,9 @@ void launch_attention(hipStream_t stream, uint32_t together, dim3 grid, size_t l
 #define VXHIP_ATTENTION(R, NC)                                                                                  \
     hipLaunchKernelGGL((gqa_attention_kernel<R, FUSED, NC>), grid, dim3(256), lds, stream, q, k_cache, v_cache, \
                        positions, t, q_heads, kv_heads, head_dim, max_seq, scale, out, cos_table, sin_table, fault)
+#define VXHIP_DECODE(R)                                                                                                  \
+    hipLaunchKernelGGL((decode_attention_kernel<R, FUSED>), grid, dim3(512), 0, stream, q, k_cache, v_cache, positions, t, \
+                       q_heads, kv_heads, max_seq, scale, out, cos_table, sin_table, fault)
 #define VXHIP_ATTENTION_HEADS(NC)     \
     do {                              \
         if (together == 4u) VXHIP_ATTENTION(4, NC); \
@@ -972,13 +1194,18 @@ void launch_attention(hipStream_t stream, uint32_t together, dim3 grid, size_t l
     } while (0)
     switch (head_dim) {
         case 32: VXHIP_ATTENTION_HEADS(1); break;
-        case 64: VXHIP_ATTENTION_HEADS(2); break;
+        case 64:
+            if (together == 4u) VXHIP_DECODE(4);
+            else if (together == 2u) VXHIP_DECODE(2);
+            else VXHIP_DECODE(1);
+            break;
         case 128: VXHIP_ATTENTION_HEADS(4); break;
         case 256: VXHIP_ATTENTION_HEADS(8); break;
         default: VXHIP_ATTENTION_HEADS(0); break;
     }
 #undef VXHIP_ATTENTION_HEADS
 #undef VXHIP_ATTENTION
+#undef VXHIP_DECODE
 }
 
 // Embedding lookup (embedding.inc:5-16): out[i] = table[tokens[i]], one workgroup per token.
@@ -1149,8 +1376,17 @@ VxHipStatus vxhip_gqa_attention(VxHipContext* ctx, const float* q_dev, const flo
     if (!device_ready(ctx)) return VXHIP_BACKEND_UNAVAILABLE;
     const float scale = (float)(1.0 / sqrt((double)head_dim));
     const uint32_t rep = q_heads / kv_heads;
-    if (t >= 8u && rep <= kPrefillQueries && (head_dim == 128u || head_dim == 64u)) {
-        // a prompt at the common head sizes: the matrix-pipe kernel
+    const uint32_t together = heads_per_workgroup(rep, rows * t * q_heads, ctx->cu_count);
+    const size_t token_lds = (size_t)together * (9u * head_dim + max_seq) * sizeof(float);  // of the per-token kernel
+    auto prompt_lds = [&](uint32_t tokens) {  // of the prompt kernel that keeps its scores
+        const size_t qw = (size_t)tokens * rep;
+        return (qw * ((max_seq + 63u) & ~63u) + (size_t)kPrefillSlots * (head_dim + 4u)) * sizeof(float);
+    };
+    constexpr size_t kTokenLds = 60u * 1024u, kPromptLds = 150u * 1024u;
+    // A prompt at the common head sizes: the matrix-pipe kernel.  (It holds no scores and would take any cache, but
+    // a cache that a decode step, or a prompt at another head size, could not serve is refused alike.)
+    if (t >= 8u && rep <= kPrefillQueries && (head_dim == 128u || head_dim == 64u) &&
+        (prompt_lds(1u) <= kPromptLds || token_lds <= kTokenLds)) {
         const uint32_t tq = kPrefillQueries / rep, blocks = (t + tq - 1u) / tq, pairs = rows * kv_heads;
         const bool split = split_prompt_slots(pairs * blocks, t, ctx->cu_count);
         const uint32_t grid = pairs * (split ? blocks : (blocks + 3u) / 4u);
@@ -1177,40 +1413,34 @@ VxHipStatus vxhip_gqa_attention(VxHipContext* ctx, const float* q_dev, const flo
     if (t >= 8u && rep <= kPrefillQueries && head_dim <= 256u) {
         // a prompt: tokens share the walk over the cache, as many per workgroup as the LDS holds
         uint32_t tq = kPrefillQueries / rep;
-        auto lds_for = [&](uint32_t tokens) {
-            const size_t qw = (size_t)tokens * rep;
-            return (qw * ((max_seq + 63u) & ~63u) + (size_t)kPrefillSlots * (head_dim + 4u)) * sizeof(float);
-        };
-        while (tq > 1u && lds_for(tq) > 150u * 1024u) tq /= 2u;
+        while (tq > 1u && prompt_lds(tq) > kPromptLds) tq /= 2u;
         // two workgroups per compute unit hide each other's staging, if four tokens or more still
         // share a walk then
-        if (lds_for(tq) > 78u * 1024u) {
+        if (prompt_lds(tq) > 78u * 1024u) {
             uint32_t fewer = tq;
-            while (fewer > 4u && lds_for(fewer) > 78u * 1024u) fewer /= 2u;
-            if (lds_for(fewer) <= 78u * 1024u) tq = fewer;
+            while (fewer > 4u && prompt_lds(fewer) > 78u * 1024u) fewer /= 2u;
+            if (prompt_lds(fewer) <= 78u * 1024u) tq = fewer;
         }
-        if (lds_for(tq) <= 150u * 1024u) {
+        if (prompt_lds(tq) <= kPromptLds) {
             static std::atomic<uint64_t> configured{0};
             if (!raise_lds_limit((const void*)gqa_prefill_kernel, 152 * 1024, configured)) {  // (plus its static 128 bytes)
                 set_error("gqa_attention: the prompt kernel's LDS limit could not be raised");
                 return VXHIP_EXECUTION_FAILED;
             }
             const dim3 grid(rows * ((t + tq - 1u) / tq), kv_heads);
-            hipLaunchKernelGGL(gqa_prefill_kernel, grid, dim3(256), lds_for(tq), ctx->stream, q_dev, k_cache_dev,
+            hipLaunchKernelGGL(gqa_prefill_kernel, grid, dim3(256), prompt_lds(tq), ctx->stream, q_dev, k_cache_dev,
                                v_cache_dev, positions_dev, t, tq, q_heads, kv_heads, head_dim, max_seq, scale, out_dev,
                                ctx->fault_dev);
             VXHIP_TRY(hipGetLastError());
             return VXHIP_OK;
         }
     }
-    const uint32_t together = heads_per_workgroup(rep, rows * t * q_heads, ctx->cu_count);
-    const size_t lds = (size_t)together * (9u * head_dim + max_seq) * sizeof(float);
-    if (lds > 60u * 1024u) {
+    if (token_lds > kTokenLds) {
         set_error("gqa_attention: head_dim/max_seq too large for the score buffer");
         return VXHIP_INVALID_ARGUMENT;
     }
     const dim3 grid(rows * t, q_heads / together);
-    launch_attention<false>(ctx->stream, together, grid, lds, q_dev, const_cast<float*>(k_cache_dev),
+    launch_attention<false>(ctx->stream, together, grid, token_lds, q_dev, const_cast<float*>(k_cache_dev),
                             const_cast<float*>(v_cache_dev), positions_dev, t, q_heads, kv_heads, head_dim, max_seq,
                             scale, out_dev, nullptr, nullptr, ctx->fault_dev);
     VXHIP_TRY(hipGetLastError());
