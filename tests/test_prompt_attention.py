@@ -75,3 +75,25 @@ def test_prompt_attention_of_infinite_scores(ctx, head_dim, t):
     assert np.isnan(got[:low]).all() and np.isnan(got[bad:]).all()  # (nothing but -inf: 0 / 0, as exp(-inf + inf) gives)
     for i in range(low, bad):
         assert np.allclose(got[i], v[0, 0, low:i + 1].astype(np.float64).mean(0), rtol=1e-5, atol=1e-6), i
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("q_heads,max_seq,taken", [(1, 30000, True), (1, 40000, False), (8, 14000, True), (8, 15000, False)])
+def test_prompt_attention_cache_limits(ctx, q_heads, max_seq, taken):
+    """The longest caches are those whose score rows fit one of the kernels that keep them, whichever kernel answers."""
+    import torch
+    import volvoxai_amd.w8a8 as vx
+    q = torch.randn(1, 8, q_heads, 64, device="cuda")
+    k, v = torch.randn(2, 1, 1, max_seq, 64, device="cuda")
+    positions = torch.arange(max_seq - 8, max_seq, device="cuda")
+    if not taken:
+        with pytest.raises(vx.VxHipError):
+            vx.gqa_attention(ctx, q, k, v, positions)
+        return
+    out = vx.gqa_attention(ctx, q, k, v, positions).reshape(8, q_heads, 64)
+    ctx.synchronize()
+    scores = torch.matmul(q[0].double(), k[0, 0].double().T) / 8.0  # [t, heads, slots]
+    scores.masked_fill_(torch.arange(max_seq, device="cuda")[None, None] > positions[:, None, None], float("-inf"))
+    want = torch.matmul(torch.softmax(scores, -1), v[0, 0].double())
+    # (30,000 terms summed in f32: each adds at most 2^-24 of a sum of probabilities times values below 1)
+    assert torch.allclose(out.double(), want, rtol=2e-5, atol=5e-6)
