@@ -97,3 +97,36 @@ def test_prompt_attention_cache_limits(ctx, q_heads, max_seq, taken):
     want = torch.matmul(torch.softmax(scores, -1), v[0, 0].double())
     # (30,000 terms summed in f32: each adds at most 2^-24 of a sum of probabilities times values below 1)
     assert torch.allclose(out.double(), want, rtol=2e-5, atol=5e-6)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,t,layers,q_heads,kv_heads,head_dim,max_seq", [
+    (1, 9, 1, 2, 2, 128, 14300),      # one row: the score buffer of the decode kernel would be too small
+    (17, 8, 1, 16, 8, 128, 6600),     # more query heads than compute units: two heads share that buffer
+    (1, 40, 2, 2, 2, 64, 14900),
+    (3, 5, 1, 4, 2, 64, 40),          # fewer tokens than the prompt kernels take
+    (2, 37, 1, 4, 2, 128, 40),
+])
+def test_decoder_prompts_behind_the_last_layer(oracle, rows, t, layers, q_heads, kv_heads, head_dim, max_seq):
+    """Behind the last layer only each row's last token is computed: the CPU restatement's logits, for every cache that
+    the layers in front take, and the same bits whatever its length.  (An activation next to a rounding boundary may
+    take the neighbouring code, one of 127: the logits then differ by less than 1 / 127 of their norm.)"""
+    import torch
+    from _decoder_ref import DecoderRef
+    from volvoxai_amd.decoder import DecoderConfig, W8A8Decoder, init_weights, rope_tables
+    sizes = dict(layers=layers, hidden=256, q_heads=q_heads, kv_heads=kv_heads, head_dim=head_dim, inter=256, vocab=300)
+    cfg, short = DecoderConfig(max_seq=max_seq, **sizes), DecoderConfig(max_seq=48, **sizes)
+    weights = init_weights(short, 3)
+    prompt = np.random.default_rng(t).integers(0, cfg.vocab, (rows, t))
+    ref = DecoderRef(short, weights, oracle, rope_tables)
+    empty = [[np.zeros((rows, kv_heads, 0, head_dim), np.float32) for _ in range(layers)] for _ in range(2)]
+    want = ref.forward(prompt, 0, *empty)
+    logits = []
+    for c in (short, cfg):
+        dec = W8A8Decoder(c, weights, rows)
+        torch.cuda.synchronize()
+        dec.prefill(torch.from_numpy(prompt).cuda())
+        logits.append(dec.last_logits.cpu().numpy())
+        dec.close()
+    assert (logits[0].view(np.uint32) == logits[1].view(np.uint32)).all()
+    assert np.linalg.norm(logits[1] - want) <= np.linalg.norm(want) / 127
