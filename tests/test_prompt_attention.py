@@ -130,3 +130,35 @@ def test_decoder_prompts_behind_the_last_layer(oracle, rows, t, layers, q_heads,
         dec.close()
     assert (logits[0].view(np.uint32) == logits[1].view(np.uint32)).all()
     assert np.linalg.norm(logits[1] - want) <= np.linalg.norm(want) / 127
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,head_dim,t", [(1, 128, 20), (1, 128, 70), (64, 64, 70), (1, 64, 70)])
+def test_values_at_the_ends_of_the_range(ctx, rows, head_dim, t):
+    """A value that is not finite reaches the tokens that see its slot and no others; values near the largest f32 leave
+    a mean of their size (probabilities of one sum to one within 2^-18 here)."""
+    import torch
+    import volvoxai_amd.w8a8 as vx
+    rng = np.random.default_rng(t)
+    q = rng.normal(0, 1, (rows, t, 2, head_dim)).astype(np.float32)
+    k = rng.normal(0, 1, (rows, 1, 96, head_dim)).astype(np.float32)
+    v = rng.normal(0, 1, (rows, 1, 96, head_dim)).astype(np.float32)
+    start = 96 - t if t < 8 else 0
+    positions = np.arange(start, start + t, dtype=np.int64)
+    nan, inf = start + t // 2, start + t - t // 4
+    v[:, 0, nan, 3] = np.nan
+    if inf < start + t:
+        v[:, 0, inf, 5] = -np.inf
+    sc = np.matmul(q.transpose(0, 2, 1, 3).astype(np.float64), k.transpose(0, 1, 3, 2)) / np.sqrt(head_dim)
+    dev = lambda a: torch.from_numpy(a).cuda()
+    got = vx.gqa_attention(ctx, dev(q), dev(k), dev(v), dev(positions)).reshape(rows, t, 2, head_dim)
+    big = vx.gqa_attention(ctx, dev(q), dev(k), torch.full((rows, 1, 96, head_dim), 3.3e38, device="cuda"), dev(positions))
+    ctx.synchronize()
+    got = got.cpu().numpy()
+    for i in range(t):
+        seen = sc[:, :, i, :positions[i] + 1]
+        p = np.exp(seen - seen.max(-1, keepdims=True))
+        with np.errstate(invalid="ignore"):
+            want = np.matmul(p / p.sum(-1, keepdims=True), v[:, 0, :positions[i] + 1].astype(np.float64))
+        assert np.allclose(got[:, i], want, rtol=2e-5, atol=5e-6, equal_nan=True), i
+    assert torch.allclose(big.double(), torch.full_like(big, 3.3e38).double(), rtol=2.0 ** -18, atol=0)

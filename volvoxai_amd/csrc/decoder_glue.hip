@@ -1090,16 +1090,68 @@ __global__ __launch_bounds__(256, 2) void gqa_prefill_mfma_kernel(const float* _
         });
     }
 
-    float* dst = out + ((size_t)(row * t + token) * q_heads + head) * HD;
-    if constexpr (SPLIT == 1) {
-        if (visible == 0u) return;
+    // Outputs that are not finite: a value that is not, of a slot that only others of the wavefront's queries see, was
+    // multiplied by the zero probability of a query that does not, or the sums over probabilities up to 1 have
+    // overflowed.  Such queries (a bit each) are computed once more over the slots they see, with the probabilities
+    // divided first; channels ch0 .. ch0 + CH - 1, by the wavefront that stores them.
+    auto recompute = [&](uint32_t queries, uint32_t ch0, auto channels_tag) {
+        constexpr uint32_t CH = decltype(channels_tag)::value;
+        for (; queries; queries &= queries - 1u) {
+            const uint32_t qi = __builtin_ctz(queries), seen = __builtin_amdgcn_readlane(visible, qi);
+            const size_t at = ((size_t)(row * t + block * tq + qi / rep) * q_heads + kvh * rep + qi % rep) * HD;
+            auto score = [&](uint32_t slot) {
+                float dot = 0.0f;
+                for (uint32_t c = 0; c < HD; c++) dot = __builtin_fmaf(q[at + c], kbase[(size_t)slot * HD + c], dot);
+                return __fmul_rn(dot, scale);
+            };
+            float best = -INFINITY, part = 0.0f;
+            for (uint32_t slot = lane; slot < seen; slot += 64u) best = fmaxf(best, score(slot));
+            best = wave_max(best);
+            for (uint32_t slot = lane; slot < seen; slot += 64u) part += expf(score(slot) - best);
+            const float total = wave_sum(part);
+            constexpr int YS = (CH + 63u) / 64u;  // channels a lane
+            float y[YS] = {};
+            for (uint32_t s0 = 0; s0 < seen; s0 += 64u) {
+                const float p = s0 + lane < seen ? __fdiv_rn(expf(score(s0 + lane) - best), total) : 0.0f;
+                for (uint32_t j = 0; j < min(64u, seen - s0); j++) {
+                    const float weight = lane_value(p, (int)j);
+                    const float* value = vbase + (size_t)(s0 + j) * HD + ch0 + lane;
 #pragma unroll
-        for (int v = 0; v < 16; v++) {
-            out_vec y;
+                    for (int i = 0; i < YS; i++)
+                        if (lane + 64u * i < CH) y[i] = __builtin_fmaf(weight, value[64 * i], y[i]);
+                }
+            }
 #pragma unroll
-            for (int c = 0; c < VW; c++) y[c] = __fdiv_rn(o[c][v], sum);
-            *reinterpret_cast<out_vec*>(dst + VW * (8u * (v / 4) + 4u * h + v % 4)) = y;
+            for (int i = 0; i < YS; i++)
+                if (lane + 64u * i < CH) out[at + ch0 + lane + 64u * i] = y[i];
         }
+    };
+    auto queries_of = [](bool lanes) {  // one bit a query from the two lanes that hold it
+        const uint64_t both = __builtin_amdgcn_ballot_w64(lanes);
+        return (uint32_t)both | (uint32_t)(both >> 32);
+    };
+
+    float* dst = out + ((size_t)(row * t + token) * q_heads + head) * HD;
+    bool finite = true;
+    if constexpr (SPLIT == 1) {
+#pragma unroll
+        for (int v = 0; v < 16; v++)
+#pragma unroll
+            for (int c = 0; c < VW; c++) {
+                o[c][v] = __fdiv_rn(o[c][v], sum);
+                finite = finite && finite_f32(o[c][v]);
+            }
+        const uint32_t again = queries_of(visible != 0u && !finite);
+        if (visible != 0u && !(again >> r & 1u)) {
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                out_vec y;
+#pragma unroll
+                for (int c = 0; c < VW; c++) y[c] = o[c][v];
+                *reinterpret_cast<out_vec*>(dst + VW * (8u * (v / 4) + 4u * h + v % 4)) = y;
+            }
+        }
+        if (again) recompute(again, 0u, IC<HD>{});
     } else {
         // [wavefront][2 + 16 * VW][64]: maximum, sum, then the outputs; wavefront w merges the registers
         // 4w .. 4w + 3 of every channel tile
@@ -1122,20 +1174,25 @@ __global__ __launch_bounds__(256, 2) void gqa_prefill_mfma_kernel(const float* _
             weight[w] = expf(parts[w * PART] - reference);
             total = __builtin_fmaf(parts[w * PART + 64], weight[w], total);
         }
-        if (visible == 0u) return;
+        out_vec y[4];
 #pragma unroll
         for (int u = 0; u < 4; u++) {
-            out_vec y;
 #pragma unroll
             for (int c = 0; c < VW; c++) {
                 float x = 0.0f;
 #pragma unroll
                 for (int w = 0; w < SPLIT; w++)
                     x = __builtin_fmaf(parts[w * PART + (2u + (4u * wave + u) * VW + c) * 64u], weight[w], x);
-                y[c] = __fdiv_rn(x, total);
+                y[u][c] = __fdiv_rn(x, total);
+                finite = finite && finite_f32(y[u][c]);
             }
-            *reinterpret_cast<out_vec*>(dst + VW * (8u * wave + 4u * h + u)) = y;
         }
+        const uint32_t again = queries_of(visible != 0u && !finite);
+        if (visible != 0u && !(again >> r & 1u)) {
+#pragma unroll
+            for (int u = 0; u < 4; u++) *reinterpret_cast<out_vec*>(dst + VW * (8u * wave + 4u * h + u)) = y[u];
+        }
+        if (again) recompute(again, 8u * VW * wave, IC<8 * VW>{});
     }
 }
 
