@@ -133,7 +133,7 @@ def test_decoder_prompts_behind_the_last_layer(oracle, rows, t, layers, q_heads,
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows,head_dim,t", [(1, 128, 20), (1, 128, 70), (64, 64, 70), (1, 64, 70)])
+@pytest.mark.parametrize("rows,head_dim,t", [(1, 128, 20), (1, 128, 70), (64, 64, 70), (1, 64, 70), (1, 64, 1), (1, 64, 3)])
 def test_values_at_the_ends_of_the_range(ctx, rows, head_dim, t):
     """A value that is not finite reaches the tokens that see its slot and no others; values near the largest f32 leave
     a mean of their size (probabilities of one sum to one within 2^-18 here)."""

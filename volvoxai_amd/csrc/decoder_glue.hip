@@ -606,6 +606,9 @@ __global__ __launch_bounds__(512, 2) void decode_attention_kernel(const float* _
         }
     }
     __syncthreads();
+    // Probabilities carry a power of two of at most one over the number of slots (it leaves with the division at the
+    // end): the sums of their products with values stay in the values' range.
+    const float unit = __uint_as_float((127u - (position ? 32u - (uint32_t)__builtin_clz(position) : 0u)) << 23);
     float4 qv[REP][KC], acc[REP][KC];
     float m[REP], sum[REP];
 #pragma unroll
@@ -641,7 +644,7 @@ __global__ __launch_bounds__(512, 2) void decode_attention_kernel(const float* _
         for (int h = 0; h < REP; h++) {
             const float grown = fmaxf(m[h], dot[h]);
             const float reference = grown == -INFINITY ? 0.0f : grown;  // (only scores of -inf so far: zeros)
-            const float keep = expf(m[h] - reference), p = expf(dot[h] - reference);
+            const float keep = expf(m[h] - reference), p = expf(dot[h] - reference) * unit;
             m[h] = grown;
             sum[h] = __builtin_fmaf(sum[h], keep, p);
 #pragma unroll
