@@ -591,15 +591,11 @@ const char* launch_fit_mode(hipStream_t s, const LinearArgs& a, int cu_count, co
     constexpr uint32_t SPB = W4 ? 2u : 1u;
     if (force && (strstr(force, "nofit") || strstr(force, "wv"))) return nullptr;  // (wv..: a general-kernel name)
     if (a.row_gain || a.row_swiglu || a.add_to || a.weight_bits != (W4 ? 4u : 8u) || a.x_flip_mask) return nullptr;
-    // One or two f32 rows of exactly the stream's length: gemv_row.hip runs them, under the name of the instance that
-    // takes such a shape's prepared rows.
-    const bool prep = a.x_f32 != nullptr;
-    if (prep && (a.rows > kMaxPrepRows || a.k != a.ksteps * 32u * SPB)) return nullptr;
     const uint32_t panels = (a.n + 31u) / 32u;
     const bool forced = force && strstr(force, "fit");
     // workgroups per panel: the general kernel's rule (and its names: c8, c16 for the channels of a workgroup)
     uint32_t split = 1;
-    if (!W4 && !prep && a.ksteps <= 128u) {
+    if (!W4 && a.ksteps <= 128u) {
         split = panels * 4u <= (uint32_t)cu_count ? 4u : panels * 2u <= (uint32_t)cu_count ? 2u : 1u;
         if (force && strstr(force, "c8")) split = 4;
         else if (force && strstr(force, "c16")) split = 2;
@@ -642,9 +638,7 @@ const char* launch_fit_mode(hipStream_t s, const LinearArgs& a, int cu_count, co
                 lds = lds_for(W, STEPS, false);
             }
             if (lds > 156u * 1024u) return;
-            if (prep) {
-                ok = launch_gemv_row(s, a, cu_count, force, gemv_dry_run) != nullptr;
-            } else if constexpr (SPLITS) {
+            if constexpr (SPLITS) {
                 if (split == 4u) ok = launch_fit<GK, W, B, W4, 4>(s, a, lds, xlds, rprod);
                 else if (split == 2u) ok = launch_fit<GK, W, B, W4, 2>(s, a, lds, xlds, rprod);
                 else ok = launch_fit<GK, W, B, W4>(s, a, lds, xlds, rprod);
@@ -653,7 +647,7 @@ const char* launch_fit_mode(hipStream_t s, const LinearArgs& a, int cu_count, co
                 ok = launch_fit<GK, W, B, W4>(s, a, lds, xlds, rprod);
             }
             taken = true;
-            snprintf(name, sizeof name, "fit%dx%d%s%s", W, B, split == 4u ? "c8" : split == 2u ? "c16" : "", prep ? "-prep" : "");
+            snprintf(name, sizeof name, "fit%dx%d%s", W, B, split == 4u ? "c8" : split == 2u ? "c16" : "");
         }
     };
     using std::integral_constant;
@@ -704,9 +698,12 @@ bool launch_split(hipStream_t s, const LinearArgs& a, size_t lds, int split) {
 template <int MODE, int GK, bool W4 = false>
 const char* launch_mode(hipStream_t s, const LinearArgs& a, int cu_count, const char* force) {
     if constexpr (MODE == (int)Epilogue::DequantF32) {
+        // f32 rows; with an instance of the kernels below named, the caller prepares them and comes back
+        if (a.x_f32)
+            return force && (strstr(force, "wv") || (strstr(force, "fit") && !strstr(force, "nofit")))
+                       ? nullptr
+                       : launch_gemv_row(s, a, cu_count, force, gemv_dry_run);
         if (const char* fit = launch_fit_mode<GK, W4>(s, a, cu_count, force)) return fit;
-        // f32 rows; with the general kernel named (wv..), the caller prepares them and comes back
-        if (a.x_f32) return force && strstr(force, "wv") ? nullptr : launch_gemv_row(s, a, cu_count, force, gemv_dry_run);
     }
     // blocks of the stream per panel, and the units a wave's run is made of
     constexpr uint32_t SPB = W4 ? 2 : 1, UNIT = GK > SPB ? GK : SPB;
