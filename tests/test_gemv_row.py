@@ -30,3 +30,24 @@ def test_rows_at_the_edges_of_the_instances(ctx, oracle, k, n, bits, group, rows
     finally:
         vx.force_variant(None)
         pl.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("no_alloc", [False, True])
+@pytest.mark.parametrize("rows,k", [(1, 1024), (2, 10240)])
+def test_rows_that_are_overwritten_by_their_output(ctx, oracle, rows, k, no_alloc):
+    """In place the workgroups of one launch would read what others have already stored: the rows are prepared first."""
+    import torch
+    import volvoxai_amd as vx
+    c = cases.packed_case(rows, k, k, 128, k, True)
+    words = oracle.pack_w8_words(c["w"])
+    _, want = oracle.packed_linear(c["x"], words, c["scales"], c["bias"], k, 128)
+    pl = vx.PackedLinear(words, c["scales"], c["bias"], k, k, 128)
+    try:
+        x = torch.from_numpy(c["x"]).cuda()
+        st, _ = pl.forward_f32(ctx, x, out=x, no_alloc=no_alloc)
+        ctx.synchronize()
+        assert st == 0 and not ctx.last_variant.endswith("-prep"), ctx.last_variant
+        assert (x.cpu().numpy().view(np.uint32) == want.view(np.uint32)).all()
+    finally:
+        pl.close()

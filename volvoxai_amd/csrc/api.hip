@@ -1200,6 +1200,17 @@ static int packed_run_f32_rows(VxHipContext* ctx, const VxHipPackedLinear* pl, c
     return 0;
 }
 
+static bool overlap(const void* a, size_t a_bytes, const void* b, size_t b_bytes) {
+    return (uintptr_t)a < (uintptr_t)b + b_bytes && (uintptr_t)b < (uintptr_t)a + a_bytes;
+}
+
+// The same for rows without operations.  Every workgroup of it reads the whole rows while others already store their
+// channels, so an output over the input goes by way of the prepared rows (which are complete before it is written).
+static bool run_rows_at_once(VxHipContext* ctx, const VxHipPackedLinear* pl, const float* x, float* y, uint32_t rows) {
+    return !overlap(x, (size_t)rows * pl->w.k * 4u, y, (size_t)rows * pl->w.n * 4u) &&
+           packed_run_f32_rows(ctx, pl, x, y, rows) == 0;
+}
+
 int vxhip_packed_linear_forward_f32(VxHipContext* ctx, const VxHipPackedLinear* pl, const float* input_dev,
                                     float* output_dev, uint32_t rows) {
     if (!ctx || !pl || !input_dev || !output_dev) {
@@ -1209,7 +1220,7 @@ int vxhip_packed_linear_forward_f32(VxHipContext* ctx, const VxHipPackedLinear* 
     if (!rows) return 0;
     if (!same_device(ctx, pl->device, "packed_linear_forward_f32") || !use_device(ctx->device)) return -1;
     const uint32_t k = pl->w.k;
-    if (packed_run_f32_rows(ctx, pl, input_dev, output_dev, rows) == 0) return 0;
+    if (run_rows_at_once(ctx, pl, input_dev, output_dev, rows)) return 0;
     const uint32_t ld = (k + 15u) / 16u * 16u;
     // the prepared rows never leave this call: up to 32 rows go to the GEMV in its operand order
     const bool operand_order = rows <= kOperandOrderRows;
@@ -1245,15 +1256,12 @@ int vxhip_packed_linear_forward_fused(VxHipContext* ctx, const VxHipPackedLinear
     // Every workgroup reads the whole input rows while others already store their channels: an input that
     // overlaps the output (or the residual it is added to, which may itself be the output) would be read
     // half updated.
-    {
-        const uintptr_t x0 = (uintptr_t)input_dev;
-        const uintptr_t x1 = x0 + (size_t)rows * (row_op == VXHIP_ROW_OP_SWIGLU ? 2u : 1u) * pl->w.k * 4u;
-        const size_t out_bytes = (size_t)rows * pl->w.n * 4u;
-        const uintptr_t y0 = (uintptr_t)output_dev, a0 = (uintptr_t)add_to_dev;
-        if ((x0 < y0 + out_bytes && y0 < x1) || (add_to_dev && x0 < a0 + out_bytes && a0 < x1)) {
-            set_error("packed_linear_forward_fused: the input rows overlap the output or the residual");
-            return -1;
-        }
+    const size_t in_bytes = (size_t)rows * (row_op == VXHIP_ROW_OP_SWIGLU ? 2u : 1u) * pl->w.k * 4u;
+    const size_t out_bytes = (size_t)rows * pl->w.n * 4u;
+    if (overlap(input_dev, in_bytes, output_dev, out_bytes) ||
+        (add_to_dev && overlap(input_dev, in_bytes, add_to_dev, out_bytes))) {
+        set_error("packed_linear_forward_fused: the input rows overlap the output or the residual");
+        return -1;
     }
     RowOps ops;
     ops.gain = row_op == VXHIP_ROW_OP_RMSNORM ? gain_dev : nullptr;
@@ -1295,7 +1303,7 @@ int vxhip_packed_linear_forward_f32_noalloc(VxHipContext* ctx, const VxHipPacked
         (void)no_alloc_scratch(ctx->device);  // sets the error text of the failed set-up
         return -1;
     }
-    if (packed_run_f32_rows(ctx, pl, input_dev, output_dev, rows) == 0) return 0;
+    if (run_rows_at_once(ctx, pl, input_dev, output_dev, rows)) return 0;
     const uint32_t k = pl->w.k;
     const uint32_t ld = (k + 15u) / 16u * 16u;
     const bool operand_order = rows <= kOperandOrderRows;
