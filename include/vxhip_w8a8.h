@@ -412,10 +412,11 @@ VxHipStatus vxhip_packed_prepare_i8(VxHipContext* context,
 
 /* vx_packed_linear_forward with normalize==8, groups in {8, 4, 3, 2}
  * (src/kernels/packed_linear_ops.inc:1545-1621) on resident f32 rows.
- * One or two rows (the reference's single-row route, :1471-1535, which prepares
- * the row and multiplies in one call) run as one launch: the streaming kernel
- * prepares the rows itself (route id ends in "-prep"); more rows are prepared
- * by a launch of their own first.  The bits are the same either way.
+ * One or two rows of k up to 14336 (the reference's single-row route, :1471-1535,
+ * which prepares the row and multiplies in one call) run as one launch whose
+ * workgroups prepare the rows themselves (route id ends in "-prep"), unless the
+ * output overlaps the input; other rows are prepared by a launch of their own
+ * first.  The bits are the same either way.
  * Returns 0 on success, -1 on a rejected descriptor (reference convention). */
 int vxhip_packed_linear_forward_f32(VxHipContext* context,
                                     const VxHipPackedLinear* linear,
@@ -456,8 +457,8 @@ int vxhip_packed_linear_forward_f32_window(VxHipContext* context,
  * The bits are those of the separate launches (vxhip_rmsnorm_prepare_i8 /
  * vxhip_swiglu_prepare_i8 / vxhip_packed_linear_forward_f32, then the add).
  * Returns 1 handled; 0 declined, nothing launched (more than two rows, k above
- * 4096 (8192 without RMSNorm), k below 1024 with RMSNorm, a panel count the
- * eight-wave kernel does not take): the caller runs the separate launches;
+ * 14336, with RMSNorm above 4096 or below 1024): the caller runs the separate
+ * launches;
  * -1 on an invalid argument, which includes input rows that overlap the output
  * or the residual (every workgroup reads the whole rows while others already
  * store; add_to_dev == output_dev is the one overlap that is safe). */

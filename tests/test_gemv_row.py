@@ -51,3 +51,30 @@ def test_rows_that_are_overwritten_by_their_output(ctx, oracle, rows, k, no_allo
         assert (x.cpu().numpy().view(np.uint32) == want.view(np.uint32)).all()
     finally:
         pl.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 2])
+@pytest.mark.parametrize("bits,group", [(8, 32), (8, 128), (4, 32), (4, 128)])
+@pytest.mark.parametrize("k,n", [(1, 40), (2, 2100), (8193, 2080), (12001, 70), (14336, 2049)])
+def test_fused_swiglu_rows_at_the_ends_of_their_lengths(ctx, oracle, k, n, bits, group, rows):
+    """From a single element to the longest row, gate and up both held: the bits of the separate launches."""
+    import torch
+    import volvoxai_amd as vx
+    from volvoxai_amd.w8a8 import swiglu_prepare_i8
+    c = cases.packed_case(rows, k, n, group, k + n + bits, True)
+    w = c["w"] if bits == 8 else cases.four_bit(c["w"])
+    words = oracle.pack_w8_words(w) if bits == 8 else oracle.pack_w4_words(w)
+    pl = vx.PackedLinear(words, c["scales"], c["bias"], k, n, group, weight_bits=bits)
+    rng = np.random.default_rng(k)
+    x = torch.from_numpy(rng.normal(0, 2, (rows, 2 * k)).astype(np.float32)).cuda()
+    resid = torch.from_numpy(rng.normal(0, 1, (rows, n)).astype(np.float32)).cuda()
+    try:
+        st, y = pl.forward_a8(ctx, *swiglu_prepare_i8(ctx, x))
+        want = resid + y
+        handled, got = pl.forward_fused(ctx, x, vx.ROW_OP_SWIGLU, add_to=resid)
+        ctx.synchronize()
+        assert st == 0 and handled == 1 and "-swiglu" in ctx.last_variant, ctx.last_variant
+        assert torch.equal(got.view(torch.int32), want.view(torch.int32)), ctx.last_variant
+    finally:
+        pl.close()

@@ -64,10 +64,17 @@ __global__ __launch_bounds__(kThreads) void gemv_row_kernel(const LinearArgs a) 
     // the rows (elements past k: zeros): a thread holds the pair 2t of every 1024 elements
     float x[ROWS][NB][2], up[OP == RowOp::Swiglu ? ROWS : 1][OP == RowOp::Swiglu ? NB : 1][2], gain[OP == RowOp::Norm ? NB : 1][2];
     auto pair_of = [&](const float* src, int b, float (&v)[2]) {
-        const uint32_t j = (uint32_t)b * 1024u + threadIdx.x * 2u, at = min(j, k - 2u);
-        const v2f_any p = *reinterpret_cast<const v2f_any*>(src + at);
-        v[0] = j < k ? (j == at ? p.x : p.y) : 0.0f;
-        v[1] = j + 1u < k ? p.y : 0.0f;
+        const uint32_t j = (uint32_t)b * 1024u + threadIdx.x * 2u;
+        if constexpr (NB == 1 && OP != RowOp::Norm) {  // (such a row may be a single element)
+            const float first = src[min(j, k - 1u)], second = src[min(j + 1u, k - 1u)];
+            v[0] = j < k ? first : 0.0f;
+            v[1] = j + 1u < k ? second : 0.0f;
+        } else {
+            const uint32_t at = min(j, k - 2u);
+            const v2f_any p = *reinterpret_cast<const v2f_any*>(src + at);
+            v[0] = j < k ? (j == at ? p.x : p.y) : 0.0f;
+            v[1] = j + 1u < k ? p.y : 0.0f;
+        }
     };
 #pragma unroll
     for (int r = 0; r < ROWS; r++) {
@@ -295,7 +302,7 @@ bool launch_group(hipStream_t s, const LinearArgs& a, uint32_t ch) {
 // (16 in between at every size.)  Workgroups of eight channels pay while they are no more than the compute
 // units, N = 2048 (3.5 | 3.6 at K = 2048); past that the row operation each of them repeats outweighs them.
 const char* launch_gemv_row(hipStream_t s, const LinearArgs& a, int cu_count, const char* force, bool dry_run) {
-    if (a.mode != Epilogue::DequantF32 || !a.x_f32 || a.rows == 0u || a.rows > kMaxPrepRows || a.k < 2u ||
+    if (a.mode != Epilogue::DequantF32 || !a.x_f32 || a.rows == 0u || a.rows > kMaxPrepRows || !a.k ||
         a.k > kMaxRowLength || (a.weight_bits != 8u && a.weight_bits != 4u))
         return nullptr;
     if (a.row_gain && (a.k < kNormBlock || a.k > 4096u)) return nullptr;
