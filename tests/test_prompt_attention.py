@@ -162,3 +162,42 @@ def test_values_at_the_ends_of_the_range(ctx, rows, head_dim, t):
             want = np.matmul(p / p.sum(-1, keepdims=True), v[:, 0, :positions[i] + 1].astype(np.float64))
         assert np.allclose(got[:, i], want, rtol=2e-5, atol=5e-6, equal_nan=True), i
     assert torch.allclose(big.double(), torch.full_like(big, 3.3e38).double(), rtol=2.0 ** -18, atol=0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale", [1.0, 3.0])
+@pytest.mark.parametrize("rows,head_dim", [(2, 64), (2, 128), (40, 64), (40, 128)])
+def test_prompt_attention_error_against_float64(ctx, rows, head_dim, scale):
+    """No further from float64 than dots summed in f32 in chains of 64 channels (fused multiply-adds), a softmax in f32 and
+    values summed slot by slot.  (65,536 outputs and more: the ratio of the two errors' norms varies by about 1 %
+    from draw to draw, and a single chain of 128 channels has 1.4 times the error.)"""
+    import torch
+    import volvoxai_amd.w8a8 as vx
+    t, heads = 128, 4
+    gen = torch.Generator(device="cuda").manual_seed(head_dim + rows)
+    q = torch.randn((rows, t, heads, head_dim), generator=gen, device="cuda") * scale
+    k = torch.randn((rows, heads, t, head_dim), generator=gen, device="cuda")
+    v = torch.randn((rows, heads, t, head_dim), generator=gen, device="cuda")
+    positions = torch.arange(t, device="cuda")
+    got = vx.gqa_attention(ctx, q, k, v, positions).reshape(rows, t, heads, head_dim).transpose(1, 2).double()
+    ctx.synchronize()
+    qt, hidden = q.transpose(1, 2).contiguous(), positions[None, :] > positions[:, None]
+    fma = lambda s, a, b: (s.double() + a.double() * b.double()).float()
+    dots = []
+    for c0 in range(0, head_dim, 64):
+        s = torch.zeros((rows, heads, t, t), device="cuda")
+        for c in range(c0, c0 + 64):
+            s = fma(s, qt[..., c, None], k[:, :, None, :, c])
+        dots.append(s)
+    inverse = float(np.float32(1.0 / np.sqrt(head_dim)))
+    p = torch.softmax((sum(dots) * inverse).masked_fill(hidden, float("-inf")), -1)
+    held = torch.zeros((rows, heads, t, head_dim), device="cuda")
+    for s in range(t):
+        held = fma(held, p[..., s, None], v[:, :, None, s])
+    exact = torch.zeros((rows, heads, t, t), device="cuda", dtype=torch.float64)
+    for c in range(head_dim):
+        exact += qt[..., c, None].double() * k[:, :, None, :, c].double()
+    p64 = torch.softmax((exact / np.sqrt(head_dim)).masked_fill(hidden, float("-inf")), -1)
+    want = sum(p64[..., s, None] * v[:, :, None, s].double() for s in range(t))
+    error, held_error = (got - want).norm().item(), (held.double() - want).norm().item()
+    assert error <= 1.1 * held_error, error / held_error

@@ -1033,18 +1033,33 @@ __global__ __launch_bounds__(256, 2) void gqa_prefill_mfma_kernel(const float* _
             else fetch(IC<e - KE - VE>{}, s0 + STEP);
             __builtin_amdgcn_sched_barrier(0);
         };
-        v16f s;
+        // A dot's error grows with the length of its chain of sums: a chain for every 32 channels, joined in pairs.
+        v16f chain[HD / 32];
 #pragma unroll
-        for (int v = 0; v < 16; v++) s[v] = 0.0f;
+        for (int n = 0; n < HD / 32; n++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) chain[n][v] = 0.0f;
+        auto join = [&](int to, int from) {
+#pragma unroll
+            for (int v = 0; v < 16; v++) chain[to][v] = __fadd_rn(chain[to][v], chain[from][v]);
+        };
         static_for<KE>([&](auto e_tag) {
-            constexpr int e = decltype(e_tag)::value;
+            constexpr int e = decltype(e_tag)::value, n = e / 4;
             const float4 kv = ring[e % RING];
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.x, qreg[e].x, s, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.y, qreg[e].y, s, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.z, qreg[e].z, s, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.w, qreg[e].w, s, 0, 0, 0);
+            chain[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.x, qreg[e].x, chain[n], 0, 0, 0);
+            chain[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.y, qreg[e].y, chain[n], 0, 0, 0);
+            chain[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.z, qreg[e].z, chain[n], 0, 0, 0);
+            chain[n] = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.w, qreg[e].w, chain[n], 0, 0, 0);
+            if constexpr (HD == 128 && e == 9) join(0, 1);  // (their last sums are out of the pipe by now)
             refill(e_tag);
         });
+        if constexpr (HD == 128) {
+            join(2, 3);
+            join(0, 2);
+        } else {
+            join(0, 1);
+        }
+        v16f s = chain[0];
         auto both_halves = [&](float x) {  // the values of the two lanes that hold a query
             return __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
         };
@@ -1103,9 +1118,12 @@ __global__ __launch_bounds__(256, 2) void gqa_prefill_mfma_kernel(const float* _
             const uint32_t qi = __builtin_ctz(queries), seen = __builtin_amdgcn_readlane(visible, qi);
             const size_t at = ((size_t)(row * t + block * tq + qi / rep) * q_heads + kvh * rep + qi % rep) * HD;
             auto score = [&](uint32_t slot) {
-                float dot = 0.0f;
-                for (uint32_t c = 0; c < HD; c++) dot = __builtin_fmaf(q[at + c], kbase[(size_t)slot * HD + c], dot);
-                return __fmul_rn(dot, scale);
+                float dot[2] = {};
+                for (uint32_t c = 0; c < HD / 2u; c++)
+#pragma unroll
+                    for (uint32_t n = 0; n < 2u; n++)
+                        dot[n] = __builtin_fmaf(q[at + HD / 2u * n + c], kbase[(size_t)slot * HD + HD / 2u * n + c], dot[n]);
+                return __fmul_rn(__fadd_rn(dot[0], dot[1]), scale);
             };
             float best = -INFINITY, part = 0.0f;
             for (uint32_t slot = lane; slot < seen; slot += 64u) best = fmaxf(best, score(slot));
