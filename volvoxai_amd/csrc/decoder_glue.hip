@@ -1079,9 +1079,7 @@ __global__ __launch_bounds__(256, 2) void gqa_prefill_mfma_kernel(const float* _
         float part = 0.0f;
 #pragma unroll
         for (int v = 0; v < 16; v++) {
-            // (a slot that is not visible counts nothing, also beside a score that makes the reference NaN or infinite)
-            const uint32_t slot = s0 + 8u * (v / 4) + 4u * h + v % 4;
-            s[v] = slot < visible ? expf(s[v] - reference) : 0.0f;
+            s[v] = expf(s[v] - reference);  // (the reference is no NaN: a maximum passes them over)
             part += s[v];
         }
         const auto parts = both_halves(part);
@@ -1114,6 +1112,8 @@ __global__ __launch_bounds__(256, 2) void gqa_prefill_mfma_kernel(const float* _
     // divided first; channels ch0 .. ch0 + CH - 1, by the wavefront that stores them.
     auto recompute = [&](uint32_t queries, uint32_t ch0, auto channels_tag) {
         constexpr uint32_t CH = decltype(channels_tag)::value;
+        __threadfence_block();  // (other lanes have stored these outputs)
+        __builtin_amdgcn_s_waitcnt(0);
         for (; queries; queries &= queries - 1u) {
             const uint32_t qi = __builtin_ctz(queries), seen = __builtin_amdgcn_readlane(visible, qi);
             const size_t at = ((size_t)(row * t + block * tq + qi / rep) * q_heads + kvh * rep + qi % rep) * HD;
@@ -1153,25 +1153,19 @@ __global__ __launch_bounds__(256, 2) void gqa_prefill_mfma_kernel(const float* _
     };
 
     float* dst = out + ((size_t)(row * t + token) * q_heads + head) * HD;
-    bool finite = true;
+    float any = 0.0f;  // stays zero while the outputs are finite
     if constexpr (SPLIT == 1) {
 #pragma unroll
-        for (int v = 0; v < 16; v++)
+        for (int v = 0; v < 16; v++) {
+            out_vec y;
 #pragma unroll
             for (int c = 0; c < VW; c++) {
-                o[c][v] = __fdiv_rn(o[c][v], sum);
-                finite = finite && finite_f32(o[c][v]);
+                y[c] = __fdiv_rn(o[c][v], sum);
+                any = __builtin_fmaf(y[c], 0.0f, any);
             }
-        const uint32_t again = queries_of(visible != 0u && !finite);
-        if (visible != 0u && !(again >> r & 1u)) {
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                out_vec y;
-#pragma unroll
-                for (int c = 0; c < VW; c++) y[c] = o[c][v];
-                *reinterpret_cast<out_vec*>(dst + VW * (8u * (v / 4) + 4u * h + v % 4)) = y;
-            }
+            if (visible != 0u) *reinterpret_cast<out_vec*>(dst + VW * (8u * (v / 4) + 4u * h + v % 4)) = y;
         }
+        const uint32_t again = queries_of(visible != 0u && any != 0.0f);
         if (again) recompute(again, 0u, IC<HD>{});
     } else {
         // [wavefront][2 + 16 * VW][64]: maximum, sum, then the outputs; wavefront w merges the registers
@@ -1195,24 +1189,21 @@ __global__ __launch_bounds__(256, 2) void gqa_prefill_mfma_kernel(const float* _
             weight[w] = expf(parts[w * PART] - reference);
             total = __builtin_fmaf(parts[w * PART + 64], weight[w], total);
         }
-        out_vec y[4];
 #pragma unroll
         for (int u = 0; u < 4; u++) {
+            out_vec y;
 #pragma unroll
             for (int c = 0; c < VW; c++) {
                 float x = 0.0f;
 #pragma unroll
                 for (int w = 0; w < SPLIT; w++)
                     x = __builtin_fmaf(parts[w * PART + (2u + (4u * wave + u) * VW + c) * 64u], weight[w], x);
-                y[u][c] = __fdiv_rn(x, total);
-                finite = finite && finite_f32(y[u][c]);
+                y[c] = __fdiv_rn(x, total);
+                any = __builtin_fmaf(y[c], 0.0f, any);
             }
+            if (visible != 0u) *reinterpret_cast<out_vec*>(dst + VW * (8u * wave + 4u * h + u)) = y;
         }
-        const uint32_t again = queries_of(visible != 0u && !finite);
-        if (visible != 0u && !(again >> r & 1u)) {
-#pragma unroll
-            for (int u = 0; u < 4; u++) *reinterpret_cast<out_vec*>(dst + VW * (8u * wave + 4u * h + u)) = y[u];
-        }
+        const uint32_t again = queries_of(visible != 0u && any != 0.0f);
         if (again) recompute(again, 8u * VW * wave, IC<8 * VW>{});
     }
 }
