@@ -361,7 +361,10 @@ __global__ __launch_bounds__(WN * WM * 64, 4) void gemm_k64_f32_kernel(const Gem
     constexpr int GPB = GK == 0 ? 4 : GK == 1 ? 2 : 1;  // scale groups that end in a k-block (GK == 4: every second block)
     constexpr int SBLK = UNI ? 0 : (GPB * BN + 63) / 64;  // loads of 64 scales
     constexpr int WLOADS = (WBLK + NWAVES - 1) / NWAVES, XLOADS = (XBLK + NWAVES - 1) / NWAVES;
-    constexpr int SLOADS = (SBLK + NWAVES - 1) / NWAVES;
+    // Wide wave tiles: the first SBLK waves load 64 scales each (and wait for one load more than they must), since a
+    // repeated load for the others costs more than that: 1137 x 6912 -> 2752 with groups of 256 66.0 -> 63.2 us.
+    constexpr bool SOME_LOAD_SCALES = TN * TM > 4 && SBLK <= NWAVES;
+    constexpr int SLOADS = SOME_LOAD_SCALES ? 0 : (SBLK + NWAVES - 1) / NWAVES;
     constexpr int SCALE_OFF = (WBLK + XBLK) * 1024;
     constexpr int STAGE_BYTES = SCALE_OFF + SBLK * 256;
     constexpr int NLOADS = WLOADS + XLOADS + SLOADS;
@@ -397,13 +400,19 @@ __global__ __launch_bounds__(WN * WM * 64, 4) void gemm_k64_f32_kernel(const Gem
     const uint32_t nkb = (ksteps_real + KS - 1) / KS;
     auto issue_block = [&](uint32_t kb, int stage) {
         char* base = lds_raw + stage * STAGE_BYTES;
+        // the scales of the groups that end in this k-block, [group][channel]: 4 bytes per lane
+        auto scales = [&](uint32_t b) {
+            const uint32_t e = b * 64u + lane, slot = e / BN;
+            const uint32_t g = GK == 0 ? kb * 4u + slot : GK == 1 ? kb * 2u + slot : GK == 2 ? kb : kb / 2u;
+            load_to_lds4(a.scales_t + (size_t)min(g, a.groups - 1u) * a.n_pad + n0 + e % BN, base + SCALE_OFF + b * 256);
+        };
+        if constexpr (SOME_LOAD_SCALES) {
+            if (wave < SBLK) scales(wave);
+        }
         static_for<NLOADS>([&](auto t_tag) {
             constexpr int t = decltype(t_tag)::value;
             if constexpr (t < SLOADS) {
-                // the scales of the groups that end in this k-block, [group][channel]: 4 bytes per lane
-                const uint32_t b = (wave + t * NWAVES) % (SBLK > 0 ? SBLK : 1), e = b * 64u + lane;
-                const uint32_t slot = e / BN, g = GK == 0 ? kb * 4u + slot : GK == 1 ? kb * 2u + slot : GK == 2 ? kb : kb / 2u;
-                load_to_lds4(a.scales_t + (size_t)min(g, a.groups - 1u) * a.n_pad + n0 + e % BN, base + SCALE_OFF + b * 256);
+                scales((wave + t * NWAVES) % (SBLK > 0 ? SBLK : 1));
             } else if constexpr (t < SLOADS + WLOADS) {
                 const uint32_t b = (wave + (t - SLOADS) * NWAVES) % WBLK;
                 const int8_t* src = w_tile + (size_t)(b / KB) * panel_bytes + (size_t)(kb * KB + b % KB) * 1024u;
