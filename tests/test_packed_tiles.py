@@ -38,3 +38,29 @@ def test_narrow_tiles_at_their_edges(ctx, oracle, rows, k, n, group, bits, group
         vx.force_variant(None)
         pl.close()
     assert seen == {"t64x64k64", "t64x32k64", "t32x32k64"}, seen
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("k", [100, 256, 300, 512, 641, 1024])
+def test_wide_tiles_in_groups_of_256(ctx, oracle, k, bits):
+    """One to eight k-blocks, the last group one or two of them: the oracle's bits."""
+    import torch
+    import volvoxai_amd as vx
+    rows, n = 161, 140
+    c = cases.packed_case(rows, k, n, 256, k + bits, True)
+    w = c["w"] if bits == 8 else cases.four_bit(c["w"])
+    words = oracle.pack_w8_words(w) if bits == 8 else oracle.pack_w4_words(w)
+    _, want = oracle.packed_linear(c["x"], words, c["scales"], c["bias"], n, 256, bits=bits)
+    pl = vx.PackedLinear(words, c["scales"], c["bias"], k, n, 256, weight_bits=bits)
+    x = torch.from_numpy(c["x"]).cuda()
+    try:
+        for tile in ["t128x128k64"] + ["t128x256k64s3"] * (bits == 8):
+            vx.force_variant("a8-mfma." + tile)
+            st, y = pl.forward_f32(ctx, x)
+            ctx.synchronize()
+            assert st == 0 and ctx.last_variant.endswith(tile), ctx.last_variant
+            assert (y.cpu().numpy().view(np.uint32) == want.view(np.uint32)).all(), ctx.last_variant
+    finally:
+        vx.force_variant(None)
+        pl.close()

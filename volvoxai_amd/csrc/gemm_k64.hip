@@ -501,8 +501,9 @@ __global__ __launch_bounds__(WN * WM * 64, 4) void gemm_k64_f32_kernel(const Gem
     static_for<NS - 1>([&](auto b_tag) { issue_block(min((uint32_t)decltype(b_tag)::value, nkb - 1u), decltype(b_tag)::value); });
     int cur = 0, refill = NS - 1;
     const v4i zero = {0, 0, 0, 0};
-    auto k_block = [&](uint32_t kb, auto ends_tag) {
+    auto k_block = [&](uint32_t kb, auto ends_tag, auto odd_tag) {
         constexpr bool ENDS = decltype(ends_tag)::value;  // may be the last k-block, with fewer groups
+        constexpr bool ODD = decltype(odd_tag)::value;    // GK == 4: the second half of a group
         wait_vmcnt<(NS - 2) * NLOADS>();
         wg_barrier();
         issue_block(min(kb + NS - 1u, nkb - 1u), refill);
@@ -550,7 +551,7 @@ __global__ __launch_bounds__(WN * WM * 64, 4) void gemm_k64_f32_kernel(const Gem
                     }
                 }
                 // first MFMA step of a scale group: accumulate onto zero instead of clearing registers
-                const bool fresh = GK == 1 || (GK == 2 && s == 0) || (GK == 4 && s == 0 && (kb & 1u) == 0u);
+                const bool fresh = GK == 1 || (GK == 2 && s == 0) || (GK == 4 && s == 0 && !ODD);
 #pragma unroll
                 for (int i = 0; i < TN; i++)
 #pragma unroll
@@ -563,7 +564,7 @@ __global__ __launch_bounds__(WN * WM * 64, 4) void gemm_k64_f32_kernel(const Gem
                 } else if constexpr (GK == 2) {
                     if (s == 1) fold(stage, 0);
                 } else {
-                    if (s == 1 && ((kb & 1u) == 1u || (ENDS && kb + 1u == nkb))) fold(stage, 0);
+                    if (s == 1 && (ODD || ENDS)) fold(stage, 0);
                 }
             }
         }
@@ -571,13 +572,22 @@ __global__ __launch_bounds__(WN * WM * 64, 4) void gemm_k64_f32_kernel(const Gem
         cur = cur + 1 == NS ? 0 : cur + 1;
     };
     // (narrow wave tiles take the last k-block by itself, so that nothing in the others is conditional; the wide
-    // ones would spill)
+    // ones would spill.  Groups of 256 take two k-blocks a round: with the half of the group as a condition of the loop
+    // 995 x 4224 -> 3168 takes 45.5 us.)
     constexpr bool PEEL = TN * TM <= 4;
     uint32_t kb = 0;
-    if constexpr (PEEL) {
-        for (; kb + 1u < nkb; kb++) k_block(kb, std::false_type{});
+    if constexpr (GK == 4) {
+        for (; kb + 1u < nkb; kb += 2u) {
+            k_block(kb, std::false_type{}, std::false_type{});
+            k_block(kb + 1u, std::false_type{}, std::true_type{});
+        }
+        if (kb < nkb) k_block(kb, std::true_type{}, std::false_type{});
+    } else {
+        if constexpr (PEEL) {
+            for (; kb + 1u < nkb; kb++) k_block(kb, std::false_type{}, std::false_type{});
+        }
+        for (; kb < nkb; kb++) k_block(kb, std::true_type{}, std::false_type{});
     }
-    for (; kb < nkb; kb++) k_block(kb, std::true_type{});
     wait_vmcnt<0>();
 
     // ---- epilogue: + bias, 16-byte stores (a lane owns row l%16 and four consecutive channels) ----
