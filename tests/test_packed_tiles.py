@@ -64,3 +64,30 @@ def test_wide_tiles_in_groups_of_256(ctx, oracle, k, bits):
     finally:
         vx.force_variant(None)
         pl.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,k,n,bits,group,grouped,tile", [
+    (333, 256, 14336, 8, 128, True, "t128x128k64"),     # the fold costs both tiles the same
+    (333, 256, 14336, 8, 128, False, "t64x64k64"),      # the products fit beside the narrow tile alone
+    (874, 4096, 5920, 8, 64, False, "t128x128k64"),
+    (874, 4096, 5920, 8, 128, False, "t128x256k64s3"),
+    (235, 256, 5120, 4, 128, True, "t32x32k64"),
+    (235, 256, 5120, 4, 256, True, "t64x32k64"),
+])
+def test_the_tile_follows_the_fold(ctx, rows, k, n, bits, group, grouped, tile):
+    """The lines of the rule at 256 compute units, where each side was the faster one."""
+    import torch
+    import volvoxai_amd as vx
+    from volvoxai_amd.decoder import pack_w4_words, pack_w8_words
+    rng = np.random.default_rng(rows)
+    words = (pack_w8_words if bits == 8 else pack_w4_words)(rng.integers(-7, 8, (n, k)).astype(np.int8))
+    scales = np.full((n, (k + group - 1) // group), 0.01, np.float32)
+    scales[0, 0] += grouped * 0.001
+    pl = vx.PackedLinear(words, scales, np.zeros(n, np.float32), k, n, group, weight_bits=bits)
+    try:
+        st, _ = pl.forward_f32(ctx, torch.ones((rows, k), device="cuda"))
+        ctx.synchronize()
+        assert st == 0 and ctx.last_variant.endswith(tile), ctx.last_variant
+    finally:
+        pl.close()

@@ -735,24 +735,33 @@ const char* launch_gemm_k64_f32(hipStream_t s, const LinearArgs& a, F32Tile tile
 //                           1000 x 8192 -> 1024   40.2 | 37.2 | 40.7 (46.4)   128 x 3000 -> 5001   16.5 | 15.3 | 13.8 (19.7)
 //   4 bits, groups of 32    64 x 4096 -> 4096     40.8 | 27.1 | 19.1 (54.9)   333 x 3000 -> 5001   41.0 | 40.0 | 39.2 (67.1)
 //                           512 x 4096 -> 4096    52.1 | 51.1 | 54.2 (94.2)   1024 x 3000 -> 5001  82.3 | 88.6 | 94.4 (227)
-// The lines: 1.5 workgroups of a tile per compute unit.
-// Past them the 128-channel tiles against 64x64, by how many a compute unit gets (in units of one 128x128 tile;
-// an odd one of those has no second workgroup to take turns with, four 64x64 tiles cost 1.2 of it -- 1.07 with four-bit
-// weights -- and one 128x256 tile 1.75 where its products fit the registers).  64x64 | 128x128 | 128x256, 8 bits,
-// one scale per channel:
+// The lines: 1.5 workgroups of a tile per compute unit; 2.5 of 64x32 with four-bit weights in groups of up to 128, whose
+// operands take longest to spread (235 x 2048 -> 5120 16.2 | 15.3 | 14.8, 302 x 9728 -> 3584 51.7 | 50.9 | 47.5).
+// Past them the 128-channel tiles against 64x64, by how many a compute unit gets, in units of one 128x128 tile (an odd
+// one of those has no second workgroup to take turns with).  What a 64x64 tile costs of it depends on the fold:
+// where both have the products s_a * s_w or neither, 0.345; one scale per channel in groups of 128, whose products
+// fit the registers beside the narrow tile alone, 0.3; four-bit weights 0.29.  64x64 | 128x128 | 128x256, 8 bits,
+// one scale per channel, groups of 128:
 //   1024 x 3000 -> 5001  43.8 | 52.7         700 x 1024 -> 4096   14.0 | 16.9 | 21.0   4096 x 1024 -> 4096  47.0 | 43.7 | 48.0
 //   333 x 4096 -> 14336  48.9 | 55.9 | 53.4  700 x 4096 -> 14336  77.7 | 81.4 | 89.9   2048 x 14336 -> 4096  211 | 195 | 172
-// 4 bits, groups of 128:  4096 x 2048 -> 1024  33.1 | 36.9   700 x 4096 -> 14336  88.5 | 96.5   2048 x 4096 -> 14336  230 | 214
+// scales of their own for every group: 1323 x 1536 -> 12800  68.8 | 62.4, 670 x 7072 -> 8832  98.5 | 91.1; groups of 256:
+// 1582 x 4768 -> 3616  68.9 | 59.9.  4 bits, groups of 128:  4096 x 2048 -> 1024  33.1 | 36.9
+//   700 x 4096 -> 14336  88.5 | 96.5   2048 x 4096 -> 14336  230 | 214   806 x 1024 -> 13824  34.4 | 33.8
+// A 128x256 tile costs 1.75 of a 128x128 one where its products fit the registers and that one's do not: groups of
+// 128.  (Groups of 64, where both have them: 2044 x 7040 -> 7616  233 | 197 | 207, 874 x 4288 -> 5920  65.7 | 64.4 | 68.8.)
 F32Tile pick_f32_tile(const LinearArgs& a, int cu_count) {
     const auto tiles = [&](uint32_t bn, uint32_t bm) { return (uint64_t)((a.n + bn - 1) / bn) * ((a.rows + bm - 1) / bm); };
     const uint64_t cu = (uint64_t)cu_count, busy = cu * 3 / 2;
-    if (tiles(64, 64) < busy) return tiles(64, 32) < busy ? F32Tile::T32x32 : F32Tile::T64x32;
+    const bool four = a.weight_bits == 4u;
+    if (tiles(64, 64) < busy)
+        return tiles(64, 32) < (four && a.group_size <= 128u ? cu * 5 / 2 + 1u : busy) ? F32Tile::T32x32 : F32Tile::T64x32;
     if (a.group_size < 64u) return F32Tile::T64x64;
     const auto per_cu = [&](uint64_t t) { return (t + cu - 1) / cu; };
     const uint64_t c128 = per_cu(tiles(128, 128));
-    const float narrow = (float)per_cu(tiles(64, 64)) * (a.weight_bits == 4u ? 0.2675f : 0.3f);
-    const float wide = (float)c128 + (c128 % 2 ? 0.15f : 0.0f);
-    if (a.uniform_group_scales && a.weight_bits == 8u && a.group_size <= 128u && a.k >= 4096u) {
+    const bool narrow_products = !four && a.uniform_group_scales && a.group_size == 128u;
+    const float narrow = (float)per_cu(tiles(64, 64)) * (four ? 0.29f : narrow_products ? 0.3f : 0.345f);
+    const float wide = (float)c128 + (c128 % 2 ? (four ? 0.2f : 0.1f) : 0.0f);
+    if (a.uniform_group_scales && a.weight_bits == 8u && a.group_size == 128u && a.k >= 4096u) {
         const float deep = 1.75f * (float)per_cu(tiles(128, 256));
         if (deep < wide && deep < narrow) return F32Tile::T128x256;
     }
