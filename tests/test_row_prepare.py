@@ -66,6 +66,14 @@ def test_row_kernels_at_their_edges(oracle, op, d, rows):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("op", ["plain", "norm", "swiglu"])
+@pytest.mark.parametrize("d", [5121, 6144, 6146, 8196, 10240, 10243, 12288, 12291])
+def test_many_long_rows(oracle, op, d):
+    """More rows than compute units, lengths on both sides of every number of passes."""
+    test_row_kernels_at_their_edges(oracle, op, d, 259)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows,d", [(3, 1022), (32, 2048), (300, 4099)])
 def test_residual_add_rides_in_front_of_the_norm(ctx, rows, d):
     import torch

@@ -13,11 +13,12 @@
 //
 // Few rows are bound by latency: a launch, the row's first touch, a reduction or two.  So a thread holds its
 // elements in registers from the load to the codes (16-byte loads, all requested before the first is used; four
-// codes per store), a reduction costs one barrier, nothing but its slots is in LDS, and a workgroup has no more
-// wavefronts than the row has 16-byte pieces.  In a recorded decode step of 32 rows, cost per launch against
+// codes per store), a reduction costs one barrier, nothing but its slots is in LDS, and a workgroup has four
+// wavefronts or, of more, no more than the row has 64 16-byte pieces.  In a recorded decode step of 32 rows, cost per launch against
 // kernels that walked LDS copies of the row an element at a time with 1024 threads: RMSNorm of 1024 elements
 // 4.65 -> 3.0 us, SwiGLU of 3072 4.5 -> 3.3, plain 2048 3.8 -> 2.9 (a launch that reads one row of its
-// predecessor and writes it back costs 2.2-2.9).  Many rows are bound by the rows' bytes.
+// predecessor and writes it back costs 2.2-2.9).  Many rows are bound by the rows' bytes
+// beside the exact divisions, some twenty instructions an element: 2048 x 14336 27.0 us, 5.4 TB/s.
 #include "common.h"
 #include "device_math.h"
 #include "row_math.h"
@@ -67,8 +68,8 @@ __device__ __forceinline__ void row_store(float* dst, uint32_t j, uint32_t d, co
     }
 }
 
-// T threads, NB passes of 4 * T elements held in registers; WHOLE: rows and their codes are whole groups of four.  Plain rows may be longer than that: the rest is read
-// again for its codes.
+// T threads, NB passes of 4 * T elements held in registers; WHOLE: rows and their codes are whole groups of four.
+// Plain rows may be longer than that: the rest is read again for its codes.
 template <RowOp OP, int T, int NB, bool WHOLE>
 __global__ __launch_bounds__(T) void row_prepare_kernel(const RowArgs a) {
     static_assert(OP != RowOp::Norm || T == 256, "the sum of squares is ordered for 16 bytes a thread of 256");
@@ -149,13 +150,17 @@ __global__ __launch_bounds__(T) void row_prepare_kernel(const RowArgs a) {
     float scale = maximum == 0.0f || bad ? 1.0f : __fdiv_rn(maximum, 127.0f);
     if (scale < 0x1p-126f) scale = 0x1p-126f;
     // (elements past d are zeros: the padding of the row's last 16-byte chunk, where the layout has one)
-    auto put = [&](uint32_t j, const v4f& t) {
+    // (a thread's codes of neighbouring passes are as far apart in either layout, whatever the row)
+    int8_t* const first = a.codes + activation_offset(a.layout, row, threadIdx.x * 4u);
+    const uint32_t step = 4u * T * (a.layout.operand_order ? kOperandOrderRows : 1u);
+    auto put = [&](uint32_t i, const v4f& t) {
+        const uint32_t j = at((int)i);
         if (j >= a.layout.ld) return;
         uint32_t q = 0u;
         if (!bad)
             q = pack4_bytes(packed_round_i8(__fdiv_rn(t[0], scale)), packed_round_i8(__fdiv_rn(t[1], scale)),
                             packed_round_i8(__fdiv_rn(t[2], scale)), packed_round_i8(__fdiv_rn(t[3], scale)));
-        int8_t* dst = a.codes + activation_offset(a.layout, row, j);
+        int8_t* dst = first + i * (size_t)step;
         if (WHOLE || j + 4u <= a.layout.ld) {
             *reinterpret_cast<u32_any*>(dst) = q;
         } else {
@@ -163,22 +168,26 @@ __global__ __launch_bounds__(T) void row_prepare_kernel(const RowArgs a) {
         }
     };
 #pragma unroll
-    for (int i = 0; i < NB; i++) put(at(i), v[i]);
+    for (int i = 0; i < NB; i++) put((uint32_t)i, v[i]);
     if constexpr (OP == RowOp::Plain)
-        for (uint32_t j = at(NB); j < a.layout.ld; j += 4u * T) put(j, row_load<WHOLE>(src, j, d));
+        for (uint32_t i = NB; at((int)i) < a.layout.ld; i++) put(i, row_load<WHOLE>(src, at((int)i), d));
     if (threadIdx.x == 0) a.scales[row] = bad ? __builtin_nanf("") : scale;
 }
 
 template <RowOp OP, int T, int NB>
 void launch(hipStream_t s, uint32_t rows, const RowArgs& a) {
+    // (Rows of 6145 to 10240 elements: LDS that nobody uses, so that six workgroups share a compute unit and not eight.
+    // With all rows of a launch resident every one of them loads first and computes then; 2048 x 8192 15.7 against 16.7 us.)
+    const size_t lds = OP == RowOp::Plain && T == 256 && (NB == 8 || NB == 10) ? 26u * 1024u : 0u;
     // (a row's codes end where the row does or at the end of a 16-byte chunk)
     if (a.d % 4u == 0u && a.layout.ld % 4u == 0u)
-        hipLaunchKernelGGL((row_prepare_kernel<OP, T, NB, true>), dim3(rows), dim3(T), 0, s, a);
+        hipLaunchKernelGGL((row_prepare_kernel<OP, T, NB, true>), dim3(rows), dim3(T), lds, s, a);
     else
-        hipLaunchKernelGGL((row_prepare_kernel<OP, T, NB, false>), dim3(rows), dim3(T), 0, s, a);
+        hipLaunchKernelGGL((row_prepare_kernel<OP, T, NB, false>), dim3(rows), dim3(T), lds, s, a);
 }
 
-// Many rows: 256 threads, as many passes as the row has.  Few rows (no more than compute units) leave a
+// Many rows: 256 threads, as many passes as the row has (or one more: an idle pass costs 2-4 %, 1246 x 9216 in fourteen
+// passes 12.3 us, in ten 11.6).  Few rows (no more than compute units) leave a
 // workgroup alone on its compute unit and latency bound: then as many threads as the row has 16-byte
 // pieces, up to 1024.
 template <RowOp OP>
@@ -197,7 +206,10 @@ void launch_op(hipStream_t s, uint32_t rows, const RowArgs& a) {
     else if (d <= 2048u) launch<OP, 256, 2>(s, rows, a);
     else if (d <= 3072u) launch<OP, 256, 3>(s, rows, a);
     else if (d <= 4096u) launch<OP, 256, 4>(s, rows, a);
+    else if (d <= 6144u) launch<OP, 256, 6>(s, rows, a);
     else if (d <= 8192u) launch<OP, 256, 8>(s, rows, a);
+    else if (d <= 10240u) launch<OP, 256, 10>(s, rows, a);
+    else if (d <= 12288u) launch<OP, 256, 12>(s, rows, a);
     else if (d <= 14336u) launch<OP, 256, 14>(s, rows, a);
     else launch<OP, 256, 15>(s, rows, a);
 }
