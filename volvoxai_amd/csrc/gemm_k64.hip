@@ -362,7 +362,8 @@ __global__ __launch_bounds__(WN * WM * 64, 4) void gemm_k64_f32_kernel(const Gem
     constexpr int SBLK = UNI ? 0 : (GPB * BN + 63) / 64;  // loads of 64 scales
     constexpr int WLOADS = (WBLK + NWAVES - 1) / NWAVES, XLOADS = (XBLK + NWAVES - 1) / NWAVES;
     // Wide wave tiles: the first SBLK waves load 64 scales each (and wait for one load more than they must), since a
-    // repeated load for the others costs more than that: 1137 x 6912 -> 2752 with groups of 256 66.0 -> 63.2 us.
+    // repeated load for the others costs more than that: 619 x 9500 -> 9861 in groups of 128 121.9 -> 119.1 us (none to
+    // see in groups of 64 and 256).
     constexpr bool SOME_LOAD_SCALES = TN * TM > 4 && SBLK <= NWAVES;
     constexpr int SLOADS = SOME_LOAD_SCALES ? 0 : (SBLK + NWAVES - 1) / NWAVES;
     constexpr int SCALE_OFF = (WBLK + XBLK) * 1024;
@@ -573,7 +574,7 @@ __global__ __launch_bounds__(WN * WM * 64, 4) void gemm_k64_f32_kernel(const Gem
     };
     // (narrow wave tiles take the last k-block by itself, so that nothing in the others is conditional; the wide
     // ones would spill.  Groups of 256 take two k-blocks a round: with the half of the group as a condition of the loop
-    // 995 x 4224 -> 3168 takes 45.5 us.)
+    // 995 x 4224 -> 3168 takes 45.0 us, so 37.8; 1137 x 6912 -> 2752 65.9 and 55.0.)
     constexpr bool PEEL = TN * TM <= 4;
     uint32_t kb = 0;
     if constexpr (GK == 4) {
