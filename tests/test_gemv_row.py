@@ -33,6 +33,14 @@ def test_rows_at_the_edges_of_the_instances(ctx, oracle, k, n, bits, group, rows
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 2])
+@pytest.mark.parametrize("bits,group", [(8, 32), (8, 256), (4, 32), (4, 128)])
+@pytest.mark.parametrize("k,n", [(4608, 40), (6144, 33), (6145, 31), (8193, 64), (10240, 40), (10241, 31), (12288, 33), (12289, 8)])
+def test_long_rows_at_the_edges_of_the_instances(ctx, oracle, k, n, bits, group, rows):
+    test_rows_at_the_edges_of_the_instances(ctx, oracle, k, n, bits, group, rows)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("no_alloc", [False, True])
 @pytest.mark.parametrize("rows,k", [(1, 1024), (2, 10240)])
 def test_rows_that_are_overwritten_by_their_output(ctx, oracle, rows, k, no_alloc):

@@ -50,7 +50,10 @@ struct PackedWeight {
 
 constexpr uint32_t kPanelRows = 32, kStepK = 32, kPanelPad = 8, kStepPad = 4;
 constexpr uint32_t kMaxGemvRows = 32;  // the MFMA operand has 32 row slots
-constexpr uint32_t kMaxPrepRows = 2;   // f32 rows a GEMV workgroup prepares by itself (every workgroup repeats them; measured: one and two rows are faster that way than as two launches, four are not)
+// f32 rows a GEMV workgroup prepares by itself (every workgroup repeats them).  One and two rows are faster that way than
+// as two launches at every length and width measured, up to 14336 x 14336 (gemv_row.hip; 2 x 13169 -> 10240 even: 40.7
+// against 39.9 us, most others 1.1 to 1.7 times as fast); four were not in a kernel before it.
+constexpr uint32_t kMaxPrepRows = 2;
 
 enum FaultBits : uint32_t {
     kFaultBadMultiplier = 1u,   // a requantization multiplier was not finite and positive

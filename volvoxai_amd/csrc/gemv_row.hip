@@ -212,8 +212,8 @@ __global__ __launch_bounds__(kThreads) void gemv_row_kernel(const LinearArgs a) 
             for (int s = 0; s < NSUB; s++) {
                 uint32_t v = (uint32_t)acc[r][s];
                 if constexpr (CH == 8) v += (uint32_t)lane_exchange<kDppRowRor8>((int)v);
-                if constexpr (CH == 16 || (CH == 8 && MEET >= 2)) v += lane_down16(v);
-                if constexpr (CH == 32 || (CH == 16 && MEET >= 2) || (CH == 8 && MEET == 4)) v += lane_down32(v);
+                if constexpr (CH == 8 && MEET >= 2) v += lane_down16(v);
+                if constexpr (CH == 32 || MEET == 4) v += lane_down32(v);
                 const int32_t dot = W4 ? (int32_t)v >> 4 : (int32_t)v;
                 if (leads && group + s < a.groups)
                     products[((group + s) * ROWS + r) * CH + c] = __fmul_rn((float)dot, __fmul_rn(rs[r], sw[u][s]));
@@ -255,12 +255,19 @@ bool launch_rows(hipStream_t s, const LinearArgs& a) {
     return a.rows == 1u ? launch<OP, GK, W4, CH, NB, 1>(s, a) : launch<OP, GK, W4, CH, NB, 2>(s, a);
 }
 
+// Lengths between the instances pay for the padding: two rows of 8704 -> 3086 took 21.5 us on the instance of 14336, 17.0
+// on that of 10240 (as two launches 18.9); of 4608 -> 2496 13.1 on that of 8192, 10.6 on that of 6144 (11.8).
 template <RowOp OP, int GK, bool W4, int CH>
 bool launch_length(hipStream_t s, const LinearArgs& a) {
     if (a.k <= 1024u) return launch_rows<OP, GK, W4, CH, 1>(s, a);
     if (a.k <= 2048u) return launch_rows<OP, GK, W4, CH, 2>(s, a);
     if (a.k <= 3072u) return launch_rows<OP, GK, W4, CH, 3>(s, a);
     if (a.k <= 4096u) return launch_rows<OP, GK, W4, CH, 4>(s, a);
+    if constexpr (OP == RowOp::Plain) {
+        if (a.k <= 6144u) return launch_rows<OP, GK, W4, CH, 6>(s, a);
+        if (a.k > 8192u && a.k <= 10240u) return launch_rows<OP, GK, W4, CH, 10>(s, a);
+        if (a.k > 8192u && a.k <= 12288u) return launch_rows<OP, GK, W4, CH, 12>(s, a);
+    }
     if constexpr (OP != RowOp::Norm) {
         if (a.k <= 8192u) return launch_rows<OP, GK, W4, CH, 8>(s, a);
         return launch_rows<OP, GK, W4, CH, 14>(s, a);
