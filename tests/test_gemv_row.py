@@ -86,3 +86,26 @@ def test_fused_swiglu_rows_at_the_ends_of_their_lengths(ctx, oracle, k, n, bits,
         assert torch.equal(got.view(torch.int32), want.view(torch.int32)), ctx.last_variant
     finally:
         pl.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,k,n,bits,group,route", [
+    (1, 8193, 4096, 8, 128, "row8-prep"), (1, 8193, 4097, 8, 128, "row32-prep"), (2, 8193, 4096, 8, 128, "row32-prep"),
+    (1, 8192, 4096, 8, 128, "row32-prep"), (1, 4097, 4096, 4, 32, "row8-prep"), (1, 4097, 4096, 4, 64, "row32-prep"),
+])
+def test_channels_of_a_workgroup(ctx, oracle, rows, k, n, bits, group, route):
+    """One long row goes on with eight channels a workgroup to N = 4096 (256 compute units): the oracle's bits there."""
+    import torch
+    import volvoxai_amd as vx
+    c = cases.packed_case(rows, k, n, group, k + n, True)
+    w = c["w"] if bits == 8 else cases.four_bit(c["w"])
+    words = oracle.pack_w8_words(w) if bits == 8 else oracle.pack_w4_words(w)
+    _, want = oracle.packed_linear(c["x"], words, c["scales"], c["bias"], n, group, bits=bits)
+    pl = vx.PackedLinear(words, c["scales"], c["bias"], k, n, group, weight_bits=bits)
+    try:
+        st, y = pl.forward_f32(ctx, torch.from_numpy(c["x"]).cuda())
+        ctx.synchronize()
+        assert st == 0 and ctx.last_variant.endswith(route), ctx.last_variant
+        assert (y.cpu().numpy().view(np.uint32) == want.view(np.uint32)).all()
+    finally:
+        pl.close()

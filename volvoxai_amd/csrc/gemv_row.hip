@@ -307,14 +307,20 @@ bool launch_group(hipStream_t s, const LinearArgs& a, uint32_t ch) {
 //   4096    4.4 |  5.8    6.5 |  6.5    8.3 |  7.2   14.6 | 11.1
 //   14336   9.8 | 14.7   15.5 | 16.9   22.6 | 19.5   44.1 | 35.0
 // (16 in between at every size.)  Workgroups of eight channels pay while they are no more than the compute
-// units, N = 2048 (3.5 | 3.6 at K = 2048); past that the row operation each of them repeats outweighs them.
+// units, N = 2048 (3.5 | 3.6 at K = 2048); past that the row operation each of them repeats outweighs them.  Two rows, four
+// bits and the other groups have that line at the same place (2 x 4096 -> 2560, 4 bits 6.6 | 6.0; 2 x 1536 -> 1760 3.8 | 4.1).
+// One row goes on with them to twice as many where the weights of a channel, or its products, are many: eight bits past
+// K = 8192 (12768 -> 3136 13.3 | 15.2, 9728 -> 2560 10.1 | 11.0; four bits 1.0 to 1.1 times the other) and groups of 32
+// past 4096 (4352 -> 2784 7.7 | 8.2, four bits 5632 -> 3579 7.9 | 8.6).
 const char* launch_gemv_row(hipStream_t s, const LinearArgs& a, int cu_count, const char* force, bool dry_run) {
     if (a.mode != Epilogue::DequantF32 || !a.x_f32 || a.rows == 0u || a.rows > kMaxPrepRows || !a.k ||
         a.k > kMaxRowLength || (a.weight_bits != 8u && a.weight_bits != 4u))
         return nullptr;
     if (a.row_gain && (a.k < kNormBlock || a.k > 4096u)) return nullptr;
     const uint32_t panels = (a.n + 31u) / 32u;
-    uint32_t ch = panels * 4u <= (uint32_t)cu_count ? 8u : 32u;
+    const bool many = a.rows == 1u && !a.row_swiglu &&
+                      ((a.weight_bits == 8u && a.k > 8192u) || (a.group_size == 32u && a.k > 4096u));
+    uint32_t ch = panels * (many ? 2u : 4u) <= (uint32_t)cu_count ? 8u : 32u;
     if (force && strstr(force, "row8")) ch = 8u;
     else if (force && strstr(force, "row32")) ch = 32u;
     if (!dry_run && !(a.weight_bits == 4u ? launch_group<true>(s, a, ch) : launch_group<false>(s, a, ch))) return nullptr;
