@@ -597,39 +597,29 @@ template <int MODE, int GK, bool W4 = false>
 const char* dispatch_tile(hipStream_t s, const LinearArgs& a, int cu_count, const char* force) {
     auto forced = [&](const char* tag) { return force && strstr(force, tag) != nullptr; };
     if constexpr (MODE == (int)Epilogue::DequantF32) {
-        // int32 tile accumulators plus f32 running sums: the wave tile is at most 64x64, and with
-        // a scale group per k-step the eight-wave tile runs out of registers.
-        const auto tiles = [&](uint32_t bn, uint32_t bm) {
-            return (uint64_t)((a.n + bn - 1) / bn) * ((a.rows + bm - 1) / bm);
-        };
-        const uint64_t enough = (uint64_t)cu_count * 3 / 4;
-        int pick = a.rows <= 64u ? 3 : tiles(128, 256) >= enough && GK > 1 ? 0 : tiles(128, 128) >= enough ? 1
-                   : tiles(64, 128) >= enough ? 2 : 3;
-        // The 16x16x64 kernel of gemm_k64.hip, unless a tile of this file is named (or it declines).
-        if (forced("k64") || !(forced("t256x") || forced("t128x") || forced("t64x"))) {
+        // The 16x16x64 kernel of gemm_k64.hip takes every launch.  The tiles of this file, its predecessors, run when
+        // one is named and serve as a second kernel to compare bits with.
+        const bool named = forced("t256x") || forced("t128x") || forced("t64x");
+        if (forced("k64") || !named) {
             const F32Tile tile = forced("t128x256k64") ? (a.weight_bits == 8u ? F32Tile::T128x256 : F32Tile::T128x128)
                                  : forced("t64x64k64") ? F32Tile::T64x64
                                  : forced("t64x32k64") ? F32Tile::T64x32
                                  : forced("t32x32k64") ? F32Tile::T32x32
                                  : forced("k64")       ? F32Tile::T128x128
                                                        : pick_f32_tile(a, cu_count);
-            if (const char* t = launch_gemm_k64_f32(s, a, tile)) return t;
+            const char* t = launch_gemm_k64_f32(s, a, tile);
+            if (t || !named) return t;
         }
-        if (forced("t256x256")) pick = GK > 1 ? 0 : 1;
-        if (forced("t128x128")) pick = 1;
-        if (forced("t64x128")) pick = 2;
-        if (forced("t64x64")) pick = 3;
+        // int32 tile accumulators plus f32 running sums: the wave tile is at most 64x64, and with
+        // a scale group per k-step the eight-wave tile runs out of registers.
         if constexpr (GK == KS) {
-            // one group per k-block: eight waves of 64x32 fold in the shadow of their MFMAs.  Measured
-            // against the plain 128x128 tile: 30 against 42 us at 4096x3072 -> 1024, 36 against 50 us
-            // at 256x4096 -> 14336; the 128x256 tile stays ahead where there is work for it.
-            if ((pick == 1 && !forced("t128x128")) || forced("t128x128p"))
-                return launch_cfg<2, 4, 2, 1, MODE, GK, W4>(s, a) ? "t128x128p" : nullptr;
+            // one group per k-block: eight waves of 64x32 fold in the shadow of their MFMAs
+            if (forced("t128x128p")) return launch_cfg<2, 4, 2, 1, MODE, GK, W4>(s, a) ? "t128x128p" : nullptr;
         }
-        if (pick == 0) return launch_cfg<2, 4, 2, 2, MODE, GK, W4>(s, a) ? "t128x256" : nullptr;
-        if (pick == 1) return launch_cfg<2, 2, 2, 2, MODE, GK, W4>(s, a) ? "t128x128" : nullptr;
-        if (pick == 2) return launch_cfg<2, 2, 1, 2, MODE, GK, W4>(s, a) ? "t64x128" : nullptr;
-        return launch_cfg<2, 2, 1, 1, MODE, GK, W4>(s, a) ? "t64x64" : nullptr;
+        if (forced("t64x128")) return launch_cfg<2, 2, 1, 2, MODE, GK, W4>(s, a) ? "t64x128" : nullptr;
+        if (forced("t64x64")) return launch_cfg<2, 2, 1, 1, MODE, GK, W4>(s, a) ? "t64x64" : nullptr;
+        if (GK == 1 || forced("t128x128")) return launch_cfg<2, 2, 2, 2, MODE, GK, W4>(s, a) ? "t128x128" : nullptr;
+        return launch_cfg<2, 4, 2, 2, MODE, GK, W4>(s, a) ? "t128x256" : nullptr;
     } else {
         // Largest tile (channels x rows) that still gives every compute unit work; names are BNxBM.
         const auto tiles = [&](uint32_t bn, uint32_t bm) {
