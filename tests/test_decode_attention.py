@@ -1,4 +1,5 @@
-"""Decode attention at head sizes 64 and 128: eight wavefronts take 16 slots each of every 128, two blocks ahead."""
+"""Decode attention at head sizes 64 (one walk over keys and values: eight wavefronts take 16 slots each of every 128, two
+blocks ahead) and 128 (the kernel that keeps its scores in LDS)."""
 import numpy as np
 import pytest
 

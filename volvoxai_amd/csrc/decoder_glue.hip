@@ -937,7 +937,7 @@ __global__ __launch_bounds__(256) void gqa_prefill_kernel(const float* __restric
 //           channel tile c is channel VW * r + c (VW = head size / 32): a value load is VW consecutive
 //           floats a lane, and the output leaves the same way.
 // Bound by the matrix pipes (128 MFMAs of 64 cycles per 32 slots and 128 channels: 17 us for 32 prompts of
-// 128 tokens, 16 query and 8 KV heads) and by 100 MB of queries, cache and outputs (20 us); measured 43 us.
+// 128 tokens, 16 query and 8 KV heads) and by 100 MB of queries, cache and outputs (20 us); measured 41.5 us.
 // With keys and values staged through LDS by four wavefronts and the scores kept there, three barriers per
 // 64 slots, the same launch took 99.7 us; heads of 64 on the vector kernel above 76.6, here 17.2.  The loads are a ring of RING 16-byte
 // registers, RING * 256 cycles of MFMAs ahead of their use; the fence behind each refill keeps the
@@ -1211,7 +1211,7 @@ __global__ __launch_bounds__(256, 2) void gqa_prefill_mfma_kernel(const float* _
 // Whether the wavefronts of a workgroup share their queries and split the slots (see the kernel above): while
 // the launch has not one wavefront for every SIMD, and more than one tile to split.  Measured, shared against
 // apart (16 query / 8 KV heads of 128): 128 tokens of 1 row 10.6 / 24.6 us, of 8 rows (512 query blocks)
-// 18.5 / 26.3, of 16 rows (1024) 33.1 / 28.2, of 32 rows 55.9 / 43.0; 190 tokens of 8 rows (768) 34.1 / 36.0;
+// 18.5 / 26.3, of 16 rows (1024) 33.1 / 28.2, of 32 rows 55.9 / 41.5; 190 tokens of 8 rows (768) 34.1 / 36.0;
 // 64 tokens of 16 rows (512) 17.9 / 17.0.  Heads of 64, 128 tokens: 512 blocks 11.6 / 16.4, 1024 20.1 / 17.2.
 bool split_prompt_slots(uint32_t query_blocks, uint32_t t, int compute_units) {
     return t > 32u && query_blocks < 4u * (uint32_t)(compute_units > 0 ? compute_units : 256);
@@ -1452,8 +1452,8 @@ VxHipStatus vxhip_gqa_attention(VxHipContext* ctx, const float* q_dev, const flo
         return (qw * ((max_seq + 63u) & ~63u) + (size_t)kPrefillSlots * (head_dim + 4u)) * sizeof(float);
     };
     constexpr size_t kTokenLds = 60u * 1024u, kPromptLds = 150u * 1024u;
-    // A prompt at the common head sizes: the matrix-pipe kernel.  (It holds no scores and would take any cache, but
-    // a cache that a decode step, or a prompt at another head size, could not serve is refused alike.)
+    // A prompt at the common head sizes: the matrix-pipe kernel.  (It holds no scores and would take any cache; those
+    // that neither the prompt kernel with scores nor the per-token kernel could hold are refused as before it.)
     if (t >= 8u && rep <= kPrefillQueries && (head_dim == 128u || head_dim == 64u) &&
         (prompt_lds(1u) <= kPromptLds || token_lds <= kTokenLds)) {
         const uint32_t tq = kPrefillQueries / rep, blocks = (t + tq - 1u) / tq, pairs = rows * kv_heads;
