@@ -33,15 +33,17 @@ def test_few_rows_at_their_edges(ctx, oracle, rows, k, bits, group):
         x[rows - 1, k - 1] = np.inf
         x[0, 0] *= 300.0
         want = oracle.packed_linear(x, words, scales, bias, n, group, bits=bits)[1]
-        for force in ("gemv.few16", "gemv.few32", "gemv.few64", None):
-            if force == "gemv.few64" and group == 32:
-                continue  # (its products do not fit the LDS at every length)
+        # what the rule takes is built: 64 channels a workgroup for up to four rows and eight bits in groups of 64 and more,
+        # 32 for up to four rows, and for more of up to 1024
+        wide = 16 if rows > 4 and k > 1024 else 32
+        widest = 64 if rows <= 4 and bits == 8 and group > 32 else wide
+        for force, ch in (("gemv.few16", 16), ("gemv.few32", wide), ("gemv.few64", widest), (None, 16)):
             vx.force_variant(force)
             st, y = pl.forward_f32(ctx, _dev(x))
             ctx.synchronize()
             vx.force_variant(None)
             got = y.cpu().numpy()
-            assert st == 0 and ".few" in ctx.last_variant, ctx.last_variant
+            assert st == 0 and ctx.last_variant.endswith(f".few{ch}"), ctx.last_variant
             nan = np.isnan(want)
             assert (np.isnan(got) == nan).all() and (got.view(np.uint32)[~nan] == want.view(np.uint32)[~nan]).all(), ctx.last_variant
         pl.close()

@@ -243,12 +243,19 @@ bool launch_length(hipStream_t s, const LinearArgs& a) {
         if (a.k <= 3072u) return launch<GK, W4, CH, 3, 4>(s, a);
         return launch<GK, W4, CH, 4, 4>(s, a);
     }
-    return a.k <= 1024u ? launch<GK, W4, CH, 1, 8>(s, a) : launch<GK, W4, CH, 2, 8>(s, a);
+    if constexpr (CH <= 32) {
+        if (a.k <= 1024u) return launch<GK, W4, CH, 1, 8>(s, a);
+        if constexpr (CH == 16) return launch<GK, W4, CH, 2, 8>(s, a);
+    }
+    return false;
 }
 
 template <int GK, bool W4>
 bool launch_channels(hipStream_t s, const LinearArgs& a, uint32_t ch) {
-    return ch == 16u ? launch_length<GK, W4, 16>(s, a) : ch == 64u ? launch_length<GK, W4, 64>(s, a) : launch_length<GK, W4, 32>(s, a);
+    if (ch == 16u) return launch_length<GK, W4, 16>(s, a);
+    if (ch == 32u) return launch_length<GK, W4, 32>(s, a);
+    if constexpr (!W4 && GK > 1) return launch_length<GK, W4, 64>(s, a);
+    return false;
 }
 
 template <bool W4>
@@ -286,12 +293,15 @@ const char* launch_gemv_few(hipStream_t s, const LinearArgs& a, int cu_count, co
     if (force && !strstr(force, "few")) return nullptr;
     if (cu_count <= 0) cu_count = 256;
     const uint32_t panels = (a.n + 31u) / 32u, cu = (uint32_t)cu_count;
-    uint32_t ch = panels * 2u <= cu ? 16u : panels > cu && a.weight_bits == 8u && a.group_size > 32u ? 64u : 32u;
+    uint32_t ch = panels * 2u <= cu ? 16u : panels > cu ? 64u : 32u;
     if (!force && a.rows > 4u && panels * (a.k <= 1024u ? 1u : 2u) > cu) return nullptr;
     if (!force && a.rows <= 4u && panels > cu && a.weight_bits == 4u && a.k > 2048u) return nullptr;
     if (force && strstr(force, "few16")) ch = 16u;
     else if (force && strstr(force, "few32")) ch = 32u;
     else if (force && strstr(force, "few64")) ch = 64u;
+    // (the widths that are built: the others are of rows, lengths and weights that the lines above keep from them)
+    if (ch == 64u && (a.weight_bits == 4u || a.group_size == 32u || a.rows > 4u)) ch = 32u;
+    if (ch == 32u && a.rows > 4u && a.k > 1024u) ch = 16u;
     if (!(a.weight_bits == 4u ? launch_group<true>(s, a, ch) : launch_group<false>(s, a, ch))) return nullptr;
     static const char* const names[2][3] = {
         {"hip.packed-linear.a8-gemv-mfma.few16", "hip.packed-linear.a8-gemv-mfma.few32", "hip.packed-linear.a8-gemv-mfma.few64"},
