@@ -1,12 +1,16 @@
 """The C-ABI library loads without a GPU, exports every declared symbol, and
 fails loudly (never silently on a CPU path) when there is no device."""
 import ctypes as C
+import re
+from pathlib import Path
 
 import numpy as np
 import pytest
 
 import volvoxai_amd as vx
 from volvoxai_amd._lib import declared_symbols, library
+
+ROOT = Path(__file__).resolve().parent.parent
 
 
 def test_library_exports_every_declared_symbol():
@@ -30,6 +34,19 @@ def test_kernel_variant_table_shape():
     # QLinear, QGemm and QMatMul share one kernel family, as upstream's cuda.qlinear.* rows do
     for fam in ("hip.qlinear.mfma-i8", "hip.qlinear.gemv-mfma"):
         assert {r["operator_kind"] for r in rows if r["id"] == fam} == {1002, 1005, 1007}
+
+
+def test_kernel_variant_table_names_every_linear_kernel():
+    """The kernels behind a family's routes, and the matrix instructions they are made of, as the sources have them."""
+    rows = vx.kernel_variants()
+    sources = [p.read_text() for p in sorted((ROOT / "volvoxai_amd" / "csrc").glob("gem*.hip"))]
+    names = {n for text in sources for n in re.findall(r"void (gem[mv]_\w*kernel)\(", text)}
+    assert len(names) == 8
+    assert names == {e.split("<")[0] for r in rows for e in r["entrypoint_id"].split("|") if e.startswith("gem")}
+    used = {n for text in sources for n in re.findall(r"__builtin_amdgcn_mfma_i32_(\w+)_i8\(", text)}
+    assert used == {n for r in rows for n in re.findall(r"mfma-i32-(\w+)-i8", r["required_features"])}
+    few = [r for r in rows if "gemv_few_kernel" in r["entrypoint_id"]]
+    assert len(few) == 2 and all("mfma-i32-16x16x64-i8" in r["required_features"] for r in few)
 
 
 def _no_gpu():
