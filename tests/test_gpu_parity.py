@@ -703,8 +703,9 @@ def test_qlinear_dequantized_equals_the_two_nodes(ctx, oracle, rows, k, n, idt, 
 @pytest.mark.parametrize("k,n,group,bits", [(4096, 14336, 128, 8), (1000, 200, 32, 8), (129, 40, 64, 8), (4096, 1024, 128, 4),
                                             (2048, 4096, 256, 8), (1024, 6144, 128, 3), (3072, 1024, 64, 2)])
 def test_few_f32_rows_are_prepared_inside_the_gemv(ctx, oracle, rows, k, n, group, bits):
-    """PackedLinear on one or two f32 rows is one launch: the streaming kernel quantizes the rows itself
-    (the reference's single-row route does both in one call, packed_linear_ops.inc:1471-1535).  Same
+    """PackedLinear on one or two f32 rows is one launch whose workgroups quantize the rows themselves (the reference's
+    single-row route does both in one call, packed_linear_ops.inc:1471-1535), and so are three and four of up to 4096,
+    but for four-bit weights of more than 2048 and 8192 channels.  Same
     bits as the oracle and as the two launches, special rows included (all zero, denormal, huge, NaN)."""
     import volvoxai_amd as vx
     c = cases.packed_case(max(rows, 5), k, n, group, 8800 + rows + n, special_rows=True)
@@ -718,14 +719,14 @@ def test_few_f32_rows_are_prepared_inside_the_gemv(ctx, oracle, rows, k, n, grou
     pl = vx.PackedLinear(words, c["scales"], c["bias"], k, n, group, weight_bits=bits)
     st, y = pl.forward_f32(ctx, dev(x))
     ctx.synchronize()
-    # (more rows keep the two launches)
-    assert st == 0 and ctx.last_variant.endswith("-prep") == (rows <= 2) and "gemv-mfma" in ctx.last_variant, ctx.last_variant
+    route = ("row8-prep" if n <= 2048 else "row32-prep") if rows <= 2 else "few16" if n <= 4096 else "few32" if n <= 8192 else "few64"
+    assert st == 0 and ctx.last_variant.endswith("gemv-mfma." + route), ctx.last_variant
     assert same_f32(y.cpu().numpy(), want)
     vx.force_variant("gemv.noprep")
     try:
         st2, y2 = pl.forward_f32(ctx, dev(x))
         ctx.synchronize()
-        assert st2 == 0 and not ctx.last_variant.endswith("-prep")
+        assert st2 == 0 and not ctx.last_variant.endswith("-prep") and ".few" not in ctx.last_variant, ctx.last_variant
     finally:
         vx.force_variant(None)
     assert same_f32(y2.cpu().numpy(), want)
