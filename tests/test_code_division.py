@@ -175,7 +175,7 @@ def test_codes_at_the_edges_of_the_reciprocal(ctx, oracle):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("exponent", [-120, 0, 127])
+@pytest.mark.parametrize("exponent", [-120, -119, 0, 127])
 def test_row_scales_of_every_mantissa(ctx, exponent):
     """Rows of one element: the scale is f32(max / 127), floored at 2^-126."""
     import torch

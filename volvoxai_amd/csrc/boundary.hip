@@ -16,7 +16,7 @@ namespace vxhip {
 // Bound by the latency of a launch and of its loads until there are tens of megabytes, so a row's pieces are all
 // requested before the first is used: a wavefront a row and 16 bytes a lane (bytes), or T threads a row and four
 // elements a thread (f32).  A byte a lane and pass, behind a quantization launch of its own, took 6.5 + 2.3 us of the
-// 15.3 us of 77 f32 rows of 1001 -> 1531 with row sums; that call is 11.2 now.  Whole calls of up to 32 rows, drawn
+// 15.3 us of 77 f32 rows of 1001 -> 1531 with row sums; that call is 10.3 now.  Whole calls of up to 32 rows, drawn
 // lengths of 256 to 4096: f32 rows to unsigned codes 10.6 -> 6.0 us, bytes with row sums 7.9 -> 5.9, bytes of odd
 // lengths 8.4 -> 6.5.
 typedef uint32_t dword_any __attribute__((aligned(1)));
@@ -126,8 +126,8 @@ __device__ __forceinline__ uint32_t codes_inside(uint32_t codes, uint32_t j, uin
     return j + 4u <= k ? codes : j >= k ? 0u : codes & ((1u << (8u * (k - j))) - 1u);
 }
 
-// Rows that are whole chunks and no sums: the elements in one run, four a thread where there are many.  (Of a few
-// hundred thousand every one has a thread of its own: the four exact divisions of a thread cost 0.3 us.)
+// Rows that are whole chunks and no sums: the elements in one run, four a thread where there are many.  (Up to a few
+// hundred thousand every one has a thread of its own: four quotients in a thread are 0.1 to 0.4 us longer than one.)
 __global__ __launch_bounds__(256) void quantize_run_kernel(const float* __restrict__ x, uint32_t quads, QuantizeRule rule,
                                                            uint32_t* __restrict__ codes) {
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
@@ -185,8 +185,9 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const float* __restr
     }
 }
 
-// (Up to here a thread an element and four a thread are the same within 1 %, past it four are up to 6 % faster: 2323 x 768
-// elements 9.9 -> 9.4 us with their linear.)
+// Where the line lies, us of a call with its linear of 1024 channels, an element a thread | four: 3 x 1024 4.6 | 5.0,
+// 8 x 4096 6.7 | 7.0, 32 x 4096 8.8 | 9.0, 512 x 256 6.5 | 6.7, 128 x 2048 9.94 | 10.03, 64 x 4096 13.66 | 13.73; past it four
+// are up to 6 % faster (2323 x 768 9.9 | 9.4).
 constexpr uint32_t kRunOfElements = 1u << 18;
 
 VxHipStatus launch_quantize_rows(hipStream_t s, const float* x, uint32_t rows, uint32_t k, float scale, int32_t zp,

@@ -521,8 +521,8 @@ __global__ __launch_bounds__(256) void gqa_attention_kernel(const float* __restr
 // first 256 slots, values too, are requested before the query is ready.
 // Bound by the latency of a launch and of its reads; the kernel above asks for its values only once the keys have
 // come, and its three phases are behind barriers.  At slot 145, 8 query and 4 KV heads: 1 row 6.0 -> 4.6 us, 32 rows
-// 7.2 -> 5.9.  (At head size 128 twice the bytes are in flight either way and the reads themselves bound it: 1 row
-// 7.4 against 7.0 us, but 32 rows 12.7 against 13.3 and at slot 220 14.7 against 16.6, so it keeps the kernel above.)
+// 7.2 -> 5.9.  (At head size 128 the kernel above stays: 1 row 7.4 against 7.0 us here, but 32 rows 12.7 against 13.3 and
+// at slot 220 14.7 against 16.6.  Its 32 rows read 37.9 MB of slots at 3.0 TB/s, half of what a GEMV's weights come at.)
 template <int REP, bool FUSED>
 __global__ __launch_bounds__(512, 2) void decode_attention_kernel(const float* __restrict__ q,
                                                                   float* __restrict__ k_cache,

@@ -85,7 +85,7 @@ __device__ __forceinline__ uint32_t magnitude_bits(float v) { return __float_as_
 constexpr uint32_t kNotFinite = 0x7f800000u;  // and everything above
 
 // scale = max|v| / 127 (1 for a zero row and for one that is not finite, floored at 2^-126): the quotient of a true
-// division for every finite maximum (all of them tried)
+// division for every finite maximum (every mantissa compared, in the middle, at the floor and at the largest exponent)
 __device__ __forceinline__ float row_code_scale(uint32_t maximum) {
     const float scale = maximum == 0u || maximum >= kNotFinite ? 1.0f : div_by_uniform(__uint_as_float(maximum), 127.0f, 0x1.020408p-7f);
     return scale < 0x1p-126f ? 0x1p-126f : scale;
@@ -106,8 +106,8 @@ struct CodeDivisor {
     __device__ __forceinline__ explicit CodeDivisor(float row_scale) {
         lift = row_scale < 0x1p-60f ? 0x1p64f : 1.0f;
         scale = __fmul_rn(row_scale, lift);
-        // the correctly rounded reciprocal of every mantissa but one from any start within two units in the last place (all
-        // tried); of the largest mantissa it may be one unit low
+        // the correctly rounded reciprocal of every mantissa but one from any start within two units in the last place
+        // (followed over all of them); of the largest mantissa it may be one unit low, and then some of its codes are others
         recip = __builtin_amdgcn_rcpf(scale);
 #pragma unroll
         for (int i = 0; i < 2; i++) recip = __fmaf_rn(__fmaf_rn(-scale, recip, 1.0f), recip, recip);

@@ -10,7 +10,7 @@
 // the accumulators as products f32(dot) * (s_a * s_w) and one thread per output adds them in ascending group order, the
 // sum the reference forms (packed_linear_ops.inc:1498-1504), bit for bit.
 //
-// Bound by latency, and by the preparation that every workgroup repeats: 16384 elements are some 20 of them a thread, 1.5 us
+// Bound by latency, and by the preparation that every workgroup repeats: of 16384 elements a thread takes 32, 1.5 us
 // beside a launch of its own that costs 2.4.
 #include "common.h"
 #include "device_math.h"
@@ -272,7 +272,8 @@ bool launch_group(hipStream_t s, const LinearArgs& a, uint32_t ch) {
 }  // namespace
 
 // Which calls, and how many channels a workgroup.  Times of a row preparation and a GEMV over those of this kernel with
-// 16 | 32 channels, means over drawn lengths, widths, groups and weight widths (behind a host that launches one by one):
+// 16 | 32 channels, means over drawn lengths, widths, groups and weight widths; replayed as a graph, and in parentheses
+// behind a host that launches one by one:
 //   rows  K up to   N up to 4096                 8192                       14336
 //   3-4   1024      1.74 | 1.71 (1.41 | 1.41)    1.35 | 1.61 (1.40 | 1.40)  1.22 | 1.44 (1.34 | 1.39)
 //   3-4   2048      1.61 | 1.49 (1.41 | 1.40)    1.36 | 1.61 (1.37 | 1.41)  1.09 | 1.19 (1.09 | 1.22)

@@ -114,8 +114,8 @@ class W8A8Decoder:
         import torch
         self.torch, self.cfg, self.rows = torch, cfg, rows
         # One row: a decode step runs the fused single-row forms (five launches per layer instead of nine)
-        # where the library takes every linear of a layer that way.  They take two rows as well, at the
-        # speed of the separate launches (fuse_rows=True asks for them; None decides by the row count).
+        # where the library takes every linear of a layer that way.  They take two rows as well, which fuse_rows=True
+        # asks for (28 layers of hidden 1024: 0.73 ms a step against 0.90); None fuses a single row only.
         wanted = rows == 1 if fuse_rows is None else bool(fuse_rows)
         self.rows_fused = False  # settled below, once the linears exist: the library is asked about each one
         self.stream = stream if stream is not None else torch.cuda.Stream()
@@ -278,7 +278,9 @@ class W8A8Decoder:
         to `next_tokens` when given; `advance` counters are incremented by the same launch)."""
         cfg = self.cfg
         rows, t = tokens.shape
-        # which linears of a prompt are tried with what follows them: fewer outputs than this never fill the tiles that do it
+        # Which linears of a prompt are tried with what follows them.  The tiles that do it are picked from 384 of 64 x 64
+        # outputs on (1.5 a compute unit); with fewer outputs than 256 whole ones that takes tiles a third empty, and
+        # the attempts are spared.
         self.takes = {name: rows * t > 32 and rows * t * self.layers[0][name].n >= 1 << 20 for name in ("qkv", "o", "gate_up", "down")}
         x2 = vx.embedding_gather(self.ctx, tokens.reshape(-1), self.embedding)
         if t == 1 and self.rows_fused:
