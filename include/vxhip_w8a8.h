@@ -414,8 +414,10 @@ VxHipStatus vxhip_packed_prepare_i8(VxHipContext* context,
  * (src/kernels/packed_linear_ops.inc:1545-1621) on resident f32 rows.
  * One or two rows of k up to 14336 (the reference's single-row route, :1471-1535,
  * which prepares the row and multiplies in one call) run as one launch whose
- * workgroups prepare the rows themselves (route id ends in "-prep"), unless the
- * output overlaps the input; other rows are prepared by a launch of their own
+ * workgroups prepare the rows themselves (route id ends in "-prep"), and so do
+ * three or four rows of k up to 4096 and five to eight of k up to 2048 where the
+ * linear is not too wide for that to pay (".few16", ".few32" or ".few64"), unless
+ * the output overlaps the input; other rows are prepared by a launch of their own
  * first.  The bits are the same either way.
  * Returns 0 on success, -1 on a rejected descriptor (reference convention). */
 int vxhip_packed_linear_forward_f32(VxHipContext* context,
