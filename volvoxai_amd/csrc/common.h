@@ -277,6 +277,13 @@ struct LinearTail {
 // nothing ran then.
 const char* launch_gemm_followed(hipStream_t s, const LinearArgs& a, After after, const LinearTail& tail, int cu_count);
 
+// decode_attention.hip: tokens = rows * t queries over the caches.  cos_table given: rotary embedding and cache append ride
+// in front (t = 1).  False where it has no kernel for the call: nothing ran.
+bool launch_decode_attention(hipStream_t s, int cu_count, uint32_t tokens, const float* q, float* k_cache, float* v_cache,
+                             const int64_t* positions, uint32_t t, uint32_t q_heads, uint32_t kv_heads, uint32_t head_dim,
+                             uint32_t max_seq, float scale, float* out, const float* cos_table, const float* sin_table,
+                             uint32_t* fault);
+
 // gemm_mfma.hip / gemv_stream.hip: return the variant id that ran, or null if
 // the shape is outside the kernel's domain (nothing launched).
 const char* launch_gemm_mfma(hipStream_t s, const LinearArgs& a, int cu_count, const char* force);

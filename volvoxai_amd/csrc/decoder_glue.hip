@@ -6,6 +6,7 @@
 //                     (native/src/kernels/llm_math.h:256-274) and the KV-cache append
 //   gqa_attention     grouped-query attention of the new tokens over the cache: f32 scores
 //                     scaled by 1/sqrt(d), causal visibility slot <= position, softmax, P.V
+//                     (of few tokens at head sizes 64 and 128: decode_attention.hip)
 //
 // All are row-sized, latency-bound kernels; none of them is on the int8 roofline.
 #include "common.h"
@@ -514,228 +515,6 @@ __global__ __launch_bounds__(256) void gqa_attention_kernel(const float* __restr
     }
 }
 
-// The same attention for head size 64 and few tokens a row (decode), in one walk over keys and values together.  Eight wavefronts a workgroup; eight lanes share a slot, key and value row alike (16-byte chunks
-// c = lane % 8 + 8 * i), so a slot's probability is in the lanes that weigh its value row and nothing is exchanged
-// but the three steps of a dot's sum: each group of eight lanes keeps its own running maximum, sum and output, and
-// the 64 groups of a workgroup meet once, at the end.  A wavefront takes 16 slots of every 128; the rows of the
-// first 256 slots, values too, are requested before the query is ready.
-// Bound by the latency of a launch and of its reads; the kernel above asks for its values only once the keys have
-// come, and its three phases are behind barriers.  At slot 145, 8 query and 4 KV heads: 1 row 6.0 -> 4.6 us, 32 rows
-// 7.2 -> 5.9.  (At head size 128 the kernel above stays: 1 row 7.4 against 7.0 us here, but 32 rows 12.7 against 13.3 and
-// at slot 220 14.7 against 16.6.  Its 32 rows read 37.9 MB of slots at 3.0 TB/s, half of what a GEMV's weights come at.)
-template <int REP, bool FUSED>
-__global__ __launch_bounds__(512, 2) void decode_attention_kernel(const float* __restrict__ q,
-                                                                  float* __restrict__ k_cache,
-                                                                  float* __restrict__ v_cache,
-                                                                  const int64_t* __restrict__ positions, uint32_t t,
-                                                                  uint32_t q_heads, uint32_t kv_heads,
-                                                                  uint32_t max_seq, float scale, float* __restrict__ out,
-                                                                  const float* __restrict__ cos_table,
-                                                                  const float* __restrict__ sin_table,
-                                                                  uint32_t* __restrict__ fault) {
-    constexpr int HD = 64, KC = HD / 32, WAVES = 8, PASSES = 2;
-    constexpr int BUFS = 2;  // blocks of 128 slots in flight
-    constexpr int STAGED = (REP + (FUSED ? 2 : 0)) * HD, ITEMS = (STAGED + 511) / 512;
-    constexpr uint32_t BLOCK = WAVES * PASSES * 8u;
-    __shared__ __attribute__((aligned(16))) float staged[STAGED];  // queries; FUSED: the appended key and value
-    __shared__ __attribute__((aligned(16))) float partial[WAVES][REP][HD];
-    __shared__ float maxima[WAVES][REP], sums[WAVES][REP];
-    const uint32_t token = blockIdx.x, head0 = blockIdx.y * REP;
-    const uint32_t row = token / t, i = token % t;
-    const uint32_t rep = q_heads / kv_heads, kvh = head0 / rep;
-    const uint64_t named = (uint64_t)positions[i];
-    if (named >= max_seq) {  // (the whole workgroup) outside the caches: touch nothing, say so
-        if (threadIdx.x == 0) atomicOr(fault, (uint32_t)kFaultBadPosition);
-        return;
-    }
-    const uint32_t position = (uint32_t)named;
-    const uint32_t cached = FUSED ? position : position + 1u;  // slots read from the caches
-    const uint32_t last_cached = max(cached, 1u) - 1u;
-    float* kbase = k_cache + ((size_t)row * kv_heads + kvh) * max_seq * HD;
-    float* vbase = v_cache + ((size_t)row * kv_heads + kvh) * max_seq * HD;
-    const uint32_t lane8 = threadIdx.x & 7u, group = (threadIdx.x >> 3) & 7u;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-
-    // operands of the queries (and of the appended row) first: loads return in order
-    float own[ITEMS], mate[ITEMS], c[ITEMS], sn[ITEMS];
-#pragma unroll
-    for (int j = 0; j < ITEMS; j++) {
-        own[j] = mate[j] = c[j] = sn[j] = 0.0f;
-        const uint32_t e = threadIdx.x + 512u * j, which = e / HD, dd = e % HD;
-        if (e < STAGED) {
-            if constexpr (FUSED) {
-                const uint32_t head = which < REP ? head0 + which : which == REP ? q_heads + kvh : q_heads + kv_heads + kvh;
-                const float* src = q + ((size_t)token * (q_heads + 2u * kv_heads) + head) * HD;
-                own[j] = src[dd];
-                mate[j] = src[dd ^ (HD / 2u)];
-                c[j] = cos_table[(size_t)position * HD + dd];
-                sn[j] = sin_table[(size_t)position * HD + dd];
-            } else {
-                own[j] = q[((size_t)token * q_heads + head0 + which) * HD + dd];
-            }
-        }
-    }
-    // Slots past the end repeat the last cached one (row 0 where there is none) and are not counted.
-    float4 kb[BUFS][PASSES][KC], vb[BUFS][PASSES][KC];
-    auto slot_of = [&](uint32_t block, int u) { return block * BLOCK + wave * (PASSES * 8u) + u * 8u + group; };
-    auto request = [&](auto b_tag, uint32_t block) {
-        constexpr int b = decltype(b_tag)::value;
-#pragma unroll
-        for (int u = 0; u < PASSES; u++) {
-            const size_t at = (size_t)min(slot_of(block, u), last_cached) * HD;
-#pragma unroll
-            for (int n = 0; n < KC; n++) kb[b][u][n] = *reinterpret_cast<const float4*>(kbase + at + 4u * (lane8 + 8u * n));
-        }
-#pragma unroll
-        for (int u = 0; u < PASSES; u++) {
-            const size_t at = (size_t)min(slot_of(block, u), last_cached) * HD;
-#pragma unroll
-            for (int n = 0; n < KC; n++) vb[b][u][n] = *reinterpret_cast<const float4*>(vbase + at + 4u * (lane8 + 8u * n));
-        }
-    };
-    static_for<BUFS>([&](auto b_tag) { request(b_tag, (uint32_t)decltype(b_tag)::value); });
-#pragma unroll
-    for (int j = 0; j < ITEMS; j++) {
-        const uint32_t e = threadIdx.x + 512u * j, which = e / HD, dd = e % HD;
-        if (e < STAGED) {
-            float y = own[j];
-            if (FUSED && which <= REP)  // the arithmetic of rope_append_kernel
-                y = __fadd_rn(__fmul_rn(own[j], c[j]), __fmul_rn(dd < HD / 2u ? -mate[j] : mate[j], sn[j]));
-            staged[e] = y;
-            if (FUSED && which >= REP && head0 % rep == 0u) (which == REP ? kbase : vbase)[(size_t)position * HD + dd] = y;
-        }
-    }
-    __syncthreads();
-    // Probabilities carry a power of two of at most one over the number of slots (it leaves with the division at the
-    // end): the sums of their products with values stay in the values' range.
-    const float unit = __uint_as_float((127u - (position ? 32u - (uint32_t)__builtin_clz(position) : 0u)) << 23);
-    float4 qv[REP][KC], acc[REP][KC];
-    float m[REP], sum[REP];
-#pragma unroll
-    for (int h = 0; h < REP; h++) {
-        m[h] = -INFINITY;
-        sum[h] = 0.0f;
-#pragma unroll
-        for (int n = 0; n < KC; n++) {
-            qv[h][n] = *reinterpret_cast<const float4*>(staged + h * HD + 4u * (lane8 + 8u * n));
-            acc[h][n] = make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-    }
-    // one slot of this group of eight lanes (all 64 lanes take part; `counts` is false for a slot past the end)
-    auto take = [&](const float4 (&kr)[KC], const float4 (&vr)[KC], bool counts) {
-        float dot[REP];
-#pragma unroll
-        for (int h = 0; h < REP; h++) {
-            float d = 0.0f;
-#pragma unroll
-            for (int n = 0; n < KC; n++) {
-                d = __builtin_fmaf(qv[h][n].x, kr[n].x, d);
-                d = __builtin_fmaf(qv[h][n].y, kr[n].y, d);
-                d = __builtin_fmaf(qv[h][n].z, kr[n].z, d);
-                d = __builtin_fmaf(qv[h][n].w, kr[n].w, d);
-            }
-            d += lane_exchange<kDppXor1>(d);
-            d += lane_exchange<kDppXor2>(d);
-            d += lane_exchange<kDppHalfMirror>(d);
-            dot[h] = __fmul_rn(d, scale);
-        }
-        if (!counts) return;
-#pragma unroll
-        for (int h = 0; h < REP; h++) {
-            const float grown = fmaxf(m[h], dot[h]);
-            const float reference = grown == -INFINITY ? 0.0f : grown;  // (only scores of -inf so far: zeros)
-            const float keep = expf(m[h] - reference), p = expf(dot[h] - reference) * unit;
-            m[h] = grown;
-            sum[h] = __builtin_fmaf(sum[h], keep, p);
-#pragma unroll
-            for (int n = 0; n < KC; n++) {
-                acc[h][n].x = __builtin_fmaf(p, vr[n].x, acc[h][n].x * keep);
-                acc[h][n].y = __builtin_fmaf(p, vr[n].y, acc[h][n].y * keep);
-                acc[h][n].z = __builtin_fmaf(p, vr[n].z, acc[h][n].z * keep);
-                acc[h][n].w = __builtin_fmaf(p, vr[n].w, acc[h][n].w * keep);
-            }
-        }
-    };
-    const uint32_t blocks = (cached + BLOCK - 1u) / BLOCK;
-    for (uint32_t block = 0; block < blocks; block += BUFS) {
-        static_for<BUFS>([&](auto b_tag) {
-            constexpr int b = decltype(b_tag)::value;
-            if (block + b < blocks) {  // (a scalar branch)
-#pragma unroll
-                for (int u = 0; u < PASSES; u++) take(kb[b][u], vb[b][u], slot_of(block + b, u) < cached);
-            }
-            request(b_tag, block + b + BUFS);
-        });
-    }
-    if constexpr (FUSED) {
-        // the appended slot, from LDS, by the group that has it in the unfused form and behind the same slots
-        if (wave == position % BLOCK / (PASSES * 8u)) {
-            float4 kr[KC], vr[KC];
-#pragma unroll
-            for (int n = 0; n < KC; n++) {
-                kr[n] = *reinterpret_cast<const float4*>(staged + REP * HD + 4u * (lane8 + 8u * n));
-                vr[n] = *reinterpret_cast<const float4*>(staged + (REP + 1) * HD + 4u * (lane8 + 8u * n));
-            }
-            take(kr, vr, group == position % 8u);
-        }
-    }
-    // The groups of a wavefront meet: lanes 32, then 16, then 8 apart.  The first step exchanges one half of the
-    // channels for the other and leaves half as many to the next.
-    constexpr int kDppRor8 = 0x128;  // lane ^ 8 within a row of 16
-    auto halves = [](float a, float b) {  // lower half: a summed over both, upper half: b
-        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-    };
-    auto row_pair = [](float a) {
-        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(a), false, false);
-        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-    };
-#pragma unroll
-    for (int h = 0; h < REP; h++) {
-        const float top = wave_max(m[h]);
-        const float keep = expf(m[h] - (top == -INFINITY ? 0.0f : top));
-        float total = sum[h] * keep;
-        total = halves(total, total);
-        total = row_pair(total);
-        total += lane_exchange<kDppRor8>(total);
-        float x[KC * 4];
-#pragma unroll
-        for (int n = 0; n < KC; n++)
-            x[4 * n] = acc[h][n].x * keep, x[4 * n + 1] = acc[h][n].y * keep, x[4 * n + 2] = acc[h][n].z * keep,
-                  x[4 * n + 3] = acc[h][n].w * keep;
-#pragma unroll
-        for (int e = 0; e < KC * 2; e++) x[e] = halves(x[e], x[e + KC * 2]);
-        const uint32_t chunk = (threadIdx.x >> 5) & 1u;
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            x[e] = row_pair(x[e]);
-            x[e] += lane_exchange<kDppRor8>(x[e]);
-        }
-        if ((threadIdx.x & 24u) == 0u)
-            *reinterpret_cast<float4*>(&partial[wave][h][4u * (lane8 + 8u * chunk)]) = make_float4(x[0], x[1], x[2], x[3]);
-        if ((threadIdx.x & 63u) == 0u) {
-            maxima[wave][h] = top;
-            sums[wave][h] = total;
-        }
-    }
-    __syncthreads();
-    for (uint32_t e = threadIdx.x; e < REP * HD; e += 512u) {
-        const uint32_t h = e / HD, dd = e % HD;
-        float top = maxima[0][h];
-#pragma unroll
-        for (int w = 1; w < WAVES; w++) top = fmaxf(top, maxima[w][h]);
-        const float reference = top == -INFINITY ? 0.0f : top;
-        float total = 0.0f, y = 0.0f;
-#pragma unroll
-        for (int w = 0; w < WAVES; w++) {
-            const float weight = expf(maxima[w][h] - reference);
-            total = __builtin_fmaf(sums[w][h], weight, total);
-            y = __builtin_fmaf(partial[w][h][dd], weight, y);
-        }
-        out[((size_t)token * q_heads + head0 + h) * HD + dd] = __fdiv_rn(y, total);
-    }
-}
-
 // Prompt attention (t > 1 tokens per row).  The kernels above give every (token, head) its own
 // workgroup, so a prompt of t tokens reads each key and value row t times.  Here a workgroup takes
 // `tq` consecutive tokens of one row and the `rep` query heads of one KV head, qw = tq * rep <= 32
@@ -1225,7 +1004,8 @@ bool split_prompt_slots(uint32_t query_blocks, uint32_t t, int compute_units) {
 // Few rows: while one head per workgroup still leaves no compute unit with two workgroups the launch
 // is latency bound again, and the heads are faster apart (28 layers of 16 query / 8 KV heads of 128,
 // per decode step: 1 row 1.13 -> 1.10 ms, 16 rows 1.385 -> 1.348; 32 rows 1.49 with two heads
-// together, 1.55 apart).
+// together, 1.55 apart).  (Measured at head size 128, which decode_attention.hip has since taken over but for the launches
+// of four; the other sizes keep these lines.)
 uint32_t heads_per_workgroup(uint32_t rep, uint32_t query_heads_in_launch, int compute_units) {
     if (query_heads_in_launch <= (uint32_t)(compute_units > 0 ? compute_units : 256)) return 1u;
     return rep >= 8u && rep % 4u == 0u ? 4u : rep % 2u == 0u ? 2u : 1u;
@@ -1243,18 +1023,18 @@ ActivationLayout prepared_layout(const VxHipContext* ctx, uint32_t rows, uint32_
     return ActivationLayout{d, 0u};
 }
 
-// Picks the instance for the query heads per workgroup (4 or 1) and the head size.
+// The query heads per workgroup (4, 2 or 1) and the head size pick the instance.
 template <bool FUSED>
-void launch_attention(hipStream_t stream, uint32_t together, dim3 grid, size_t lds, const float* q, float* k_cache,
+void launch_attention(VxHipContext* ctx, uint32_t together, dim3 grid, size_t lds, const float* q, float* k_cache,
                       float* v_cache, const int64_t* positions, uint32_t t, uint32_t q_heads, uint32_t kv_heads,
                       uint32_t head_dim, uint32_t max_seq, float scale, float* out, const float* cos_table,
-                      const float* sin_table, uint32_t* fault) {
-#define VXHIP_ATTENTION(R, NC)                                                                                  \
-    hipLaunchKernelGGL((gqa_attention_kernel<R, FUSED, NC>), grid, dim3(256), lds, stream, q, k_cache, v_cache, \
-                       positions, t, q_heads, kv_heads, head_dim, max_seq, scale, out, cos_table, sin_table, fault)
-#define VXHIP_DECODE(R)                                                                                                  \
-    hipLaunchKernelGGL((decode_attention_kernel<R, FUSED>), grid, dim3(512), 0, stream, q, k_cache, v_cache, positions, t, \
-                       q_heads, kv_heads, max_seq, scale, out, cos_table, sin_table, fault)
+                      const float* sin_table) {
+    if (launch_decode_attention(ctx->stream, ctx->cu_count, grid.x, q, k_cache, v_cache, positions, t, q_heads, kv_heads,
+                                head_dim, max_seq, scale, out, cos_table, sin_table, ctx->fault_dev))
+        return;
+#define VXHIP_ATTENTION(R, NC)                                                                                       \
+    hipLaunchKernelGGL((gqa_attention_kernel<R, FUSED, NC>), grid, dim3(256), lds, ctx->stream, q, k_cache, v_cache, \
+                       positions, t, q_heads, kv_heads, head_dim, max_seq, scale, out, cos_table, sin_table, ctx->fault_dev)
 #define VXHIP_ATTENTION_HEADS(NC)     \
     do {                              \
         if (together == 4u) VXHIP_ATTENTION(4, NC); \
@@ -1263,18 +1043,12 @@ void launch_attention(hipStream_t stream, uint32_t together, dim3 grid, size_t l
     } while (0)
     switch (head_dim) {
         case 32: VXHIP_ATTENTION_HEADS(1); break;
-        case 64:
-            if (together == 4u) VXHIP_DECODE(4);
-            else if (together == 2u) VXHIP_DECODE(2);
-            else VXHIP_DECODE(1);
-            break;
-        case 128: VXHIP_ATTENTION_HEADS(4); break;
+        case 128: VXHIP_ATTENTION(4, 4); break;  // (the only ones that are not taken above)
         case 256: VXHIP_ATTENTION_HEADS(8); break;
         default: VXHIP_ATTENTION_HEADS(0); break;
     }
 #undef VXHIP_ATTENTION_HEADS
 #undef VXHIP_ATTENTION
-#undef VXHIP_DECODE
 }
 
 // Embedding lookup (embedding.inc:5-16): out[i] = table[tokens[i]], one workgroup per token.
@@ -1509,9 +1283,9 @@ VxHipStatus vxhip_gqa_attention(VxHipContext* ctx, const float* q_dev, const flo
         return VXHIP_INVALID_ARGUMENT;
     }
     const dim3 grid(rows * t, q_heads / together);
-    launch_attention<false>(ctx->stream, together, grid, token_lds, q_dev, const_cast<float*>(k_cache_dev),
+    launch_attention<false>(ctx, together, grid, token_lds, q_dev, const_cast<float*>(k_cache_dev),
                             const_cast<float*>(v_cache_dev), positions_dev, t, q_heads, kv_heads, head_dim, max_seq,
-                            scale, out_dev, nullptr, nullptr, ctx->fault_dev);
+                            scale, out_dev, nullptr, nullptr);
     VXHIP_TRY(hipGetLastError());
     return VXHIP_OK;
 }
@@ -1537,8 +1311,8 @@ VxHipStatus vxhip_rope_gqa_attention_decode(VxHipContext* ctx, const float* qkv_
         return VXHIP_INVALID_ARGUMENT;
     }
     const dim3 grid(rows, q_heads / together);
-    launch_attention<true>(ctx->stream, together, grid, lds, qkv_dev, k_cache_dev, v_cache_dev, position_dev, 1u,
-                           q_heads, kv_heads, head_dim, max_seq, scale, out_dev, cos_dev, sin_dev, ctx->fault_dev);
+    launch_attention<true>(ctx, together, grid, lds, qkv_dev, k_cache_dev, v_cache_dev, position_dev, 1u,
+                           q_heads, kv_heads, head_dim, max_seq, scale, out_dev, cos_dev, sin_dev);
     VXHIP_TRY(hipGetLastError());
     return VXHIP_OK;
 }
