@@ -1,0 +1,99 @@
+"""The dequantizing linear with K split over a workgroup's wavefronts (gemm_slabs.hip) at the edges of its slabs, passes and tiles,
+and the calls that take it."""
+import numpy as np
+import pytest
+
+import _cases as cases
+
+
+def _linear(oracle, k, n, group, bits, c):
+    import volvoxai_amd as vx
+    w = c["w"] if bits == 8 else cases.four_bit(c["w"])
+    words = oracle.pack_w8_words(w) if bits == 8 else oracle.pack_w4_words(w)
+    return words, vx.PackedLinear(words, c["scales"], c["bias"], k, n, group, weight_bits=bits)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("group", [32, 64, 128, 256])
+@pytest.mark.parametrize("rows,k,n", [(1, 1, 1), (16, 32, 16), (17, 33, 17), (32, 128, 32), (33, 129, 33), (31, 300, 47), (5, 1023, 63),
+                                      (47, 1025, 64), (64, 2048, 65), (65, 2079, 257), (70, 2500, 300)])
+def test_tiles_at_their_edges(ctx, oracle, rows, k, n, group, bits):
+    """One column to more than two passes of every group size, last passes of one wavefront and of all, an odd group in the last slab of
+    two and half a group of 256, rows and channels that end inside a tile, rows that are not finite: the oracle's bits on every tile."""
+    import torch
+    import volvoxai_amd as vx
+    c = cases.packed_case(rows, k, n, group, rows + k + n + bits, True, special_rows=rows == 47)
+    words, pl = _linear(oracle, k, n, group, bits, c)
+    _, want = oracle.packed_linear(c["x"], words, c["scales"], c["bias"], n, group, bits=bits)
+    nan = np.isnan(want)
+    x = torch.from_numpy(c["x"]).cuda()
+    try:
+        for tile in ("slab16x16", "slab16x32", "slab32x32"):
+            vx.force_variant("a8-mfma." + tile)
+            st, y = pl.forward_f32(ctx, x, out=torch.full((rows, n), 7.0, device="cuda"))
+            ctx.synchronize()
+            got = y.cpu().numpy()
+            # (up to two rows, and a few more short ones, go in one launch whatever tile is named)
+            assert st == 0 and (ctx.last_variant.endswith(tile) or rows <= 2), ctx.last_variant
+            assert (np.isnan(got) == nan).all() and (got.view(np.uint32)[~nan] == want.view(np.uint32)[~nan]).all(), ctx.last_variant
+    finally:
+        vx.force_variant(None)
+        pl.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,k,n,bits,group,tile", [
+    (64, 4096, 512, 8, 128, "slab16x16"), (64, 4096, 4096, 8, 128, "slab32x32"), (32, 4096, 4096, 8, 128, "slab16x32"),
+    (128, 4096, 4096, 8, 128, None), (257, 4096, 64, 8, 128, None), (96, 1279, 64, 8, 128, None), (96, 1280, 64, 8, 128, "slab16x16"),
+    (8, 4096, 64, 8, 128, None), (8, 2500, 64, 8, 128, "slab16x16"), (4, 4096, 64, 8, 128, None), (4, 4097, 64, 8, 128, "slab16x16"),
+    (16, 2000, 8000, 4, 128, "slab16x16"), (24, 4096, 14336, 8, 128, None), (24, 4000, 8192, 8, 128, None)])
+def test_which_calls_take_it(ctx, rows, k, n, bits, group, tile):
+    """The lines of the rule at 256 compute units; both entry points agree bit for bit, and with the kernel that took the call before."""
+    import torch
+    import volvoxai_amd as vx
+    from volvoxai_amd.decoder import pack_w4_words, pack_w8_words
+    rng = np.random.default_rng(rows)
+    words = (pack_w8_words if bits == 8 else pack_w4_words)(rng.integers(-7, 8, (n, k)).astype(np.int8))
+    scales = rng.uniform(0.002, 0.01, (n, (k + group - 1) // group)).astype(np.float32)
+    pl = vx.PackedLinear(words, scales, rng.normal(0, 0.1, n).astype(np.float32), k, n, group, weight_bits=bits)
+    x = torch.from_numpy(rng.normal(0, 1, (rows, k)).astype(np.float32)).cuda()
+    try:
+        st, y = pl.forward_f32(ctx, x)
+        assert st == 0 and ("slab" in ctx.last_variant) == bool(tile) and (not tile or ctx.last_variant.endswith(tile)), ctx.last_variant
+        st, again = pl.forward_f32(ctx, x, out=torch.empty_like(y), no_alloc=True)
+        assert st == 0 and ("slab" in ctx.last_variant) == bool(tile), ctx.last_variant
+        vx.force_variant("a8-mfma.t64x64k64")
+        st, plain = pl.forward_f32(ctx, x)
+        vx.force_variant(None)
+        ctx.synchronize()
+        assert st == 0 and torch.equal(y.view(torch.int32), again.view(torch.int32)) and torch.equal(y.view(torch.int32), plain.view(torch.int32))
+    finally:
+        vx.force_variant(None)
+        pl.close()
+
+
+@pytest.mark.gpu
+def test_scratch_with_room_for_the_rows_alone(oracle):
+    """225 rows of 18000 fit the fixed scratch array (4 MiB) and a scratch reserved for them, eight tiles of 32 rows do not: the call is
+    taken as before, and by the slab kernel where its scratch may grow."""
+    import torch
+    import volvoxai_amd as vx
+    rows, k, n, group = 225, 18000, 40, 128
+    c = cases.packed_case(rows, k, n, group, 5, True)
+    words, pl = _linear(oracle, k, n, group, 8, c)
+    _, want = oracle.packed_linear(c["x"], words, c["scales"], c["bias"], n, group)
+    x = torch.from_numpy(c["x"]).cuda()
+    fixed, reserved, growing = vx.Context(0, None), vx.Context(0, None), vx.Context(0, None)
+    try:
+        reserved.reserve_scratch(3 << 20)  # (in whole MiB, with one to spare)
+        out = torch.empty((rows, n), device="cuda")
+        for context, slabs, no_alloc in ((fixed, False, True), (reserved, False, False), (growing, True, False)):
+            out.fill_(7.0)
+            torch.cuda.synchronize()
+            st, _ = pl.forward_f32(context, x, out=out, no_alloc=no_alloc)
+            context.synchronize()
+            assert st == 0 and ("slab" in context.last_variant) == slabs, context.last_variant
+            assert (out.cpu().numpy().view(np.uint32) == want.view(np.uint32)).all()
+    finally:
+        pl.close(), fixed.close(), reserved.close(), growing.close()

@@ -1274,6 +1274,34 @@ static bool run_rows_at_once(VxHipContext* ctx, const VxHipPackedLinear* pl, con
     return id != nullptr;
 }
 
+// The same for calls that gemm_slabs.hip takes: the rows are prepared into tiles of 32.  Where those would outgrow a scratch that has
+// room for the rows themselves (`fixed`: the scratch array, which cannot grow), the caller goes the way that needs no more.
+static int packed_run_slabs(VxHipContext* ctx, const VxHipPackedLinear* pl, const float* x, float* y, uint32_t rows, bool fixed) {
+    const SlabTile tile = pick_slab_tile(f32_row_args(ctx, pl, x, y, rows), ctx->cu_count, forced_variant());
+    if (tile == SlabTile::None) return -2;
+    const uint32_t k = pl->w.k, ld = (k + 15u) / 16u * 16u;
+    const size_t tiled_rows = ((size_t)rows + kOperandOrderRows - 1u) / kOperandOrderRows * kOperandOrderRows;
+    Carver sizes{nullptr}, without{nullptr};
+    sizes.take<float>(rows);
+    sizes.take<int8_t>(tiled_rows * ld);
+    without.take<float>(rows);
+    without.take<int8_t>((size_t)rows * ld);
+    if (fixed ? sizes.off > kNoAllocScratchBytes
+              : sizes.off + 256u > ctx->scratch_bytes && without.off + 256u <= ctx->scratch_bytes)
+        return -2;
+    if (!fixed && ensure_scratch(ctx, sizes.off + 256u) != VXHIP_OK) return -1;
+    Carver c{(char*)(fixed ? ctx->no_alloc_scratch : ctx->scratch)};
+    float* row_scales = c.take<float>(rows);
+    int8_t* prepared = c.take<int8_t>(tiled_rows * ld);
+    if (launch_prepare_i8(ctx->stream, x, rows, k, prepared, ActivationLayout{ld, 1u}, row_scales) != VXHIP_OK) return -1;
+    LinearArgs a = prepared_args(ctx, pl, prepared, ld, row_scales, y, rows);
+    a.x_operand_order = 1u;
+    const char* id = launch_gemm_slabs(ctx->stream, a, tile);
+    if (!id) return -1;
+    set_last_variant(ctx, id);
+    return 0;
+}
+
 int vxhip_packed_linear_forward_f32(VxHipContext* ctx, const VxHipPackedLinear* pl, const float* input_dev,
                                     float* output_dev, uint32_t rows) {
     if (!ctx || !pl || !input_dev || !output_dev) {
@@ -1284,6 +1312,7 @@ int vxhip_packed_linear_forward_f32(VxHipContext* ctx, const VxHipPackedLinear* 
     if (!same_device(ctx, pl->device, "packed_linear_forward_f32") || !use_device(ctx->device)) return -1;
     const uint32_t k = pl->w.k;
     if (run_rows_at_once(ctx, pl, input_dev, output_dev, rows)) return 0;
+    if (const int taken = packed_run_slabs(ctx, pl, input_dev, output_dev, rows, false); taken != -2) return taken;
     const uint32_t ld = (k + 15u) / 16u * 16u;
     // the prepared rows never leave this call: up to 32 rows go to the GEMV in its operand order
     const bool operand_order = rows <= kOperandOrderRows;
@@ -1367,6 +1396,7 @@ int vxhip_packed_linear_forward_f32_noalloc(VxHipContext* ctx, const VxHipPacked
         return -1;
     }
     if (run_rows_at_once(ctx, pl, input_dev, output_dev, rows)) return 0;
+    if (const int taken = packed_run_slabs(ctx, pl, input_dev, output_dev, rows, true); taken != -2) return taken;
     const uint32_t k = pl->w.k;
     const uint32_t ld = (k + 15u) / 16u * 16u;
     const bool operand_order = rows <= kOperandOrderRows;

@@ -218,9 +218,8 @@ void launch_op(hipStream_t s, uint32_t rows, const RowArgs& a) {
 VxHipStatus launch_row_prepare(hipStream_t s, RowOp op, float* x, const float* delta, const float* gain, double eps,
                                uint32_t rows, uint32_t d, int8_t* codes, ActivationLayout layout, float* scales,
                                float* values) {
-    // (operand order has room for 32 rows, and its rows are whole 16-byte chunks)
-    if (layout.operand_order && (rows > kOperandOrderRows || layout.ld != (d + 15u) / 16u * 16u))
-        return VXHIP_INVALID_ARGUMENT;
+    // (the rows of operand order are whole 16-byte chunks)
+    if (layout.operand_order && layout.ld != (d + 15u) / 16u * 16u) return VXHIP_INVALID_ARGUMENT;
     if (op != RowOp::Plain && d > kMaxRowOpLength) return VXHIP_INVALID_ARGUMENT;
     const RowArgs a{x, delta, gain, eps, d, codes, layout, scales, values};
     switch (op) {
