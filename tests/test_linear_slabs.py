@@ -1,4 +1,4 @@
-"""The dequantizing linear with K split over a workgroup's wavefronts (gemm_slabs.hip) at the edges of its slabs, passes and tiles,
+"""The dequantizing linear with K split over a workgroup's wavefronts (linear_slabs.hip) at the edges of its slabs, passes and tiles,
 and the calls that take it."""
 import numpy as np
 import pytest

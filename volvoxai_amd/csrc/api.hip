@@ -1274,7 +1274,7 @@ static bool run_rows_at_once(VxHipContext* ctx, const VxHipPackedLinear* pl, con
     return id != nullptr;
 }
 
-// The same for calls that gemm_slabs.hip takes: the rows are prepared into tiles of 32.  Where those would outgrow a scratch that has
+// The same for calls that linear_slabs.hip takes: the rows are prepared into tiles of 32.  Where those would outgrow a scratch that has
 // room for the rows themselves (`fixed`: the scratch array, which cannot grow), the caller goes the way that needs no more.
 static int packed_run_slabs(VxHipContext* ctx, const VxHipPackedLinear* pl, const float* x, float* y, uint32_t rows, bool fixed) {
     const SlabTile tile = pick_slab_tile(f32_row_args(ctx, pl, x, y, rows), ctx->cu_count, forced_variant());
@@ -1296,7 +1296,7 @@ static int packed_run_slabs(VxHipContext* ctx, const VxHipPackedLinear* pl, cons
     if (launch_prepare_i8(ctx->stream, x, rows, k, prepared, ActivationLayout{ld, 1u}, row_scales) != VXHIP_OK) return -1;
     LinearArgs a = prepared_args(ctx, pl, prepared, ld, row_scales, y, rows);
     a.x_operand_order = 1u;
-    const char* id = launch_gemm_slabs(ctx->stream, a, tile);
+    const char* id = launch_linear_slabs(ctx->stream, a, tile);
     if (!id) return -1;
     set_last_variant(ctx, id);
     return 0;

@@ -151,7 +151,7 @@ VxHipStatus launch_stage_activations(hipStream_t s, const void* x, uint32_t rows
 // ((j / 16) * 32 + row) * 16 + j % 16, which is how a wavefront of the streaming GEMV wants them:
 // the 64 lanes' loads of one k-step are then 1 KiB in a row (8 cache lines) instead of 32 bytes
 // from each of 32 lines.  Such a buffer always holds whole tiles of 32 rows of ceil(k / 16) chunks.
-// (What callers exchange has one tile; gemm_slabs.hip takes more.)
+// (What callers exchange has one tile; linear_slabs.hip takes more.)
 struct ActivationLayout {
     uint32_t ld;
     uint32_t operand_order;
@@ -307,12 +307,12 @@ const char* launch_gemv_row(hipStream_t s, const LinearArgs& a, int cu_count, co
 // gemv_few.hip: three to eight f32 rows of a DequantF32 linear, prepared by the kernel itself; null where it does not take
 // the call
 const char* launch_gemv_few(hipStream_t s, const LinearArgs& a, int cu_count, const char* force);
-// gemm_slabs.hip: a DequantF32 linear on prepared rows in operand order, tiles of 32 of them one after the other, for launches of
+// linear_slabs.hip: a DequantF32 linear on prepared rows in operand order, tiles of 32 of them one after the other, for launches of
 // few tiles.  pick_slab_tile says which tile a call should take (channels x rows), or None: nothing but a's extents, group
 // size and weight width is looked at.
 enum class SlabTile : int { None = 0, T16x16 = 1, T16x32 = 2, T32x32 = 3 };
 SlabTile pick_slab_tile(const LinearArgs& a, int cu_count, const char* force);
-const char* launch_gemm_slabs(hipStream_t s, const LinearArgs& a, SlabTile tile);
+const char* launch_linear_slabs(hipStream_t s, const LinearArgs& a, SlabTile tile);
 // While on (per thread), launch_gemv_stream chooses as always and launches nothing: its result tells
 // whether a call of that description would be taken.
 void set_gemv_dry_run(bool on);

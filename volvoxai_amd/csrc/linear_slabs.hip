@@ -38,7 +38,7 @@ struct SlabLds {
 
 // A tile of 16 * TN channels and 16 * TM rows, TN and TM of 1 and 2.
 template <int GROUP, bool W4, int TN, int TM>
-__global__ __launch_bounds__(WAVES * 64, 4) void gemm_slab_kernel(const GemmParams p) {
+__global__ __launch_bounds__(WAVES * 64, 4) void linear_slab_kernel(const GemmParams p) {
     constexpr int STEPS = GROUP <= 64 ? 1 : 2;    // MFMA steps of 64 columns in a slab
     constexpr int GPS = GROUP == 32 ? 2 : 1;      // scale groups that end in a slab (GROUP == 256: in every second one)
     constexpr int HALVES = GROUP == 256 ? 2 : 1;  // slabs of a unit, which is what a wavefront takes of a pass
@@ -220,7 +220,7 @@ template <int GROUP, bool W4, int TN, int TM>
 bool launch(hipStream_t s, const LinearArgs& a) {
     constexpr int LDS = SlabLds<GROUP, TN, TM>::BYTES;
     static std::atomic<uint64_t> configured{0};
-    auto kern = gemm_slab_kernel<GROUP, W4, TN, TM>;
+    auto kern = linear_slab_kernel<GROUP, W4, TN, TM>;
     if (!raise_lds_limit((const void*)kern, LDS, configured)) return false;
     GemmParams p;
     p.a = a;
@@ -296,7 +296,7 @@ SlabTile pick_slab_tile(const LinearArgs& a, int cu_count, const char* force) {
 }
 
 // a.x: operand order in tiles of 32 rows, ldx = the columns rounded up to 16.
-const char* launch_gemm_slabs(hipStream_t s, const LinearArgs& a, SlabTile tile) {
+const char* launch_linear_slabs(hipStream_t s, const LinearArgs& a, SlabTile tile) {
     if (a.mode != Epilogue::DequantF32 || !a.x || !a.x_operand_order || !a.y || !a.rows || a.acc_out || a.add_to || a.x_flip_mask ||
         a.ldx != (a.k + 15u) / 16u * 16u || (uintptr_t)a.x % 16u)
         return nullptr;
