@@ -552,6 +552,49 @@ int vxhip_packed_linear_add_a8(VxHipContext* context,
                                const float* row_scales_dev, float* residual_dev,
                                uint32_t rows);
 
+/* A small prompt of a pre-norm decoder (RMSNorm, q/k/v, rotary embedding and cache
+ * append, grouped-query attention, output projection, residual add, RMSNorm,
+ * gate/up, SwiGLU, down projection, residual add; then RMSNorm, lm_head, ArgMax)
+ * as one call: the launches of the entry points of this header, issued without
+ * the host in between, with the same bits.  (Of any size; a prompt large enough
+ * for vxhip_packed_linear_rope_append_a8 and its neighbours is faster with
+ * them.)  No counterpart in the reference, whose graph executor plays this part.
+ *   tokens_dev [rows, t] int32 ids, t of 2 to max_seq; positions_dev [t]; caches
+ *   [rows, kv_heads, max_seq, head_dim]; logits_dev [rows, lm_head channels] and
+ *   next_dev [rows] of each row's last token.
+ * workspace_dev: vxhip_decoder_prompt_workspace bytes on a 256-byte boundary,
+ * the caller's, in use until the launches have run.  That function returns 0,
+ * and the call VXHIP_INVALID_ARGUMENT with nothing launched, where an argument
+ * is NULL or extents do not fit each other. */
+typedef struct VxHipDecoderLayer {
+    const float* gain1_dev;
+    const float* gain2_dev;
+    const VxHipPackedLinear* qkv;
+    const VxHipPackedLinear* output;
+    const VxHipPackedLinear* gate_up;
+    const VxHipPackedLinear* down;
+    float* k_cache_dev;
+    float* v_cache_dev;
+} VxHipDecoderLayer;
+typedef struct VxHipDecoderPrompt {
+    const VxHipDecoderLayer* layers;
+    const int32_t* tokens_dev;
+    const float* embedding_dev;
+    const float* final_gain_dev;
+    const VxHipPackedLinear* lm_head;
+    const float* cos_dev;
+    const float* sin_dev;
+    const int64_t* positions_dev;
+    void* workspace_dev;
+    size_t workspace_bytes;
+    float* logits_dev;
+    int32_t* next_dev;
+    double eps;
+    uint32_t layer_count, rows, t, hidden, vocab, q_heads, kv_heads, head_dim, max_seq;
+} VxHipDecoderPrompt;
+size_t vxhip_decoder_prompt_workspace(const VxHipContext* context, const VxHipDecoderPrompt* prompt);
+VxHipStatus vxhip_decoder_prompt(VxHipContext* context, const VxHipDecoderPrompt* prompt);
+
 /* Field-for-field layout of the PackedLinear part of VxLLMOpArgs
  * (src/kernels/llm_ops.h:38-53) is not reproduced here; this one-shot HOST
  * entry takes the same values as plain arguments: x=input f32 [rows,k],

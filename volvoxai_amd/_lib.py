@@ -105,6 +105,8 @@ def _declare(L: C.CDLL) -> None:
         "vxhip_packed_linear_rope_append_a8": (C.c_int, [vp, vp, vp, vp, vp, vp, vp, u32, u32, u32, u32, u32, u32, vp, vp, vp]),
         "vxhip_packed_linear_swiglu_a8": (C.c_int, [vp, vp, vp, vp, vp, u32]),
         "vxhip_packed_linear_add_a8": (C.c_int, [vp, vp, vp, vp, vp, u32]),
+        "vxhip_decoder_prompt_workspace": (sz, [vp, vp]),
+        "vxhip_decoder_prompt": (i32, [vp, vp]),
         "vxhip_packed_linear_f32": (C.c_int, [vp, vp, vp, vp, vp, u64, i32, i32, i32, i32, i32, u64, u64]),
         "vxhip_packed_linear_forward_f32_window": (C.c_int, [vp, vp, vp, vp, u32, u64, u64]),
         "vxhip_quantize_typed_f32_i8u8": (C.c_int, [vp, u32, vp, f32, i32, u32]),

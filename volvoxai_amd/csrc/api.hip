@@ -402,6 +402,7 @@ void vxhip_context_destroy(VxHipContext* ctx) {
     if (ctx->scratch) (void)hipFree(ctx->scratch);
     for (int i = 0; i < ctx->retired_count; i++) (void)hipFree(ctx->retired[i]);
     if (ctx->fault_dev) (void)hipFree(ctx->fault_dev);
+    if (ctx->fault_host) (void)hipHostFree(ctx->fault_host);
     if (ctx->div_proof_dev) (void)hipFree(ctx->div_proof_dev);
     if (ctx->io_in) (void)hipFree(ctx->io_in);
     if (ctx->io_out) (void)hipFree(ctx->io_out);
@@ -490,8 +491,14 @@ const char* vxhip_context_last_variant(const VxHipContext* ctx) { return ctx ? c
 
 VxHipStatus vxhip_context_fault_flags(VxHipContext* ctx, uint32_t* flags) {
     if (!ctx || !flags || !not_recording(ctx, "context_fault_flags")) return VXHIP_INVALID_ARGUMENT;
-    VXHIP_TRY(hipMemcpyAsync(flags, ctx->fault_dev, sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream));
+    if (!use_device(ctx->device)) return VXHIP_BACKEND_UNAVAILABLE;
+    // A copy of the word to the caller's memory takes the stream 10 us longer than this store, once in every decode step
+    // whose ids a program chooses.  (Pinned when it is first asked for: that takes 70 us.)
+    if (!ctx->fault_host) VXHIP_TRY(hipHostMalloc((void**)&ctx->fault_host, sizeof(uint32_t), hipHostMallocDefault));
+    const VxHipStatus published = launch_publish_u32(ctx->stream, ctx->fault_dev, ctx->fault_host);
+    if (published != VXHIP_OK) return published;
     VXHIP_TRY(hipStreamSynchronize(ctx->stream));
+    *flags = __atomic_load_n(ctx->fault_host, __ATOMIC_RELAXED);
     return VXHIP_OK;
 }
 

@@ -257,6 +257,16 @@ VxHipStatus launch_fill_u32(hipStream_t s, uint32_t* p, uint32_t count, uint32_t
     return VXHIP_OK;
 }
 
+__global__ void publish_u32_kernel(const uint32_t* p, uint32_t* host) {
+    __hip_atomic_store(host, *p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+VxHipStatus launch_publish_u32(hipStream_t s, const uint32_t* p, uint32_t* host) {
+    hipLaunchKernelGGL(publish_u32_kernel, dim3(1), dim3(1), 0, s, p, host);
+    VXHIP_TRY(hipGetLastError());
+    return VXHIP_OK;
+}
+
 // ---- exactness proof of the short division ------------------------------------
 // Division by a fixed divisor scales exactly with the dividend's exponent (as long as nothing
 // leaves the normal range), so trying all 2^23 mantissas at one exponent decides it for every

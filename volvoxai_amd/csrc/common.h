@@ -77,6 +77,7 @@ struct VxHipContext {
     void* retired[kRetiredSlots] = {};
     int retired_count = 0;
     uint32_t* fault_dev = nullptr;
+    uint32_t* fault_host = nullptr;  // pinned, where vxhip_context_fault_flags has the word written to
     void* no_alloc_scratch = nullptr;  // this device's address of the fixed scratch array (api.hip), or null
     // Exhaustive exactness proofs of the short division sequences, one pair of mismatch
     // counters per divisor seen (the output scales of the calls made on this context).
@@ -181,6 +182,7 @@ VxHipStatus launch_unblock_activations(hipStream_t s, const int8_t* blocked, uin
 VxHipStatus launch_requantize(hipStream_t s, const void* x, uint32_t n, void* y, float multiplier, int32_t zp_in,
                               int32_t zp_out, bool in_i8, bool out_i8);
 VxHipStatus launch_fill_u32(hipStream_t s, uint32_t* p, uint32_t count, uint32_t value);
+VxHipStatus launch_publish_u32(hipStream_t s, const uint32_t* p, uint32_t* host);  // *host = *p, host pinned
 // Counts, over every f32 mantissa of the dividend, where the one- and the two-correction
 // division by `divisor` differ from IEEE division: counters[0] and counters[1].
 VxHipStatus launch_division_proof(hipStream_t s, float divisor, float recip, uint32_t* counters);

@@ -278,7 +278,13 @@ class W8A8Decoder:
         to `next_tokens` when given; `advance` counters are incremented by the same launch)."""
         cfg = self.cfg
         rows, t = tokens.shape
-        # Which linears of a prompt are tried with what follows them.  The tiles that do it are picked from 384 of 64 x 64
+        # A small prompt is bound by the host: one call issues its launches, without the linears that take what follows them.  4
+        # layers of hidden 1024 that way | a call a launch, with those linears: 180 tokens 232 | 410 us, 340 274 | 384, 500 314 | 371,
+        # 800 389 | 391, 1200 477 | 449; of hidden 512 1200 tokens 265 | 397.
+        if t > 1 and next_tokens is None and advance is None and rows * t * self.layers[0]["qkv"].n < 1 << 21:
+            return vx.decoder_prompt(self.ctx, tokens, self.embedding, self.layers, self.gain_f, self.lm_head, self.cos, self.sin, positions,
+                                     cfg.q_heads, cfg.kv_heads, cfg.head_dim, cfg.eps, self.k_cache, self.v_cache)
+        # Which linears of a larger one are tried with what follows them.  The tiles that do it are picked from 384 of 64 x 64
         # outputs on (1.5 a compute unit); with fewer outputs than 256 whole ones that takes tiles a third empty, and
         # the attempts are spared.
         self.takes = {name: rows * t > 32 and rows * t * self.layers[0][name].n >= 1 << 20 for name in ("qkv", "o", "gate_up", "down")}

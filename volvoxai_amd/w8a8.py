@@ -610,6 +610,58 @@ def packed_prepare_i8(ctx: Context, x):
     return a8, scales
 
 
+class _DecoderLayer(C.Structure):
+    _fields_ = [(name, C.c_void_p) for name in ("gain1", "gain2", "qkv", "output", "gate_up", "down", "k_cache", "v_cache")]
+
+
+class _DecoderPrompt(C.Structure):
+    _fields_ = ([("layers", C.POINTER(_DecoderLayer))] +
+                [(name, C.c_void_p) for name in ("tokens", "embedding", "final_gain", "lm_head", "cos", "sin", "positions", "workspace")] +
+                [("workspace_bytes", C.c_size_t), ("logits", C.c_void_p), ("next", C.c_void_p), ("eps", C.c_double)] +
+                [(name, C.c_uint32) for name in ("layer_count", "rows", "t", "hidden", "vocab", "q_heads", "kv_heads", "head_dim", "max_seq")])
+
+
+def decoder_prompt(ctx: Context, tokens, embedding, layers, final_gain, lm_head, cos, sin, positions, q_heads, kv_heads, head_dim, eps,
+                   k_cache, v_cache):
+    """A pre-norm decoder's prompt as one call (vxhip_decoder_prompt): tokens int32 [rows, t], t of 2 and more; layers: dicts of the
+    PackedLinears "qkv", "o", "gate_up", "down" and the f32 vectors "gain1", "gain2"; caches [layers, rows, kv_heads, max_seq, head_dim].
+    Returns the logits of each row's last token and their argmax (int32)."""
+    import torch
+    rows, t = tokens.shape
+    vocab, hidden = embedding.shape
+    if k_cache.ndim != 5 or k_cache.shape[0] != len(layers) or v_cache.shape != k_cache.shape:
+        raise ValueError(f"k_cache, v_cache: shapes {tuple(k_cache.shape)}, {tuple(v_cache.shape)}, expected [{len(layers)}, rows, kv_heads, "
+                         "max_seq, head_dim]")
+    _dp(k_cache, "k_cache", torch.float32), _dp(v_cache, "v_cache", torch.float32)
+    max_seq = _check_caches(k_cache[0], v_cache[0], cos, sin, rows, kv_heads, head_dim)
+    next_tokens = torch.empty((rows,), dtype=torch.int32, device=embedding.device)
+    logits = torch.empty((rows, lm_head.n), dtype=torch.float32, device=embedding.device)
+    filled = (_DecoderLayer * len(layers))()
+    k_at, v_at, cache_bytes = k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(0) * 4
+    for i, (layer, to) in enumerate(zip(layers, filled)):
+        to.gain1, to.gain2 = _dp(layer["gain1"], "gain1", torch.float32, numel=hidden), _dp(layer["gain2"], "gain2", torch.float32, numel=hidden)
+        to.qkv, to.output, to.gate_up, to.down = layer["qkv"]._h, layer["o"]._h, layer["gate_up"]._h, layer["down"]._h
+        to.k_cache, to.v_cache = k_at + i * cache_bytes, v_at + i * cache_bytes
+    p = _DecoderPrompt(layers=filled, tokens=_dp(tokens, "tokens", torch.int32), embedding=_dp(embedding, "embedding", torch.float32),
+                       final_gain=_dp(final_gain, "final_gain", torch.float32, numel=hidden), lm_head=lm_head._h, cos=_dp(cos), sin=_dp(sin),
+                       positions=_dp(positions, "positions", torch.int64, numel=t), logits=_dp(logits),
+                       next=_dp(next_tokens), eps=float(eps), layer_count=len(layers), rows=rows, t=t,
+                       hidden=hidden, vocab=vocab, q_heads=q_heads, kv_heads=kv_heads, head_dim=head_dim, max_seq=max_seq)
+    p.workspace_bytes = library().vxhip_decoder_prompt_workspace(ctx._h, C.byref(p))
+    # (the workspace goes back to the allocator at return: it has to belong to the stream that uses it)
+    if ctx._stream is not None:
+        with torch.cuda.stream(ctx._stream):
+            workspace = torch.empty((p.workspace_bytes,), dtype=torch.uint8, device=embedding.device)
+    else:
+        workspace = torch.empty((p.workspace_bytes,), dtype=torch.uint8, device=embedding.device)
+        torch.cuda.current_stream().synchronize()
+    p.workspace = workspace.data_ptr()
+    _check(library().vxhip_decoder_prompt(ctx._h, C.byref(p)), "vxhip_decoder_prompt")
+    if ctx._stream is None:
+        ctx.synchronize()
+    return logits, next_tokens
+
+
 # ---- host-pointer drop-ins (numpy in, numpy out) -------------------------------
 
 def qlinear_i8u8(input, weight, weight_scales, weight_zero_points, bias, rows, d_in, d_out,
