@@ -47,7 +47,7 @@ def test_tiles_at_their_edges(ctx, oracle, rows, k, n, group, bits):
     (64, 4096, 512, 8, 128, "slab16x16"), (64, 4096, 4096, 8, 128, "slab32x32"), (32, 4096, 4096, 8, 128, "slab16x32"),
     (128, 4096, 4096, 8, 128, None), (257, 4096, 64, 8, 128, None), (96, 1279, 64, 8, 128, None), (96, 1280, 64, 8, 128, "slab16x16"),
     (8, 4096, 64, 8, 128, None), (8, 2500, 64, 8, 128, "slab16x16"), (4, 4096, 64, 8, 128, None), (4, 4097, 64, 8, 128, "slab16x16"),
-    (16, 2000, 8000, 4, 128, "slab16x16"), (24, 4096, 14336, 8, 128, None), (24, 4000, 8192, 8, 128, None)])
+    (16, 2000, 8000, 4, 128, "slab16x16"), (24, 4096, 14336, 8, 128, None), (24, 4000, 8192, 8, 128, None), (16, 2048, 14336, 8, 64, None), (16, 4096, 6144, 8, 64, "slab16x16")])
 def test_which_calls_take_it(ctx, rows, k, n, bits, group, tile):
     """The lines of the rule at 256 compute units; both entry points agree bit for bit, and with the kernel that took the call before."""
     import torch

@@ -261,7 +261,7 @@ bool launch_bits(hipStream_t s, const LinearArgs& a) {
 // in groups of 32 and 64 are slower up to 2.7 (16 x 4096 -> 14336 in groups of 64 28.9 | 20.2 | 21.0 | 18.8).  Groups of 256 have the
 // cheapest fold there (150 x 2500 -> 1500 9.1 | 11.7 | 10.2 | 9.2), short rows the fewest k-blocks (207 x 1440 -> 1056 7.5 us, 32x32 9.3).
 // The straight-line instances keep their calls up to eight rows (6 x 3000 -> 1531 6.2 | 6.5, but 8 x 2500 -> 1500, which has none,
-// 9.3 | 6.8) and on whole panels (16 x 4096 -> 8192 10.5 | 13.1).
+// 9.3 | 6.8) and on whole panels (16 x 4096 -> 8192 10.5 | 13.1, 16 x 2048 -> 14336 in groups of 64 12.0 | 13.6).
 // 110 drawn calls of 3 to 256 rows, K from 1024: the 68 that come here take 0.76 of their time (geometric mean), the worst 1.02.
 SlabTile pick_slab_tile(const LinearArgs& a, int cu_count, const char* force) {
     if (a.weight_bits != 8u && a.weight_bits != 4u) return SlabTile::None;
@@ -279,7 +279,8 @@ SlabTile pick_slab_tile(const LinearArgs& a, int cu_count, const char* force) {
     const bool fits = a.rows <= (four ? 8u : 32u) && (shared || enough) &&
                       (columns == 1024u || columns == 2048u || columns == 3072u || columns == 4096u || columns == 8192u || columns == 14336u);
     if (a.k < (a.rows <= 4u ? 4097u : a.rows <= 8u ? 2049u : fits ? 2048u : 1280u)) return SlabTile::None;
-    if (fits && (a.rows <= 8u || (enough && a.group_size >= 128u))) return SlabTile::None;
+    // (whole panels: its products of all groups leave a compute unit room for two workgroups, or are at least few)
+    if (fits && (a.rows <= 8u || (enough && (a.group_size >= 128u || a.groups * a.rows * 128u <= 80u * 1024u)))) return SlabTile::None;
     const auto cost = [&](uint32_t tile_n, uint32_t tile_m, float one) {
         const float per = (float)((uint64_t)((a.n + tile_n - 1u) / tile_n) * ((a.rows + tile_m - 1u) / tile_m)) / (float)cu;
         return one * (per > 1.0f ? 1.0f + 0.6f * (per - 1.0f) : 1.0f);
