@@ -97,3 +97,20 @@ def test_scratch_with_room_for_the_rows_alone(oracle):
             assert (out.cpu().numpy().view(np.uint32) == want.view(np.uint32)).all()
     finally:
         pl.close(), fixed.close(), reserved.close(), growing.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,n,tile", [(1000, 1531, "t64x32k64"), (640, 4096, "t64x32k64"), (900, 4096, "t64x64k64"), (768, 4096, "t64x64k64")])
+def test_tiles_of_groups_of_32(ctx, oracle, rows, n, tile):
+    """More 64x64 tiles than 1.5 a compute unit (256 of them): the half tiles where they need an odd number of rounds of the device."""
+    import torch
+    c = cases.packed_case(rows, 96, n, 32, rows, True)
+    words, pl = _linear(oracle, 96, n, 32, 8, c)
+    _, want = oracle.packed_linear(c["x"], words, c["scales"], c["bias"], n, 32)
+    try:
+        st, y = pl.forward_f32(ctx, torch.from_numpy(c["x"]).cuda())
+        ctx.synchronize()
+        assert st == 0 and ctx.last_variant.endswith(tile), ctx.last_variant
+        assert (y.cpu().numpy().view(np.uint32) == want.view(np.uint32)).all()
+    finally:
+        pl.close()
