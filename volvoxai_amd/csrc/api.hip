@@ -302,6 +302,10 @@ static const char* run_linear(VxHipContext* ctx, const LinearArgs& a) {
     const char* id = nullptr;
     if (force_gemv) return launch_gemv_stream(ctx->stream, a, ctx->cu_count, force);
     if (force_gemm || force_gemm_f) return launch_gemm_mfma(ctx->stream, a, ctx->cu_count, force);
+    // (rows that the streaming kernel takes, but not as fast: see launch_requant_split)
+    if (!force && a.rows > kMaxGemvRows / 2u && a.rows <= kMaxGemvRows && a.mode != Epilogue::DequantF32 &&
+        launch_requant_split(ctx->stream, a, ctx->cu_count, nullptr))
+        return a.mode == Epilogue::RequantRow ? "hip.qlinear.mfma-i8-rowscale.t32x32split" : "hip.qlinear.mfma-i8.t32x32split";
     if (a.rows <= kMaxGemvRows) id = launch_gemv_stream(ctx->stream, a, ctx->cu_count, force);
     if (!id) id = launch_gemm_mfma(ctx->stream, a, ctx->cu_count, force);
     return id;

@@ -291,6 +291,9 @@ bool launch_decode_attention(hipStream_t s, int cu_count, uint32_t tokens, const
 // gemm_mfma.hip / gemv_stream.hip: return the variant id that ran, or null if
 // the shape is outside the kernel's domain (nothing launched).
 const char* launch_gemm_mfma(hipStream_t s, const LinearArgs& a, int cu_count, const char* force);
+// qlinear_split.hip: requantizing linears of few tiles of output, K split over a workgroup's wavefronts: the tile's name, or null where it
+// does not take the call
+const char* launch_requant_split(hipStream_t s, const LinearArgs& a, int cu_count, const char* force);
 // A kernel's dynamic-LDS limit is an attribute per device: raised once per device and kernel
 // (`done` holds one bit per device ordinal; a racing second call only repeats the request).
 inline bool raise_lds_limit(const void* kernel, int bytes, std::atomic<uint64_t>& done) {

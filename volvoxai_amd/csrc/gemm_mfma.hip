@@ -621,6 +621,7 @@ const char* dispatch_tile(hipStream_t s, const LinearArgs& a, int cu_count, cons
         if (GK == 1 || forced("t128x128")) return launch_cfg<2, 2, 2, 2, MODE, GK, W4>(s, a) ? "t128x128" : nullptr;
         return launch_cfg<2, 4, 2, 2, MODE, GK, W4>(s, a) ? "t128x256" : nullptr;
     } else {
+        if (const char* split = launch_requant_split(s, a, cu_count, force)) return split;
         // Largest tile (channels x rows) that still gives every compute unit work; names are BNxBM.
         const auto tiles = [&](uint32_t bn, uint32_t bm) {
             return (uint64_t)((a.n + bn - 1) / bn) * ((a.rows + bm - 1) / bm);

@@ -15,10 +15,10 @@ constexpr int kQuantizeLinear = 0, kDequantizeLinear = 0;  // boundary ops carry
 
 const VxHipKernelVariant kVariants[] = {
     // (tile suffixes ending in k64 are gemm_k64_kernel, the 16x16x64 form of the large tiles)
-    QROWS("hip.qlinear.mfma-i8", "gemm_mfma_kernel<RequantTensor>|gemm_k64_kernel<RequantTensor>",
+    QROWS("hip.qlinear.mfma-i8", "gemm_mfma_kernel<RequantTensor>|gemm_k64_kernel<RequantTensor>|requant_split_kernel<RequantTensor>",
           "hip.qlinear.canonical-resident-int32-bound-rows-gt32-any-k-tail",
           "hip.gfx950-mfma-i32-32x32x32-i8,hip.gfx950-mfma-i32-16x16x64-i8,hip.global-load-lds-b128", 300),
-    QROWS("hip.qlinear.mfma-i8-rowscale", "gemm_mfma_kernel<RequantRow>|gemm_k64_kernel<RequantRow>",
+    QROWS("hip.qlinear.mfma-i8-rowscale", "gemm_mfma_kernel<RequantRow>|gemm_k64_kernel<RequantRow>|requant_split_kernel<RequantRow>",
           "hip.qlinear.per-row-input-scale-i8-zero-input-zp-int32-bound-rows-gt32",
           "hip.gfx950-mfma-i32-32x32x32-i8,hip.gfx950-mfma-i32-16x16x64-i8,hip.global-load-lds-b128", 300),
     QROWS("hip.qlinear.gemv-mfma", "gemv_panel_kernel<RequantTensor>",
