@@ -107,3 +107,25 @@ def test_structures_as_the_header_lays_them_out():
     assert C.sizeof(_DecoderLayer) == 64 and C.sizeof(_DecoderPrompt) == 144
     assert (_DecoderPrompt.workspace_bytes.offset, _DecoderPrompt.logits.offset, _DecoderPrompt.eps.offset,
             _DecoderPrompt.layer_count.offset, _DecoderPrompt.max_seq.offset) == (72, 80, 96, 104, 136)
+
+
+@pytest.mark.gpu
+def test_fault_words_of_many_contexts():
+    """More contexts than the pinned page has lines, destroyed and created again: every one reads its own fault word."""
+    import torch
+    from volvoxai_amd import w8a8 as vx
+    table = torch.ones((4, 8), device="cuda")
+    good, bad = torch.tensor([1], dtype=torch.int32, device="cuda"), torch.tensor([9], dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    contexts = [vx.Context(0, None) for _ in range(70)]
+    for turn in range(2):
+        for i, context in enumerate(contexts):
+            vx.embedding_gather(context, bad if i % 3 == turn else good, table, out=torch.empty((1, 8), device="cuda"))
+        assert [c.fault_flags() for c in contexts] == [2 if i % 3 == turn else 0 for i in range(70)]
+        for c in contexts[::2]:
+            c.close()
+        for c in contexts[1::2]:
+            c.clear_fault_flags()
+        contexts[::2] = [vx.Context(0, None) for _ in range(35)]
+    for c in contexts:
+        c.close()

@@ -78,6 +78,38 @@ VxHipStatus ensure_scratch(VxHipContext* ctx, size_t bytes) {
     return VXHIP_OK;
 }
 
+// Pinned words of the contexts (fault_host), a 64-byte line each.  Pinning takes 70 us, so the lines are those of one page that is pinned
+// with the first context and kept; contexts past its 64 pin a word of their own.
+struct PinnedWords {
+    std::mutex lock;
+    char* page = nullptr;
+    uint64_t taken = 0;
+};
+static PinnedWords g_pinned_words;
+constexpr size_t kPinnedLine = 64u;
+
+static hipError_t take_pinned_word(uint32_t** word) {
+    std::lock_guard<std::mutex> guard(g_pinned_words.lock);
+    if (!g_pinned_words.page) {
+        const hipError_t e = hipHostMalloc((void**)&g_pinned_words.page, 64u * kPinnedLine, hipHostMallocPortable);
+        if (e != hipSuccess) return e;
+    }
+    if (~g_pinned_words.taken) {
+        const int line = __builtin_ctzll(~g_pinned_words.taken);
+        g_pinned_words.taken |= 1ull << line;
+        *word = (uint32_t*)(g_pinned_words.page + (size_t)line * kPinnedLine);
+        return hipSuccess;
+    }
+    return hipHostMalloc((void**)word, sizeof(uint32_t), hipHostMallocPortable);
+}
+// (the context's stream has been waited for: nothing writes the word any more)
+static void give_pinned_word(uint32_t* word) {
+    std::lock_guard<std::mutex> guard(g_pinned_words.lock);
+    const ptrdiff_t at = (char*)word - g_pinned_words.page;
+    if (at >= 0 && at < (ptrdiff_t)(64u * kPinnedLine)) g_pinned_words.taken &= ~(1ull << (at / (ptrdiff_t)kPinnedLine));
+    else (void)hipHostFree(word);
+}
+
 void set_last_variant(VxHipContext* ctx, const char* id) {
     // (no formatting: this is on every call's path)
     const size_t length = id ? strnlen(id, sizeof ctx->last_variant - 1u) : 0u;
@@ -384,6 +416,7 @@ VxHipStatus vxhip_context_create(int32_t device, void* stream, uint32_t flags, V
     }
     hipError_t e = hipMalloc((void**)&ctx->fault_dev, 256);
     if (e == hipSuccess) e = hipMemset(ctx->fault_dev, 0, 256);
+    if (e == hipSuccess) e = take_pinned_word(&ctx->fault_host);
     if (e == hipSuccess)
         e = hipMalloc((void**)&ctx->div_proof_dev, VxHipContext::kDivisorSlots * 2 * sizeof(uint32_t));
     if (e != hipSuccess) {
@@ -406,7 +439,7 @@ void vxhip_context_destroy(VxHipContext* ctx) {
     if (ctx->scratch) (void)hipFree(ctx->scratch);
     for (int i = 0; i < ctx->retired_count; i++) (void)hipFree(ctx->retired[i]);
     if (ctx->fault_dev) (void)hipFree(ctx->fault_dev);
-    if (ctx->fault_host) (void)hipHostFree(ctx->fault_host);
+    if (ctx->fault_host) give_pinned_word(ctx->fault_host);
     if (ctx->div_proof_dev) (void)hipFree(ctx->div_proof_dev);
     if (ctx->io_in) (void)hipFree(ctx->io_in);
     if (ctx->io_out) (void)hipFree(ctx->io_out);
@@ -497,8 +530,7 @@ VxHipStatus vxhip_context_fault_flags(VxHipContext* ctx, uint32_t* flags) {
     if (!ctx || !flags || !not_recording(ctx, "context_fault_flags")) return VXHIP_INVALID_ARGUMENT;
     if (!use_device(ctx->device)) return VXHIP_BACKEND_UNAVAILABLE;
     // A copy of the word to the caller's memory takes the stream 10 us longer than this store, once in every decode step
-    // whose ids a program chooses.  (Pinned when it is first asked for: that takes 70 us.)
-    if (!ctx->fault_host) VXHIP_TRY(hipHostMalloc((void**)&ctx->fault_host, sizeof(uint32_t), hipHostMallocDefault));
+    // whose ids a program chooses.
     const VxHipStatus published = launch_publish_u32(ctx->stream, ctx->fault_dev, ctx->fault_host);
     if (published != VXHIP_OK) return published;
     VXHIP_TRY(hipStreamSynchronize(ctx->stream));
