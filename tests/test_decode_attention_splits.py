@@ -16,3 +16,12 @@ from test_decode_attention import ctx  # noqa: F401
 ])
 def test_decode_attention_splits(ctx, rows, q_heads, kv_heads, head_dim, position):  # noqa: F811
     blocks.test_decode_attention_blocks(ctx, rows, q_heads, kv_heads, head_dim, position)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("position", [256, 319, 320, 383, 384, 447, 448, 511, 512, 519])
+@pytest.mark.parametrize("rows,q_heads,kv_heads,head_dim", [(3, 8, 4, 128), (9, 16, 8, 128), (50, 3, 1, 128), (5, 8, 4, 64), (65, 8, 4, 64), (130, 8, 1, 64)])
+def test_first_blocks_that_are_not_whole(ctx, rows, q_heads, kv_heads, head_dim, position):  # noqa: F811
+    """Past 256 slots: one to four rounds of 64 in the first block, the last round with strips of one wavefront and of all, two
+    blocks and three."""
+    blocks.test_decode_attention_blocks(ctx, rows, q_heads, kv_heads, head_dim, position)

@@ -6,7 +6,7 @@
 // nothing else.  Few rows are bound by the latency of a launch (1.7), of the position and behind it of the rows (1.5), and
 // by what a compute unit takes in: its address unit needs 16 cycles a load of 1 KiB, a microsecond for the 148 KB of a
 // head.  So one walk asks for everything that is in sight, values too, before the query is ready, holds it in registers (256
-// slots: 128 of a lane's at head size 128), and asks for nothing else; and scores, sums and outputs cross the
+// slots: 128 of a lane's at head size 128), and up to there asks for nothing else; and scores, sums and outputs cross the
 // workgroup twice.  At slot 145, against a kernel that kept its scores in LDS and asked for its values behind them (head size 128)
 // and one walk of blocks of 128 slots with their requests clamped (64), 16 query and 8 KV heads of 128: 1 row
 // 7.3 -> 4.1 us, 8 rows 8.0 -> 5.2, 16 rows 8.9 -> 6.9, 32 rows 12.3 -> 9.3; 8 and 4 of 64: 1 row 4.6 -> 3.3, 32 rows 5.7 -> 4.9.
@@ -23,12 +23,14 @@
 namespace vxhip {
 namespace {
 
+constexpr int kWaitLoads = 0x0f70;  // s_waitcnt vmcnt(0), the other counters at their largest
+
 // grid (rows * t, kv_heads, query heads of a KV head / REP * VS); a workgroup has REP query heads of a KV head and 1 / VS of
 // their channels (the scores want whole rows of keys, and each share makes them again).  The cache is cut into strips of eight slots, dealt to eight
 // wavefronts in turn; two wavefronts are a part.  In a wavefront eight lanes share a slot, key and value row alike: 16-byte
 // chunks c = lane % 8 + 8 * n, so a load of the wavefront covers a strip in whole 128-byte lines, and a slot's
-// probability is in the lanes that weigh its value row.  A part has one running maximum (its wavefronts meet once
-// in 256 slots), which its probabilities refer to; the four parts are weighed against each other at the end.
+// probability is in the lanes that weigh its value row.  A wavefront's probabilities refer to its running maximum; up to 256 slots,
+// and behind the last one, it shares it with the other of its part, and the four parts are weighed against each other at the end.
 template <int HD, int REP, int VS, bool FUSED, bool STREAM>
 __global__ __launch_bounds__(512) void decode_attention_kernel(
     const float* __restrict__ q, float* __restrict__ k_cache, float* __restrict__ v_cache,
@@ -86,8 +88,6 @@ __global__ __launch_bounds__(512) void decode_attention_kernel(
             to[n] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(
                 rows, (int)(first + (block * BLOCK + u * PASS) * (HD * 4u) + n * 128u), 0, STREAM ? 2 : 0));
     };
-    auto key_row = [&](uint32_t block, int u, v4f (&to)[KC]) { row_of(k_rows, lane_at, block, u, to); };
-    auto value_row = [&](uint32_t block, int u, v4f (&to)[VC]) { row_of(v_rows, lane_at + share * (OWN * 4u), block, u, to); };
     auto stage = [&] {
         if (STAGED == THREADS || threadIdx.x < STAGED) {
             float y = own;
@@ -110,9 +110,9 @@ __global__ __launch_bounds__(512) void decode_attention_kernel(
 #pragma unroll
         for (int n = 0; n < VC; n++) acc[h][n] = v4f{0.f, 0.f, 0.f, 0.f};
     }
-    // `ends`: this strip may hold the appended slot, and slots behind it
-    auto score = [&](uint32_t block, int u, bool ends, const v4f (&qv)[REP][KC], v4f (&kr)[KC], float (&dot)[REP], float (&top)[REP]) {
-        const uint32_t slot = strip_of(block, u) + group;
+    // `strip`: its first slot.  `ends`: it may hold the appended slot; `masked`: and slots out of sight
+    auto score = [&](uint32_t strip, bool ends, bool masked, const v4f (&qv)[REP][KC], v4f (&kr)[KC], float (&dot)[REP], float (&top)[REP]) {
+        const uint32_t slot = strip + group;
         if (FUSED && ends && slot == position) {
 #pragma unroll
             for (int n = 0; n < KC; n++) kr[n] = *reinterpret_cast<const v4f*>(staged + REP * HD + 4u * lane8 + 32 * n);
@@ -128,12 +128,12 @@ __global__ __launch_bounds__(512) void decode_attention_kernel(
             d += lane_exchange<kDppXor2>(d);
             d += lane_exchange<kDppHalfMirror>(d);
             d = __fmul_rn(d, scale);
-            dot[h] = ends && slot > position ? -INFINITY : d;
+            dot[h] = masked && slot > position ? -INFINITY : d;
             top[h] = fmaxf(top[h], dot[h]);
         }
     };
-    auto weigh = [&](uint32_t block, int u, bool ends, v4f (&vr)[VC], const float (&p)[REP]) {
-        if (FUSED && ends && strip_of(block, u) + group == position) {
+    auto weigh = [&](uint32_t strip, bool ends, v4f (&vr)[VC], const float (&p)[REP]) {
+        if (FUSED && ends && strip + group == position) {
 #pragma unroll
             for (int n = 0; n < VC; n++) vr[n] = *reinterpret_cast<const v4f*>(staged + (REP + 1) * HD + share * OWN + 4u * lane8 + 32 * n);
         }
@@ -191,10 +191,10 @@ __global__ __launch_bounds__(512) void decode_attention_kernel(
             constexpr int P = decltype(passes_tag)::value, N = P > 0 ? P : 1;
             v4f kb[N][KC], vb[N][VC];
 #pragma unroll
-            for (int u = 0; u < P; u++) key_row(0u, u, kb[u]);
+            for (int u = 0; u < P; u++) row_of(k_rows, lane_at, 0u, u, kb[u]);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int u = 0; u < P; u++) value_row(0u, u, vb[u]);
+            for (int u = 0; u < P; u++) row_of(v_rows, lane_at + share * (OWN * 4u), 0u, u, vb[u]);
             __builtin_amdgcn_sched_barrier(0);
             stage();
             float dot[N][REP], top[REP], grown[REP];
@@ -204,12 +204,12 @@ __global__ __launch_bounds__(512) void decode_attention_kernel(
                 v4f qv[REP][KC];
                 queries(qv);
 #pragma unroll
-                for (int u = 0; u < P; u++) score(0u, u, u == P - 1, qv, kb[u], dot[u], top);
+                for (int u = 0; u < P; u++) score(strip_of(0u, u), u == P - 1, u == P - 1, qv, kb[u], dot[u], top);
             }
             meet(0u, top, grown);
             settle(std::true_type{}, grown, dot, passes_tag);
 #pragma unroll
-            for (int u = 0; u < P; u++) weigh(0u, u, u == P - 1, vb[u], dot[u]);
+            for (int u = 0; u < P; u++) weigh(strip_of(0u, u), u == P - 1, vb[u], dot[u]);
         };
         const uint32_t passes = position >= wave * STRIP ? (position - wave * STRIP) / PASS + 1u : 0u;
         switch (passes) {
@@ -220,15 +220,37 @@ __global__ __launch_bounds__(512) void decode_attention_kernel(
             default: whole(std::integral_constant<int, 4>{}); break;
         }
     } else {
-        // More: a block's rows are requested as soon as the registers of the one before are free.
+        // More: a block's rows are requested as soon as the registers of the one before are free, and the wavefronts meet behind
+        // the last one only.  The first block is the one that is not whole: its first `missing` rounds of 64 slots would lie in front
+        // of slot 0, so that only strips of the last round are asked for out of sight.  (With the last block not whole, all of it
+        // asked for, and a meeting a block: 16 heads on 8 of 128 at slot 256 1 row 6.5 -> 5.8 us, 16 rows 13.4 -> 10.6, 32 rows 17.8 -> 15.1;
+        // 32 heads on 4, 8 rows, slot 256 9.6 -> 8.6, 1000 21.8 -> 20.5, 2000 39.3 -> 35.6.  Copies of the last two blocks for
+        // each number of strips, as above, spill.)
+        const uint32_t missing = blocks * PASSES - (position / PASS + 1u), back = missing * PASS;
+        const uint32_t lane_back = lane_at - back * (HD * 4u);
         v4f kb[PASSES][KC], vb[PASSES][VC];
+        auto request_first = [&](auto whole_tag) {
+            constexpr bool WHOLE = decltype(whole_tag)::value;
+            auto requested = [&](int u) { return WHOLE || u + 1 == PASSES || (uint32_t)u >= missing; };  // (scalar)
 #pragma unroll
-        for (int u = 0; u < PASSES; u++) key_row(0u, u, kb[u]);
-        __builtin_amdgcn_sched_barrier(0);
+            for (int u = 0; u < PASSES; u++) {
+                if (requested(u)) row_of(k_rows, lane_back, 0u, u, kb[u]);
+                else for (auto& chunk : kb[u]) chunk = v4f{0.f, 0.f, 0.f, 0.f};
+            }
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int u = 0; u < PASSES; u++) value_row(0u, u, vb[u]);
-        __builtin_amdgcn_sched_barrier(0);
-        stage();
+            for (int u = 0; u < PASSES; u++) {
+                if (requested(u)) row_of(v_rows, lane_back + share * (OWN * 4u), 0u, u, vb[u]);
+                else for (auto& chunk : vb[u]) chunk = v4f{0.f, 0.f, 0.f, 0.f};
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            stage();
+            // Requests under a condition make the number in flight unknown, and the first use would wait for all of them, in either
+            // case: here is that wait, so that the other has none.
+            if constexpr (!WHOLE) __builtin_amdgcn_s_waitcnt(kWaitLoads);
+        };
+        if (missing == 0u) request_first(std::true_type{});
+        else request_first(std::false_type{});
         v4f qv[REP][KC];
         queries(qv);
         uint32_t block = 0u;
@@ -239,22 +261,33 @@ __global__ __launch_bounds__(512) void decode_attention_kernel(
             for (int h = 0; h < REP; h++) top[h] = -INFINITY;
 #pragma unroll
             for (int u = 0; u < PASSES; u++) {
-                score(block, u, ENDS, qv, kb[u], dot[u], top);
+                score(strip_of(block, u) - back, ENDS && u + 1 == PASSES, true, qv, kb[u], dot[u], top);
                 __builtin_amdgcn_sched_barrier(0);
-                if constexpr (!ENDS) key_row(block + 1u, u, kb[u]);
+                if constexpr (!ENDS) row_of(k_rows, lane_back, block + 1u, u, kb[u]);
             }
-            meet(block, top, grown);
+#pragma unroll
+            for (int h = 0; h < REP; h++) grown[h] = fmaxf(m[h], wave_max(top[h]));
             settle(std::false_type{}, grown, dot, std::integral_constant<int, PASSES>{});
 #pragma unroll
             for (int u = 0; u < PASSES; u++) {
-                weigh(block, u, ENDS, vb[u], dot[u]);
+                weigh(strip_of(block, u) - back, ENDS && u + 1 == PASSES, vb[u], dot[u]);
                 __builtin_amdgcn_sched_barrier(0);
-                if constexpr (!ENDS) value_row(block + 1u, u, vb[u]);
+                if constexpr (!ENDS) row_of(v_rows, lane_back + share * (OWN * 4u), block + 1u, u, vb[u]);
             }
         };
 #pragma clang loop unroll(disable)
         for (; block + 1u < blocks; block++) one(std::false_type{});
         one(std::true_type{});
+        float common[REP];
+        meet(block, m, common);
+#pragma unroll
+        for (int h = 0; h < REP; h++) {
+            const float keep = expf(m[h] - reference(common[h]));
+            sum[h] *= keep;
+#pragma unroll
+            for (int n = 0; n < VC; n++) acc[h][n] *= keep;
+            m[h] = common[h];
+        }
     }
     // The groups of a wavefront meet: lanes 32, then 16, then 8 apart.  A step that can exchanges one half of the channels
     // for the other, so a lane is left with one chunk.
