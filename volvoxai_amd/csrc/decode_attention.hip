@@ -25,7 +25,11 @@ namespace {
 
 constexpr int kWaitLoads = 0x0f70;  // s_waitcnt vmcnt(0), the other counters at their largest
 
-// grid (rows * t, kv_heads, query heads of a KV head / REP * VS); a workgroup has REP query heads of a KV head and 1 / VS of
+// What a grid's x, y and z count: tokens are rows * t, those of a row in turn or, where rows come first, the rows' first ones, then their
+// second ones; parts are the workgroups of a KV head, its query heads / REP * VS.
+enum class GridOrder : uint32_t { TokensHeadsParts, HeadsPartsTokens, RowsPartsHeads };
+
+// A workgroup has REP query heads of a KV head and 1 / VS of
 // their channels (the scores want whole rows of keys, and each share makes them again).  The cache is cut into strips of eight slots, dealt to eight
 // wavefronts in turn; two wavefronts are a part.  In a wavefront eight lanes share a slot, key and value row alike: 16-byte
 // chunks c = lane % 8 + 8 * n, so a load of the wavefront covers a strip in whole 128-byte lines, and a slot's
@@ -34,8 +38,8 @@ constexpr int kWaitLoads = 0x0f70;  // s_waitcnt vmcnt(0), the other counters at
 template <int HD, int REP, int VS, bool FUSED, bool STREAM>
 __global__ __launch_bounds__(512) void decode_attention_kernel(
     const float* __restrict__ q, float* __restrict__ k_cache, float* __restrict__ v_cache,
-    const int64_t* __restrict__ positions, uint32_t t, uint32_t rep, uint32_t max_seq, float scale, float* __restrict__ out,
-    const float* __restrict__ cos_table, const float* __restrict__ sin_table, uint32_t* __restrict__ fault) {
+    const int64_t* __restrict__ positions, GridOrder order, uint32_t t, uint32_t kv_heads, uint32_t rep, uint32_t max_seq, float scale,
+    float* __restrict__ out, const float* __restrict__ cos_table, const float* __restrict__ sin_table, uint32_t* __restrict__ fault) {
     constexpr int KC = HD / 32, OWN = HD / VS, VC = KC / VS, PASSES = 4, PARTS = 4, PART_WAVES = 2, WAVES = PARTS * PART_WAVES, THREADS = WAVES * 64;
     constexpr uint32_t STRIP = 8u, PASS = WAVES * STRIP, BLOCK = PASSES * PASS;
     constexpr int STAGED = (REP + (FUSED ? 2 : 0)) * HD;
@@ -44,10 +48,20 @@ __global__ __launch_bounds__(512) void decode_attention_kernel(
     __shared__ __attribute__((aligned(16))) float partial[WAVES][REP][OWN];
     __shared__ __attribute__((aligned(8))) float maxima[2][REP][WAVES];
     __shared__ float sums[WAVES][REP];
+    const uint32_t x = order == GridOrder::HeadsPartsTokens ? blockIdx.z : blockIdx.x;
+    const uint32_t kvh = order == GridOrder::TokensHeadsParts   ? blockIdx.y
+                         : order == GridOrder::HeadsPartsTokens ? blockIdx.x
+                                                                : blockIdx.z;
+    const uint32_t part = order == GridOrder::TokensHeadsParts ? blockIdx.z : blockIdx.y;
     // (no division stands in front of the first load of a decode step: three of them take a tenth of a microsecond)
-    const uint32_t token = blockIdx.x, row = FUSED ? token : token / t, i = FUSED ? 0u : token % t;
-    const uint32_t kvh = blockIdx.y, kv_heads = gridDim.y, q_heads = kv_heads * rep;
-    const uint32_t head0 = kvh * rep + blockIdx.z / VS * REP, share = blockIdx.z % VS;
+    uint32_t row = x, i = 0u;
+    if constexpr (!FUSED) {
+        const uint32_t per = order == GridOrder::RowsPartsHeads ? gridDim.x / t : t;
+        row = order == GridOrder::RowsPartsHeads ? x % per : x / per;
+        i = order == GridOrder::RowsPartsHeads ? x / per : x % per;
+    }
+    const uint32_t token = FUSED ? row : row * t + i, q_heads = kv_heads * rep;
+    const uint32_t head0 = kvh * rep + part / VS * REP, share = part % VS;
     const uint64_t named = (uint64_t)positions[i];
     if (named >= max_seq) {  // (the whole workgroup) outside the caches: touch nothing, say so
         if (threadIdx.x == 0) atomicOr(fault, (uint32_t)kFaultBadPosition);
@@ -94,7 +108,7 @@ __global__ __launch_bounds__(512) void decode_attention_kernel(
             if (FUSED && which <= REP)  // the arithmetic of rope_append_kernel
                 y = __fadd_rn(__fmul_rn(own, c), __fmul_rn(dd < HD / 2u ? -mate : mate, sn));
             staged[threadIdx.x] = y;
-            if (FUSED && which >= REP && blockIdx.z == 0u) (which == REP ? kbase : vbase)[(size_t)position * HD + dd] = y;
+            if (FUSED && which >= REP && part == 0u) (which == REP ? kbase : vbase)[(size_t)position * HD + dd] = y;
         }
         __syncthreads();
     };
@@ -353,6 +367,13 @@ __global__ __launch_bounds__(512) void decode_attention_kernel(
 // Eight query heads a KV head and more than four heads a compute unit: four heads a workgroup read their rows half as
 // often (64 rows of 32 heads of 128 at slot 255: 23.3, here 47; 32 rows 15.7 both, at slot 145 13.6 and 11.2).  At head size 128
 // their registers do not fit this kernel: false, and the caller launches the one that keeps its scores.
+// Workgroups that read the same rows -- the parts of a KV head, the tokens of a row -- share them where they run on one XCD (of
+// consecutive workgroups every eighth) and soon after each other.  With the parts last, a device's worth of workgroups and more
+// apart, each read its rows from HBM again: 24 heads on 8 of 128, 32 rows, slot 255 34.3 us against 20.7, 2000 259 against 125 (the kernel
+// that this one replaced 22.3 and 132); 32 on 8, 32 rows, slot 2000 179 against 98.  Below one and a half workgroups a compute
+// unit they run at once (32 on 8, 17 rows 10.8 against 12.0), and eight heads a KV head gain only past the lengths that the
+// four-heads kernels have (32 on 4, 24 rows 14.3 against 15.6).  Several tokens a row: 16 heads on 8 of 128, 32 rows of 4 at
+// slot 255 47 us against 30.
 // Non-temporal loads where a row's reader is alone: 32 rows 9.3 against 10.4 us; where two workgroups read it, plain ones
 // (17 rows of 16 heads on 2: 6.8 against 7.2).
 bool launch_decode_attention(hipStream_t s, int cu_count, uint32_t tokens, const float* q, float* k_cache, float* v_cache,
@@ -362,9 +383,25 @@ bool launch_decode_attention(hipStream_t s, int cu_count, uint32_t tokens, const
     const uint32_t rep = q_heads / kv_heads;
     const uint64_t cu = cu_count > 0 ? (uint64_t)cu_count : 256u, heads = (uint64_t)tokens * q_heads;
     const bool four = rep >= 8u && rep % 4u == 0u && heads > 4u * cu;
-#define VXHIP_DECODE_AS(HD, REP, VS, FUSED, STREAM)                                                                        \
-    hipLaunchKernelGGL((decode_attention_kernel<HD, REP, VS, FUSED, STREAM>), dim3(tokens, kv_heads, rep / REP * VS), dim3(512), \
-                       0, s, q, k_cache, v_cache, positions, t, rep, max_seq, scale, out, cos_table, sin_table, fault)
+    GridOrder order = GridOrder::TokensHeadsParts;
+    auto grid_of = [&](uint32_t parts) {
+        const bool shared = t > 1u || (parts > 1u && !(rep >= 8u && rep % 4u == 0u) && (uint64_t)tokens * kv_heads * parts * 2u >= cu * 3u);
+        if (shared && kv_heads % 8u == 0u && tokens <= 0xffffu) {
+            order = GridOrder::HeadsPartsTokens;
+            return dim3(kv_heads, parts, tokens);
+        }
+        if (shared && tokens / t % 8u == 0u) {
+            order = GridOrder::RowsPartsHeads;
+            return dim3(tokens, parts, kv_heads);
+        }
+        return dim3(tokens, kv_heads, parts);
+    };
+#define VXHIP_DECODE_AS(HD, REP, VS, FUSED, STREAM)                                                                            \
+    do {                                                                                                                       \
+        const dim3 grid = grid_of(rep / REP * VS);                                                                             \
+        hipLaunchKernelGGL((decode_attention_kernel<HD, REP, VS, FUSED, STREAM>), grid, dim3(512), 0, s, q, k_cache, v_cache,  \
+                           positions, order, t, kv_heads, rep, max_seq, scale, out, cos_table, sin_table, fault);              \
+    } while (0)
 #define VXHIP_DECODE(HD, REP, VS)                                                            \
     do {                                                                                     \
         constexpr bool kAlone = VS == 1 && REP < 4; /* (may be) */                           \
