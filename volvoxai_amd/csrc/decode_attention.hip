@@ -375,7 +375,8 @@ __global__ __launch_bounds__(512) void decode_attention_kernel(
 // four-heads kernels have (32 on 4, 24 rows 14.3 against 15.6).  Several tokens a row: 16 heads on 8 of 128, 32 rows of 4 at
 // slot 255 47 us against 30.
 // Non-temporal loads where a row's reader is alone: 32 rows 9.3 against 10.4 us; where two workgroups read it, plain ones
-// (17 rows of 16 heads on 2: 6.8 against 7.2).
+// (17 rows of 16 heads on 2: 6.8 against 7.2), and where several tokens do (8 heads on 8 of 128, 32 rows of 7 at slot 600 86.5
+// against 79.8; 4 on 4 of 64 27.1 against 21.0; two tokens gain and lose up to a tenth).
 bool launch_decode_attention(hipStream_t s, int cu_count, uint32_t tokens, const float* q, float* k_cache, float* v_cache,
                              const int64_t* positions, uint32_t t, uint32_t q_heads, uint32_t kv_heads, uint32_t head_dim,
                              uint32_t max_seq, float scale, float* out, const float* cos_table, const float* sin_table,
@@ -405,7 +406,7 @@ bool launch_decode_attention(hipStream_t s, int cu_count, uint32_t tokens, const
 #define VXHIP_DECODE(HD, REP, VS)                                                            \
     do {                                                                                     \
         constexpr bool kAlone = VS == 1 && REP < 4; /* (may be) */                           \
-        if (kAlone && rep == REP) {                                                          \
+        if (kAlone && rep == REP && t == 1u) {                                               \
             if (cos_table) VXHIP_DECODE_AS(HD, REP, VS, true, kAlone);                       \
             else VXHIP_DECODE_AS(HD, REP, VS, false, kAlone);                                \
         } else {                                                                             \
