@@ -13,6 +13,8 @@ from test_decode_attention import ctx  # noqa: F401
     (130, 8, 1, 128),                                  # four heads a workgroup, by way of scores in LDS
     (5, 8, 4, 64), (24, 8, 4, 64), (90, 3, 1, 64),     # a head on two, on one
     (65, 8, 4, 64), (130, 8, 1, 64),                   # two and four heads a workgroup
+    (20, 32, 4, 64), (33, 16, 4, 64),                  # four from two heads a compute unit on
+    (20, 32, 4, 128),                                  # by way of scores in LDS, the cache longer than 256 slots
 ])
 def test_decode_attention_splits(ctx, rows, q_heads, kv_heads, head_dim, position):  # noqa: F811
     blocks.test_decode_attention_blocks(ctx, rows, q_heads, kv_heads, head_dim, position)

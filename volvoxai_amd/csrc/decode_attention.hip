@@ -364,9 +364,13 @@ __global__ __launch_bounds__(512) void decode_attention_kernel(
 //   128   1 row  4.6 | 4.2 | 4.1 | 5.5    8 rows  5.8 | 5.2 | 6.2 | 6.4    16 rows  6.9 | 8.6 | 10.3 | 6.9    32 rows  14.0 | 16.5 | 19.4 | 9.5
 //         (steps of 28 layers, ms: 12 rows 1.027 | 1.077 | 1.098 | 1.017, 16 rows 1.046 | 1.094 | 1.147 | 1.019)
 //    64   1 row  3.9 | 3.3 | - | 4.2      8 rows  4.2 | 4.0 | - | 4.8      16 rows  4.5 | 4.2 | - | 5.0         32 rows  4.8 | 5.6 | - | 5.3
-// Eight query heads a KV head and more than four heads a compute unit: four heads a workgroup read their rows half as
-// often (64 rows of 32 heads of 128 at slot 255: 23.3, here 47; 32 rows 15.7 both, at slot 145 13.6 and 11.2).  At head size 128
-// their registers do not fit this kernel: false, and the caller launches the one that keeps its scores.
+// Four heads a workgroup read their rows half as often.  At head size 64, in groups of four heads, from two heads a compute
+// unit on (two heads a workgroup | four: 32 heads on 4, 16 rows, slot 145 4.6 | 5.8 us, 20 rows 6.7 | 6.0, slot 2000 38.7 | 30.5; 32 on 8,
+// 24 rows, slot 145 8.6 | 7.3, 2000 48.5 | 39.3).  At head size 128 their registers do not fit this kernel: false, and the caller launches
+// the one that keeps its scores, in groups of eight heads: more than four heads a compute unit (64 rows of 32 heads on 4 at slot
+// 255 47 | 23.3), and from two and a half on where the cache may hold more than 256 slots (32 on 4, 24 rows, slot 145 10.6 | 13.2, 256
+// 17.2 | 15.3, 2000 79.6 | 65.3; 32 rows, slot 145 11.4 | 13.6, 256 19.0 | 15.8, 2000 89 | 68; 17 rows, slot 256 16.9 | 15.7, 300 17.2 | 18.2,
+// 2000 63.6 | 64.1).
 // Workgroups that read the same rows -- the parts of a KV head, the tokens of a row -- share them where they run on one XCD (of
 // consecutive workgroups every eighth) and soon after each other.  With the parts last, a device's worth of workgroups and more
 // apart, each read its rows from HBM again: 24 heads on 8 of 128, 32 rows, slot 255 34.3 us against 20.7, 2000 259 against 125 (the kernel
@@ -383,7 +387,8 @@ bool launch_decode_attention(hipStream_t s, int cu_count, uint32_t tokens, const
                              uint32_t* fault) {
     const uint32_t rep = q_heads / kv_heads;
     const uint64_t cu = cu_count > 0 ? (uint64_t)cu_count : 256u, heads = (uint64_t)tokens * q_heads;
-    const bool four = rep >= 8u && rep % 4u == 0u && heads > 4u * cu;
+    const bool four = rep % 4u == 0u && (head_dim == 64u ? heads > 2u * cu
+                                                         : rep >= 8u && (heads > 4u * cu || (max_seq > 256u && heads * 2u >= cu * 5u)));
     GridOrder order = GridOrder::TokensHeadsParts;
     auto grid_of = [&](uint32_t parts) {
         const bool shared = t > 1u || (parts > 1u && !(rep >= 8u && rep % 4u == 0u) && (uint64_t)tokens * kv_heads * parts * 2u >= cu * 3u);
