@@ -114,3 +114,28 @@ def test_tiles_of_groups_of_32(ctx, oracle, rows, n, tile):
         assert (y.cpu().numpy().view(np.uint32) == want.view(np.uint32)).all()
     finally:
         pl.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("rows,n,tile", [(1000, 1531, "t64x32k64"), (720, 4500, "t64x64k64"), (1500, 3000, "t64x64k64"), (2048, 5184, "t64x64k64"), (2048, 13888, "t64x64k64")])
+def test_tiles_of_groups_of_32_in_many_rounds(ctx, rows, n, bits, tile):
+    """An odd number of rounds of half tiles saves less and less of the launch, and a half tile costs more than half: three against two are
+    taken, seven against four and more are not.  The same bits as the other tile."""
+    import torch
+    import volvoxai_amd as vx
+    from volvoxai_amd.decoder import pack_w4_words, pack_w8_words
+    rng = np.random.default_rng(n)
+    words = (pack_w8_words if bits == 8 else pack_w4_words)(rng.integers(-7, 8, (n, 64)).astype(np.int8))
+    pl = vx.PackedLinear(words, rng.uniform(0.002, 0.01, (n, 2)).astype(np.float32), np.zeros(n, np.float32), 64, n, 32, weight_bits=bits)
+    x = torch.from_numpy(rng.normal(0, 1, (rows, 64)).astype(np.float32)).cuda()
+    try:
+        st, y = pl.forward_f32(ctx, x)
+        assert st == 0 and ctx.last_variant.endswith(tile), ctx.last_variant
+        vx.force_variant("a8-mfma." + {"t64x32k64": "t64x64k64", "t64x64k64": "t64x32k64"}[tile])
+        st, other = pl.forward_f32(ctx, x)
+        ctx.synchronize()
+        assert st == 0 and not ctx.last_variant.endswith(tile) and torch.equal(y.view(torch.int32), other.view(torch.int32))
+    finally:
+        vx.force_variant(None)
+        pl.close()

@@ -951,9 +951,11 @@ const char* launch_gemm_k64_f32(hipStream_t s, const LinearArgs& a, F32Tile tile
 //                           512 x 4096 -> 4096    52.1 | 51.1 | 54.2 (94.2)   1024 x 3000 -> 5001  82.3 | 88.6 | 94.4 (227)
 // The lines: 1.5 workgroups of a tile per compute unit; 2.5 of 64x32 with four-bit weights in groups of up to 128, whose
 // operands take longest to spread (235 x 2048 -> 5120 16.2 | 15.3 | 14.8, 302 x 9728 -> 3584 51.7 | 50.9 | 47.5).
-// Past them groups of 32, whose fold is most of their time: 64x32 tiles where they end a round of the device earlier (8 bits, 64x64 | 64x32
-// 1000 x 2000 -> 1531 28.9 | 24.6, 640 x 1500 -> 4096 28.8 | 27.6, 720 x 1500 -> 4500 36.5 | 35.0; where they do not,
-// 900 x 1500 -> 4096 38.2 | 39.6).  The other groups: the 128-channel tiles against 64x64, by how many a compute unit gets, in units of one 128x128 tile (an odd
+// Past them groups of 32, whose fold is most of their time: 64x32 tiles where a compute unit's share of them, 0.595 of a 64x64 tile each,
+// is the smaller one: three against two and five against three, and where rows end in a tile's first half up to ten against six (64x64 | 64x32, 8 bits and then 4: 1000 x 2000 ->
+// 1531 28.0 | 24.4 and 29.6 | 25.5, 640 x 1500 -> 4096 27.2 | 27.6 and 28.7 | 28.0; where they are not, 720 x 1500 -> 4500 34.8 | 34.8
+// and 33.7 | 34.3, 1500 x 1000 -> 3000 30.7 | 33.1 and 31.6 | 32.2, 2048 x 1024 -> 5184 56.8 | 67.8 and 55.6 | 63.0, -> 13888 130 | 160 and
+// 129 | 154).  The other groups: the 128-channel tiles against 64x64, by how many a compute unit gets, in units of one 128x128 tile (an odd
 // one of those has no second workgroup to take turns with).  What a 64x64 tile costs of it depends on the fold:
 // where both have the products s_a * s_w or neither, 0.345; one scale per channel in groups of 128, whose products
 // fit the registers beside the narrow tile alone, 0.3; four-bit weights 0.29.  64x64 | 128x128 | 128x256, 8 bits,
@@ -972,7 +974,7 @@ F32Tile pick_f32_tile(const LinearArgs& a, int cu_count) {
     if (tiles(64, 64) < busy)
         return tiles(64, 32) < (four && a.group_size <= 128u ? cu * 5 / 2 + 1u : busy) ? F32Tile::T32x32 : F32Tile::T64x32;
     const auto per_cu = [&](uint64_t t) { return (t + cu - 1) / cu; };
-    if (a.group_size < 64u) return per_cu(tiles(64, 32)) < 2 * per_cu(tiles(64, 64)) ? F32Tile::T64x32 : F32Tile::T64x64;
+    if (a.group_size < 64u) return 0.595f * (float)per_cu(tiles(64, 32)) < (float)per_cu(tiles(64, 64)) ? F32Tile::T64x32 : F32Tile::T64x64;
     const uint64_t c128 = per_cu(tiles(128, 128));
     const bool narrow_products = !four && a.uniform_group_scales && a.group_size == 128u;
     const float narrow = (float)per_cu(tiles(64, 64)) * (four ? 0.29f : narrow_products ? 0.3f : 0.345f);
