@@ -74,6 +74,20 @@ def test_which_calls_take_it(ctx, rows, k, n, bits, group, tile):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows,k,n,bits,group,tile", [
+    (24, 8192, 8192, 8, 128, "slab32x32"), (16, 14336, 8192, 8, 128, "slab16x16"),  # no instance: its LDS does not suffice
+    (6, 3000, 1531, 8, 64, "slab16x16"), (8, 3000, 7000, 8, 64, "slab16x16"),       # none: the last group is half a group
+    (8, 14336, 8192, 8, 128, "slab16x16"), (8, 8192, 8192, 4, 128, "slab16x16"),    # one that reads its rows from memory
+    (8, 4096, 14336, 8, 64, "slab16x16"), (16, 8192, 14336, 8, 128, "slab16x16"),
+    (4, 8192, 14336, 8, 128, None), (8, 4096, 8192, 8, 128, None),                  # one that has them in LDS
+    (10, 6000, 8192, 8, 128, None), (3, 10000, 5055, 8, 128, None), (24, 6000, 5055, 8, 128, None), (8, 13000, 4096, 8, 128, "slab16x16"),
+    (8, 10000, 8192, 4, 256, None), (8, 6000, 8192, 4, 128, "slab16x16"), (24, 10000, 5055, 8, 128, "slab16x32")])  # the general kernel, and not
+def test_calls_that_no_straight_line_instance_holds(ctx, rows, k, n, bits, group, tile):
+    """What the rule takes to stand behind a call is what the streaming kernel's launcher has for it."""
+    test_which_calls_take_it(ctx, rows, k, n, bits, group, tile)
+
+
+@pytest.mark.gpu
 def test_scratch_with_room_for_the_rows_alone(oracle):
     """225 rows of 18000 fit the fixed scratch array (4 MiB) and a scratch reserved for them, eight tiles of 32 rows do not: the call is
     taken as before, and by the slab kernel where its scratch may grow."""

@@ -314,13 +314,17 @@ const char* launch_gemv_row(hipStream_t s, const LinearArgs& a, int cu_count, co
 const char* launch_gemv_few(hipStream_t s, const LinearArgs& a, int cu_count, const char* force);
 // linear_slabs.hip: a DequantF32 linear on prepared rows in operand order, tiles of 32 of them one after the other, for launches of
 // few tiles.  pick_slab_tile says which tile a call should take (channels x rows), or None: nothing but a's extents, group
-// size and weight width is looked at.
+// size, weight width and what the streaming kernel has for them is looked at.
 enum class SlabTile : int { None = 0, T16x16 = 1, T16x32 = 2, T32x32 = 3 };
 SlabTile pick_slab_tile(const LinearArgs& a, int cu_count, const char* force);
 const char* launch_linear_slabs(hipStream_t s, const LinearArgs& a, SlabTile tile);
 // While on (per thread), launch_gemv_stream chooses as always and launches nothing: its result tells
 // whether a call of that description would be taken.
 void set_gemv_dry_run(bool on);
+// What launch_gemv_stream has for a DequantF32 call of a's extents on prepared rows in operand order: nothing, its general kernel, or a
+// straight-line instance, which reads the rows from memory or keeps them in LDS (a workgroup's share then leaves room for a second one).
+enum class Streams : int { None, General, RowsInMemory, RowsInLds };
+Streams streaming_kernel(LinearArgs a, int cu_count);
 
 const char* forced_variant();
 

@@ -39,6 +39,7 @@ namespace {
 // While set on the calling thread the launchers of this file decide as always but launch nothing: what
 // launch_gemv_stream then returns tells whether (and as which variant) a call would run.
 thread_local bool gemv_dry_run = false;
+thread_local Streams gemv_fit = Streams::None;  // the straight-line instance chosen last
 
 extern __shared__ __attribute__((aligned(16))) char gemv_lds[];
 
@@ -626,10 +627,11 @@ const char* launch_fit_mode(hipStream_t s, const LinearArgs& a, int cu_count, co
         if constexpr (STEPS % GK == 0) {
             if (taken || a.ksteps != (uint32_t)(W * B)) return;
             // (an instance named in full, "fit12x8", rules the others out)
-            char id[16];
-            snprintf(id, sizeof id, "fit%dx%d", W, B);
-            if (const char* named = force ? strstr(force, "fit") : nullptr)
+            if (const char* named = force ? strstr(force, "fit") : nullptr) {
+                char id[16];
+                snprintf(id, sizeof id, "fit%dx%d", W, B);
                 if (named[3] >= '0' && named[3] <= '9' && strncmp(named, id, strlen(id)) != 0) return;
+            }
             // the activation rows go through LDS while two workgroups still fit a compute unit that way
             bool xlds = a.rows <= kFitLdsRows;
             size_t lds = lds_for(W, STEPS, xlds);
@@ -647,7 +649,8 @@ const char* launch_fit_mode(hipStream_t s, const LinearArgs& a, int cu_count, co
                 ok = launch_fit<GK, W, B, W4>(s, a, lds, xlds, rprod);
             }
             taken = true;
-            snprintf(name, sizeof name, "fit%dx%d%s", W, B, split == 4u ? "c8" : split == 2u ? "c16" : "");
+            gemv_fit = xlds ? Streams::RowsInLds : Streams::RowsInMemory;
+            if (!gemv_dry_run) snprintf(name, sizeof name, "fit%dx%d%s", W, B, split == 4u ? "c8" : split == 2u ? "c16" : "");
         }
     };
     using std::integral_constant;
@@ -774,6 +777,17 @@ const char* launch_mode(hipStream_t s, const LinearArgs& a, int cu_count, const 
 }  // namespace
 
 void set_gemv_dry_run(bool on) { gemv_dry_run = on; }
+
+Streams streaming_kernel(LinearArgs a, int cu_count) {
+    a.x = nullptr;
+    a.x_f32 = nullptr;
+    a.x_operand_order = 1u;
+    gemv_fit = Streams::None;
+    set_gemv_dry_run(true);
+    const bool taken = launch_gemv_stream(nullptr, a, cu_count, nullptr) != nullptr;
+    set_gemv_dry_run(false);
+    return !taken ? Streams::None : gemv_fit != Streams::None ? gemv_fit : Streams::General;
+}
 
 const char* launch_gemv_stream(hipStream_t s, const LinearArgs& a, int cu_count, const char* force) {
     if (cu_count <= 0) cu_count = 256;

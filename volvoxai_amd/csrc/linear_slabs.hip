@@ -256,13 +256,23 @@ bool launch_bits(hipStream_t s, const LinearArgs& a) {
 //                            64 x 14336 -> 1024 30.1 | 13.1 | 15.9 | 20.9    200 x 14336 -> 1024 32.5 | 29.0 | 24.7 | 23.6
 //   4 bits, groups of 32     32 x 14336 -> 4096 55.9 | 27.4 | 27.1 | 44.4    64 x 2500 -> 1500   13.2 |  8.6 |  8.9 | 12.3
 //   4 bits, groups of 128    16 x 2000 -> 8000   8.1 |  7.2 |  8.3 |  8.3    32 x 4096 -> 14336  21.3 | 21.6 | 19.5 | 17.1
-// Past a cost of 2 the tiles of gemm_k64.hip and the streaming kernel's straight-line instances are as fast or faster (128 x 4096 ->
-// 4096 13.9 | 19.8 | 16.9 | 14.4, 32 x 4096 -> 14336 19.4 | 25.5 | 22.8 | 19.7); the general streaming kernel and the straight-line one
-// in groups of 32 and 64 are slower up to 2.7 (16 x 4096 -> 14336 in groups of 64 28.9 | 20.2 | 21.0 | 18.8).  Groups of 256 have the
-// cheapest fold there (150 x 2500 -> 1500 9.1 | 11.7 | 10.2 | 9.2), short rows the fewest k-blocks (207 x 1440 -> 1056 7.5 us, 32x32 9.3).
-// The straight-line instances keep their calls up to eight rows (6 x 3000 -> 1531 6.2 | 6.5, but 8 x 2500 -> 1500, which has none,
-// 9.3 | 6.8) and on whole panels (16 x 4096 -> 8192 10.5 | 13.1, 16 x 2048 -> 14336 in groups of 64 12.0 | 13.6).
-// 110 drawn calls of 3 to 256 rows, K from 1024: the 68 that come here take 0.76 of their time (geometric mean), the worst 1.02.
+// Past a cost of 2 the tiles of gemm_k64.hip and the streaming kernel's straight-line instances up to K = 4096 are as fast or faster
+// (128 x 4096 -> 4096 13.9 | 19.8 | 16.9 | 14.4, 32 x 4096 -> 14336 19.4 | 25.5 | 22.8 | 19.7); the general streaming kernel, the straight-line
+// one in groups of 32 and 64 and the longer ones are slower up to 2.7 (16 x 4096 -> 14336 in groups of 64 28.9 | 20.2 | 21.0 | 18.8, 16 x 8192 ->
+// 14336 36.3 | 32.8 | 34.2 | 30.0).  Groups of 256 have the cheapest fold there (150 x 2500 -> 1500 9.1 | 11.7 | 10.2 | 9.2), short rows the
+// fewest k-blocks (207 x 1440 -> 1056 7.5 us, 32x32 9.3).
+// What stands behind a call is asked of its launcher (streaming_kernel).  Up to eight rows a straight-line instance that has them
+// in LDS keeps its calls (6 x 3000 -> 1531 6.2 | 6.5, 4 x 8192 -> 14336 25.6 | 28.9); one that reads them from memory does not (8 x 4096 ->
+// 14336 in groups of 64 23.6 | 18.6; 8 x 14336 -> 8192 36.5 | 26.7, with four bits 44.6 | 21.3).  With more rows whole panels up to K = 4096 stay
+// (16 x 4096 -> 8192 10.5 | 13.1, 16 x 2048 -> 14336 in groups of 64 12.0 | 13.6); past it none do, and where the instance's LDS does not
+// suffice there was no streaming kernel either (16 x 14336 -> 8192 41.1 | 30.2 | 31.3 | 26.6, 24 x 8192 -> 8192 25.6 | 25.3 | 21.8 | 18.5).
+// The general kernel keeps weights of more than 26 MB once a compute unit gets a second tile (10 x 6000 -> 8192 14.7 | 17.5, 8 x 10000 ->
+// 5055 17.4 | 19.0, in groups of 256 8 x 3500 -> 8192 10.7 | 11.6, 20 x 4384 -> 6433 12.6 | - | 16.2; before that 8 x 13000 -> 4096 19.6 | 17.2; fewer
+// bytes, in groups of 64 6 x 3000 -> 1531, whose last group is half a group, 9.2 | 7.3, 8 x 2500 -> 8192 9.7 | 8.5, of four bits 8 x 6000 ->
+// 8192 12.4 | 11.9), where each of its workgroups has a compute unit or its products leave room for a second one (10 x 2784 -> 13830
+// 13.7 | 16.1, in groups of 256 8 x 4115 -> 10232 15.3 | 16.5; not 13 x 10240 -> 8704 32.7 | 30.1, in groups of 64 9 x 6176 -> 8376 26.9 | 21.6).
+// 150 drawn calls, most of 3 to 32 rows of long K: all take 0.84 of the time they took before these kernels (geometric mean), the worst 1.03.
+constexpr uint64_t kStreamedWeights = 26000000u;
 SlabTile pick_slab_tile(const LinearArgs& a, int cu_count, const char* force) {
     if (a.weight_bits != 8u && a.weight_bits != 4u) return SlabTile::None;
     if (force) {
@@ -274,13 +284,16 @@ SlabTile pick_slab_tile(const LinearArgs& a, int cu_count, const char* force) {
     const bool four = a.weight_bits == 4u;
     if (a.rows <= kMaxPrepRows || a.rows > 256u) return SlabTile::None;
     const uint32_t panels = (a.n + 31u) / 32u, cu = cu_count > 0 ? (uint32_t)cu_count : 256u, columns = a.ksteps * (four ? 64u : 32u);
-    // a straight-line instance of gemv_stream.hip (launch_fit_mode) stands behind the call
-    const bool shared = !four && columns <= 4096u, enough = panels * 4u >= cu * 3u;
-    const bool fits = a.rows <= (four ? 8u : 32u) && (shared || enough) &&
-                      (columns == 1024u || columns == 2048u || columns == 3072u || columns == 4096u || columns == 8192u || columns == 14336u);
-    if (a.k < (a.rows <= 4u ? 4097u : a.rows <= 8u ? 2049u : fits ? 2048u : 1280u)) return SlabTile::None;
-    // (whole panels: its products of all groups leave a compute unit room for two workgroups, or are at least few)
-    if (fits && (a.rows <= 8u || (enough && (a.group_size >= 128u || a.groups * a.rows * 128u <= 80u * 1024u)))) return SlabTile::None;
+    if (a.k < (a.rows <= 4u ? 4097u : a.rows <= 8u ? 2049u : 1280u)) return SlabTile::None;
+    const Streams behind = a.rows <= 32u ? streaming_kernel(a, cu_count) : Streams::None;
+    if (a.rows <= 8u && behind == Streams::RowsInLds) return SlabTile::None;
+    if (behind == Streams::General && panels * 2u > cu && (panels <= cu || a.groups * (a.rows + 1u) * 128u <= 80u * 1024u) &&
+        (uint64_t)a.n * a.k * a.weight_bits > kStreamedWeights * 8u)
+        return SlabTile::None;
+    const bool fits = a.rows > 8u && (behind == Streams::RowsInMemory || behind == Streams::RowsInLds) && columns <= 4096u;
+    if (fits && a.k < 2048u) return SlabTile::None;
+    // (whole panels: the products of all groups leave a compute unit room for two workgroups, or are at least few)
+    if (fits && panels * 4u >= cu * 3u && (a.group_size >= 128u || a.groups * a.rows * 128u <= 80u * 1024u)) return SlabTile::None;
     const auto cost = [&](uint32_t tile_n, uint32_t tile_m, float one) {
         const float per = (float)((uint64_t)((a.n + tile_n - 1u) / tile_n) * ((a.rows + tile_m - 1u) / tile_m)) / (float)cu;
         return one * (per > 1.0f ? 1.0f + 0.6f * (per - 1.0f) : 1.0f);
@@ -288,10 +301,11 @@ SlabTile pick_slab_tile(const LinearArgs& a, int cu_count, const char* force) {
     const bool fine = a.group_size == 32u;
     const float c0 = cost(16u, 16u, 1.0f), c1 = cost(16u, 32u, fine ? 1.25f : 1.38f), c2 = cost(32u, 32u, fine ? 2.2f : 1.95f);
     const float least = c0 <= c1 && c0 <= c2 ? c0 : c1 <= c2 ? c1 : c2;
-    const float line = a.rows > 8u && a.rows <= 32u && !(fits && a.group_size >= 128u) ? 2.7f
-                       : a.rows > 32u && a.k < 2048u                                   ? 1.6f
-                       : a.group_size == 256u && a.k < 4096u                           ? 1.9f
-                                                                                       : 2.0f;
+    const bool slow_stream = a.rows <= 8u ? behind == Streams::RowsInMemory : a.rows <= 32u && !(fits && a.group_size >= 128u);
+    const float line = slow_stream                          ? 2.7f
+                       : a.rows > 32u && a.k < 2048u        ? 1.6f
+                       : a.group_size == 256u && a.k < 4096u ? 1.9f
+                                                            : 2.0f;
     if (least > line) return SlabTile::None;
     return least == c0 ? SlabTile::T16x16 : least == c1 ? SlabTile::T16x32 : SlabTile::T32x32;
 }
