@@ -81,9 +81,11 @@ def test_which_calls_take_it(ctx, rows, k, n, bits, group, tile):
     (8, 4096, 14336, 8, 64, "slab16x16"), (16, 8192, 14336, 8, 128, "slab16x16"),
     (4, 8192, 14336, 8, 128, None), (8, 4096, 8192, 8, 128, None),                  # one that has them in LDS
     (10, 6000, 8192, 8, 128, None), (3, 10000, 5055, 8, 128, None), (24, 6000, 5055, 8, 128, None), (8, 13000, 4096, 8, 128, "slab16x16"),
-    (8, 10000, 8192, 4, 256, None), (8, 6000, 8192, 4, 128, "slab16x16"), (24, 10000, 5055, 8, 128, "slab16x32")])  # the general kernel, and not
-def test_calls_that_no_straight_line_instance_holds(ctx, rows, k, n, bits, group, tile):
-    """What the rule takes to stand behind a call is what the streaming kernel's launcher has for it."""
+    (8, 10000, 8192, 4, 256, None), (8, 6000, 8192, 4, 128, "slab16x16"), (24, 10000, 5055, 8, 128, "slab16x32"),   # the general kernel, and not
+    (239, 2304, 736, 8, 256, None), (112, 2304, 736, 8, 256, "slab16x16"), (118, 1536, 1280, 8, 128, None), (118, 1536, 1024, 8, 128, "slab16x32")])  # cheap folds
+def test_what_stands_behind_a_call(ctx, rows, k, n, bits, group, tile):
+    """What the rule takes to stand behind a call is what the streaming kernel's launcher has for it; short walks and cheap folds are left to
+    the tiles of gemm_k64.hip."""
     test_which_calls_take_it(ctx, rows, k, n, bits, group, tile)
 
 

@@ -259,8 +259,8 @@ bool launch_bits(hipStream_t s, const LinearArgs& a) {
 // Past a cost of 2 the tiles of gemm_k64.hip and the streaming kernel's straight-line instances up to K = 4096 are as fast or faster
 // (128 x 4096 -> 4096 13.9 | 19.8 | 16.9 | 14.4, 32 x 4096 -> 14336 19.4 | 25.5 | 22.8 | 19.7); the general streaming kernel, the straight-line
 // one in groups of 32 and 64 and the longer ones are slower up to 2.7 (16 x 4096 -> 14336 in groups of 64 28.9 | 20.2 | 21.0 | 18.8, 16 x 8192 ->
-// 14336 36.3 | 32.8 | 34.2 | 30.0).  Groups of 256 have the cheapest fold there (150 x 2500 -> 1500 9.1 | 11.7 | 10.2 | 9.2), short rows the
-// fewest k-blocks (207 x 1440 -> 1056 7.5 us, 32x32 9.3).
+// 14336 36.3 | 32.8 | 34.2 | 30.0).  Groups of 256 have the cheapest fold there (150 x 2500 -> 1500 9.1 | 11.7 | 10.2 | 9.2, 239 x 2304 -> 736, a cost
+// of 1.74, 8.4 | - | 9.6), short rows the fewest k-blocks (207 x 1440 -> 1056 7.5 us, 32x32 9.3; 118 x 1536 -> 1280, 1.59, 7.3 | - | 7.7).
 // What stands behind a call is asked of its launcher (streaming_kernel).  Up to eight rows a straight-line instance that has them
 // in LDS keeps its calls (6 x 3000 -> 1531 6.2 | 6.5, 4 x 8192 -> 14336 25.6 | 28.9); one that reads them from memory does not (8 x 4096 ->
 // 14336 in groups of 64 23.6 | 18.6; 8 x 14336 -> 8192 36.5 | 26.7, with four bits 44.6 | 21.3).  With more rows whole panels up to K = 4096 stay
@@ -303,8 +303,8 @@ SlabTile pick_slab_tile(const LinearArgs& a, int cu_count, const char* force) {
     const float least = c0 <= c1 && c0 <= c2 ? c0 : c1 <= c2 ? c1 : c2;
     const bool slow_stream = a.rows <= 8u ? behind == Streams::RowsInMemory : a.rows <= 32u && !(fits && a.group_size >= 128u);
     const float line = slow_stream                          ? 2.7f
-                       : a.rows > 32u && a.k < 2048u        ? 1.6f
-                       : a.group_size == 256u && a.k < 4096u ? 1.9f
+                       : a.rows > 32u && a.k < 2048u        ? 1.5f
+                       : a.group_size == 256u && a.k < 4096u ? 1.6f
                                                             : 2.0f;
     if (least > line) return SlabTile::None;
     return least == c0 ? SlabTile::T16x16 : least == c1 ? SlabTile::T16x32 : SlabTile::T32x32;
