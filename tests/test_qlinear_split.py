@@ -95,3 +95,10 @@ def test_which_calls_take_it(ctx, rows, k, n, taken):
     finally:
         vx.force_variant(None)
         lin.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,k,n,taken", [(70, 256, 512, False), (70, 257, 512, True), (67, 200, 256, False), (52, 256, 3840, True)])
+def test_two_k_blocks(ctx, rows, k, n, taken):
+    """Few tiles of up to two k-blocks stay with the tiles of 64 x 64."""
+    test_which_calls_take_it(ctx, rows, k, n, taken)

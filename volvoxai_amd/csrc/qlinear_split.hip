@@ -142,6 +142,9 @@ bool launch(hipStream_t s, const LinearArgs& a) {
 //   256   1536 -> 1536  1.5   5.94 -> 5.72             256   3001 -> 1531  1.5  13.87 -> 12.05 (with its staging launch)
 //   128   4096 -> 4096  2    11.29 -> 9.42 taken       256   2048 -> 2048  2     6.88 -> 7.19 not taken
 //   512   4096 -> 2048  4    11.46 -> 16.68 not taken
+// Two k-blocks are walked as fast by the tiles of 64 x 64, up to half a tile a compute unit by 0.3 us (70 x 256 -> 512 3.44 -> 3.72, 67 x 256 ->
+// 256 with per-row scales 4.03 -> 4.33; not 52 x 256 -> 3840 6.5 -> 5.8, nor unsigned bytes, which those tiles want flipped first: 124 x 256 ->
+// 512 5.8 -> 3.7).
 // From 17 rows on also in place of the streaming kernel: 32 x 2048 -> 2048 6.2 -> 4.6, 32 x 4096 -> 512 7.7 -> 5.4 (16 rows 6.2); 32 x
 // 1024 -> 1024 3.9 -> 4.2 and 24 x 1536 -> 1536 4.5 are left there.  105 calls of 17 to 500 rows, bytes, per-row scales and f32 rows: 0.79 of their
 // time before (geometric mean of graph replays).
@@ -153,6 +156,7 @@ const char* launch_requant_split(hipStream_t s, const LinearArgs& a, int cu_coun
         if (!strstr(force, "t32x32split")) return nullptr;
     } else {
         const uint64_t tiles = (uint64_t)((a.n + 31u) / 32u) * ((a.rows + 31u) / 32u), cu = cu_count > 0 ? (uint64_t)cu_count : 256u;
+        if (a.k <= 256u && tiles * 2u <= cu && !a.x_flip_mask) return nullptr;
         if (tiles > (a.k >= 2560u ? cu * 2u : a.k >= 1536u ? cu * 3u / 2u : cu)) return nullptr;
         if (a.rows <= kMaxGemvRows && (a.rows <= 16u || a.k < 2048u || tiles > cu)) return nullptr;
     }
