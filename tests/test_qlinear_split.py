@@ -102,3 +102,31 @@ def test_which_calls_take_it(ctx, rows, k, n, taken):
 def test_two_k_blocks(ctx, rows, k, n, taken):
     """Few tiles of up to two k-blocks stay with the tiles of 64 x 64."""
     test_which_calls_take_it(ctx, rows, k, n, taken)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("unsigned", [False, True])
+@pytest.mark.parametrize("zero_points", [False, True])
+@pytest.mark.parametrize("rows,k,n,taken", [(17, 4096, 512, True), (32, 2048, 2048, True), (24, 2056, 100, True), (16, 4096, 512, False),
+                                            (17, 2032, 512, False), (33, 512, 64, True)])
+def test_both_activation_types_take_it(ctx, oracle, rows, k, n, taken, zero_points, unsigned):
+    """Signed and unsigned bytes of the same extents run on the same kernels, where the rows are read in place and where they are staged:
+    the oracle's bytes."""
+    import torch
+    import volvoxai_amd as vx
+    rng = np.random.default_rng(rows + k)
+    w, zps = rng.integers(-127, 128, (n, k)).astype(np.int8), rng.integers(-9, 10, n).astype(np.int32) * int(zero_points)
+    scales, bias = rng.uniform(0.005, 0.02, n).astype(np.float32), rng.integers(-2000, 2001, n).astype(np.int32)
+    lo, kind, dtype, zp_in = (0, np.uint8, vx.DTYPE_U8, 121) if unsigned else (-128, np.int8, vx.DTYPE_I8, -3)
+    x = rng.integers(lo, lo + 256, (rows, k)).astype(kind)
+    s_out = float(0.02 * 0.0125 * 74 * 74 * np.sqrt(k) / 40)
+    ok, want = oracle.qlinear(x, w, bias, scales, zps, 0.02, zp_in, s_out, 5, dtype, vx.DTYPE_I8, vx.DTYPE_I8)
+    assert ok == 1
+    lin = vx.QLinear(w, scales, zps, bias, vx.DTYPE_I8)
+    try:
+        ok, y = lin.forward(ctx, torch.from_numpy(x).cuda(), 0.02, zp_in, s_out, 5, input_dtype=dtype)
+        ctx.synchronize()
+        assert ok == 1 and ("t32x32split" in ctx.last_variant) == taken, ctx.last_variant
+        assert (y.cpu().numpy() == want).all()
+    finally:
+        lin.close()

@@ -325,6 +325,14 @@ static bool same_device(const VxHipContext* ctx, int handle_device, const char* 
     return false;
 }
 
+// Rows that the streaming kernel takes, but not as fast (see launch_requant_split): the variant that ran, or null.
+static const char* run_split_rows(VxHipContext* ctx, const LinearArgs& a, const char* force) {
+    if (force || a.rows <= kMaxGemvRows / 2u || a.rows > kMaxGemvRows || a.mode == Epilogue::DequantF32 ||
+        !launch_requant_split(ctx->stream, a, ctx->cu_count, nullptr))
+        return nullptr;
+    return a.mode == Epilogue::RequantRow ? "hip.qlinear.mfma-i8-rowscale.t32x32split" : "hip.qlinear.mfma-i8.t32x32split";
+}
+
 // Picks the kernel family for the shape and launches it.
 static const char* run_linear(VxHipContext* ctx, const LinearArgs& a) {
     const char* force = forced_variant();
@@ -334,10 +342,7 @@ static const char* run_linear(VxHipContext* ctx, const LinearArgs& a) {
     const char* id = nullptr;
     if (force_gemv) return launch_gemv_stream(ctx->stream, a, ctx->cu_count, force);
     if (force_gemm || force_gemm_f) return launch_gemm_mfma(ctx->stream, a, ctx->cu_count, force);
-    // (rows that the streaming kernel takes, but not as fast: see launch_requant_split)
-    if (!force && a.rows > kMaxGemvRows / 2u && a.rows <= kMaxGemvRows && a.mode != Epilogue::DequantF32 &&
-        launch_requant_split(ctx->stream, a, ctx->cu_count, nullptr))
-        return a.mode == Epilogue::RequantRow ? "hip.qlinear.mfma-i8-rowscale.t32x32split" : "hip.qlinear.mfma-i8.t32x32split";
+    if (const char* split = run_split_rows(ctx, a, force)) return split;
     if (a.rows <= kMaxGemvRows) id = launch_gemv_stream(ctx->stream, a, ctx->cu_count, force);
     if (!id) id = launch_gemm_mfma(ctx->stream, a, ctx->cu_count, force);
     return id;
@@ -849,14 +854,15 @@ static int qlinear_run(VxHipContext* ctx, const VxHipQLinear* lin, const void* i
         id = launch_gemv_stream(ctx->stream, a, ctx->cu_count, force);
         a.x_f32 = nullptr;
     }
-    // Unsigned bytes in whole aligned 16-byte chunks, few rows, no row sums wanted: the streaming kernel
-    // flips the top bits itself and the staging launch is saved.
+    // Unsigned bytes in whole aligned 16-byte chunks, few rows, no row sums wanted: the streaming and the split kernel
+    // flip the top bits themselves and the staging launch is saved.
     if (!id && !input_f32_dev && flip && rows <= kMaxGemvRows && (k % 16u) == 0u && ((uintptr_t)input_dev % 16u) == 0u &&
         !lin->any_zero_point && !(force && !strstr(force, "gemv"))) {
         a.x = (const int8_t*)input_dev;
         a.ldx = k;
         a.x_flip_mask = 0x80808080u;
-        id = launch_gemv_stream(ctx->stream, a, ctx->cu_count, force);
+        id = run_split_rows(ctx, a, force);
+        if (!id) id = launch_gemv_stream(ctx->stream, a, ctx->cu_count, force);
         a.x_flip_mask = 0u;
     }
     // ... and so do the large-tile GEMM kernels (gemm_k64.hip, FLIP) for more rows
