@@ -122,7 +122,8 @@ VxHipStatus vxhip_context_clear_fault_flags(VxHipContext* context);
  * `bytes` now instead of inside a later call.  Entry points size the scratch by
  * themselves; a block that is outgrown is kept until vxhip_context_destroy, so a
  * HIP graph captured on this context stays valid when a later, larger call
- * grows it.  Reserving up front only avoids holding the outgrown blocks.  No
+ * grows it.  Reserving up front only avoids holding the outgrown blocks; a call
+ * that can run in what is reserved does not grow it for a faster kernel.  No
  * counterpart in the reference. */
 VxHipStatus vxhip_context_reserve_scratch(VxHipContext* context, size_t bytes);
 /* Layout of prepared activations (int8 codes) handed between entry points on

@@ -116,6 +116,60 @@ def test_scratch_with_room_for_the_rows_alone(oracle):
 
 
 @pytest.mark.gpu
+def test_scratch_grows_for_the_tiles_outside_a_recording(oracle):
+    """A context whose scratch, sized by a smaller call, holds 70 rows of 14336 and not three tiles of 32 of them: it grows, unless the
+    launches are being recorded, by the context or by the owner of its stream, which is refused nothing it was given before."""
+    import torch
+    import volvoxai_amd as vx
+    rows, k, n, group = 70, 14336, 40, 128
+    c = cases.packed_case(rows, k, n, group, 5, True)
+    words, pl = _linear(oracle, k, n, group, 8, c)
+    _, want = oracle.packed_linear(c["x"], words, c["scales"], c["bias"], n, group)
+    x, out = torch.from_numpy(c["x"]).cuda(), torch.empty((rows, n), device="cuda")
+
+    def context(stream):
+        made = vx.Context(0, stream)
+        st, _ = pl.forward_f32(made, x[:40].contiguous(), out=torch.empty((40, n), device="cuda"))
+        made.synchronize()
+        assert st == 0
+        return made
+
+    def same():
+        torch.cuda.synchronize()
+        equal = (out.cpu().numpy().view(np.uint32) == want.view(np.uint32)).all()
+        out.fill_(7.0)
+        torch.cuda.synchronize()
+        return equal
+
+    stream = torch.cuda.Stream()
+    recording, capturing, growing = context(None), context(stream), context(None)
+    try:
+        recording.begin_recording()
+        st, _ = pl.forward_f32(recording, x, out=out)
+        replay = recording.end_recording()
+        assert st == 0 and "slab" not in recording.last_variant, recording.last_variant
+        for _ in range(2):
+            replay.launch(recording)
+            assert same()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            st, _ = pl.forward_f32(capturing, x, out=out)
+        assert st == 0 and "slab" not in capturing.last_variant, capturing.last_variant
+        for _ in range(2):
+            graph.replay()
+            assert same()
+        for made in (growing, recording, capturing):
+            st, _ = pl.forward_f32(made, x, out=out)
+            made.synchronize()
+            assert st == 0 and "slab" in made.last_variant and same(), made.last_variant
+        replay.launch(recording)  # (its block is kept)
+        assert same()
+        replay.close()
+    finally:
+        pl.close(), recording.close(), capturing.close(), growing.close()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows,n,tile", [(1000, 1531, "t64x32k64"), (640, 4096, "t64x32k64"), (900, 4096, "t64x64k64"), (768, 4096, "t64x64k64")])
 def test_tiles_of_groups_of_32(ctx, oracle, rows, n, tile):
     """More 64x64 tiles than 1.5 a compute unit (256 of them): the half tiles where they need an odd number of rounds of the device."""

@@ -553,7 +553,9 @@ VxHipStatus vxhip_context_clear_fault_flags(VxHipContext* ctx) {
 VxHipStatus vxhip_context_reserve_scratch(VxHipContext* ctx, size_t bytes) {
     if (!ctx) return VXHIP_INVALID_ARGUMENT;
     if (!use_device(ctx->device)) return VXHIP_BACKEND_UNAVAILABLE;
-    return ensure_scratch(ctx, bytes);
+    const VxHipStatus status = ensure_scratch(ctx, bytes);
+    if (status == VXHIP_OK) ctx->scratch_reserved = ctx->scratch_bytes;
+    return status;
 }
 
 VxHipStatus vxhip_context_set_activation_layout(VxHipContext* ctx, uint32_t layout) {
@@ -1323,20 +1325,32 @@ static bool run_rows_at_once(VxHipContext* ctx, const VxHipPackedLinear* pl, con
     return id != nullptr;
 }
 
+// Whether a call that could do with the scratch as it is may have it grown: not while launches are being recorded, by this context or
+// by the stream's owner, and not past what the caller has reserved.
+static bool may_grow_scratch(const VxHipContext* ctx) {
+    if (ctx->recording || ctx->scratch_bytes <= ctx->scratch_reserved) return false;
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &status) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return status == hipStreamCaptureStatusNone;
+}
+
 // The same for calls that linear_slabs.hip takes: the rows are prepared into tiles of 32.  Where those would outgrow a scratch that has
-// room for the rows themselves (`fixed`: the scratch array, which cannot grow), the caller goes the way that needs no more.
+// room for what the other kernels want, and cannot grow (`fixed`: the scratch array never can), the caller goes their way.
 static int packed_run_slabs(VxHipContext* ctx, const VxHipPackedLinear* pl, const float* x, float* y, uint32_t rows, bool fixed) {
     const SlabTile tile = pick_slab_tile(f32_row_args(ctx, pl, x, y, rows), ctx->cu_count, forced_variant());
     if (tile == SlabTile::None) return -2;
     const uint32_t k = pl->w.k, ld = (k + 15u) / 16u * 16u;
     const size_t tiled_rows = ((size_t)rows + kOperandOrderRows - 1u) / kOperandOrderRows * kOperandOrderRows;
-    Carver sizes{nullptr}, without{nullptr};
+    Carver sizes{nullptr}, others{nullptr};
     sizes.take<float>(rows);
     sizes.take<int8_t>(tiled_rows * ld);
-    without.take<float>(rows);
-    without.take<int8_t>((size_t)rows * ld);
+    others.take<float>(rows);
+    others.take<int8_t>((rows <= kOperandOrderRows ? tiled_rows : rows) * ld);
     if (fixed ? sizes.off > kNoAllocScratchBytes
-              : sizes.off + 256u > ctx->scratch_bytes && without.off + 256u <= ctx->scratch_bytes)
+              : sizes.off + 256u > ctx->scratch_bytes && others.off + 256u <= ctx->scratch_bytes && !may_grow_scratch(ctx))
         return -2;
     if (!fixed && ensure_scratch(ctx, sizes.off + 256u) != VXHIP_OK) return -1;
     Carver c{(char*)(fixed ? ctx->no_alloc_scratch : ctx->scratch)};

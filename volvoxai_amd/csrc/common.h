@@ -73,6 +73,7 @@ struct VxHipContext {
     // context has the block's address baked into its kernel nodes and may be replayed later.
     void* scratch = nullptr;
     size_t scratch_bytes = 0;
+    size_t scratch_reserved = 0;  // its size when the caller last asked for one (vxhip_context_reserve_scratch)
     static constexpr int kRetiredSlots = 48;  // sizes at least double, so this is never reached
     void* retired[kRetiredSlots] = {};
     int retired_count = 0;
