@@ -566,7 +566,8 @@ int vxhip_packed_linear_add_a8(VxHipContext* context,
  * workspace_dev: vxhip_decoder_prompt_workspace bytes on a 256-byte boundary,
  * the caller's, in use until the launches have run.  That function returns 0,
  * and the call VXHIP_INVALID_ARGUMENT with nothing launched, where an argument
- * is NULL or extents do not fit each other. */
+ * is NULL, extents do not fit each other or one of the entry points would
+ * refuse them, or a linear is another device's. */
 typedef struct VxHipDecoderLayer {
     const float* gain1_dev;
     const float* gain2_dev;

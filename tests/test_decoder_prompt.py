@@ -92,6 +92,48 @@ def test_refusals():
     dec.close()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("t,changes", [(5, dict(max_seq=16384)), (4, dict(head_dim=128, max_seq=16384)), (9, dict(head_dim=6)), (9, dict(hidden=15364)),
+                                       (9, dict(inter=15364)), (9, dict(head_dim=128, q_heads=8, kv_heads=4, max_seq=20000))])
+def test_what_a_step_would_refuse_is_refused_before_the_first(t, changes):
+    """Caches past the per-token attention's scores and past the prompt's, head sizes and rows that no step takes: an error, and the caches
+    are as they were."""
+    import torch
+    from volvoxai_amd.decoder import DecoderConfig
+    cfg = DecoderConfig(**{**dict(layers=2, hidden=64, q_heads=4, kv_heads=2, head_dim=64, inter=96, vocab=50, max_seq=16), **changes})
+    dec = _decoder(1, cfg, 3)
+    try:
+        dec.k_cache.fill_(3.0), dec.v_cache.fill_(3.0)
+        torch.cuda.synchronize()
+        with pytest.raises(RuntimeError, match="vxhip_decoder_prompt"):
+            dec.prefill(torch.zeros((1, t), dtype=torch.int64, device="cuda"))
+        torch.cuda.synchronize()
+        assert bool((dec.k_cache == 3.0).all()) and bool((dec.v_cache == 3.0).all())
+    finally:
+        dec.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layers,t,max_seq", [(2, 9, 16384), (1, 5, 14000), (2, 5, 14000)])
+def test_long_caches_that_are_taken(layers, t, max_seq):
+    """The longest caches of a prompt of eight tokens and more, and of fewer, go on being taken."""
+    import torch
+    from volvoxai_amd.decoder import DecoderConfig
+    cfg = DecoderConfig(layers=layers, hidden=64, q_heads=4, kv_heads=2, head_dim=64, inter=96, vocab=50, max_seq=max_seq)
+    dec = _decoder(1, cfg, 3)
+    try:
+        ids = torch.randint(0, 50, (1, t), generator=torch.Generator().manual_seed(t)).cuda()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(dec.stream):
+            logits, _, _, _ = _one_by_one(dec, ids.to(torch.int32))
+        torch.cuda.synchronize()
+        dec.prefill(ids)
+        torch.cuda.synchronize()
+        assert torch.equal(dec.last_logits.view(torch.int32), logits.view(torch.int32))
+    finally:
+        dec.close()
+
+
 def test_null_arguments_without_a_device():
     from volvoxai_amd._lib import library
     from volvoxai_amd.w8a8 import _DecoderPrompt

@@ -169,6 +169,7 @@ constexpr uint32_t kOperandOrderRows = 32;
 // (not Plain, may be null) receives the f32 rows the codes are made of.
 enum class RowOp : int { Plain = 0, Norm = 1, Swiglu = 2 };
 constexpr uint32_t kMaxRowOpLength = 15360;  // Norm and Swiglu hold the whole row in registers
+constexpr uint32_t kMaxRopeHead = 1024;      // of the rotary embedding's heads
 VxHipStatus launch_row_prepare(hipStream_t s, RowOp op, float* x, const float* delta, const float* gain, double eps,
                                uint32_t rows, uint32_t d, int8_t* codes, ActivationLayout layout, float* scales,
                                float* values);
@@ -281,6 +282,10 @@ struct LinearTail {
 // The variant id, or null where the call is not taken (few rows, weights or extents that these tiles do not have):
 // nothing ran then.
 const char* launch_gemm_followed(hipStream_t s, const LinearArgs& a, After after, const LinearTail& tail, int cu_count);
+
+// decoder_glue.hip: whether vxhip_gqa_attention has a kernel for these extents (none of them zero, whole KV groups)
+bool gqa_takes(const VxHipContext* ctx, uint32_t rows, uint32_t t, uint32_t q_heads, uint32_t kv_heads, uint32_t head_dim,
+               uint32_t max_seq);
 
 // decode_attention.hip: tokens = rows * t queries over the caches.  cos_table given: rotary embedding and cache append ride
 // in front (t = 1).  False where it has no kernel for the call: nothing ran.

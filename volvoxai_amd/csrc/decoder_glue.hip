@@ -1023,6 +1023,46 @@ ActivationLayout prepared_layout(const VxHipContext* ctx, uint32_t rows, uint32_
     return ActivationLayout{d, 0u};
 }
 
+// Which kernel an attention over the caches runs on, and what it needs.
+enum class GqaRoute { None, PromptMfma, PromptScores, Token };
+struct GqaPlan {
+    GqaRoute route;
+    uint32_t tokens;    // of a workgroup's walk (prompt kernels)
+    uint32_t together;  // query heads a workgroup (per-token kernel)
+    size_t lds;         // (dynamic) of the kernels that keep their scores
+};
+
+GqaPlan plan_gqa(const VxHipContext* ctx, uint32_t rows, uint32_t t, uint32_t q_heads, uint32_t kv_heads, uint32_t head_dim,
+                 uint32_t max_seq) {
+    const uint32_t rep = q_heads / kv_heads;
+    const uint32_t together = heads_per_workgroup(rep, rows * t * q_heads, ctx->cu_count);
+    const size_t token_lds = (size_t)together * (9u * head_dim + max_seq) * sizeof(float);  // of the per-token kernel
+    auto prompt_lds = [&](uint32_t tokens) {  // of the prompt kernel that keeps its scores
+        const size_t qw = (size_t)tokens * rep;
+        return (qw * ((max_seq + 63u) & ~63u) + (size_t)kPrefillSlots * (head_dim + 4u)) * sizeof(float);
+    };
+    constexpr size_t kTokenLds = 60u * 1024u, kPromptLds = 150u * 1024u;
+    // A prompt at the common head sizes: the matrix-pipe kernel.  (It holds no scores and would take any cache; those
+    // that neither the prompt kernel with scores nor the per-token kernel could hold are refused as before it.)
+    if (t >= 8u && rep <= kPrefillQueries && (head_dim == 128u || head_dim == 64u) &&
+        (prompt_lds(1u) <= kPromptLds || token_lds <= kTokenLds))
+        return {GqaRoute::PromptMfma, kPrefillQueries / rep, together, 0u};
+    if (t >= 8u && rep <= kPrefillQueries && head_dim <= 256u) {
+        // a prompt: tokens share the walk over the cache, as many per workgroup as the LDS holds
+        uint32_t tq = kPrefillQueries / rep;
+        while (tq > 1u && prompt_lds(tq) > kPromptLds) tq /= 2u;
+        // two workgroups per compute unit hide each other's staging, if four tokens or more still
+        // share a walk then
+        if (prompt_lds(tq) > 78u * 1024u) {
+            uint32_t fewer = tq;
+            while (fewer > 4u && prompt_lds(fewer) > 78u * 1024u) fewer /= 2u;
+            if (prompt_lds(fewer) <= 78u * 1024u) tq = fewer;
+        }
+        if (prompt_lds(tq) <= kPromptLds) return {GqaRoute::PromptScores, tq, together, prompt_lds(tq)};
+    }
+    return {token_lds > kTokenLds ? GqaRoute::None : GqaRoute::Token, 0u, together, token_lds};
+}
+
 // The query heads per workgroup (4, 2 or 1) and the head size pick the instance.
 template <bool FUSED>
 void launch_attention(VxHipContext* ctx, uint32_t together, dim3 grid, size_t lds, const float* q, float* k_cache,
@@ -1139,6 +1179,12 @@ __global__ __launch_bounds__(1024) void argmax_rows_kernel(const float* __restri
 }
 
 }  // namespace
+
+bool gqa_takes(const VxHipContext* ctx, uint32_t rows, uint32_t t, uint32_t q_heads, uint32_t kv_heads, uint32_t head_dim,
+               uint32_t max_seq) {
+    return head_dim % 4u == 0u && plan_gqa(ctx, rows, t, q_heads, kv_heads, head_dim, max_seq).route != GqaRoute::None;
+}
+
 }  // namespace vxhip
 
 using namespace vxhip;
@@ -1189,7 +1235,7 @@ VxHipStatus vxhip_rope_append_kv(VxHipContext* ctx, const float* qkv_dev, const 
                                  uint32_t kv_heads, uint32_t head_dim, uint32_t max_seq, float* q_out_dev,
                                  float* k_cache_dev, float* v_cache_dev) {
     if (!ctx || !qkv_dev || !cos_dev || !sin_dev || !positions_dev || !q_out_dev || !k_cache_dev || !v_cache_dev ||
-        !q_heads || !kv_heads || q_heads % kv_heads || !head_dim || head_dim % 2u || head_dim > 1024u || !max_seq) {
+        !q_heads || !kv_heads || q_heads % kv_heads || !head_dim || head_dim % 2u || head_dim > kMaxRopeHead || !max_seq) {
         set_error("rope_append_kv: null argument or unsupported head geometry");
         return VXHIP_INVALID_ARGUMENT;
     }
@@ -1218,19 +1264,10 @@ VxHipStatus vxhip_gqa_attention(VxHipContext* ctx, const float* q_dev, const flo
     if (!rows || !t) return VXHIP_OK;
     if (!device_ready(ctx)) return VXHIP_BACKEND_UNAVAILABLE;
     const float scale = (float)(1.0 / sqrt((double)head_dim));
-    const uint32_t rep = q_heads / kv_heads;
-    const uint32_t together = heads_per_workgroup(rep, rows * t * q_heads, ctx->cu_count);
-    const size_t token_lds = (size_t)together * (9u * head_dim + max_seq) * sizeof(float);  // of the per-token kernel
-    auto prompt_lds = [&](uint32_t tokens) {  // of the prompt kernel that keeps its scores
-        const size_t qw = (size_t)tokens * rep;
-        return (qw * ((max_seq + 63u) & ~63u) + (size_t)kPrefillSlots * (head_dim + 4u)) * sizeof(float);
-    };
-    constexpr size_t kTokenLds = 60u * 1024u, kPromptLds = 150u * 1024u;
-    // A prompt at the common head sizes: the matrix-pipe kernel.  (It holds no scores and would take any cache; those
-    // that neither the prompt kernel with scores nor the per-token kernel could hold are refused as before it.)
-    if (t >= 8u && rep <= kPrefillQueries && (head_dim == 128u || head_dim == 64u) &&
-        (prompt_lds(1u) <= kPromptLds || token_lds <= kTokenLds)) {
-        const uint32_t tq = kPrefillQueries / rep, blocks = (t + tq - 1u) / tq, pairs = rows * kv_heads;
+    const GqaPlan plan = plan_gqa(ctx, rows, t, q_heads, kv_heads, head_dim, max_seq);
+    const uint32_t tq = plan.tokens;
+    if (plan.route == GqaRoute::PromptMfma) {
+        const uint32_t blocks = (t + tq - 1u) / tq, pairs = rows * kv_heads;
         const bool split = split_prompt_slots(pairs * blocks, t, ctx->cu_count);
         const uint32_t grid = pairs * (split ? blocks : (blocks + 3u) / 4u);
         const size_t lds = split ? 4u * (2u + head_dim / 2u) * 64u * sizeof(float) : 0u;
@@ -1253,37 +1290,25 @@ VxHipStatus vxhip_gqa_attention(VxHipContext* ctx, const float* q_dev, const flo
         VXHIP_TRY(hipGetLastError());
         return VXHIP_OK;
     }
-    if (t >= 8u && rep <= kPrefillQueries && head_dim <= 256u) {
-        // a prompt: tokens share the walk over the cache, as many per workgroup as the LDS holds
-        uint32_t tq = kPrefillQueries / rep;
-        while (tq > 1u && prompt_lds(tq) > kPromptLds) tq /= 2u;
-        // two workgroups per compute unit hide each other's staging, if four tokens or more still
-        // share a walk then
-        if (prompt_lds(tq) > 78u * 1024u) {
-            uint32_t fewer = tq;
-            while (fewer > 4u && prompt_lds(fewer) > 78u * 1024u) fewer /= 2u;
-            if (prompt_lds(fewer) <= 78u * 1024u) tq = fewer;
+    if (plan.route == GqaRoute::PromptScores) {
+        static std::atomic<uint64_t> configured{0};
+        if (!raise_lds_limit((const void*)gqa_prefill_kernel, 152 * 1024, configured)) {  // (plus its static 128 bytes)
+            set_error("gqa_attention: the prompt kernel's LDS limit could not be raised");
+            return VXHIP_EXECUTION_FAILED;
         }
-        if (prompt_lds(tq) <= kPromptLds) {
-            static std::atomic<uint64_t> configured{0};
-            if (!raise_lds_limit((const void*)gqa_prefill_kernel, 152 * 1024, configured)) {  // (plus its static 128 bytes)
-                set_error("gqa_attention: the prompt kernel's LDS limit could not be raised");
-                return VXHIP_EXECUTION_FAILED;
-            }
-            const dim3 grid(rows * ((t + tq - 1u) / tq), kv_heads);
-            hipLaunchKernelGGL(gqa_prefill_kernel, grid, dim3(256), prompt_lds(tq), ctx->stream, q_dev, k_cache_dev,
-                               v_cache_dev, positions_dev, t, tq, q_heads, kv_heads, head_dim, max_seq, scale, out_dev,
-                               ctx->fault_dev);
-            VXHIP_TRY(hipGetLastError());
-            return VXHIP_OK;
-        }
+        const dim3 grid(rows * ((t + tq - 1u) / tq), kv_heads);
+        hipLaunchKernelGGL(gqa_prefill_kernel, grid, dim3(256), plan.lds, ctx->stream, q_dev, k_cache_dev,
+                           v_cache_dev, positions_dev, t, tq, q_heads, kv_heads, head_dim, max_seq, scale, out_dev,
+                           ctx->fault_dev);
+        VXHIP_TRY(hipGetLastError());
+        return VXHIP_OK;
     }
-    if (token_lds > kTokenLds) {
+    if (plan.route == GqaRoute::None) {
         set_error("gqa_attention: head_dim/max_seq too large for the score buffer");
         return VXHIP_INVALID_ARGUMENT;
     }
-    const dim3 grid(rows * t, q_heads / together);
-    launch_attention<false>(ctx, together, grid, token_lds, q_dev, const_cast<float*>(k_cache_dev),
+    const dim3 grid(rows * t, q_heads / plan.together);
+    launch_attention<false>(ctx, plan.together, grid, plan.lds, q_dev, const_cast<float*>(k_cache_dev),
                             const_cast<float*>(v_cache_dev), positions_dev, t, q_heads, kv_heads, head_dim, max_seq,
                             scale, out_dev, nullptr, nullptr);
     VXHIP_TRY(hipGetLastError());

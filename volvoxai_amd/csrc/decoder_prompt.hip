@@ -70,18 +70,29 @@ Workspace carve(const VxHipContext* ctx, const VxHipDecoderPrompt* p, char* base
     return w;
 }
 
+// Tokens a row that go through the last layer's attention: the last eight, the fewest that run on the prompt kernels, which take caches
+// that the per-token form does not (its limit is 60 KiB of scores, theirs 150).  The rows do not depend on each other: the same bits.
+uint32_t tokens_seen_last(uint32_t t) { return t >= 8u ? 8u : 1u; }
+
+// Everything that a step could refuse, so that no launch of a prompt runs where another will not.
 bool admitted(const VxHipContext* ctx, const VxHipDecoderPrompt* p) {
     if (!ctx || !p || !p->tokens_dev || !p->embedding_dev || !p->layers || !p->layer_count || !p->final_gain_dev || !p->lm_head ||
         !p->cos_dev || !p->sin_dev || !p->positions_dev || !p->rows || p->t < 2u || !p->hidden || !p->q_heads || !p->kv_heads ||
         p->q_heads % p->kv_heads || !p->head_dim || !p->max_seq || p->t > p->max_seq ||
-        (uint64_t)p->rows * p->t > 0xffffffffull || p->lm_head->w.k != p->hidden)
+        (uint64_t)p->rows * p->t > 0xffffffffull || p->lm_head->w.k != p->hidden || !p->vocab || p->hidden > kMaxRowOpLength ||
+        p->head_dim > kMaxRopeHead ||
+        (p->layer_count > 1u && !gqa_takes(ctx, p->rows, p->t, p->q_heads, p->kv_heads, p->head_dim, p->max_seq)) ||
+        !gqa_takes(ctx, p->rows, tokens_seen_last(p->t), p->q_heads, p->kv_heads, p->head_dim, p->max_seq) ||
+        p->lm_head->device != ctx->device)
         return false;
     const uint64_t q_dim = (uint64_t)p->q_heads * p->head_dim, qkv = q_dim + 2ull * p->kv_heads * p->head_dim;
     for (uint32_t i = 0; i < p->layer_count; i++) {
         const VxHipDecoderLayer& L = p->layers[i];
         if (!L.gain1_dev || !L.gain2_dev || !L.qkv || !L.output || !L.gate_up || !L.down || !L.k_cache_dev || !L.v_cache_dev ||
             L.qkv->w.k != p->hidden || L.qkv->w.n != qkv || L.output->w.k != q_dim || L.output->w.n != p->hidden ||
-            L.gate_up->w.k != p->hidden || L.gate_up->w.n % 2u || L.down->w.k != L.gate_up->w.n / 2u || L.down->w.n != p->hidden)
+            L.gate_up->w.k != p->hidden || L.gate_up->w.n % 2u || L.down->w.k != L.gate_up->w.n / 2u || L.down->w.n != p->hidden ||
+            L.down->w.k > kMaxRowOpLength || L.qkv->device != ctx->device || L.output->device != ctx->device ||
+            L.gate_up->device != ctx->device || L.down->device != ctx->device)
             return false;
     }
     return true;
@@ -97,7 +108,7 @@ size_t vxhip_decoder_prompt_workspace(const VxHipContext* ctx, const VxHipDecode
 
 VxHipStatus vxhip_decoder_prompt(VxHipContext* ctx, const VxHipDecoderPrompt* p) {
     if (!admitted(ctx, p) || !p->workspace_dev || (uintptr_t)p->workspace_dev % 256u || !p->logits_dev || !p->next_dev) {
-        set_error("decoder_prompt: a null argument, or extents that do not fit each other");
+        set_error("decoder_prompt: a null argument, extents that do not fit each other or that a step does not take, or a linear of another device");
         return VXHIP_INVALID_ARGUMENT;
     }
     const Workspace w = carve(ctx, p, (char*)p->workspace_dev);
@@ -134,11 +145,9 @@ VxHipStatus vxhip_decoder_prompt(VxHipContext* ctx, const VxHipDecoderPrompt* p)
                                         p->head_dim, p->max_seq, w.q, L.k_cache_dev, L.v_cache_dev));
         const float *q = w.q, *attention = w.attention;
         uint32_t seen = t;
-        // Behind the cache append of the last layer only each row's last token goes on to the logits.  The attention takes
-        // the last eight, the fewest that run on the prompt kernels: a single one would go to the decode kernel, which refuses caches
-        // that a prompt may have (its score buffer holds 60 KiB, theirs 150).  The rows do not depend on each other: the same bits.
+        // Behind the cache append of the last layer only each row's last token goes on to the logits.
         if (last) {
-            seen = t >= 8u ? 8u : 1u;
+            seen = tokens_seen_last(t);
             if (seen != t) {
                 if (!last_tokens(ctx->stream, w.q, rows, t, seen, q_dim, w.last_q)) return VXHIP_INTERNAL;
                 q = w.last_q;
