@@ -86,3 +86,35 @@ def test_argument_validation_happens_before_any_device_work():
     words = np.zeros((2, 8), np.uint32)
     assert lib.vxhip_packed_linear_create(p(words), p(s), None, 32, 2, 32, 4, C.byref(h)) == -7
     assert lib.vxhip_packed_linear_create(p(words), p(s), None, 32, 2, 48, 8, C.byref(h)) == -1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 3, 8, 17, 32, 33, 64])
+def test_routes_lie_in_the_row_domains_of_the_table(ctx, rows):
+    """The ids that calls report, against the rows their records declare: few rows on the split and the slab kernels too."""
+    import torch
+    table = {r["id"]: r["predicate_id"] for r in vx.kernel_variants()}
+    rng = np.random.default_rng(rows)
+    n = 512
+
+    def admitted():
+        family = max((i for i in table if ctx.last_variant.startswith(i + ".")), key=len)
+        least, most = re.search(r"rows-g[te](\d+)", table[family]), re.search(r"rows-le(\d+)", table[family])
+        if least and rows < int(least.group(1)) + ("rows-gt" in table[family]):
+            return False
+        return not (most and rows > int(most.group(1)))
+
+    for k in (2500, 4608):
+        scales = rng.uniform(0.002, 0.01, (n, (k + 127) // 128)).astype(np.float32)
+        q = vx.QLinear(rng.integers(-127, 128, (n, k)).astype(np.int8), scales[:, 0].copy(), np.zeros(n, np.int32), np.zeros(n, np.int32), vx.DTYPE_I8)
+        words = np.full((n, (k + 3) // 4), 0x81818181, np.uint32)
+        p = vx.PackedLinear(words, scales, None, k, n, 128)
+        x = torch.ones((rows, k), device="cuda")
+        try:
+            ok, _ = q.forward(ctx, x.to(torch.int8), 0.02, 0, 1.0, 0, input_dtype=vx.DTYPE_I8)
+            assert ok == 1 and admitted(), ctx.last_variant
+            st, _ = p.forward_f32(ctx, x)
+            assert st == 0 and admitted(), ctx.last_variant
+        finally:
+            ctx.synchronize()
+            q.close(), p.close()
