@@ -1,5 +1,5 @@
-"""Decode attention at head sizes 64 (one walk over keys and values: eight wavefronts take 16 slots each of every 128, two
-blocks ahead) and 128 (the kernel that keeps its scores in LDS)."""
+"""Decode attention at head sizes 64 and 128: one walk over keys and values, blocks of 256 slots, eight wavefronts that take eight
+slots of every 64 each, and four query heads a workgroup by way of scores in LDS at head size 128."""
 import numpy as np
 import pytest
 

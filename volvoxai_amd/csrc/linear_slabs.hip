@@ -249,7 +249,7 @@ bool launch_bits(hipStream_t s, const LinearArgs& a) {
 // Which calls (f32 rows, so that the preparation can write operand order), and which tile.  A tile's time is about constant
 // while there are no more of them than compute units and grows by 0.6 of that for each further one a compute unit gets; a 16x32
 // tile (channels x rows) costs 1.38 of a 16x16 one and a 32x32 tile 1.95 (groups of 32, whose products are four times as
-// many: 1.25 and 2.2).  us, preparation included, with the kernels that took the call before | 16x16 | 16x32 | 32x32:
+// many: 1.25 and 2.2, which the rule never takes: by name only).  us, preparation included, with the kernels that took the call before | 16x16 | 16x32 | 32x32:
 //   8 bits, groups of 128    32 x 2048 -> 1024   6.3 |  5.5 |  6.0 |  6.9    32 x 4096 -> 4096    9.4 |  9.4 |  8.7 | 10.2
 //                            64 x 3000 -> 1531  10.6 |  8.2 |  7.6 |  8.8    64 x 4096 -> 4096   12.3 | 12.8 | 11.3 | 10.5
 //                            32 x 14336 -> 4096 35.4 | 25.5 | 22.6 | 26.4    64 x 14336 -> 4096  32.2 | 37.7 | 31.4 | 27.0

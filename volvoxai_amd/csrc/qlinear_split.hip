@@ -146,7 +146,8 @@ bool launch(hipStream_t s, const LinearArgs& a) {
 // 256 with per-row scales 4.03 -> 4.33; not 52 x 256 -> 3840 6.5 -> 5.8, nor unsigned bytes, which those tiles want flipped first: 124 x 256 ->
 // 512 5.8 -> 3.7).
 // From 17 rows on also in place of the streaming kernel: 32 x 2048 -> 2048 6.2 -> 4.6, 32 x 4096 -> 512 7.7 -> 5.4 (16 rows 6.2); 32 x
-// 1024 -> 1024 3.9 -> 4.2 and 24 x 1536 -> 1536 4.5 are left there.  105 calls of 17 to 500 rows, bytes, per-row scales and f32 rows: 0.79 of their
+// 1024 -> 1024 3.9 -> 4.2 and 24 x 1536 -> 1536 4.5 are left there.  (17 to 23 rows of K below 2900 and few channels take it 4.2 or 5.3, by where
+// their operands lie, and these tiles 4.6: 18 x 2064 -> 1120, 23 x 2656 -> 448.)  105 calls of 17 to 500 rows, bytes, per-row scales and f32 rows: 0.79 of their
 // time before (geometric mean of graph replays).
 const char* launch_requant_split(hipStream_t s, const LinearArgs& a, int cu_count, const char* force) {
     if (a.mode == Epilogue::DequantF32 || a.weight_bits != 8u || a.x_f32 || a.x_operand_order || a.ldx < 16u || a.ldx % 16u ||
