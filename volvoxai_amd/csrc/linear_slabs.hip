@@ -285,6 +285,16 @@ SlabTile pick_slab_tile(const LinearArgs& a, int cu_count, const char* force) {
     if (a.rows <= kMaxPrepRows || a.rows > 256u) return SlabTile::None;
     const uint32_t panels = (a.n + 31u) / 32u, cu = cu_count > 0 ? (uint32_t)cu_count : 256u, columns = a.ksteps * (four ? 64u : 32u);
     if (a.k < (a.rows <= 4u ? 4097u : a.rows <= 8u ? 2049u : 1280u)) return SlabTile::None;
+    const auto cost = [&](uint32_t tile_n, uint32_t tile_m, float one) {
+        const float per = (float)((uint64_t)((a.n + tile_n - 1u) / tile_n) * ((a.rows + tile_m - 1u) / tile_m)) / (float)cu;
+        return one * (per > 1.0f ? 1.0f + 0.6f * (per - 1.0f) : 1.0f);
+    };
+    const bool fine = a.group_size == 32u;
+    const float c0 = cost(16u, 16u, 1.0f), c1 = cost(16u, 32u, fine ? 1.25f : 1.38f), c2 = cost(32u, 32u, fine ? 2.2f : 1.95f);
+    const float least = c0 <= c1 && c0 <= c2 ? c0 : c1 <= c2 ? c1 : c2;
+    const SlabTile cheapest = least == c0 ? SlabTile::T16x16 : least == c1 ? SlabTile::T16x32 : SlabTile::T32x32;
+    // (nothing below declines these, and asking takes the host a tenth of a microsecond)
+    if (a.rows > 8u && a.rows <= 32u && a.k >= 2048u && panels * 2u <= cu && least <= 1.6f) return cheapest;
     const Streams behind = a.rows <= 32u ? streaming_kernel(a, cu_count) : Streams::None;
     if (a.rows <= 8u && behind == Streams::RowsInLds) return SlabTile::None;
     if (behind == Streams::General && panels * 2u > cu && (panels <= cu || a.groups * (a.rows + 1u) * 128u <= 80u * 1024u) &&
@@ -294,20 +304,12 @@ SlabTile pick_slab_tile(const LinearArgs& a, int cu_count, const char* force) {
     if (fits && a.k < 2048u) return SlabTile::None;
     // (whole panels: the products of all groups leave a compute unit room for two workgroups, or are at least few)
     if (fits && panels * 4u >= cu * 3u && (a.group_size >= 128u || a.groups * a.rows * 128u <= 80u * 1024u)) return SlabTile::None;
-    const auto cost = [&](uint32_t tile_n, uint32_t tile_m, float one) {
-        const float per = (float)((uint64_t)((a.n + tile_n - 1u) / tile_n) * ((a.rows + tile_m - 1u) / tile_m)) / (float)cu;
-        return one * (per > 1.0f ? 1.0f + 0.6f * (per - 1.0f) : 1.0f);
-    };
-    const bool fine = a.group_size == 32u;
-    const float c0 = cost(16u, 16u, 1.0f), c1 = cost(16u, 32u, fine ? 1.25f : 1.38f), c2 = cost(32u, 32u, fine ? 2.2f : 1.95f);
-    const float least = c0 <= c1 && c0 <= c2 ? c0 : c1 <= c2 ? c1 : c2;
     const bool slow_stream = a.rows <= 8u ? behind == Streams::RowsInMemory : a.rows <= 32u && !(fits && a.group_size >= 128u);
     const float line = slow_stream                          ? 2.7f
                        : a.rows > 32u && a.k < 2048u        ? 1.5f
                        : a.group_size == 256u && a.k < 4096u ? 1.6f
                                                             : 2.0f;
-    if (least > line) return SlabTile::None;
-    return least == c0 ? SlabTile::T16x16 : least == c1 ? SlabTile::T16x32 : SlabTile::T32x32;
+    return least > line ? SlabTile::None : cheapest;
 }
 
 // a.x: operand order in tiles of 32 rows, ldx = the columns rounded up to 16.
